@@ -189,9 +189,10 @@ struct dsm_engine {
   PinnedBuf<ApplyCtl> h_actl;
   // DFS
   DevBuf<DfsCtl> ctl;
-  PinnedBuf<DfsCtl> h_ctl;
-  DevBuf<Task> queue;
-  uint32_t qcap = 0, epoch = 0;
+  DevBuf<Mailbox> mail;          // one per wave of the largest grid
+  DevBuf<IdleWord> idle;         // their waiting states
+  PinnedBuf<BlockRec> h_rec;     // what each block of the last DFS launch did
+  uint32_t epoch = 0;            // of the last DFS launch
   DevBuf<uint32_t> seed_plan, seed_s, seed_d, seed_tag;
   uint32_t seed_cap = 0;
   DevBuf<unsigned long long> counts;
@@ -201,7 +202,7 @@ struct dsm_engine {
   bool tuples_host = false;
   unsigned long long tuple_cap = 0;
   uint32_t dfs_blocks = 0, dfs_wpb = 4, max_qn = 2;
-  uint32_t donate_min = 256, lane_work = 16, donate_every = 8, donate_min_n2 = 64, leaf_budget = 2048;
+  uint32_t donate_min = 256, lane_work = 16, donate_every = 4, donate_min_n2 = 64, leaf_budget = 2048;
   bool leaf_sets = true;
   bool bit_probe_last = false;
   bool graph_rounds = true;
@@ -231,11 +232,9 @@ struct dsm_engine {
   std::vector<uint32_t> last_touched, last_relabel;
   DevBuf<uint32_t> d_last_touched, d_last_relabel, sync_q, sync_ctl;
   int cu_lds = 160 * 1024;   // LDS bytes per CU
-  // per-wave task time of the last DFS launch (balance statistics)
-  DevBuf<unsigned long long> wave_busy;
-  PinnedBuf<unsigned long long> h_wave_busy;
   DevBuf<unsigned long long> query_busy;  // per query: DFS task ticks since the last read
-  uint32_t wave_slots = 0, last_blocks = 0, last_wpb = 0;
+  uint32_t wave_slots = 0;       // waves of the largest grid
+  uint32_t last_blocks = 0, last_wpb = 0;  // grid of the last DFS launch
   // the DFS round as a HIP graph (graph_round)
   hipGraph_t rg_graph = nullptr;
   hipGraphExec_t rg_exec = nullptr;
@@ -750,10 +749,6 @@ int upload_tables(dsm_engine *e) {
   HIPCHK(hipMemset(e->query_busy.p, 0, (size_t)nq * 8));
   HIPCHK(e->h_counts.ensure((size_t)nq * 2 * kMaxSlots));
   HIPCHK(e->ctl.alloc(1));
-  HIPCHK(e->h_ctl.ensure(1));
-  e->qcap = e->opt.queue_capacity ? e->opt.queue_capacity : (1u << 20);
-  HIPCHK(e->queue.alloc(e->qcap));
-  HIPCHK(hipMemset(e->queue.p, 0, (size_t)e->qcap * sizeof(Task)));  // ready = 0: no epoch
   HIPCHK(e->tuple_count.alloc(1));
   if (e->opt.tuple_capacity) {
     e->tuple_cap = e->opt.tuple_capacity;
@@ -827,8 +822,9 @@ DfsArgs dfs_args(dsm_engine *e) {
   da.seed_s = e->seed_s.p;
   da.seed_d = e->seed_d.p;
   da.seed_tag = e->seed_tag.p;
-  da.queue = e->queue.p;
-  da.qcap = e->qcap;
+  da.mail = e->mail.p;
+  da.idle = e->idle.p;
+  da.donate_cap = 0xFFFFFFFFu;
   da.epoch = ++e->epoch;
   da.donate_min = e->donate_min;
   da.lane_work = e->lane_work;
@@ -848,9 +844,8 @@ DfsArgs dfs_args(dsm_engine *e) {
   da.tuples = e->tuples;
   da.tuple_cap = e->tuple_cap;
   da.tuple_count = e->tuple_count.p;
-  da.wave_busy = e->wave_busy.p;
+  da.rec = e->h_rec.p;
   da.query_busy = e->query_busy.p;
-  da.wave_slots = e->wave_slots;
   return da;
 }
 
@@ -859,11 +854,15 @@ DfsArgs dfs_args(dsm_engine *e) {
 uint32_t dfs_grid(dsm_engine *e, uint32_t nrec) {
   const uint64_t want =
       ((uint64_t)nrec * std::max<uint32_t>(e->max_plans_per_key, 1) * 8 + e->dfs_wpb - 1) / e->dfs_wpb;
-  const uint32_t b = (uint32_t)std::min<uint64_t>(e->dfs_blocks, std::max<uint64_t>(want, (uint64_t)e->num_cu));
-  e->last_blocks = b;
+  uint32_t b = (uint32_t)std::min<uint64_t>(e->dfs_blocks, std::max<uint64_t>(want, (uint64_t)e->num_cu));
   e->last_wpb = e->tuples ? 4u : e->dfs_wpb;
+  b = std::min(b, e->wave_slots / e->last_wpb);  // a mailbox for every wave
+  e->last_blocks = b;
   return b;
 }
+
+// The waiting words of a grid.
+uint32_t idle_words(uint32_t waves) { return (waves + kIdleGroup - 1) / kIdleGroup; }
 
 void drop_round_graph(dsm_engine *e) {
   if (e->rg_exec) (void)hipGraphExecDestroy(e->rg_exec);
@@ -872,8 +871,14 @@ void drop_round_graph(dsm_engine *e) {
   e->rg_graph = nullptr;
 }
 
-// The round as one HIP graph: ctl reset -> seed list 0 -> seed list 1 -> DFS ->
-// control block to the host. Built once per launch shape (waves per block,
+// queue_capacity bounds the tasks a round hands to waiting waves: an equal share
+// for every wave of the grid.
+void cap_donations(dsm_engine *e, DfsArgs &da) {
+  if (e->opt.queue_capacity) da.donate_cap = e->opt.queue_capacity / (e->last_blocks * e->last_wpb);
+}
+
+// The round as one HIP graph: ctl reset -> seed list 0 -> seed list 1 -> DFS,
+// whose blocks write their records to pinned host memory. Built once per launch shape (waves per block,
 // tuples or not); every later round updates the kernel nodes' arguments and
 // grids in the executable graph and launches it.
 int graph_round(dsm_engine *e, const RoundPart *parts, int nparts, uint32_t nrec) {
@@ -884,7 +889,11 @@ int graph_round(dsm_engine *e, const RoundPart *parts, int nparts, uint32_t nrec
   st.seed[1] = seed_args(e, nparts > 1 ? parts[1] : none);
   st.dfs = dfs_args(e);
   hipKernelNodeParams pr, p0, p1, pd;
-  round_node_params(st, dfs_grid(e, nrec), e->dfs_wpb, e->max_qn, &pr, &p0, &p1, &pd);
+  const uint32_t blocks = dfs_grid(e, nrec);
+  cap_donations(e, st.dfs);
+  st.idle = e->idle.p;
+  st.nidle = idle_words(e->wave_slots);
+  round_node_params(st, blocks, e->dfs_wpb, e->max_qn, &pr, &p0, &p1, &pd);
   const uint32_t key = (e->tuples ? 16u : 0u) | e->dfs_wpb;
   if (!e->rg_exec || e->rg_key != key) {
     drop_round_graph(e);
@@ -893,11 +902,6 @@ int graph_round(dsm_engine *e, const RoundPart *parts, int nparts, uint32_t nrec
     HIPCHK(hipGraphAddKernelNode(&e->rg_seed0, e->rg_graph, &e->rg_reset, 1, &p0));
     HIPCHK(hipGraphAddKernelNode(&e->rg_seed1, e->rg_graph, &e->rg_seed0, 1, &p1));
     HIPCHK(hipGraphAddKernelNode(&e->rg_dfs, e->rg_graph, &e->rg_seed1, 1, &pd));
-    hipGraphNode_t cp, cw;
-    HIPCHK(hipGraphAddMemcpyNode1D(&cp, e->rg_graph, &e->rg_dfs, 1, e->h_ctl.p, e->ctl.p, sizeof(DfsCtl),
-                                   hipMemcpyDeviceToHost));
-    HIPCHK(hipGraphAddMemcpyNode1D(&cw, e->rg_graph, &cp, 1, e->h_wave_busy.p, e->wave_busy.p,
-                                   (size_t)e->wave_slots * 24, hipMemcpyDeviceToHost));
     HIPCHK(hipGraphInstantiate(&e->rg_exec, e->rg_graph, nullptr, nullptr, 0));
     e->rg_key = key;
   } else {
@@ -922,14 +926,14 @@ int dfs_round(dsm_engine *e, const RoundPart *parts, int nparts, hipEvent_t ev0,
     int rc = graph_round(e, parts, nparts, nrec);
     if (rc) return rc;
   } else {
-    HIPCHK(launch_ctl_reset(e->ctl.p, nullptr, nullptr, nullptr, 0, e->stream));
+    HIPCHK(launch_ctl_reset(e->ctl.p, nullptr, nullptr, nullptr, 0, e->idle.p, idle_words(e->wave_slots), e->stream));
     for (int i = 0; i < nparts; i++)
       if (parts[i].n) HIPCHK(launch_seed(seed_args(e, parts[i]), e->stream));
     if (ev1) HIPCHK(hipEventRecord(ev1, e->stream));
-    HIPCHK(launch_dfs(dfs_args(e), dfs_grid(e, nrec), e->dfs_wpb, e->max_qn, e->stream));
-    HIPCHK(hipMemcpyAsync(e->h_ctl.p, e->ctl.p, sizeof(DfsCtl), hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipMemcpyAsync(e->h_wave_busy.p, e->wave_busy.p, (size_t)e->wave_slots * 24, hipMemcpyDeviceToHost,
-                          e->stream));
+    DfsArgs da = dfs_args(e);
+    const uint32_t blocks = dfs_grid(e, nrec);
+    cap_donations(e, da);
+    HIPCHK(launch_dfs(da, blocks, e->dfs_wpb, e->max_qn, e->stream));
   }
   if (ev2) HIPCHK(hipEventRecord(ev2, e->stream));
   return DSM_OK;
@@ -941,58 +945,48 @@ int run_round(dsm_engine *e, const uint32_t *rs, const uint32_t *rd, uint32_t nr
   return dfs_round(e, &p, 1, ev0, ev1, ev2);
 }
 
+// The last round's errors: the records of its blocks, which have ended.
+int round_error(dsm_engine *e) {
+  for (uint32_t b = 0; b < e->last_blocks; b++) {
+    const BlockRec &r = e->h_rec.p[b];
+    if (r.epoch != e->epoch) return e->fail_msg(DSM_EDEVICE, "DFS: block %u of %u left no record", b, e->last_blocks);
+    if (r.seed_overflow)
+      return e->fail_msg(DSM_ELIMIT, "seed table overflow (%llu seeds dropped)", r.seed_overflow);
+    if (r.abort) return e->fail_msg(DSM_EDEVICE, "DFS watchdog: a wave waited more than %u ms for work", e->watchdog_ms);
+  }
+  return DSM_OK;
+}
+
+// The last round's errors, and its work and balance into the statistics.
 int check_round(dsm_engine *e, uint64_t *seeds) {
-  const DfsCtl &c = *e->h_ctl.p;
-  if (c.seed_overflow.v)
-    return e->fail_msg(DSM_ELIMIT, "seed table overflow (%u seeds dropped)", c.seed_overflow.v);
-  if (c.abort.v)
-    return e->fail_msg(DSM_EDEVICE, "DFS watchdog: a wave waited more than %u ms for work (%d tasks left)",
-                       e->watchdog_ms, c.work_left.v);
-  *seeds = c.nseeds.v;
-  e->stats.tasks_donated += std::min(c.q_tail.v, e->qcap);
-  e->stats.dfs_entries += c.scanned.v;
-  e->stats.dfs_search_loads += c.loads.v;
-  e->stats.dfs_merge_bytes += c.mbytes.v;
-  // balance: per-block task time of the launch
-  {
-    const uint32_t nb = e->last_blocks, wpb = e->last_wpb;
-    if (nb && (uint64_t)nb * wpb <= e->wave_slots) {
-      double tot = 0, mx = 0;
-      for (uint32_t b = 0; b < nb; b++) {
-        double s = 0;
-        for (uint32_t w = 0; w < wpb; w++) s += (double)e->h_wave_busy.p[(size_t)b * wpb + w];
-        tot += s;
-        mx = std::max(mx, s);
-      }
-      const double to_ms = 1.0 / (double)e->wall_khz;
-      e->stats.dfs_busy_ms += tot * to_ms;
-      e->stats.dfs_waves += (uint64_t)nb * wpb;
-      if (tot > 0) e->stats.dfs_block_imbalance += mx / (tot / nb);
-      // head and tail idle: a wave without tasks counts as idle in the tail
-      const unsigned long long *first = e->h_wave_busy.p + e->wave_slots;
-      const unsigned long long *last = first + e->wave_slots;
-      const uint32_t nw = nb * wpb;
-      unsigned long long t0 = ~0ull, t1 = 0;
-      for (uint32_t w = 0; w < nw; w++)
-        if (first[w]) {
-          t0 = std::min(t0, first[w]);
-          t1 = std::max(t1, last[w]);
-        }
-      if (t1 > t0) {
-        const double span = (double)(t1 - t0);
-        double head = 0, tail = 0;
-        for (uint32_t w = 0; w < nw; w++) {
-          if (!first[w]) {
-            tail += span;
-            continue;
-          }
-          head += (double)(first[w] - t0);
-          tail += (double)(t1 - last[w]);
-        }
-        e->stats.dfs_head_idle += head / (span * nw);
-        e->stats.dfs_tail_idle += tail / (span * nw);
-      }
-    }
+  if (int rc = round_error(e)) return rc;
+  const uint32_t nb = e->last_blocks, nw = nb * e->last_wpb;
+  *seeds = nb ? e->h_rec.p[0].nseeds : 0;
+  unsigned long long busy = 0, busiest = 0, active = 0, t0 = ~0ull, t1 = 0;
+  double first = 0, last = 0;  // summed over the active waves
+  for (uint32_t b = 0; b < nb; b++) {
+    const BlockRec &r = e->h_rec.p[b];
+    e->stats.tasks_donated += r.donated;
+    e->stats.dfs_entries += r.scanned;
+    e->stats.dfs_search_loads += r.loads;
+    e->stats.dfs_merge_bytes += r.mbytes;
+    busy += r.busy;
+    busiest = std::max(busiest, r.busy);
+    if (!r.active) continue;
+    active += r.active;
+    t0 = std::min(t0, r.first_min);
+    t1 = std::max(t1, r.last_max);
+    first += (double)r.first_sum;
+    last += (double)r.last_sum;
+  }
+  e->stats.dfs_busy_ms += (double)busy / (double)e->wall_khz;
+  e->stats.dfs_waves += nw;
+  if (busy) e->stats.dfs_block_imbalance += (double)busiest / ((double)busy / nb);
+  // head and tail idle: a wave without tasks counts as idle in the tail
+  if (t1 > t0) {
+    const double span = (double)(t1 - t0), na = (double)active;
+    e->stats.dfs_head_idle += (first - na * (double)t0) / (span * nw);
+    e->stats.dfs_tail_idle += (na * (double)t1 - last + span * (nw - na)) / (span * nw);
   }
   e->stats.dfs_launches += 1;
   return DSM_OK;
@@ -1303,7 +1297,7 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const SortedSync 
   int rc;
   e->shadow_delta_ok = false;
   e->grew = false;
-  HIPCHK(launch_ctl_reset(nullptr, e->actl.p, nullptr, nullptr, 0, e->stream));
+  HIPCHK(launch_ctl_reset(nullptr, e->actl.p, nullptr, nullptr, 0, nullptr, 0, e->stream));
   if ((rc = do_apply_delta(e, d))) return rc;
   // the catch-up's deferred label-sorted copies: this update's dirty bits are
   // all set and the dirty list still holds the last update's vertices. After
@@ -1390,14 +1384,15 @@ int create_impl(dsm_engine *e, const dsm_graph_desc *graph, const dsm_query_desc
     uint32_t most = 0;
     for (uint32_t w : {1u, 2u, 4u, 8u}) most = std::max<uint32_t>(most, (uint32_t)dfs_max_blocks_per_cu(w, e->max_qn) * w);
     e->wave_slots = most * (uint32_t)e->num_cu;
-    // per wave: task time, first task start, last task end
-    HIPCHK(e->wave_busy.alloc(3 * (size_t)e->wave_slots));
-    HIPCHK(e->h_wave_busy.ensure(3 * (size_t)e->wave_slots));
+    HIPCHK(e->mail.alloc(e->wave_slots));
+    HIPCHK(hipMemset(e->mail.p, 0, (size_t)e->wave_slots * sizeof(Mailbox)));  // stop = 0: no epoch
+    HIPCHK(e->idle.alloc(idle_words(e->wave_slots)));
+    HIPCHK(e->h_rec.ensure(e->wave_slots));
   }
   e->donate_min = e->opt.donate_min ? e->opt.donate_min : 256;
   e->lane_work = e->opt.lane_work ? e->opt.lane_work : 16;
   e->leaf_budget = e->opt.leaf_budget ? e->opt.leaf_budget : 2048;
-  e->donate_every = e->opt.donate_every ? e->opt.donate_every : 8;
+  e->donate_every = e->opt.donate_every ? e->opt.donate_every : 4;
   e->donate_min_n2 = e->opt.donate_min_n2 ? e->opt.donate_min_n2 : 64;
   e->leaf_sets = e->opt.leaf_sets != 0;
   e->bit_probe_last = e->opt.bit_probe_last != 0;
@@ -1667,7 +1662,7 @@ int dsm_apply_batch(dsm_engine *e, const dsm_change *changes, uint32_t k) {
     }
   }
   const uint32_t nq = (uint32_t)e->queries.size();
-  HIPCHK(launch_ctl_reset(nullptr, nullptr, e->tuple_count.p, e->counts.p, nq * 2, e->stream));
+  HIPCHK(launch_ctl_reset(nullptr, nullptr, e->tuple_count.p, e->counts.p, nq * 2, nullptr, 0, e->stream));
   int rc;
   bool applied = false;
   // 1. negatives in the pre-batch graph; with overlap_apply the batch is
@@ -1920,7 +1915,7 @@ int dsm_autotune(dsm_engine *e, const dsm_change *sample, uint32_t k, dsm_tune_r
     e->donate_every = c.dev;
     e->bit_probe_last = c.pl;
     if (loaded) HIPCHK(hipEventRecord(e->ev_pre, e->stream));
-    HIPCHK(launch_ctl_reset(nullptr, nullptr, e->tuple_count.p, e->counts.p, nq * 2, e->stream));
+    HIPCHK(launch_ctl_reset(nullptr, nullptr, e->tuple_count.p, e->counts.p, nq * 2, nullptr, 0, e->stream));
     int rc2 = run_round(e, rb.p, rb.p + k, k, 0, e->ev[9], e->ev[10], e->ev[11]);
     if (rc2) return rc2;
     if (loaded && (rc2 = overlap_apply(e, load, true, false))) return rc2;
@@ -2247,7 +2242,7 @@ int pipe_round(dsm_engine *e, PinnedBuf<uint32_t> &h_rec, DevBuf<uint32_t> &d_re
   if (applied) *applied = false;
   if (overlap) HIPCHK(hipEventRecord(e->ev_pre, e->stream));
   if (R) HIPCHK(launch_ctl_reset(nullptr, nullptr, nullptr, e->counts.p + (size_t)R->slot * nq * 2, nq * 2,
-                                 e->stream));
+                                 nullptr, 0, e->stream));
   if (np + nn) {
     if ((rc = ensure_seed_cap(e, np + nn))) return rc;
     HIPCHK(h_rec.ensure(2 * (size_t)(np + nn) + 2));
@@ -2280,10 +2275,7 @@ int pipe_round(dsm_engine *e, PinnedBuf<uint32_t> &h_rec, DevBuf<uint32_t> &d_re
   }
   HIPCHK(hipStreamSynchronize(e->stream));
   if (np + nn) {
-    const DfsCtl &c = *e->h_ctl.p;
-    if (c.seed_overflow.v) return e->fail_msg(DSM_ELIMIT, "seed table overflow in a pipelined round");
-    if (c.abort.v)
-      return e->fail_msg(DSM_EDEVICE, "DFS watchdog: a wave waited more than %u ms for work", e->watchdog_ms);
+    if (!stats && (rc = round_error(e))) return rc;
     if (stats) {
       uint64_t seeds = 0;
       if ((rc = check_round(e, &seeds))) return rc;

@@ -47,18 +47,22 @@ struct alignas(8) SigReq {
 };
 
 // A unit of DFS work: levels [0, level) are fixed in f; level `level` scans
-// source-list indices [lo, hi). One 128-byte queue slot each; `ready` holds
-// the launch epoch once the slot is published.
-struct alignas(128) Task {
+// source-list indices [lo, hi). Every wave of the grid has a mailbox of its own
+// (a 128-byte line): a busy wave that has claimed it while its owner waits
+// (IdleWord) writes a task there and adds one to `mail`; `stop` takes the
+// launch's epoch once no wave of the grid has work left.
+struct alignas(128) Mailbox {
   uint32_t plan;
   uint32_t level;
   uint32_t lo, hi;
   uint32_t f[kMaxQ];
   uint32_t tag;          // count slot << 1 | sign (1 positive, 0 negative)
-  uint32_t ready;
-  uint32_t pad[10];
+  uint32_t pad0;
+  uint32_t mail;         // tasks delivered so far (never reset); read with stop as one 8-byte word
+  uint32_t stop;
+  uint32_t pad[8];
 };
-static_assert(sizeof(Task) == 128, "task slot layout");
+static_assert(sizeof(Mailbox) == 128, "mailbox layout");
 constexpr int kTaskWords = 5 + kMaxQ;  // payload words (21)
 constexpr uint32_t kMaxSlots = 64;     // count slots: requests served in one step
 
@@ -72,16 +76,33 @@ struct alignas(128) CtlLine {
 };
 struct DfsCtl {
   CtlLine<uint32_t> nseeds;        // seeds written by the seed kernel
-  CtlLine<uint32_t> seed_head;     // next seed to claim
-  CtlLine<uint32_t> q_head;        // queue tickets taken by waves out of work
-  CtlLine<uint32_t> q_tail;        // queue slots reserved by donors (= tasks donated)
-  CtlLine<int32_t> work_left;      // seeds + donated tasks not yet finished
+  CtlLine<uint32_t> seed_head;     // seed parts claimed beyond every wave's first
   CtlLine<uint32_t> seed_overflow; // seeds dropped for lack of capacity (must stay 0)
   CtlLine<uint32_t> abort;         // set when an idle wave outlived the watchdog
-  CtlLine<unsigned long long> scanned;  // source-list entries tested
-  CtlLine<unsigned long long> loads;    // 4-byte reads of membership searches
-  CtlLine<unsigned long long> mbytes;   // 4 B x degree of every backward list of every expanded partial match
 };
+// The waiting state of 16 waves of the grid (wave w is in word w mod ngroups),
+// a line each: bits 0..15 waiting for work, bits 16..31 started, bits 32..63 the
+// number of claims so far. Busy waves look at one word after another for a
+// waiting wave, so that no line is polled by the whole grid.
+using IdleWord = CtlLine<unsigned long long>;
+constexpr uint32_t kIdleGroup = 16;
+
+// What a block of a DFS launch did, written to pinned host memory by the block
+// when it ends; valid when epoch is the launch's. Times are wall-clock ticks.
+struct alignas(128) BlockRec {
+  unsigned long long epoch;
+  unsigned long long active;       // waves that had a task
+  unsigned long long busy;         // their time on tasks, summed
+  unsigned long long first_min, first_sum;  // start of a wave's first task
+  unsigned long long last_max, last_sum;    // end of its last one
+  unsigned long long donated;      // tasks handed to waiting waves
+  unsigned long long scanned;      // source-list entries tested
+  unsigned long long loads;        // 4-byte reads of membership searches
+  unsigned long long mbytes;       // 4 B x degree of every backward list of every expanded partial match
+  unsigned long long nseeds, seed_overflow, abort;  // the control block as the block saw it last
+  unsigned long long pad[2];
+};
+static_assert(sizeof(BlockRec) == 128, "block record layout");
 
 // Status of the apply kernels of one batch.
 struct alignas(64) ApplyCtl {
@@ -165,8 +186,9 @@ struct DfsArgs {
   const uint32_t *seed_plan;
   const uint32_t *seed_s;
   const uint32_t *seed_d;
-  Task *queue;
-  uint32_t qcap;
+  Mailbox *mail;                 // [waves of the grid]
+  IdleWord *idle;                // [ceil(waves / kIdleGroup)]
+  uint32_t donate_cap;           // most tasks a wave may hand out
   uint32_t epoch;
   uint32_t donate_min;
   uint32_t lane_work;            // longest leaf list one lane scans alone
@@ -186,8 +208,7 @@ struct DfsArgs {
   uint32_t *tuples;              // [tuple_cap][kMaxQ+2] or null
   unsigned long long tuple_cap;
   unsigned long long *tuple_count;  // tuples found this batch
-  unsigned long long *wave_busy;    // per wave of the grid: wall-clock ticks on tasks (or null)
-  uint32_t wave_slots;              // entries of wave_busy
+  BlockRec *rec;                    // [blocks of the grid], pinned host memory
   unsigned long long *query_busy;   // per query: wall-clock ticks of its tasks (or null)
 };
 
@@ -372,10 +393,12 @@ hipError_t launch_filter_dirty(const DevGraph &g, const FilterTables &ft, const 
 hipError_t launch_seed(const SeedArgs &a, hipStream_t s);
 hipError_t launch_dfs(const DfsArgs &a, uint32_t blocks, uint32_t waves_per_block, uint32_t max_query_vertices,
                       hipStream_t s);
-// Resets the DFS control block (ctl) and/or the per-batch state (actl's
-// counters, the tuple counter and the nq*2 match counts); null pointers are skipped.
+// Resets the DFS control block (ctl) with the nidle waiting words and/or the
+// per-batch state (actl's counters, the tuple counter and the nq*2 match
+// counts); null pointers are skipped.
 hipError_t launch_ctl_reset(DfsCtl *ctl, ApplyCtl *actl, unsigned long long *tuple_count,
-                            unsigned long long *counts, uint32_t ncounts, hipStream_t s);
+                            unsigned long long *counts, uint32_t ncounts, IdleWord *idle, uint32_t nidle,
+                            hipStream_t s);
 hipError_t launch_scratch_reset(ApplyCtl *actl, hipStream_t s);
 hipError_t launch_pool_move(const uint32_t *old_pool, uint32_t *new_pool, const uint32_t *old_start,
                             const uint32_t *new_start, const uint32_t *deg, uint32_t n,
@@ -393,10 +416,12 @@ struct RoundNodeArgs {
   unsigned long long *no_tc;
   unsigned long long *no_counts;
   uint32_t no_ncounts;
+  IdleWord *idle;
+  uint32_t nidle;
   SeedArgs seed[2];
   DfsArgs dfs;
   uint32_t chunk_levels;
-  void *reset_params[5];
+  void *reset_params[7];
   void *seed_params[2][1];
   void *dfs_params[2];
 };

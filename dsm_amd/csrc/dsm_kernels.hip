@@ -19,6 +19,8 @@
 //   k_dfs                           persistent wave64 DFS with per-wave LDS
 //                                   stacks, work donation and shared leaf sets
 //                                   (gpu_match.cu:96-876 restated for CDNA)
+#include <cstddef>
+
 #include "dsm_device.h"
 #include "dsm_internal.h"
 
@@ -1037,7 +1039,6 @@ __global__ __launch_bounds__(256) void k_seed(SeedArgs a) {
       atomicAdd(&a.ctl->seed_overflow.v, cnt);
       continue;
     }
-    atomicAdd(&a.ctl->work_left.v, (int)cnt);
     uint32_t o = base;
     for (uint32_t p = p0; p < p1; p++) {
       const Plan &pl = a.plans[p];
@@ -1053,21 +1054,16 @@ __global__ __launch_bounds__(256) void k_seed(SeedArgs a) {
 }
 
 __global__ void k_ctl_reset(DfsCtl *ctl, ApplyCtl *actl, unsigned long long *tuple_count,
-                            unsigned long long *counts, uint32_t ncounts) {
+                            unsigned long long *counts, uint32_t ncounts, IdleWord *idle, uint32_t nidle) {
   for (uint32_t i = threadIdx.x; counts && i < ncounts; i += blockDim.x) counts[i] = 0;
+  for (uint32_t i = threadIdx.x; i < nidle; i += blockDim.x) idle[i].v = 0;
   if (threadIdx.x == 0) {
     if (tuple_count) *tuple_count = 0;
     if (ctl) {
       ctl->nseeds.v = 0;
       ctl->seed_head.v = 0;
-      ctl->q_head.v = 0;
-      ctl->q_tail.v = 0;
-      ctl->work_left.v = 0;
       ctl->seed_overflow.v = 0;
       ctl->abort.v = 0;
-      ctl->scanned.v = 0;
-      ctl->loads.v = 0;
-      ctl->mbytes.v = 0;
     }
     if (actl) {
       actl->scratch_used = 0;
@@ -1259,7 +1255,7 @@ __device__ __forceinline__ bool test_chunk(const WaveMem &M, const DfsArgs &a, u
 // that carry the leaf's signature bit and differ from the earlier images of
 // its label. F is sorted. Sets fstate: kFReady (F in fbuf), kFLarge (shortest
 // such list longer than kFCap) or kFNone (no such neighbour).
-__device__ void compute_leaf_set(const WaveMem &M, const DfsArgs &a, uint32_t leaf, uint32_t &scanned,
+__device__ __forceinline__ void compute_leaf_set(const WaveMem &M, const DfsArgs &a, uint32_t leaf, uint32_t &scanned,
                                  uint32_t &loads) {
   WaveHdr &S = *M.h;
   const uint32_t lane = lane_id();
@@ -1479,7 +1475,7 @@ __device__ __forceinline__ uint32_t leaf_count_wave(const WaveMem &M, const DfsA
   return c;
 }
 
-__device__ void emit_tuples(const WaveHdr &S, const DfsArgs &a, uint32_t l, uint32_t w, bool ok) {
+__device__ __forceinline__ void emit_tuples(const WaveHdr &S, const DfsArgs &a, uint32_t l, uint32_t w, bool ok) {
   const uint64_t m = ballot(ok);
   if (m == 0) return;
   unsigned long long base = 0;
@@ -1496,7 +1492,7 @@ __device__ void emit_tuples(const WaveHdr &S, const DfsArgs &a, uint32_t l, uint
   t[2 + S.qv[l]] = w;
 }
 
-// Hands half of some remaining work to the queue when waves are waiting.
+// Hands ranges of the wave's unscanned work to waiting waves.
 //
 // Levels shallower than the current one give away work when enough entries
 // remain there (fetched-but-unconsumed chunk entries count: their source
@@ -1504,13 +1500,36 @@ __device__ void emit_tuples(const WaveHdr &S, const DfsArgs &a, uint32_t l, uint
 // more above the leaf; sixteen one level above it. The level being scanned
 // gives away work only when at least donate_min source entries remain. The
 // receiver re-fetches and re-filters the donated source range [mid, end).
-// Hands ranges of the wave's unscanned work to waiting waves: up to
-// min(waiting, kDonateBurst) of them per call, each half of what is left at
-// the shallowest level that still holds enough, so that when most of the grid
-// runs dry at once the work spreads in fewer check periods.
+//
+// Up to kDonateBurst ranges go out per call, each half of what is left at the
+// shallowest level that still holds enough, so that when most of the grid runs
+// dry at once the work spreads in fewer check periods.
+//
+// Words that the whole grid reads or counts on bound the search once it is
+// spread: with one pair of ticket counters, read by every busy wave every eight
+// scan steps, 1,024 waves on 128 or on 256 CUs took the same time, 2,048 waves
+// 14.0 ms per launch (1M vertices, 64 queries, batches of 4,096) and their time
+// on tasks fell by 30% when they looked 32 times less often. With a waiting word
+// per 16 waves, each busy wave looking at another one each time, a mailbox per
+// wave and work counted in registers, the same launches take 10.1 ms, and
+// looking every fourth step costs nothing (9.9 ms).
 constexpr uint32_t kDonateBurst = DSM_DONATE_BURST;
+constexpr uint32_t kMaxParts = 64;  // shares a seed is cut into at most
+constexpr unsigned long long kIdleBits = (1ull << kIdleGroup) - 1;
 
-__device__ __forceinline__ bool donate_one(WaveHdr &S, const DfsArgs &a, uint32_t L0, uint32_t l, uint32_t n) {
+// The waves of the grid as try_donate and the waiting waves see them.
+struct Crew {
+  uint32_t nwaves, ngroups;
+  uint32_t me;       // this wave
+  uint32_t look;     // the waiting word it looks at next
+  uint32_t donated;  // tasks it has handed out
+};
+
+// One range to a wave that waits in word g; `word` (lane 0) is what lane 0 last
+// saw of it. The claim is a compare-and-swap of the word: its owner is no longer
+// waiting from then on, and finds the task in its mailbox.
+__device__ __forceinline__ bool donate_one(WaveHdr &S, const DfsArgs &a, uint32_t L0, uint32_t l, uint32_t n,
+                                           Crew &cr, uint32_t g, unsigned long long &word) {
   uint32_t lv = 0xFFFFFFFFu, mid = 0, keep_cn = 0;
   for (uint32_t k = L0; k <= l; k++) {
     const uint32_t p = S.pos[k], e = S.end[k];
@@ -1552,30 +1571,35 @@ __device__ __forceinline__ bool donate_one(WaveHdr &S, const DfsArgs &a, uint32_
   }
   if (lv == 0xFFFFFFFFu) return false;
   const uint32_t e = S.end[lv];
-  uint32_t slot = 0, ok = 0;
+  uint32_t who = 0xFFFFFFFFu;
   if (lane_id() == 0) {
-    const uint32_t t = atomicAdd(&a.ctl->q_tail.v, 1u);
-    if (t < a.qcap) {
-      ok = 1;
-      slot = t;
-      atomicAdd(&a.ctl->work_left.v, 1);
+    while (word & kIdleBits) {
+      const uint32_t b = (uint32_t)__builtin_ctzll(word);
+      const unsigned long long next = (word & ~(1ull << b)) + (1ull << 32);
+      const unsigned long long was = atomicCAS(&a.idle[g].v, word, next);
+      if (was == word) {
+        who = b * cr.ngroups + g;
+        word = next;
+        break;
+      }
+      word = was;
     }
   }
-  ok = bcast(ok);
-  if (!ok) return false;
-  slot = bcast(slot);
+  who = bcast(who);
+  if (who == 0xFFFFFFFFu) return false;
+  cr.donated++;
   const uint32_t lane = lane_id();
-  uint32_t word = 0;
-  if (lane == 0) word = S.plan;
-  else if (lane == 1) word = lv;
-  else if (lane == 2) word = mid;
-  else if (lane == 3) word = e;
-  else if (lane < 4u + kMaxQ) word = S.f[lane - 4];
-  else if (lane == 4u + kMaxQ) word = S.tag;
-  if (lane < (uint32_t)kTaskWords) reinterpret_cast<uint32_t *>(&a.queue[slot])[lane] = word;
+  uint32_t pay = 0;
+  if (lane == 0) pay = S.plan;
+  else if (lane == 1) pay = lv;
+  else if (lane == 2) pay = mid;
+  else if (lane == 3) pay = e;
+  else if (lane < 4u + kMaxQ) pay = S.f[lane - 4];
+  else if (lane == 4u + kMaxQ) pay = S.tag;
+  if (lane < (uint32_t)kTaskWords) reinterpret_cast<uint32_t *>(&a.mail[who])[lane] = pay;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   if (lane == 0) {
-    st_release(&a.queue[slot].ready, a.epoch);
+    atomicAdd(&a.mail[who].mail, 1u);
     // the donor keeps source indices below mid; after a split inside the
     // chunk, mid <= pos, so nothing is left to fetch at this level and a later
     // split there donates [mid', mid) only
@@ -1586,16 +1610,93 @@ __device__ __forceinline__ bool donate_one(WaveHdr &S, const DfsArgs &a, uint32_
   return true;
 }
 
-__device__ void try_donate(WaveHdr &S, const DfsArgs &a, uint32_t L0, uint32_t l, uint32_t n) {
-  // waves waiting for work = tickets taken - slots reserved
-  uint32_t waiting = 0;
-  if (lane_id() == 0) {
-    const uint32_t h = ld_relaxed(&a.ctl->q_head.v), t = ld_relaxed(&a.ctl->q_tail.v);
-    waiting = (h > t && t < a.qcap) ? h - t : 0u;
+__device__ __forceinline__ void try_donate(WaveHdr &S, const DfsArgs &a, uint32_t L0, uint32_t l, uint32_t n, Crew &cr) {
+  const uint32_t g = cr.look;
+  cr.look = g + 1 < cr.ngroups ? g + 1 : 0u;
+  unsigned long long word = 0;
+  if (lane_id() == 0) word = ld_relaxed(&a.idle[g].v);
+  const uint32_t waiting = bcast((uint32_t)__popcll(word & kIdleBits));
+  for (uint32_t k = 0; k < waiting && k < kDonateBurst && cr.donated < a.donate_cap; k++)
+    if (!donate_one(S, a, L0, l, n, cr, g, word)) break;
+}
+
+// No started wave has work: every waiting word has all its started waves
+// waiting, twice in a row with no claim between. Work can only come from a
+// busy wave, so nothing is left then, apart from waves that start later, which
+// bring a seed of their own and finish it alone.
+__device__ __forceinline__ bool all_waiting(const DfsArgs &a, const Crew &cr) {
+  uint32_t claims = 0;
+  for (int pass = 0; pass < 2; pass++) {
+    wave_sync();  // keeps the passes apart; the words are read past the caches
+    uint32_t c = 0;
+    bool all = true;
+    for (uint32_t g = lane_id(); g < cr.ngroups; g += 64) {
+      const unsigned long long v = ld_relaxed(&a.idle[g].v);
+      all = all && (v & kIdleBits) == (v >> kIdleGroup & kIdleBits);
+      c += (uint32_t)(v >> 32);
+    }
+    if (pass == 1) all = all && c == claims;
+    claims = c;
+    if (ballot(!all)) return false;
   }
-  waiting = bcast(waiting);
-  for (uint32_t k = 0; k < waiting && k < kDonateBurst; k++)
-    if (!donate_one(S, a, L0, l, n)) break;
+  return true;
+}
+
+// A wave out of work: marks itself waiting in its word and polls its mailbox.
+// Returns true with a task in it, false when the launch is over (or aborted).
+// The wave whose mark completes its word looks at all of them, and when no wave
+// has work it tells every mailbox to stop. A wave that stops takes its mark
+// back first; if a busy wave claimed it in the meantime (one that started late,
+// after the others had been told to stop), it takes that task instead.
+__device__ __forceinline__ bool wait_for_task(const DfsArgs &a, const Crew &cr, uint32_t &seen) {
+  const uint32_t lane = lane_id();
+  unsigned long long *word = &a.idle[cr.me % cr.ngroups].v;
+  const uint32_t b = cr.me / cr.ngroups;
+  const unsigned long long bits = 1ull << b | 1ull << (b + kIdleGroup);
+  uint32_t full = 0;
+  if (lane == 0) {
+    const unsigned long long v = atomicOr(word, bits) | bits;
+    full = (v & kIdleBits) == (v >> kIdleGroup & kIdleBits);
+  }
+  bool look = bcast(full) != 0;
+  Mailbox *mb = &a.mail[cr.me];
+  const uint64_t since = wall_clock64();
+  for (uint32_t naps = 0;; naps++) {
+    if (look && all_waiting(a, cr))
+      for (uint32_t w = lane; w < cr.nwaves; w += 64)
+        __hip_atomic_store(&a.mail[w].stop, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    look = false;
+    // relaxed poll: an acquire here would invalidate the CU's L1 on every poll
+    // of every waiting wave; the acquire fence follows a hit instead
+    unsigned long long ms = 0;
+    if (lane == 0) ms = ld_relaxed(reinterpret_cast<unsigned long long *>(&mb->mail));
+    ms = bcast64(ms);
+    if ((uint32_t)ms != seen) {
+      seen = (uint32_t)ms;
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      return true;
+    }
+    if ((uint32_t)(ms >> 32) == a.epoch) {
+      uint32_t mine = 0;
+      if (lane == 0) mine = (uint32_t)(atomicAnd(word, ~bits) >> b) & 1u;
+      if (bcast(mine)) return false;
+    }
+    if ((naps & 63) == 63) {
+      // the abort flag and the watchdog; one wave per word looks at the words again
+      look = b == 0;
+      uint32_t out = 0;
+      if (lane == 0) {
+        out = ld_relaxed(&a.ctl->abort.v);
+        if (!out && wall_clock64() - since > a.watchdog) {
+          st_release(&a.ctl->abort.v, 1u);
+          out = 1;
+        }
+      }
+      if (bcast(out)) return false;
+    }
+    const uint32_t reps = (1u << (naps < 4 ? naps : 4u)) < a.poll_max ? (1u << (naps < 4 ? naps : 4u)) : a.poll_max;
+    for (uint32_t r = 0; r < reps; r++) __builtin_amdgcn_s_sleep(8);
+  }
 }
 
 template <int WPB, bool TUP>
@@ -1616,88 +1717,63 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
   WaveHdr &S = *M.h;
   if (lane == 0) S.plan = 0xFFFFFFFFu;
   wave_sync();
+  const uint32_t wv = threadIdx.x >> 6;
+  // what the block's waves did, for its record
+  __shared__ unsigned long long s_rec[WPB][7];
+  Crew cr;
+  cr.nwaves = gridDim.x * WPB;
+  cr.ngroups = (cr.nwaves + kIdleGroup - 1) / kIdleGroup;
+  cr.me = blockIdx.x * WPB + wv;
+  cr.look = (cr.me + 1) % cr.ngroups;
+  cr.donated = 0;
   // a seed table overflow leaves unwritten slots: match nothing, the host
   // reports the error (the table is sized so that it cannot happen)
-  if (a.ctl->seed_overflow.v) return;
-  const uint32_t nseeds = a.ctl->nseeds.v;
-  // Seeds are claimed from a counter, never assigned by wave index: the grid
-  // is sized to what the occupancy query says fits, but nothing guarantees
-  // that every block is resident at once, and a seed reserved for a block
-  // that has not started would keep the resident waves waiting for it.
-  bool seeds_left = true;
-  // Donated tasks are handed out by ticket: a wave out of work takes the next
-  // ticket with one atomic add and then waits on the ready flag inside that
-  // queue slot (a 128-byte line of its own), so publishing a task wakes exactly
-  // one wave and idle waves never contend on a shared counter.
-  uint32_t ticket = 0xFFFFFFFFu;
-  uint32_t naps = 0;            // polls of the current ticket (backoff)
-  uint64_t idle_since = 0;      // wall clock when the wave ran out of work (watchdog)
+  const uint32_t nseeds = a.ctl->seed_overflow.v ? 0u : a.ctl->nseeds.v;
+  // With fewer seeds than waves, every seed is cut into `parts` shares of its
+  // first level's source range, so that the grid starts with work for all
+  // instead of spreading it by halves (100,000 vertices, 4 queries, batches of
+  // 256, about 30 seeds a launch: 230 -> 96 us, with the waiting words). A wave's first share is the one of its
+  // own index; the rest are claimed from a counter. A share whose wave has not
+  // started (nothing guarantees that every block is resident at once) keeps
+  // nobody waiting: waves that have started end without it, and its own wave
+  // does it when it starts.
+  const uint32_t parts = nseeds && nseeds < cr.nwaves ? min(cr.nwaves / nseeds, kMaxParts) : 1u;
+  const uint32_t total = nseeds * parts;
+  uint32_t first = cr.me;
+  bool seeds_left = total > cr.nwaves;
+  uint32_t seen = 0;  // mail taken so far
+  if (lane == 0) {
+    seen = ld_relaxed(&a.mail[cr.me].mail);
+    if (first < total) atomicOr(&a.idle[cr.me % cr.ngroups].v, 1ull << (cr.me / cr.ngroups + kIdleGroup));
+  }
+  seen = bcast(seen);
   uint64_t busy = 0;            // wall-clock ticks spent on tasks
   uint64_t first_t = 0, last_t = 0;  // start of the first task, end of the last
+  uint64_t wscanned = 0, wloads = 0, wmbytes = 0;  // work of all its tasks
   for (;;) {
-    // lane 0 claims work; every decision is then broadcast so that all
-    // control flow below stays wave-uniform
-    uint32_t got = 0, slot = 0, took = 0;
-    if (lane == 0) {
-      if (seeds_left) {
-        const uint32_t i = atomicAdd(&a.ctl->seed_head.v, 1u);
-        if (i < nseeds) {
-          got = 2;
-          slot = i;
-        } else {
-          seeds_left = false;
-        }
-      }
-      if (!got) {
-        if (ticket == 0xFFFFFFFFu) {
-          ticket = atomicAdd(&a.ctl->q_head.v, 1u);
-          took = 1;
-        }
-        // relaxed poll: an acquire here would invalidate the CU's L1 on every
-        // poll of every waiting wave; the acquire fence follows a hit instead
-        if (ticket < a.qcap && ld_relaxed(&a.queue[ticket].ready) == a.epoch) {
-          got = 1;
-          slot = ticket;
-          ticket = 0xFFFFFFFFu;
-        }
-      }
+    uint32_t got = 0, slot = 0;
+    if (total == 0) break;
+    if (first < total) {
+      got = 2;
+      slot = first;
+      first = 0xFFFFFFFFu;
+    } else if (seeds_left) {
+      if (lane == 0) slot = cr.nwaves + atomicAdd(&a.ctl->seed_head.v, 1u);
+      slot = bcast(slot);
+      if (slot < total) got = 2;
+      else seeds_left = false;
     }
-    got = bcast(got);
-    slot = bcast(slot);
-    if (bcast(took)) {
-      naps = 0;
-      idle_since = wall_clock64();
-    }
-    if (got == 0) {
-      // waiting for the ticket's task: exponential backoff; the termination
-      // counter, the abort flag and the watchdog every eighth poll
-      if ((naps & 7) == 7) {
-        int32_t left = 0;
-        uint32_t ab = 0, expired = 0;
-        if (lane == 0) {
-          left = ld_relaxed(&a.ctl->work_left.v);
-          ab = ld_relaxed(&a.ctl->abort.v);
-          expired = wall_clock64() - idle_since > a.watchdog;
-          if (expired && left > 0) st_release(&a.ctl->abort.v, 1u);
-        }
-        left = (int32_t)bcast((uint32_t)left);
-        ab = bcast(ab);
-        expired = bcast(expired);
-        if (left <= 0 || ab || expired) break;
-      }
-      const uint32_t reps = (1u << (naps < 4 ? naps : 4u)) < a.poll_max ? (1u << (naps < 4 ? naps : 4u)) : a.poll_max;
-      for (uint32_t r = 0; r < reps; r++) __builtin_amdgcn_s_sleep(8);
-      naps++;
-      continue;
+    if (!got) {
+      if (!wait_for_task(a, cr, seen)) break;
+      got = 1;
     }
     // ---- load the task
     const uint64_t t_task = wall_clock64();
     if (first_t == 0) first_t = t_task;
-    uint32_t plan, L0, lo, hi, tag, fw = 0;
+    uint32_t plan, L0, lo, hi, tag, fw = 0, part = 0;
     if (got == 1) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
       const uint32_t word =
-          lane < (uint32_t)kTaskWords ? reinterpret_cast<const uint32_t *>(&a.queue[slot])[lane] : 0u;
+          lane < (uint32_t)kTaskWords ? reinterpret_cast<const uint32_t *>(&a.mail[cr.me])[lane] : 0u;
       plan = __builtin_amdgcn_readlane(word, 0);
       L0 = __builtin_amdgcn_readlane(word, 1);
       lo = __builtin_amdgcn_readlane(word, 2);
@@ -1705,6 +1781,8 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
       tag = __builtin_amdgcn_readlane(word, 4 + kMaxQ);
       fw = __shfl(word, (int)((lane + 4) & 63));
     } else {
+      part = slot / nseeds;
+      slot -= part * nseeds;
       plan = a.seed_plan[slot];
       tag = a.seed_tag[slot];
       L0 = 2;
@@ -1740,13 +1818,28 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
     uint32_t scanned = 0, loads = 0;  // per lane: source entries read, search loads
     if (L0 >= n) {
       // complete embedding (two-vertex query seeded by its only edge)
-      if (lane == 0) lcount = 1;
-      if (TUP) emit_tuples(S, a, n - 1, S.f[n - 1], lane == 0);
+      if (lane == 0 && part == 0) lcount = 1;
+      if (TUP) emit_tuples(S, a, n - 1, S.f[n - 1], lane == 0 && part == 0);
     } else {
       // a seed expands its partial match here; a donated task continues one
       // whose expansion the donor counted
-      if (got == 2 && lane == 0) mbytes += list_bytes(S, S.back[L0]);
+      if (got == 2 && lane == 0 && part == 0) mbytes += list_bytes(S, S.back[L0]);
       init_level(S, a.g, L0, lo, hi);
+      if (got == 2 && parts > 1) {
+        // the share of the source range, in pieces of what a hand-off is worth:
+        // an entry two or more levels above the leaf, 16 one level above it,
+        // a chunk of 64 at the leaf
+        const uint32_t piece = L0 + 3 <= n ? 1u : L0 + 2 == n ? 16u : 64u;
+        const uint32_t len = bcast(S.end[L0]), np = (len + piece - 1) / piece;
+        lo = (uint32_t)((uint64_t)np * part / parts) * piece;
+        hi = min((uint32_t)((uint64_t)np * (part + 1) / parts) * piece, len);
+        wave_sync();
+        if (lane == 0) {
+          S.pos[L0] = lo;
+          S.end[L0] = hi;
+        }
+        wave_sync();
+      }
       uint32_t l = L0;
       // highest position the leaf set F depends on (-1: none)
       int fdep = -1;
@@ -1761,7 +1854,7 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
           for (;;) {
             if (++tick >= a.donate_every) {
               tick = 0;
-              try_donate(S, a, L0, l, n);
+              try_donate(S, a, L0, l, n, cr);
             }
             const uint32_t p = bcast(S.pos[l]), e = bcast(S.end[l]);
             if (p >= e) break;
@@ -1809,7 +1902,7 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
           for (;;) {
             if (++tick >= a.donate_every) {
               tick = 0;
-              try_donate(S, a, L0, l, n);
+              try_donate(S, a, L0, l, n, cr);
             }
             const uint32_t p = bcast(S.pos[l]), e = bcast(S.end[l]);
             if (p >= e) break;
@@ -1887,7 +1980,7 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
         }
         if (++tick >= a.donate_every) {
           tick = 0;
-          try_donate(S, a, L0, l, n);
+          try_donate(S, a, L0, l, n, cr);
         }
         const uint32_t p = bcast(S.pos[l]), e = bcast(S.end[l]);
         if (p < e) {
@@ -1935,22 +2028,53 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
       const uint32_t tg = S.tag;
       if (tot)
         atomicAdd(&a.counts[((size_t)(tg >> 1) * a.nq + S.query) * 2 + (tg & 1)], (unsigned long long)tot);
-      atomicAdd(&a.ctl->scanned.v, (unsigned long long)sc);
-      atomicAdd(&a.ctl->loads.v, (unsigned long long)ld);
-      atomicAdd(&a.ctl->mbytes.v, (unsigned long long)mb);
-      atomicSub(&a.ctl->work_left.v, 1);
     }
+    wscanned += sc;
+    wloads += ld;
+    wmbytes += mb;
     last_t = wall_clock64();
     busy += last_t - t_task;
     if (a.query_busy && lane == 0) atomicAdd(&a.query_busy[S.query], (unsigned long long)(last_t - t_task));
   }
-  // time this wave spent on tasks (not waiting) and when its first task
-  // started and its last ended, for the balance statistics
-  const uint32_t slot_w = blockIdx.x * WPB + (threadIdx.x >> 6);
-  if (a.wave_busy && lane == 0 && slot_w < a.wave_slots) {
-    a.wave_busy[slot_w] = busy;
-    a.wave_busy[a.wave_slots + slot_w] = first_t;
-    a.wave_busy[2 * (size_t)a.wave_slots + slot_w] = last_t;
+  // the block's record: the time its waves
+  // spent on tasks (not waiting), when their first task started and their last
+  // ended, and their work
+  if (lane == 0) {
+    s_rec[wv][0] = busy;
+    s_rec[wv][1] = first_t;
+    s_rec[wv][2] = last_t;
+    s_rec[wv][3] = cr.donated;
+    s_rec[wv][4] = wscanned;
+    s_rec[wv][5] = wloads;
+    s_rec[wv][6] = wmbytes;
+  }
+  __syncthreads();
+  if (wv == 0) {
+    // a lane per word of the record, so that it leaves as one write over the bus
+    unsigned long long x = 0;
+    const unsigned long long field = lane;
+    if (field == offsetof(BlockRec, first_min) / 8) x = ~0ull;
+    for (int w = 0; w < WPB; w++) {
+      const unsigned long long *r = s_rec[w];
+      const bool act = r[1] != 0;
+      switch (field) {
+        case offsetof(BlockRec, active) / 8: x += act; break;
+        case offsetof(BlockRec, busy) / 8: x += r[0]; break;
+        case offsetof(BlockRec, first_min) / 8: x = act ? min(x, r[1]) : x; break;
+        case offsetof(BlockRec, first_sum) / 8: x += r[1]; break;
+        case offsetof(BlockRec, last_max) / 8: x = max(x, r[2]); break;
+        case offsetof(BlockRec, last_sum) / 8: x += r[2]; break;
+        case offsetof(BlockRec, donated) / 8: x += r[3]; break;
+        case offsetof(BlockRec, scanned) / 8: x += r[4]; break;
+        case offsetof(BlockRec, loads) / 8: x += r[5]; break;
+        case offsetof(BlockRec, mbytes) / 8: x += r[6]; break;
+      }
+    }
+    if (field == offsetof(BlockRec, epoch) / 8) x = a.epoch;
+    if (field == offsetof(BlockRec, nseeds) / 8) x = a.ctl->nseeds.v;
+    if (field == offsetof(BlockRec, seed_overflow) / 8) x = a.ctl->seed_overflow.v;
+    if (field == offsetof(BlockRec, abort) / 8) x = ld_relaxed(&a.ctl->abort.v);
+    if (lane < sizeof(BlockRec) / 8) reinterpret_cast<unsigned long long *>(&a.rec[blockIdx.x])[lane] = x;
   }
 }
 
@@ -2205,6 +2329,8 @@ void round_node_params(RoundNodeArgs &st, uint32_t blocks, uint32_t waves_per_bl
   st.reset_params[2] = &st.no_tc;
   st.reset_params[3] = &st.no_counts;
   st.reset_params[4] = &st.no_ncounts;
+  st.reset_params[5] = &st.idle;
+  st.reset_params[6] = &st.nidle;
   *reset = hipKernelNodeParams{};
   reset->func = reinterpret_cast<void *>(&k_ctl_reset);
   reset->gridDim = dim3(1);
@@ -2262,8 +2388,9 @@ int dfs_max_blocks_per_cu(uint32_t waves_per_block, uint32_t max_query_vertices)
 }
 
 hipError_t launch_ctl_reset(DfsCtl *ctl, ApplyCtl *actl, unsigned long long *tuple_count,
-                            unsigned long long *counts, uint32_t ncounts, hipStream_t s) {
-  hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(256), 0, s, ctl, actl, tuple_count, counts, ncounts);
+                            unsigned long long *counts, uint32_t ncounts, IdleWord *idle, uint32_t nidle,
+                            hipStream_t s) {
+  hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(256), 0, s, ctl, actl, tuple_count, counts, ncounts, idle, nidle);
   return hipGetLastError();
 }
 

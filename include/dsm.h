@@ -76,7 +76,8 @@ typedef struct {
   uint32_t waves_per_block;  /* DFS launch shape; 0 = default */
   uint32_t blocks_per_cu;    /* 0 = as many as occupancy allows */
   uint32_t donate_min;       /* smallest source range split off to an idle wave (0 = default) */
-  uint32_t queue_capacity;   /* donated-task queue slots (0 = default) */
+  uint32_t queue_capacity;   /* most tasks a round hands to idle waves, shared evenly by
+                                its waves (0 = no limit) */
   uint32_t watchdog_ms;      /* an idle DFS wave that waits longer than this for
                                 work aborts the round with DSM_EDEVICE (0 = 60 s) */
   uint32_t lane_work;        /* one level above the leaf: longest list a lane scans
@@ -84,7 +85,7 @@ typedef struct {
   int leaf_sets;             /* 1: one level above the leaf, candidates count their
                                 leaf images against a leaf set shared by the parent;
                                 0: one descent per candidate */
-  uint32_t donate_every;     /* scan steps between a busy wave's checks for idle waves (0 = 8) */
+  uint32_t donate_every;     /* scan steps between a busy wave's checks for idle waves (0 = 4) */
   uint32_t donate_min_n2;    /* smallest range one level above the leaf that is split
                                 off to an idle wave (0 = 64) */
   uint32_t poll_max;         /* a wave waiting for donated work sleeps at most this many

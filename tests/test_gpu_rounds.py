@@ -1,0 +1,64 @@
+"""How a DFS round spreads its work: seeds cut into shares, hand-offs between
+waves and the end of the launch, at the grid's edges."""
+import numpy as np
+import pytest
+
+from dsm_amd import engine as E
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {"edge": [(0, 1)], "path3": [(0, 1), (1, 2)], "tri_pendant": [(0, 1), (1, 2), (0, 2), (1, 3)],
+          "house": [(0, 1), (1, 2), (2, 3), (3, 0), (0, 4), (1, 4)]}
+
+
+def one_label(shape):
+    e = np.array(SHAPES[shape], np.uint32)
+    n = int(e.max()) + 1
+    return n, np.zeros(n, np.uint32), e[:, 0].copy(), e[:, 1].copy()
+
+
+@pytest.mark.parametrize("records", [1, 2, 127, 128, 129, 512, 513, 1025])
+@pytest.mark.parametrize("queue_capacity", [0, 1])
+def test_seed_shares_around_the_grid_size(records, queue_capacity):
+    """One record to one per wave and beyond (a query edge gives two seeds per
+    record, a path four, ...: 1,024 waves are met from both sides), with and
+    without hand-offs, for queries of two vertices (a share holds a whole
+    match) to five."""
+    rng = np.random.default_rng(records)
+    n, m = 150, 900
+    key = rng.permutation(n * n)
+    key = key[key // n < key % n][:m]
+    u, v = (key // n).astype(np.uint32), (key % n).astype(np.uint32)
+    queries = [one_label(s) for s in sorted(SHAPES)]
+    labels = np.zeros(n, np.uint32)
+    # re-inserted present edges: each seeds, and the graph stays as it is
+    pick = rng.integers(0, len(u), records)
+    z = np.zeros(records, np.uint32)
+    batch = (np.ones(records, np.uint8), u[pick], v[pick], z)
+    want = O.run_stream(O.Graph(n, labels, u, v), [O.Query(*q) for q in queries], [batch], relabel=False)[0]
+    eng = E.Engine((n, labels, u, v), queries, relabel=False, queue_capacity=queue_capacity)
+    try:
+        for _ in range(3):  # the mailboxes are used again by every round
+            pos, neg = eng.process_batch(*batch)
+            assert pos.tolist() == want["pos"] and neg.tolist() == want["neg"]
+        if queue_capacity:
+            assert eng.stats()["tasks_donated"] == 0
+    finally:
+        eng.close()
+
+
+def test_watchdog_ends_a_round_whose_waves_wait():
+    """A round that keeps some waves waiting past watchdog_ms (long shares of
+    one seed, hand-offs off) ends by itself with DSM_EDEVICE."""
+    n = 300
+    u, v = np.triu_indices(n, 1)
+    u, v = u.astype(np.uint32), v.astype(np.uint32)
+    eng = E.Engine((n, np.zeros(n, np.uint32), u, v), [one_label("house")], relabel=False, queue_capacity=1,
+                   watchdog_ms=1, leaf_sets=False)
+    try:
+        with pytest.raises(E.DsmError) as ei:
+            eng.process_batch(np.ones(1, np.uint8), u[:1], v[:1], np.zeros(1, np.uint32))
+        assert ei.value.code == E.DSM_EDEVICE and "watchdog" in str(ei.value)
+    finally:
+        eng.close()
