@@ -26,6 +26,55 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Wave-wide scans and reductions over DPP: row shifts by 1, 2, 4 and 8 inside
+// the rows of 16 lanes, then lane 15 of a row to the next row and lane 31 to the
+// upper half. Six vector instructions where a ladder of shuffles makes six
+// dependent trips through LDS. All 64 lanes must be active.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_from(uint32_t none, uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, CTRL, ROWS, 0xF, false);
+}
+// inclusive sum over the lanes
+__device__ __forceinline__ uint32_t wave_incl_sum(uint32_t x) {
+  x += dpp_from<0x111, 0xF>(0, x);
+  x += dpp_from<0x112, 0xF>(0, x);
+  x += dpp_from<0x114, 0xF>(0, x);
+  x += dpp_from<0x118, 0xF>(0, x);
+  x += dpp_from<0x142, 0xA>(0, x);
+  x += dpp_from<0x143, 0xC>(0, x);
+  return x;
+}
+__device__ __forceinline__ uint32_t wave_or(uint32_t x) {
+  x |= dpp_from<0x111, 0xF>(0, x);
+  x |= dpp_from<0x112, 0xF>(0, x);
+  x |= dpp_from<0x114, 0xF>(0, x);
+  x |= dpp_from<0x118, 0xF>(0, x);
+  x |= dpp_from<0x142, 0xA>(0, x);
+  x |= dpp_from<0x143, 0xC>(0, x);
+  return __builtin_amdgcn_readlane(x, 63);
+}
+// the least value of lanes 0 .. 15
+__device__ __forceinline__ uint32_t row0_min(uint32_t x) {
+  x = min(x, dpp_from<0x111, 0xF>(0xFFFFFFFFu, x));
+  x = min(x, dpp_from<0x112, 0xF>(0xFFFFFFFFu, x));
+  x = min(x, dpp_from<0x114, 0xF>(0xFFFFFFFFu, x));
+  x = min(x, dpp_from<0x118, 0xF>(0xFFFFFFFFu, x));
+  return __builtin_amdgcn_readlane(x, 15);
+}
+// Exclusive sum over the lanes; the total comes back in *total.
+__device__ __forceinline__ uint32_t wave_excl_sum(uint32_t c, uint32_t *total) {
+  const uint32_t incl = wave_incl_sum(c);
+  *total = __builtin_amdgcn_readlane(incl, 63);
+  return incl - c;
+}
+
+// Sum over the lanes, in every lane.
+__device__ __forceinline__ uint64_t wave_sum(uint64_t x) {
+  if (ballot(x >> 26 != 0) == 0) return __builtin_amdgcn_readlane(wave_incl_sum((uint32_t)x), 63);
+  for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o);
+  return x;
+}
+
 template <typename T>
 __device__ __forceinline__ T ld_relaxed(T *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -63,6 +112,30 @@ __device__ __forceinline__ bool contains(const uint32_t *a, uint32_t n, uint32_t
     n -= half;
   }
   return a[lo] == x;
+}
+
+// contains() of K values at once: the searches' loads are in flight together.
+template <int K>
+__device__ __forceinline__ void contains_each(const uint32_t *a, uint32_t n, const uint32_t (&x)[K], bool (&in)[K]) {
+  uint32_t lo[K];
+#pragma unroll
+  for (int u = 0; u < K; u++) {
+    lo[u] = 0;
+    in[u] = false;
+  }
+  if (n == 0) return;
+  uint32_t m = n;
+  while (m > 1) {
+    const uint32_t half = m >> 1;
+    uint32_t v[K];
+#pragma unroll
+    for (int u = 0; u < K; u++) v[u] = a[lo[u] + half];
+#pragma unroll
+    for (int u = 0; u < K; u++) lo[u] = v[u] <= x[u] ? lo[u] + half : lo[u];
+    m -= half;
+  }
+#pragma unroll
+  for (int u = 0; u < K; u++) in[u] = a[lo[u]] == x[u];
 }
 
 // The search window staged in LDS per membership test (entries).
@@ -129,8 +202,8 @@ __device__ __forceinline__ bool window_member(const uint32_t *L, uint32_t d, uin
   const uint32_t lane = lane_id();
   const uint64_t alive = ballot(ok);
   if (alive == 0) return false;
-  const uint32_t wmin = __shfl(w, (int)__builtin_ctzll(alive));
-  const uint32_t wmax = __shfl(w, (int)(63 - __builtin_clzll(alive)));
+  const uint32_t wmin = __builtin_amdgcn_readlane(w, __builtin_ctzll(alive));
+  const uint32_t wmax = __builtin_amdgcn_readlane(w, 63 - __builtin_clzll(alive));
   uint32_t lo, hi;
   bounds2(L, d, wmin, wmax + 1, lo, hi, loads);
   const uint32_t W = hi - lo;

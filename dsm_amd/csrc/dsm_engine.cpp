@@ -202,7 +202,7 @@ struct dsm_engine {
   bool tuples_host = false;
   unsigned long long tuple_cap = 0;
   uint32_t dfs_blocks = 0, dfs_wpb = 4, max_qn = 2;
-  uint32_t donate_min = 256, lane_work = 16, donate_every = 4, donate_min_n2 = 64, leaf_budget = 2048;
+  uint32_t donate_min = 256, lane_work = 16, donate_every = 4, donate_min_n2 = 64, leaf_budget = 8192;
   bool leaf_sets = true;
   bool bit_probe_last = false;
   bool graph_rounds = true;
@@ -1391,7 +1391,7 @@ int create_impl(dsm_engine *e, const dsm_graph_desc *graph, const dsm_query_desc
   }
   e->donate_min = e->opt.donate_min ? e->opt.donate_min : 256;
   e->lane_work = e->opt.lane_work ? e->opt.lane_work : 16;
-  e->leaf_budget = e->opt.leaf_budget ? e->opt.leaf_budget : 2048;
+  e->leaf_budget = e->opt.leaf_budget ? e->opt.leaf_budget : 8192;
   e->donate_every = e->opt.donate_every ? e->opt.donate_every : 4;
   e->donate_min_n2 = e->opt.donate_min_n2 ? e->opt.donate_min_n2 : 64;
   e->leaf_sets = e->opt.leaf_sets != 0;

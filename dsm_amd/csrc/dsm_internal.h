@@ -74,9 +74,10 @@ struct alignas(128) CtlLine {
   T v;
   uint32_t pad[(128 - sizeof(T)) / 4];
 };
+constexpr uint32_t kSeedHeads = 16;
 struct DfsCtl {
   CtlLine<uint32_t> nseeds;        // seeds written by the seed kernel
-  CtlLine<uint32_t> seed_head;     // seed parts claimed beyond every wave's first
+  CtlLine<uint32_t> seed_head[kSeedHeads];  // seed shares claimed: head h counts shares h, h + kSeedHeads, ...
   CtlLine<uint32_t> seed_overflow; // seeds dropped for lack of capacity (must stay 0)
   CtlLine<uint32_t> abort;         // set when an idle wave outlived the watchdog
 };

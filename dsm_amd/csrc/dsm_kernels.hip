@@ -707,19 +707,6 @@ __device__ __forceinline__ void bucket_scatter(const DevGraph &g, const uint8_t 
   }
 }
 
-// Exclusive prefix sum over the lanes (a wave-wide scan of shuffles); the
-// inclusive total comes back in *total.
-__device__ __forceinline__ uint32_t wave_excl_sum(uint32_t c, uint32_t *total) {
-  const uint32_t lane = lane_id();
-  uint32_t incl = c;
-  for (uint32_t off = 1; off < 64; off <<= 1) {
-    const uint32_t y = __shfl_up(incl, off);
-    if (lane >= off) incl += y;
-  }
-  *total = __builtin_amdgcn_readlane(incl, 63);
-  return incl - c;
-}
-
 constexpr uint32_t kLbuildBlock = 4096;  // lists longer than this are sorted by a whole block
 constexpr uint32_t kLbuildWaves = 16;    // waves of that block
 
@@ -1061,7 +1048,7 @@ __global__ void k_ctl_reset(DfsCtl *ctl, ApplyCtl *actl, unsigned long long *tup
     if (tuple_count) *tuple_count = 0;
     if (ctl) {
       ctl->nseeds.v = 0;
-      ctl->seed_head.v = 0;
+      for (uint32_t h = 0; h < kSeedHeads; h++) ctl->seed_head[h].v = 0;
       ctl->seed_overflow.v = 0;
       ctl->abort.v = 0;
     }
@@ -1111,13 +1098,21 @@ struct WaveHdr {
   uint32_t n, query, plan, tag;
   uint32_t fstate, fn;       // leaf set F of the current positions 0..n-3 (see leaf_count)
 };
-constexpr uint32_t kFCap = 2048;  // largest leaf set F kept in LDS
-// F is indexed by id range: bucket b = id >> DfsArgs::fshift (fshift makes the
-// graph's ids fit kFIdx buckets), fidx[b] = first entry of F at or past the
-// bucket. A membership test reads two offsets and binary-searches only the
-// bucket's entries (a few, ids being spread over the range) instead of
-// log2 |F| dependent LDS reads over all of F.
+constexpr uint32_t kFCap = 1024;   // largest leaf set F kept in LDS
+constexpr uint32_t kFScan = 2048;  // longest list it is computed from
+// Membership in F goes through a table beside it, of one of two kinds.
+// - Up to kFBits entries: a bitmap of kFBitWords x 32 bits with the hashed ids of
+//   F set. One read settles almost every id outside F (at most 256 of 8,192 bits
+//   are set); the few left search F. Clearing and setting it costs five LDS
+//   writes a lane.
+// - More: F indexed by id range: bucket b = id >> DfsArgs::fshift (fshift makes the
+//   graph's ids fit kFIdx buckets), fidx[b] = first entry of F at or past the
+//   bucket. A test reads two offsets and searches the bucket's few entries.
+//   Filling the buckets between two entries is a loop per entry, as long as F is
+//   short, which is why the short sets, nearly all of them, take the bitmap.
 constexpr uint32_t kFIdx = 512;
+constexpr uint32_t kFBits = 256;
+constexpr uint32_t kFBitWords = 256;
 // One level above the leaf, the candidates of a 64-entry window count their
 // leaf images inline until their summed scan or search work passes
 // DfsArgs::leaf_budget entries; the candidate that passes it descends to the
@@ -1125,8 +1120,8 @@ constexpr uint32_t kFIdx = 512;
 // count cannot), and the window resumes after it.
 // states of the leaf set F
 constexpr uint32_t kFStale = 0;  // not computed for the current positions
-constexpr uint32_t kFReady = 1;  // fbuf[0, fn) holds F
-constexpr uint32_t kFLarge = 2;  // the shortest fixed list exceeds kFCap: per-candidate descent
+constexpr uint32_t kFReady = 1;  // fbuf[0, fn) holds F, ftab its table
+constexpr uint32_t kFLarge = 2;  // the shortest fixed list exceeds kFScan, or F kFCap: per-candidate descent
 constexpr uint32_t kFNone = 3;   // the leaf's only backward neighbour is position n-2
 
 struct WaveMem {
@@ -1136,12 +1131,13 @@ struct WaveMem {
   uint32_t *cst;    // [levels][64] list start of each candidate
   uint32_t *cdg;    // [levels][64] degree of each candidate
   uint32_t *fbuf;   // [kFCap] leaf set F, ascending
-  uint16_t *fidx;   // [kFIdx + 1] bucket offsets into fbuf
+  uint32_t *ftab;   // F's table: kFBitWords words of bits, or kFIdx + 1 16-bit bucket offsets into fbuf
 };
+constexpr uint32_t kFTabBytes = ((kFIdx + 1) * 2 + 15) / 16 * 16;
+static_assert(kFBitWords * 4 <= kFTabBytes, "the bits fit the table");
 
 __host__ __device__ constexpr uint32_t wave_lds_bytes(uint32_t chunk_levels) {
-  return (uint32_t)((sizeof(WaveHdr) + 15) / 16 * 16) + kWin * 4 + kFCap * 4 + chunk_levels * 64 * 12 +
-         ((kFIdx + 1) * 2 + 15) / 16 * 16;
+  return (uint32_t)((sizeof(WaveHdr) + 15) / 16 * 16) + kWin * 4 + kFCap * 4 + chunk_levels * 64 * 12 + kFTabBytes;
 }
 
 // 4 B per entry of the full lists of the positions in `mask`: what a merge
@@ -1159,34 +1155,29 @@ __device__ __forceinline__ uint64_t list_bytes(const WaveHdr &S, uint32_t mask) 
 // Among the lists of the positions in `mask`, the one with the fewest entries
 // of label index li: for a vertex of degree > kLabelSorted, its label bucket in
 // the label-sorted copy; otherwise the whole list. Lane j examines position j;
-// a wave minimum picks the shortest, lowest position on ties. Wave-uniform
+// a minimum over lanes 0 .. 15 picks the shortest, lowest position on ties. Wave-uniform
 // results; an empty mask gives length 0.
 __device__ __forceinline__ void pick_source(const WaveHdr &S, const DevGraph &g, uint32_t mask, uint32_t li,
                                             const uint32_t *&src, uint32_t &len, uint32_t &j) {
   const uint32_t lane = lane_id();
-  uint64_t key = ~0ull;
-  uint32_t off = 0, sorted = 0;
-  if (lane < (uint32_t)kMaxQ && (mask >> lane & 1)) {
-    const uint32_t d = S.fd[lane];
-    uint32_t n = d;
+  uint32_t n = 0xFFFFFFFFu, off = 0, sorted = 0;
+  if (mask >> (lane & 31) & 1 && lane < (uint32_t)kMaxQ) {
+    n = S.fd[lane];
     off = S.fs[lane];
-    if (d > kLabelSorted) {
+    if (n > kLabelSorted) {
       const uint32_t *row = g.loff + (size_t)S.f[lane] * (g.nbuckets + 1);
       const uint32_t b0 = row[li], b1 = row[li + 1];
       n = b1 - b0;
       off += b0;
       sorted = 1;
     }
-    key = ((uint64_t)n << 32) | lane;
   }
-  for (int o = 32; o >= 1; o >>= 1) {
-    const uint64_t y = __shfl_xor(key, o);
-    key = y < key ? y : key;
-  }
-  j = key == ~0ull ? 0u : (uint32_t)(key & 0xFFFFFFFFu);
-  len = key == ~0ull ? 0u : (uint32_t)(key >> 32);
-  const uint32_t boff = __shfl(off, (int)j);
-  const uint32_t bsorted = __shfl(sorted, (int)j);
+  len = row0_min(n);
+  j = 0;
+  if (len == 0xFFFFFFFFu) len = 0;
+  else j = (uint32_t)__builtin_ctzll(ballot(lane < (uint32_t)kMaxQ && n == len));
+  const uint32_t boff = __builtin_amdgcn_readlane(off, j);
+  const uint32_t bsorted = __builtin_amdgcn_readlane(sorted, j);
   src = (bsorted ? g.lpool : g.pool) + boff;
 }
 
@@ -1249,12 +1240,15 @@ __device__ __forceinline__ bool test_chunk(const WaveMem &M, const DfsArgs &a, u
   return test_entries(M, a, S.src[l], S.back[l] & ~(1u << S.srcj[l]), S.inj[l], S.sig[l], p, e, w, loads);
 }
 
+// An id's bit in the table of a short leaf set (13 bits, kFBitWords words).
+__device__ __forceinline__ uint32_t f_hash(uint32_t y) { return (y * 0x9E3779B1u) >> 19; }
+
 // Leaf set F for positions 0..n-3 (leaf = n-1): the images the leaf may take
 // judging only by its backward neighbours other than position n-2, i.e. the
 // entries of the intersection of their lists (label bucket of the shortest)
 // that carry the leaf's signature bit and differ from the earlier images of
 // its label. F is sorted. Sets fstate: kFReady (F in fbuf), kFLarge (shortest
-// such list longer than kFCap) or kFNone (no such neighbour).
+// such list longer than kFScan, or F than kFCap) or kFNone (no such neighbour).
 __device__ __forceinline__ void compute_leaf_set(const WaveMem &M, const DfsArgs &a, uint32_t leaf, uint32_t &scanned,
                                  uint32_t &loads) {
   WaveHdr &S = *M.h;
@@ -1268,7 +1262,7 @@ __device__ __forceinline__ void compute_leaf_set(const WaveMem &M, const DfsArgs
     const uint32_t *src;
     uint32_t len, j;
     pick_source(S, a.g, bp, S.lix[leaf], src, len, j);
-    if (len > kFCap) {
+    if (len > kFScan) {
       state = kFLarge;
     } else {
       const uint32_t oth = bp & ~(1u << j);
@@ -1279,23 +1273,35 @@ __device__ __forceinline__ void compute_leaf_set(const WaveMem &M, const DfsArgs
         const bool ok = test_entries(M, a, src, oth, inj, sig, p, len, w, loads);
         scanned += p + lane < len ? 1u : 0u;
         const uint64_t m = ballot(ok);
+        if (cnt + (uint32_t)__popcll(m) > kFCap) {
+          state = kFLarge;
+          break;
+        }
         if (ok) M.fbuf[cnt + mbcnt(m)] = w;
         cnt += (uint32_t)__popcll(m);
       }
     }
   }
   wave_sync();
-  if (state == kFReady) {
+  if (state == kFReady && cnt <= kFBits) {
+    reinterpret_cast<uint4 *>(M.ftab)[lane] = uint4{0, 0, 0, 0};
+    wave_sync();
+    for (uint32_t i = lane; i < cnt; i += 64) {
+      const uint32_t h = f_hash(M.fbuf[i]);
+      atomicOr(&M.ftab[h >> 5], 1u << (h & 31));
+    }
+  } else if (state == kFReady) {
     // bucket offsets: entry i opens every bucket after its predecessor's up
     // to its own; buckets past the last entry start at cnt
+    uint16_t *fidx = reinterpret_cast<uint16_t *>(M.ftab);
     const uint32_t sh = a.fshift;
     for (uint32_t i = lane; i < cnt; i += 64) {
       const uint32_t b = M.fbuf[i] >> sh;
       const uint32_t pb = i ? (M.fbuf[i - 1] >> sh) + 1 : 0u;
-      for (uint32_t k = pb; k <= b; k++) M.fidx[k] = (uint16_t)i;
+      for (uint32_t k = pb; k <= b; k++) fidx[k] = (uint16_t)i;
     }
-    const uint32_t last = cnt ? (M.fbuf[cnt - 1] >> sh) + 1 : 0u;
-    for (uint32_t k = last + lane; k <= kFIdx; k += 64) M.fidx[k] = (uint16_t)cnt;
+    const uint32_t last = (M.fbuf[cnt - 1] >> sh) + 1;
+    for (uint32_t k = last + lane; k <= kFIdx; k += 64) fidx[k] = (uint16_t)cnt;
   }
   wave_sync();
   if (lane == 0) {
@@ -1305,10 +1311,15 @@ __device__ __forceinline__ void compute_leaf_set(const WaveMem &M, const DfsArgs
   wave_sync();
 }
 
-// y in F (state kFReady), through the bucket index.
-__device__ __forceinline__ bool in_leaf_set(const WaveMem &M, const DfsArgs &a, uint32_t y) {
+// y in F (state kFReady, fn entries), through F's table.
+__device__ __forceinline__ bool in_leaf_set(const WaveMem &M, const DfsArgs &a, uint32_t fn, uint32_t y) {
+  if (fn <= kFBits) {
+    const uint32_t h = f_hash(y);
+    return (M.ftab[h >> 5] >> (h & 31) & 1) && lds_contains(M.fbuf, fn, y);
+  }
+  const uint16_t *fidx = reinterpret_cast<const uint16_t *>(M.ftab);
   const uint32_t b = y >> a.fshift;
-  const uint32_t lo = M.fidx[b], hi = M.fidx[b + 1];
+  const uint32_t lo = fidx[b], hi = fidx[b + 1];
   return lds_contains(M.fbuf + lo, hi - lo, y);
 }
 
@@ -1318,8 +1329,10 @@ __device__ __forceinline__ bool in_leaf_set(const WaveMem &M, const DfsArgs &a, 
 // with F, the entries that lie in F; with no other backward neighbour
 // (kFNone), the entries that carry the leaf's signature and differ from the
 // earlier images of its label. Injectivity against w itself applies when the
-// leaf has w's label. A lane whose scan would take more than a.lane_work
-// steps leaves it to the wave (leaf_count_wave) and reports its list instead.
+// leaf has w's label. The lanes' scans are shared by the wave
+// (leaf_scan_segments); a list much longer than F is left to leaf_count_wave,
+// which searches F's elements in it. Without leaf_segments a lane scans a list
+// of up to a.lane_work entries itself and leaves longer ones to the wave.
 
 struct LeafList {
   const uint32_t *L;
@@ -1327,18 +1340,88 @@ struct LeafList {
   bool by_f;  // search F's elements in L instead of scanning L
 };
 
-__device__ __forceinline__ bool leaf_accept(const WaveHdr &S, const DfsArgs &a, const WaveMem &M, uint32_t leaf,
-                                            uint32_t st, uint32_t fn, bool injw, uint32_t w, uint32_t y) {
-  if (injw && y == w) return false;
-  if (st == kFReady) return in_leaf_set(M, a, y);
-  if (!bit_of(a.bm, a.words, S.sig[leaf], y)) return false;
-  uint32_t m = S.inj[leaf] & ~(1u << (leaf - 1));
+// Reads of one search for each of F's elements in a list of len entries.
+__device__ __forceinline__ uint32_t search_reads(uint32_t len) { return 33u - (uint32_t)__builtin_clz(len | 1u); }
+
+// F's elements are searched in the list when that is fewer dependent steps for
+// the wave: a search takes search_reads(len) of them for up to 256 elements (four
+// a lane), a scan one for 256 entries, which come in whole lines. The line lies
+// at kScanPerStep entries a step.
+constexpr uint32_t kScanPerStep = 128;
+__device__ __forceinline__ bool search_f(uint32_t fn, uint32_t len) {
+  return len > kScanPerStep * search_reads(len) * ((fn + 255) / 256);
+}
+
+// A leaf level's constants, read once per scan.
+struct LeafRule {
+  uint32_t st, fn, sig, inj;
+  bool injw;
+};
+__device__ __forceinline__ LeafRule leaf_rule(const WaveHdr &S, uint32_t leaf) {
+  const uint32_t inj = S.inj[leaf];
+  return LeafRule{S.fstate, S.fn, S.sig[leaf], inj & ~(1u << (leaf - 1)), (bool)(inj >> (leaf - 1) & 1)};
+}
+
+// Whether y is a leaf image; w is the image of position n-2 it belongs to.
+__device__ __forceinline__ bool leaf_accept_one(const WaveMem &M, const DfsArgs &a, const LeafRule &r, uint32_t w,
+                                                uint32_t y) {
+  if (r.injw && y == w) return false;
+  if (r.st == kFReady) return in_leaf_set(M, a, r.fn, y);
+  if (!bit_of(a.bm, a.words, r.sig, y)) return false;
+  uint32_t m = r.inj;
   while (m) {
     const uint32_t j = __builtin_ctz(m);
     m &= m - 1;
-    if (S.f[j] == y) return false;
+    if (M.h->f[j] == y) return false;
   }
   return true;
+}
+
+// How many of a lane's K entries y are leaf images; w is the image of position
+// n-2 each belongs to, ok the entries that exist.
+template <int K>
+__device__ __forceinline__ uint32_t leaf_accept(const WaveMem &M, const DfsArgs &a, const LeafRule &r,
+                                                const uint32_t (&w)[K], const uint32_t (&y)[K], bool (&ok)[K]) {
+  const WaveHdr &S = *M.h;
+  uint32_t c = 0;
+  if (r.st == kFReady) {
+    if (r.fn <= kFBits) {
+      uint32_t t[K];
+      bool any = false;
+#pragma unroll
+      for (int u = 0; u < K; u++) t[u] = M.ftab[f_hash(y[u]) >> 5];
+#pragma unroll
+      for (int u = 0; u < K; u++) {
+        ok[u] = ok[u] && (t[u] >> (f_hash(y[u]) & 31) & 1) && !(r.injw && y[u] == w[u]);
+        any = any || ok[u];
+      }
+      if (ballot(any) == 0) return 0;
+#pragma unroll
+      for (int u = 0; u < K; u++)
+        if (ballot(ok[u])) c += ok[u] && lds_contains(M.fbuf, r.fn, y[u]) ? 1u : 0u;
+    } else {
+#pragma unroll
+      for (int u = 0; u < K; u++)
+        c += ok[u] && !(r.injw && y[u] == w[u]) && in_leaf_set(M, a, r.fn, y[u]) ? 1u : 0u;
+    }
+    return c;
+  }
+  uint64_t bw[K];
+#pragma unroll
+  for (int u = 0; u < K; u++) bw[u] = a.bm[(size_t)r.sig * a.words + (ok[u] ? y[u] >> 6 : 0u)];
+#pragma unroll
+  for (int u = 0; u < K; u++) ok[u] = ok[u] && (bw[u] >> (y[u] & 63) & 1) && !(r.injw && y[u] == w[u]);
+  uint32_t m = r.inj;
+  while (m) {
+    const uint32_t j = __builtin_ctz(m);
+    m &= m - 1;
+    const uint32_t f = S.f[j];
+#pragma unroll
+    for (int u = 0; u < K; u++) ok[u] = ok[u] && f != y[u];
+  }
+#pragma unroll
+  for (int u = 0; u < K; u++) c += ok[u] ? 1u : 0u;
+  return c;
 }
 
 __device__ __forceinline__ uint32_t leaf_count_lane(const WaveMem &M, const DfsArgs &a, uint32_t leaf, uint32_t w,
@@ -1347,127 +1430,143 @@ __device__ __forceinline__ uint32_t leaf_count_lane(const WaveMem &M, const DfsA
   const WaveHdr &S = *M.h;
   const uint32_t pv = leaf - 1;
   const uint32_t back = S.back[leaf];
-  const bool injw = (S.inj[leaf] >> pv) & 1;
-  const uint32_t st = S.fstate, fn = S.fn;
+  const LeafRule r = leaf_rule(S, leaf);
   defer = false;
   if (!((back >> pv) & 1)) {
-    uint32_t c = fn;
-    if (injw && in_leaf_set(M, a, w)) c--;
+    uint32_t c = r.fn;
+    if (r.injw && in_leaf_set(M, a, r.fn, w)) c--;
     return c;
   }
   const uint32_t ws = a.g.start[w], wd = a.g.deg[w];
   wdeg = wd;
-  const uint32_t *L = a.g.pool + ws;
-  uint32_t len = wd;
+  out.L = a.g.pool + ws;
+  out.len = wd;
   if (wd > kLabelSorted) {
     const uint32_t *row = a.g.loff + (size_t)w * (a.g.nbuckets + 1);
     const uint32_t li = S.lix[leaf];
     const uint32_t b0 = row[li], b1 = row[li + 1];
-    L = a.g.lpool + ws + b0;
-    len = b1 - b0;
+    out.L = a.g.lpool + ws + b0;
+    out.len = b1 - b0;
     loads += 2;
   }
-  const uint32_t lg = 33u - (uint32_t)__builtin_clz(len | 1u);
-  const bool by_f = st == kFReady && (uint64_t)fn * lg < len;
-  if (!by_f && a.leaf_segments) {
-    // scanned with every other lane's list as one segmented array (leaf_scan_segments)
-    scan = true;
-    out.L = L;
-    out.len = len;
-    out.by_f = false;
+  out.by_f = r.st == kFReady && search_f(r.fn, out.len);
+  if (out.by_f || (!a.leaf_segments && out.len > a.lane_work)) {
+    defer = true;
     return 0;
   }
-  const uint32_t work = by_f ? fn * lg : len;
-  if (work > a.lane_work) {
-    defer = true;
-    out.L = L;
-    out.len = len;
-    out.by_f = by_f;
+  if (a.leaf_segments) {
+    scan = true;
     return 0;
   }
   uint32_t c = 0;
-  if (by_f) {
-    for (uint32_t k = 0; k < fn; k++) {
-      const uint32_t x = M.fbuf[k];
-      c += (!(injw && x == w) && contains(L, len, x)) ? 1u : 0u;
-    }
-    loads += fn * lg;
-  } else {
-    for (uint32_t k = 0; k < len; k++) c += leaf_accept(S, a, M, leaf, st, fn, injw, w, L[k]) ? 1u : 0u;
-    scanned += len;
-  }
+  for (uint32_t k = 0; k < out.len; k++) c += leaf_accept_one(M, a, r, w, out.L[k]) ? 1u : 0u;
+  scanned += out.len;
   return c;
 }
 
 // The lists of the lanes with `has`, scanned as one segmented array: entry k
-// of the concatenation is read by lane k mod 64, which finds the list it falls
-// in by a binary search over the lanes' exclusive prefix sums (shuffles). Short
-// lists thus share each 64-entry step instead of keeping their lanes in a
-// serial loop, and consecutive entries of a list are read by consecutive
-// lanes. Returns this lane's share of the count (the task sums the wave).
+// of the concatenation is read by lane k mod 64. Short lists thus share each
+// 64-entry step instead of keeping their lanes in a serial loop, and
+// consecutive entries of a list are read by consecutive lanes. Four steps are
+// taken at a time, their reads in flight together. The lists that are not empty
+// sit in the window buffer (where its entry 0 would be, and w); the list of an
+// entry is the number of list starts at or before it, from a bit mask of the
+// starts in its step. Returns this lane's share of the count (the task sums the
+// wave).
+//
+// Bound by the latency of the reads and of the LDS steps between them: a step of
+// 64 entries took 2,460 cycles one at a time, with the list found by a binary
+// search over shuffles, and was 27% of the search (1M vertices, 64 queries). With
+// it, the bit tables, searches four at a time and the DPP scans, the waves' time
+// on tasks fell from 19.4 to 15.2 s per launch at 2,048 waves.
 __device__ __forceinline__ uint32_t leaf_scan_segments(const WaveMem &M, const DfsArgs &a, uint32_t leaf, uint32_t w,
                                                        bool has, const LeafList &ll, uint32_t &scanned) {
-  const WaveHdr &S = *M.h;
+  constexpr int K = 4;
   const uint32_t lane = lane_id();
-  const bool injw = (S.inj[leaf] >> (leaf - 1)) & 1;
-  const uint32_t st = S.fstate, fn = S.fn;
   const uint32_t n = has ? ll.len : 0u;
-  uint32_t incl = n;
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(incl, o);
-    if (lane >= (uint32_t)o) incl += y;
+  const uint64_t lists = ballot(n > 0);
+  if (lists == 0) return 0;
+  uint32_t total;
+  const uint32_t excl = wave_excl_sum(n, &total);
+  const LeafRule r = leaf_rule(*M.h, leaf);
+  uint4 *seg = reinterpret_cast<uint4 *>(M.win);  // [64]
+  wave_sync();
+  if (n > 0) {
+    const unsigned long long p = (unsigned long long)ll.L - 4ull * excl;
+    seg[mbcnt(lists)] = uint4{(uint32_t)p, (uint32_t)(p >> 32), w, 0};
   }
-  const uint32_t total = __shfl(incl, 63);
-  const uint32_t excl = incl - n;
-  const unsigned long long lp = has ? (unsigned long long)ll.L : 0ull;
-  uint32_t c = 0;
-  for (uint32_t base = 0; base < total; base += 64) {
-    const uint32_t k = base + lane;
-    // the owner is the last lane whose list starts at or before k
-    uint32_t o = 0;
-    for (uint32_t step = 32; step; step >>= 1) {
-      const uint32_t cand = o + step;
-      if (__shfl(excl, (int)cand) <= k) o = cand;
+  wave_sync();
+  uint32_t c = 0, before = 0;  // list starts before the step
+  for (uint32_t base = 0; base < total; base += 64 * K) {
+    uint32_t li[K], wo[K], y[K];
+    bool ok[K];
+    const uint32_t at = excl - base;
+    if (ballot(n > 0 && at < 64 * K) == 0) {
+      // one list goes through all steps
+#pragma unroll
+      for (int u = 0; u < K; u++) li[u] = before - 1;
+    } else {
+#pragma unroll
+      for (int u = 0; u < K; u++) {
+        const uint32_t q = at - 64 * u;
+        const uint32_t lo = wave_or(n > 0 && q < 32 ? 1u << q : 0u);
+        const uint32_t hi = wave_or(n > 0 && q >= 32 && q < 64 ? 1u << (q - 32) : 0u);
+        const uint64_t starts = (uint64_t)hi << 32 | lo;
+        // starts at or before this lane's entry
+        li[u] = before + mbcnt(starts) + (uint32_t)(starts >> lane & 1) - 1;
+        before += (uint32_t)__popcll(starts);
+      }
     }
-    const uint32_t start = __shfl(excl, (int)o);
-    const uint32_t *L = (const uint32_t *)__shfl(lp, (int)o);
-    const uint32_t wo = __shfl(w, (int)o);
-    if (k < total) {
-      c += leaf_accept(S, a, M, leaf, st, fn, injw, wo, L[k - start]) ? 1u : 0u;
-      scanned++;
+#pragma unroll
+    for (int u = 0; u < K; u++) {
+      const uint32_t k = base + 64 * u + lane;
+      const uint4 s = seg[li[u]];
+      const uint32_t *L = reinterpret_cast<const uint32_t *>((unsigned long long)s.y << 32 | s.x);
+      wo[u] = s.z;
+      ok[u] = k < total;
+      y[u] = ok[u] ? L[k] : 0u;
     }
+    c += leaf_accept(M, a, r, wo, y, ok);
   }
+  scanned += n;
+  wave_sync();  // the window buffer is free again
   return c;
 }
 
-// The deferred lanes' lists, one after another, 64 entries (or F elements) at
-// a time across the wave; returns this lane's share of the count.
+// The deferred lanes' lists, one after another, 256 F elements (or list entries)
+// at a time across the wave; returns this lane's share of the count.
 __device__ __forceinline__ uint32_t leaf_count_wave(const WaveMem &M, const DfsArgs &a, uint32_t leaf, uint32_t w,
                                                     bool defer, const LeafList &ll, uint32_t &scanned,
                                                     uint32_t &loads) {
-  const WaveHdr &S = *M.h;
+  constexpr int K = 4;
   const uint32_t lane = lane_id();
-  const bool injw = (S.inj[leaf] >> (leaf - 1)) & 1;
-  const uint32_t st = S.fstate, fn = S.fn;
   uint32_t c = 0;
   uint64_t dm = ballot(defer);
+  if (dm == 0) return 0;
+  const LeafRule r = leaf_rule(*M.h, leaf);
+  const uint32_t llo = (uint32_t)(unsigned long long)ll.L, lhi = (uint32_t)((unsigned long long)ll.L >> 32);
   while (dm) {
-    const int src = (int)__builtin_ctzll(dm);
+    const uint32_t src = (uint32_t)__builtin_ctzll(dm);
     dm &= dm - 1;
-    const uint32_t *L = (const uint32_t *)__shfl((unsigned long long)ll.L, src);
-    const uint32_t len = __shfl(ll.len, src);
-    const uint32_t ww = __shfl(w, src);
-    const bool by_f = __shfl((uint32_t)ll.by_f, src) != 0;
+    const uint32_t *L = reinterpret_cast<const uint32_t *>(
+        (unsigned long long)__builtin_amdgcn_readlane(lhi, src) << 32 | (uint32_t)__builtin_amdgcn_readlane(llo, src));
+    const uint32_t len = __builtin_amdgcn_readlane(ll.len, src);
+    const uint32_t ww = __builtin_amdgcn_readlane(w, src);
+    const bool by_f = __builtin_amdgcn_readlane((uint32_t)ll.by_f, src) != 0;
     if (by_f) {
-      const uint32_t lg = 33u - (uint32_t)__builtin_clz(len | 1u);
-      for (uint32_t k = lane; k < fn; k += 64) {
-        const uint32_t x = M.fbuf[k];
-        c += (!(injw && x == ww) && contains(L, len, x)) ? 1u : 0u;
-        loads += lg;
+      for (uint32_t k0 = 0; k0 < r.fn; k0 += 64 * K) {
+        uint32_t x[K];
+        bool in[K];
+#pragma unroll
+        for (int u = 0; u < K; u++) x[u] = k0 + 64 * u + lane < r.fn ? M.fbuf[k0 + 64 * u + lane] : 0xFFFFFFFFu;
+        contains_each(L, len, x, in);
+#pragma unroll
+        for (int u = 0; u < K; u++) c += in[u] && !(r.injw && x[u] == ww) ? 1u : 0u;
       }
+      for (uint32_t k = lane; k < r.fn; k += 64) loads += search_reads(len);
     } else {
       for (uint32_t k = lane; k < len; k += 64) {
-        c += leaf_accept(S, a, M, leaf, st, fn, injw, ww, L[k]) ? 1u : 0u;
+        c += leaf_accept_one(M, a, r, ww, L[k]) ? 1u : 0u;
         scanned++;
       }
     }
@@ -1699,25 +1798,34 @@ __device__ __forceinline__ bool wait_for_task(const DfsArgs &a, const Crew &cr, 
   }
 }
 
+// Bound by latency: dependent scattered reads and LDS steps, on few waves. What
+// counts is how many waves fit. Registers: the wave's index is made uniform, so
+// that its LDS addresses live in scalar registers (135 -> 96 vector registers; at
+// most 128 leave room for the 16-wave blocks of an update beside three blocks
+// per CU, which otherwise wait for the round to end). LDS: 10.3 KB a wave with a
+// leaf set of 1,024 entries, three blocks of four waves per CU beside an update;
+// 14.3 KB, two blocks, with 2,048. Per launch (1M vertices, 64 queries, batches
+// of 4,096, beside the update): 8.1 ms at two blocks, 6.1 at three, 5.9 at four
+// (a 512-entry leaf set), where the update falls behind.
 template <int WPB, bool TUP>
-__global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_levels) {
+__global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_levels) {
   extern __shared__ __align__(16) uint8_t s_dyn[];
   const uint32_t lane = lane_id();
+  const uint32_t wv = bcast(threadIdx.x >> 6);
   WaveMem M;
   {
-    uint8_t *base = s_dyn + (threadIdx.x >> 6) * wave_lds_bytes(chunk_levels);
+    uint8_t *base = s_dyn + wv * wave_lds_bytes(chunk_levels);
     M.h = reinterpret_cast<WaveHdr *>(base);
     M.win = reinterpret_cast<uint32_t *>(base + (sizeof(WaveHdr) + 15) / 16 * 16);
     M.cand = M.win + kWin;
     M.cst = M.cand + chunk_levels * 64;
     M.cdg = M.cst + chunk_levels * 64;
     M.fbuf = M.cdg + chunk_levels * 64;
-    M.fidx = reinterpret_cast<uint16_t *>(M.fbuf + kFCap);
+    M.ftab = M.fbuf + kFCap;
   }
   WaveHdr &S = *M.h;
   if (lane == 0) S.plan = 0xFFFFFFFFu;
   wave_sync();
-  const uint32_t wv = threadIdx.x >> 6;
   // what the block's waves did, for its record
   __shared__ unsigned long long s_rec[WPB][7];
   Crew cr;
@@ -1732,36 +1840,43 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
   // With fewer seeds than waves, every seed is cut into `parts` shares of its
   // first level's source range, so that the grid starts with work for all
   // instead of spreading it by halves (100,000 vertices, 4 queries, batches of
-  // 256, about 30 seeds a launch: 230 -> 96 us, with the waiting words). A wave's first share is the one of its
-  // own index; the rest are claimed from a counter. A share whose wave has not
-  // started (nothing guarantees that every block is resident at once) keeps
-  // nobody waiting: waves that have started end without it, and its own wave
-  // does it when it starts.
+  // 256, about 30 seeds a launch: 230 -> 96 us, with the waiting words).
+  // Shares are claimed, never assigned by wave index: the grid is sized to what
+  // the occupancy query says fits, but nothing guarantees that every block is
+  // resident at once (an update may run beside the round). They are claimed from
+  // kSeedHeads counters, a wave starting at one of its own, so that the grid's
+  // first claims do not queue up on one line. With more shares than waves a wave
+  // whose counter has run out moves on to one that has not.
   const uint32_t parts = nseeds && nseeds < cr.nwaves ? min(cr.nwaves / nseeds, kMaxParts) : 1u;
   const uint32_t total = nseeds * parts;
-  uint32_t first = cr.me;
-  bool seeds_left = total > cr.nwaves;
+  uint32_t head = cr.me % kSeedHeads;
+  bool seeds_left = total > 0;
   uint32_t seen = 0;  // mail taken so far
   if (lane == 0) {
     seen = ld_relaxed(&a.mail[cr.me].mail);
-    if (first < total) atomicOr(&a.idle[cr.me % cr.ngroups].v, 1ull << (cr.me / cr.ngroups + kIdleGroup));
+    if (seeds_left) atomicOr(&a.idle[cr.me % cr.ngroups].v, 1ull << (cr.me / cr.ngroups + kIdleGroup));
   }
   seen = bcast(seen);
   uint64_t busy = 0;            // wall-clock ticks spent on tasks
   uint64_t first_t = 0, last_t = 0;  // start of the first task, end of the last
-  uint64_t wscanned = 0, wloads = 0, wmbytes = 0;  // work of all its tasks
+  if (lane < 7) s_rec[wv][lane] = 0;
   for (;;) {
     uint32_t got = 0, slot = 0;
     if (total == 0) break;
-    if (first < total) {
-      got = 2;
-      slot = first;
-      first = 0xFFFFFFFFu;
-    } else if (seeds_left) {
-      if (lane == 0) slot = cr.nwaves + atomicAdd(&a.ctl->seed_head.v, 1u);
+    while (seeds_left) {
+      if (lane == 0) slot = head + kSeedHeads * atomicAdd(&a.ctl->seed_head[head].v, 1u);
       slot = bcast(slot);
-      if (slot < total) got = 2;
-      else seeds_left = false;
+      if (slot < total) {
+        got = 2;
+        break;
+      }
+      uint64_t open = 0;
+      if (total > cr.nwaves) {
+        const uint32_t h = lane % kSeedHeads;
+        open = ballot(lane < kSeedHeads && h + kSeedHeads * ld_relaxed(&a.ctl->seed_head[h].v) < total);
+      }
+      if (open == 0) seeds_left = false;
+      else head = (uint32_t)__builtin_ctzll(open >> head ? open >> head << head : open);
     }
     if (!got) {
       if (!wait_for_task(a, cr, seen)) break;
@@ -1931,12 +2046,8 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
             // inline work of the lanes up to this one; the first lane past the
             // budget descends, the lanes after it are tested again later
             uint32_t wk = 0;
-            if (scan || defer) wk = ll.by_f ? S.fn * (33u - (uint32_t)__builtin_clz(ll.len | 1u)) : ll.len;
-            uint32_t incl = wk;
-            for (int o = 1; o < 64; o <<= 1) {
-              const uint32_t y = __shfl_up(incl, o);
-              if (lane >= (uint32_t)o) incl += y;
-            }
+            if (scan || defer) wk = ll.by_f ? S.fn * search_reads(ll.len) : ll.len;
+            const uint32_t incl = wave_incl_sum(wk);
             const uint64_t dm = ballot(wk > 0 && incl > a.leaf_budget);
             const uint32_t k0 = dm ? (uint32_t)__builtin_ctzll(dm) : 64u;
             if (lane >= k0) {
@@ -1950,7 +2061,7 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
             lcount += leaf_count_wave(M, a, l + 1, w, defer, ll, scanned, loads);
             if (dm) {
               // lane k0's candidate as a one-entry chunk at source index p + k0
-              const uint32_t w0 = __shfl(w, (int)k0);
+              const uint32_t w0 = __builtin_amdgcn_readlane(w, k0);
               wave_sync();
               if (lane == 0) {
                 const uint32_t c = (l - 2) * 64;
@@ -2015,23 +2126,17 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
         l--;
       }
     }
-    // wave sum of the lane counts
-    uint64_t tot = lcount;
-    uint64_t sc = scanned, ld = loads, mb = mbytes;
-    for (int off = 32; off >= 1; off >>= 1) {
-      tot += __shfl_xor(tot, off);
-      sc += __shfl_xor(sc, off);
-      ld += __shfl_xor(ld, off);
-      mb += __shfl_xor(mb, off);
-    }
-    if (lane == 0) {
+    const uint64_t tot = wave_sum(lcount);
+    if (lane == 0 && tot) {
       const uint32_t tg = S.tag;
-      if (tot)
-        atomicAdd(&a.counts[((size_t)(tg >> 1) * a.nq + S.query) * 2 + (tg & 1)], (unsigned long long)tot);
+      atomicAdd(&a.counts[((size_t)(tg >> 1) * a.nq + S.query) * 2 + (tg & 1)], (unsigned long long)tot);
     }
-    wscanned += sc;
-    wloads += ld;
-    wmbytes += mb;
+    const uint64_t sc = wave_sum(scanned), ld = wave_sum(loads), mb = wave_sum(mbytes);
+    if (lane == 0) {
+      s_rec[wv][4] += sc;
+      s_rec[wv][5] += ld;
+      s_rec[wv][6] += mb;
+    }
     last_t = wall_clock64();
     busy += last_t - t_task;
     if (a.query_busy && lane == 0) atomicAdd(&a.query_busy[S.query], (unsigned long long)(last_t - t_task));
@@ -2044,9 +2149,6 @@ __global__ __launch_bounds__(WPB * 64) void k_dfs(DfsArgs a, uint32_t chunk_leve
     s_rec[wv][1] = first_t;
     s_rec[wv][2] = last_t;
     s_rec[wv][3] = cr.donated;
-    s_rec[wv][4] = wscanned;
-    s_rec[wv][5] = wloads;
-    s_rec[wv][6] = wmbytes;
   }
   __syncthreads();
   if (wv == 0) {

@@ -104,7 +104,7 @@ typedef struct {
   uint32_t leaf_budget;      /* one level above the leaf: inline leaf-count work (list
                                 entries) of a 64-candidate window before a candidate
                                 descends so that its scan can be shared with idle waves
-                                (0 = 2048; 0xFFFFFFFF = never) */
+                                (0 = 8192; 0xFFFFFFFF = never) */
   int cluster_filter;        /* 1: after every update the candidates are refined by the
                                 cluster encoding of the reference's clusterFilter
                                 (filter.cu:1525-1654: spanning tree, vertex cover,

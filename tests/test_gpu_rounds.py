@@ -62,3 +62,38 @@ def test_watchdog_ends_a_round_whose_waves_wait():
         assert ei.value.code == E.DSM_EDEVICE and "watchdog" in str(ei.value)
     finally:
         eng.close()
+
+
+@pytest.mark.parametrize("da,db", [(5, 5000), (70, 20000), (256, 300), (257, 700), (258, 257), (900, 40000),
+                                   (1024, 1500), (1025, 1026), (1026, 2047), (2048, 2049), (2050, 2051)])
+@pytest.mark.parametrize("labels", [1, 2])
+def test_leaf_sets_at_their_limits(da, db, labels):
+    """Squares between two hubs of da and db neighbours: leaf sets of up to and
+    past 256 entries (bitmap or id buckets), 1,024 (kept or descended) and lists
+    past 2,048 entries; lists short and long enough that the set's elements are
+    searched in them; with the leaf's label that of other positions or not."""
+    rng = np.random.default_rng(da + db)
+    n = max(da, db) + 2
+    xs = np.arange(2, n, dtype=np.uint32)
+    pa, pb = rng.choice(xs, da, replace=False), rng.choice(xs, db, replace=False)
+    extra = rng.choice(xs, (400, 2))
+    u = np.concatenate([np.zeros(da, np.uint32), np.ones(db, np.uint32), extra[:, 0]]).astype(np.uint32)
+    v = np.concatenate([pa, pb, extra[:, 1]]).astype(np.uint32)
+    keep = u != v
+    u, v = u[keep], v[keep]
+    lab = np.zeros(n, np.uint32)
+    lab[2:] = labels - 1
+    sq = np.array([(0, 1), (1, 2), (2, 3), (3, 0)], np.uint32)
+    queries = [(4, np.array([0, labels - 1] * 2, np.uint32), sq[:, 0].copy(), sq[:, 1].copy())]
+    both = np.intersect1d(pa, pb)
+    x = (both if len(both) else pa)[:2].astype(np.uint32)
+    batch = (np.ones(4, np.uint8), np.array([0, 0, 1, 1], np.uint32),
+             np.resize(x, 4).astype(np.uint32), np.zeros(4, np.uint32))
+    want = O.run_stream(O.Graph(n, lab, u, v), [O.Query(*q) for q in queries], [batch], relabel=False)[0]
+    for kw in ({}, {"leaf_segments": False}, {"leaf_budget": 64}):
+        eng = E.Engine((n, lab, u, v), queries, relabel=False, **kw)
+        try:
+            pos, neg = eng.process_batch(*batch)
+            assert pos.tolist() == want["pos"] and neg.tolist() == want["neg"], kw
+        finally:
+            eng.close()
