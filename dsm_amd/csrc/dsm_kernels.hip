@@ -1101,18 +1101,18 @@ struct WaveHdr {
 constexpr uint32_t kFCap = 1024;   // largest leaf set F kept in LDS
 constexpr uint32_t kFScan = 2048;  // longest list it is computed from
 // Membership in F goes through a table beside it, of one of two kinds.
-// - Up to kFBits entries: a bitmap of kFBitWords x 32 bits with the hashed ids of
-//   F set. One read settles almost every id outside F (at most 256 of 8,192 bits
-//   are set); the few left search F. Clearing and setting it costs five LDS
-//   writes a lane.
+// - Up to kFHash entries: a hash set of the ids, kFBuckets buckets of four, a full
+//   bucket going on to the next. One 16-byte read settles almost every id (F has
+//   21 entries in the mean on the 64-query stream, and a bucket a third of one).
 // - More: F indexed by id range: bucket b = id >> DfsArgs::fshift (fshift makes the
 //   graph's ids fit kFIdx buckets), fidx[b] = first entry of F at or past the
 //   bucket. A test reads two offsets and searches the bucket's few entries.
 //   Filling the buckets between two entries is a loop per entry, as long as F is
-//   short, which is why the short sets, nearly all of them, take the bitmap.
+//   short, which is why the short sets, nearly all of them, take the hash set.
 constexpr uint32_t kFIdx = 512;
-constexpr uint32_t kFBits = 256;
-constexpr uint32_t kFBitWords = 256;
+constexpr uint32_t kFHash = 128;
+constexpr uint32_t kFBuckets = 64;
+constexpr uint32_t kFEmpty = 0xFFFFFFFFu;
 // One level above the leaf, the candidates of a 64-entry window count their
 // leaf images inline until their summed scan or search work passes
 // DfsArgs::leaf_budget entries; the candidate that passes it descends to the
@@ -1131,10 +1131,10 @@ struct WaveMem {
   uint32_t *cst;    // [levels][64] list start of each candidate
   uint32_t *cdg;    // [levels][64] degree of each candidate
   uint32_t *fbuf;   // [kFCap] leaf set F, ascending
-  uint32_t *ftab;   // F's table: kFBitWords words of bits, or kFIdx + 1 16-bit bucket offsets into fbuf
+  uint32_t *ftab;   // F's table: kFBuckets x 4 ids, or kFIdx + 1 16-bit bucket offsets into fbuf
 };
 constexpr uint32_t kFTabBytes = ((kFIdx + 1) * 2 + 15) / 16 * 16;
-static_assert(kFBitWords * 4 <= kFTabBytes, "the bits fit the table");
+static_assert(kFBuckets * 16 <= kFTabBytes && kFBuckets == 64, "the hash set fits the table, a bucket per lane");
 
 __host__ __device__ constexpr uint32_t wave_lds_bytes(uint32_t chunk_levels) {
   return (uint32_t)((sizeof(WaveHdr) + 15) / 16 * 16) + kWin * 4 + kFCap * 4 + chunk_levels * 64 * 12 + kFTabBytes;
@@ -1142,14 +1142,10 @@ __host__ __device__ constexpr uint32_t wave_lds_bytes(uint32_t chunk_levels) {
 
 // 4 B per entry of the full lists of the positions in `mask`: what a merge
 // intersection over those lists reads (the work measure of the expansion).
-__device__ __forceinline__ uint64_t list_bytes(const WaveHdr &S, uint32_t mask) {
-  uint64_t b = 0;
-  while (mask) {
-    const uint32_t j = __builtin_ctz(mask);
-    mask &= mask - 1;
-    b += 4ull * S.fd[j];
-  }
-  return b;
+// Lane j's share: position j's list.
+__device__ __forceinline__ uint32_t list_bytes(const WaveHdr &S, uint32_t mask) {
+  const uint32_t lane = lane_id();
+  return lane < (uint32_t)kMaxQ && (mask >> lane & 1) ? 4u * S.fd[lane] : 0u;
 }
 
 // Among the lists of the positions in `mask`, the one with the fewest entries
@@ -1240,8 +1236,8 @@ __device__ __forceinline__ bool test_chunk(const WaveMem &M, const DfsArgs &a, u
   return test_entries(M, a, S.src[l], S.back[l] & ~(1u << S.srcj[l]), S.inj[l], S.sig[l], p, e, w, loads);
 }
 
-// An id's bit in the table of a short leaf set (13 bits, kFBitWords words).
-__device__ __forceinline__ uint32_t f_hash(uint32_t y) { return (y * 0x9E3779B1u) >> 19; }
+// An id's first bucket in the hash set of a short leaf set.
+__device__ __forceinline__ uint32_t f_hash(uint32_t y) { return (y * 0x9E3779B1u) >> 26; }
 
 // Leaf set F for positions 0..n-3 (leaf = n-1): the images the leaf may take
 // judging only by its backward neighbours other than position n-2, i.e. the
@@ -1283,12 +1279,13 @@ __device__ __forceinline__ void compute_leaf_set(const WaveMem &M, const DfsArgs
     }
   }
   wave_sync();
-  if (state == kFReady && cnt <= kFBits) {
-    reinterpret_cast<uint4 *>(M.ftab)[lane] = uint4{0, 0, 0, 0};
+  if (state == kFReady && cnt <= kFHash) {
+    reinterpret_cast<uint4 *>(M.ftab)[lane] = uint4{kFEmpty, kFEmpty, kFEmpty, kFEmpty};
     wave_sync();
     for (uint32_t i = lane; i < cnt; i += 64) {
-      const uint32_t h = f_hash(M.fbuf[i]);
-      atomicOr(&M.ftab[h >> 5], 1u << (h & 31));
+      const uint32_t y = M.fbuf[i];
+      uint32_t at = f_hash(y) * 4;
+      while (atomicCAS(&M.ftab[at], kFEmpty, y) != kFEmpty) at = (at + 1) % (kFBuckets * 4);
     }
   } else if (state == kFReady) {
     // bucket offsets: entry i opens every bucket after its predecessor's up
@@ -1311,11 +1308,19 @@ __device__ __forceinline__ void compute_leaf_set(const WaveMem &M, const DfsArgs
   wave_sync();
 }
 
+// Looks a lane's id y up in bucket h of the hash set. Returns true when that
+// settles it: the bucket holds y (found) or is not full.
+__device__ __forceinline__ bool f_look(const uint4 &t, uint32_t y, bool &found) {
+  found = t.x == y || t.y == y || t.z == y || t.w == y;
+  return found || t.w == kFEmpty;
+}
+
 // y in F (state kFReady, fn entries), through F's table.
 __device__ __forceinline__ bool in_leaf_set(const WaveMem &M, const DfsArgs &a, uint32_t fn, uint32_t y) {
-  if (fn <= kFBits) {
-    const uint32_t h = f_hash(y);
-    return (M.ftab[h >> 5] >> (h & 31) & 1) && lds_contains(M.fbuf, fn, y);
+  if (fn <= kFHash) {
+    bool found;
+    for (uint32_t h = f_hash(y); !f_look(reinterpret_cast<const uint4 *>(M.ftab)[h], y, found);) h = (h + 1) % kFBuckets;
+    return found;
   }
   const uint16_t *fidx = reinterpret_cast<const uint16_t *>(M.ftab);
   const uint32_t b = y >> a.fshift;
@@ -1385,20 +1390,16 @@ __device__ __forceinline__ uint32_t leaf_accept(const WaveMem &M, const DfsArgs 
   const WaveHdr &S = *M.h;
   uint32_t c = 0;
   if (r.st == kFReady) {
-    if (r.fn <= kFBits) {
-      uint32_t t[K];
-      bool any = false;
+    if (r.fn <= kFHash) {
+      uint4 t[K];
 #pragma unroll
-      for (int u = 0; u < K; u++) t[u] = M.ftab[f_hash(y[u]) >> 5];
+      for (int u = 0; u < K; u++) t[u] = reinterpret_cast<const uint4 *>(M.ftab)[f_hash(y[u])];
 #pragma unroll
       for (int u = 0; u < K; u++) {
-        ok[u] = ok[u] && (t[u] >> (f_hash(y[u]) & 31) & 1) && !(r.injw && y[u] == w[u]);
-        any = any || ok[u];
+        bool found;
+        if (!f_look(t[u], y[u], found)) found = in_leaf_set(M, a, r.fn, y[u]);
+        c += ok[u] && found && !(r.injw && y[u] == w[u]) ? 1u : 0u;
       }
-      if (ballot(any) == 0) return 0;
-#pragma unroll
-      for (int u = 0; u < K; u++)
-        if (ballot(ok[u])) c += ok[u] && lds_contains(M.fbuf, r.fn, y[u]) ? 1u : 0u;
     } else {
 #pragma unroll
       for (int u = 0; u < K; u++)
@@ -1437,14 +1438,13 @@ __device__ __forceinline__ uint32_t leaf_count_lane(const WaveMem &M, const DfsA
     if (r.injw && in_leaf_set(M, a, r.fn, w)) c--;
     return c;
   }
-  const uint32_t ws = a.g.start[w], wd = a.g.deg[w];
+  // the bucket offsets are read beside the degree that says whether they count
+  const uint32_t *row = a.g.loff + (size_t)w * (a.g.nbuckets + 1) + S.lix[leaf];
+  const uint32_t ws = a.g.start[w], wd = a.g.deg[w], b0 = row[0], b1 = row[1];
   wdeg = wd;
   out.L = a.g.pool + ws;
   out.len = wd;
   if (wd > kLabelSorted) {
-    const uint32_t *row = a.g.loff + (size_t)w * (a.g.nbuckets + 1);
-    const uint32_t li = S.lix[leaf];
-    const uint32_t b0 = row[li], b1 = row[li + 1];
     out.L = a.g.lpool + ws + b0;
     out.len = b1 - b0;
     loads += 2;
@@ -1477,8 +1477,10 @@ __device__ __forceinline__ uint32_t leaf_count_lane(const WaveMem &M, const DfsA
 // Bound by the latency of the reads and of the LDS steps between them: a step of
 // 64 entries took 2,460 cycles one at a time, with the list found by a binary
 // search over shuffles, and was 27% of the search (1M vertices, 64 queries). With
-// it, the bit tables, searches four at a time and the DPP scans, the waves' time
-// on tasks fell from 19.4 to 15.2 s per launch at 2,048 waves.
+// it, the hash sets, searches four at a time and the DPP scans, the waves' time
+// on tasks fell from 19.4 to 12.5 s per launch at 2,048 waves. Fetching the next
+// four steps ahead of the tests takes 14 more registers and gave 2%; the update
+// beside the round then waits for room, so it is not done.
 __device__ __forceinline__ uint32_t leaf_scan_segments(const WaveMem &M, const DfsArgs &a, uint32_t leaf, uint32_t w,
                                                        bool has, const LeafList &ll, uint32_t &scanned) {
   constexpr int K = 4;
@@ -1524,7 +1526,7 @@ __device__ __forceinline__ uint32_t leaf_scan_segments(const WaveMem &M, const D
       const uint32_t *L = reinterpret_cast<const uint32_t *>((unsigned long long)s.y << 32 | s.x);
       wo[u] = s.z;
       ok[u] = k < total;
-      y[u] = ok[u] ? L[k] : 0u;
+      y[u] = L[ok[u] ? k : total - 1];
     }
     c += leaf_accept(M, a, r, wo, y, ok);
   }
@@ -1806,7 +1808,8 @@ __device__ __forceinline__ bool wait_for_task(const DfsArgs &a, const Crew &cr, 
 // leaf set of 1,024 entries, three blocks of four waves per CU beside an update;
 // 14.3 KB, two blocks, with 2,048. Per launch (1M vertices, 64 queries, batches
 // of 4,096, beside the update): 8.1 ms at two blocks, 6.1 at three, 5.9 at four
-// (a 512-entry leaf set), where the update falls behind.
+// (a 512-entry leaf set), where the update falls behind; 5.6 at three with hash
+// sets for the short leaf sets.
 template <int WPB, bool TUP>
 __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_levels) {
   extern __shared__ __align__(16) uint8_t s_dyn[];
@@ -1938,7 +1941,7 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
     } else {
       // a seed expands its partial match here; a donated task continues one
       // whose expansion the donor counted
-      if (got == 2 && lane == 0 && part == 0) mbytes += list_bytes(S, S.back[L0]);
+      if (got == 2 && part == 0) mbytes += list_bytes(S, S.back[L0]);
       init_level(S, a.g, L0, lo, hi);
       if (got == 2 && parts > 1) {
         // the share of the source range, in pieces of what a hand-off is worth:
@@ -2005,7 +2008,7 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
           }
           wave_sync();
           l++;
-          mbytes += lane == 0 ? list_bytes(S, S.back[l]) : 0ull;
+          mbytes += list_bytes(S, S.back[l]);
           init_level(S, a.g, l, 0, 0xFFFFFFFFu);
           continue;
         }
@@ -2033,7 +2036,7 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
             if (bcast(S.fstate) == kFStale) compute_leaf_set(M, a, l + 1, scanned, loads);
             // backward lists of the leaf other than position n-2, read by a
             // merge for every candidate of this level
-            const uint64_t fixed_leaf_bytes = list_bytes(S, S.back[l + 1] & ~(1u << l));
+            const uint64_t fixed_leaf_bytes = list_bytes(S, S.back[l + 1] & ~(1u << l));  // this lane's share
             if (bcast(S.fstate) == kFLarge) {
               // this chunk and the rest of the level take the descent path
               large = true;
@@ -2054,8 +2057,9 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
               lc = 0;
               scan = defer = false;
             } else if (ok) {
-              mbytes += fixed_leaf_bytes + 4ull * wdeg;
+              mbytes += 4ull * wdeg;
             }
+            mbytes += fixed_leaf_bytes * (uint32_t)__popcll(ballot(ok && lane < k0));
             lcount += lc;
             if (a.leaf_segments) lcount += leaf_scan_segments(M, a, l + 1, w, scan, ll, scanned);
             lcount += leaf_count_wave(M, a, l + 1, w, defer, ll, scanned, loads);

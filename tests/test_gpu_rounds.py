@@ -64,12 +64,12 @@ def test_watchdog_ends_a_round_whose_waves_wait():
         eng.close()
 
 
-@pytest.mark.parametrize("da,db", [(5, 5000), (70, 20000), (256, 300), (257, 700), (258, 257), (900, 40000),
+@pytest.mark.parametrize("da,db", [(5, 5000), (70, 20000), (128, 300), (129, 700), (130, 131), (900, 40000),
                                    (1024, 1500), (1025, 1026), (1026, 2047), (2048, 2049), (2050, 2051)])
 @pytest.mark.parametrize("labels", [1, 2])
 def test_leaf_sets_at_their_limits(da, db, labels):
     """Squares between two hubs of da and db neighbours: leaf sets of up to and
-    past 256 entries (bitmap or id buckets), 1,024 (kept or descended) and lists
+    past 128 entries (hash set or id ranges), 1,024 (kept or descended) and lists
     past 2,048 entries; lists short and long enough that the set's elements are
     searched in them; with the leaf's label that of other positions or not."""
     rng = np.random.default_rng(da + db)
