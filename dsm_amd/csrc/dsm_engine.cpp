@@ -181,8 +181,11 @@ struct dsm_engine {
   DevBuf<uint32_t> scratch;
   unsigned long long scratch_cap = 0;
   DevBuf<uint32_t> dirty_bits, dirty_list, heavy_list;
-  DevBuf<uint32_t> bbuf;              // batch arrays (device)
-  PinnedBuf<uint32_t> hbuf;           // batch arrays (pinned staging)
+  DevBuf<uint32_t> bbuf;              // an update's arrays (device)
+  PinnedBuf<uint32_t> hbuf;           // the same (pinned staging)
+  PinnedBuf<uint32_t> hrec;           // a round's records (pinned staging)
+  // the copies out of hbuf / hrec: done before either is filled again
+  hipEvent_t ev_hbuf = nullptr, ev_hrec = nullptr;
   DevBuf<uint32_t> ndeg, fail;
   DevBuf<unsigned long long> soff;
   DevBuf<ApplyCtl> actl;
@@ -195,9 +198,14 @@ struct dsm_engine {
   uint32_t epoch = 0;            // of the last DFS launch
   DevBuf<uint32_t> seed_plan, seed_s, seed_d, seed_tag;
   uint32_t seed_cap = 0;
-  DevBuf<unsigned long long> counts;
-  PinnedBuf<unsigned long long> h_counts;
-  DevBuf<unsigned long long> tuple_count;
+  // the tuple counter, then the match counts; both are cleared by the reset of
+  // the round that follows counts_stale
+  DevBuf<unsigned long long> results;
+  PinnedBuf<unsigned long long> h_results;
+  unsigned long long *tuple_count() { return results.p; }
+  unsigned long long *counts() { return results.p + 1; }
+  unsigned long long *h_counts() { return h_results.p + 1; }
+  bool counts_stale = false;
   uint32_t *tuples = nullptr;
   bool tuples_host = false;
   unsigned long long tuple_cap = 0;
@@ -230,7 +238,7 @@ struct dsm_engine {
   bool shadow_delta_ok = false;
   bool grew = false;  // the pool grew during the update being applied
   std::vector<uint32_t> last_touched, last_relabel;
-  DevBuf<uint32_t> d_last_touched, d_last_relabel, sync_q, sync_ctl;
+  DevBuf<uint32_t> sync_q;
   int cu_lds = 160 * 1024;   // LDS bytes per CU
   DevBuf<unsigned long long> query_busy;  // per query: DFS task ticks since the last read
   uint32_t wave_slots = 0;       // waves of the largest grid
@@ -238,7 +246,7 @@ struct dsm_engine {
   // the DFS round as a HIP graph (graph_round)
   hipGraph_t rg_graph = nullptr;
   hipGraphExec_t rg_exec = nullptr;
-  hipGraphNode_t rg_reset = nullptr, rg_seed0 = nullptr, rg_seed1 = nullptr, rg_dfs = nullptr;
+  hipGraphNode_t rg_reset = nullptr, rg_seed = nullptr, rg_dfs = nullptr;
   uint32_t rg_key = 0;
   uint32_t watchdog_ms = 60000;
   int wall_khz = 100000;
@@ -275,7 +283,8 @@ struct dsm_engine {
       if (tuples_host) (void)hipHostFree(tuples);
       else (void)hipFree(tuples);
     }
-    if (ev_pre) (void)hipEventDestroy(ev_pre);
+    for (hipEvent_t x : {ev_pre, ev_hbuf, ev_hrec})
+      if (x) (void)hipEventDestroy(x);
     if (stream2) (void)hipStreamDestroy(stream2);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -328,6 +337,7 @@ struct dsm_engine {
     // the merge scratch (at least one entry per pool entry) is idle while the
     // label-sorted copies are rebuilt
     h.bucket_bytes = scratch_cap >= pool_cap ? reinterpret_cast<uint8_t *>(scratch.p) : nullptr;
+    h.actl = actl.p;
     return h;
   }
   DirtyArgs dirty() {
@@ -716,6 +726,7 @@ int upload_graph(dsm_engine *e, const dsm_graph_desc *g) {
   HIPCHK(e->h_actl.ensure(1));
   ApplyCtl a0{};
   a0.pool_used = total;
+  a0.max_deg = n ? *std::max_element(dg.begin(), dg.end()) : 0;
   HIPCHK(hipMemcpy(e->actl.p, &a0, sizeof a0, hipMemcpyHostToDevice));
   *e->h_actl.p = a0;
   HIPCHK(e->dirty_bits.alloc((n + 31) / 32));
@@ -744,12 +755,11 @@ int upload_tables(dsm_engine *e) {
   HIPCHK(e->d_plan_key.alloc(e->plan_key.size()));
   HIPCHK(hipMemcpy(e->d_plan_key.p, e->plan_key.data(), e->plan_key.size() * 4, hipMemcpyHostToDevice));
   const uint32_t nq = (uint32_t)e->queries.size();
-  HIPCHK(e->counts.alloc((size_t)nq * 2 * kMaxSlots));
+  HIPCHK(e->results.alloc((size_t)nq * 2 * kMaxSlots + 1));
   HIPCHK(e->query_busy.alloc(nq));
   HIPCHK(hipMemset(e->query_busy.p, 0, (size_t)nq * 8));
-  HIPCHK(e->h_counts.ensure((size_t)nq * 2 * kMaxSlots));
+  HIPCHK(e->h_results.ensure((size_t)nq * 2 * kMaxSlots + 1));
   HIPCHK(e->ctl.alloc(1));
-  HIPCHK(e->tuple_count.alloc(1));
   if (e->opt.tuple_capacity) {
     e->tuple_cap = e->opt.tuple_capacity;
     size_t bytes = (size_t)e->tuple_cap * (kMaxQ + 2) * 4;
@@ -782,16 +792,20 @@ int ensure_seed_cap(dsm_engine *e, uint32_t nrec) {
   return DSM_OK;
 }
 
-// A DFS round: reset the control block, seed up to two record lists (each
-// with its count tag, slot << 1 | sign), one persistent DFS launch over all
-// their seeds, and a copy of the control block to the host. The seed table
-// must hold the seeds of every list.
+// A DFS round: reset the control block (and the results with counts_stale, or
+// a count slot), seed up to two record lists (each with its count tag, slot << 1
+// | sign), one persistent DFS launch over all their seeds. The seed table must
+// hold the seeds of both lists.
 struct RoundPart {
   const uint32_t *rs, *rd;
   uint32_t n, tag;
 };
+struct ClearSpan {
+  unsigned long long *tuple_count, *counts;
+  uint32_t ncounts;
+};
 
-SeedArgs seed_args(dsm_engine *e, const RoundPart &p) {
+SeedArgs seed_args(dsm_engine *e, const RoundPart *parts, int nparts) {
   SeedArgs sa;
   sa.g = e->dev_graph();
   sa.bm = e->bm.p;
@@ -799,15 +813,17 @@ SeedArgs seed_args(dsm_engine *e, const RoundPart &p) {
   sa.plans = e->d_plans.p;
   sa.plan_key = e->d_plan_key.p;
   sa.nplans = (uint32_t)e->plans.size();
-  sa.rs = p.rs;
-  sa.rd = p.rd;
-  sa.nrec = p.n;
+  for (int i = 0; i < 2; i++) {
+    sa.rs[i] = i < nparts ? parts[i].rs : nullptr;
+    sa.rd[i] = i < nparts ? parts[i].rd : nullptr;
+    sa.nrec[i] = i < nparts ? parts[i].n : 0;
+    sa.tag[i] = i < nparts ? parts[i].tag : 0;
+  }
   sa.seed_plan = e->seed_plan.p;
   sa.seed_s = e->seed_s.p;
   sa.seed_d = e->seed_d.p;
   sa.seed_tag = e->seed_tag.p;
   sa.seed_cap = e->seed_cap;
-  sa.tag = p.tag;
   sa.ctl = e->ctl.p;
   return sa;
 }
@@ -840,10 +856,10 @@ DfsArgs dfs_args(dsm_engine *e) {
   da.nq = (uint32_t)e->queries.size();
   da.watchdog = (unsigned long long)e->wall_khz * e->watchdog_ms;
   da.ctl = e->ctl.p;
-  da.counts = e->counts.p;
+  da.counts = e->counts();
   da.tuples = e->tuples;
   da.tuple_cap = e->tuple_cap;
-  da.tuple_count = e->tuple_count.p;
+  da.tuple_count = e->tuple_count();
   da.rec = e->h_rec.p;
   da.query_busy = e->query_busy.p;
   return da;
@@ -877,36 +893,36 @@ void cap_donations(dsm_engine *e, DfsArgs &da) {
   if (e->opt.queue_capacity) da.donate_cap = e->opt.queue_capacity / (e->last_blocks * e->last_wpb);
 }
 
-// The round as one HIP graph: ctl reset -> seed list 0 -> seed list 1 -> DFS,
-// whose blocks write their records to pinned host memory. Built once per launch shape (waves per block,
+// The round as one HIP graph: reset -> seeding -> DFS, whose blocks write their
+// records to pinned host memory. Built once per launch shape (waves per block,
 // tuples or not); every later round updates the kernel nodes' arguments and
 // grids in the executable graph and launches it.
-int graph_round(dsm_engine *e, const RoundPart *parts, int nparts, uint32_t nrec) {
+int graph_round(dsm_engine *e, const RoundPart *parts, int nparts, uint32_t nrec, const ClearSpan &clear) {
   RoundNodeArgs st;
   st.ctl = e->ctl.p;
-  const RoundPart none{nullptr, nullptr, 0, 0};
-  st.seed[0] = seed_args(e, nparts > 0 ? parts[0] : none);
-  st.seed[1] = seed_args(e, nparts > 1 ? parts[1] : none);
+  st.tuple_count = clear.tuple_count;
+  st.counts = clear.counts;
+  st.ncounts = clear.ncounts;
+  st.seed = seed_args(e, parts, nparts);
   st.dfs = dfs_args(e);
-  hipKernelNodeParams pr, p0, p1, pd;
+  hipKernelNodeParams pr, ps, pd;
   const uint32_t blocks = dfs_grid(e, nrec);
   cap_donations(e, st.dfs);
   st.idle = e->idle.p;
-  st.nidle = idle_words(e->wave_slots);
-  round_node_params(st, blocks, e->dfs_wpb, e->max_qn, &pr, &p0, &p1, &pd);
+  st.nidle = idle_words(e->last_blocks * e->last_wpb);
+  round_node_params(st, blocks, e->dfs_wpb, e->max_qn, &pr, &ps, &pd);
   const uint32_t key = (e->tuples ? 16u : 0u) | e->dfs_wpb;
   if (!e->rg_exec || e->rg_key != key) {
     drop_round_graph(e);
     HIPCHK(hipGraphCreate(&e->rg_graph, 0));
     HIPCHK(hipGraphAddKernelNode(&e->rg_reset, e->rg_graph, nullptr, 0, &pr));
-    HIPCHK(hipGraphAddKernelNode(&e->rg_seed0, e->rg_graph, &e->rg_reset, 1, &p0));
-    HIPCHK(hipGraphAddKernelNode(&e->rg_seed1, e->rg_graph, &e->rg_seed0, 1, &p1));
-    HIPCHK(hipGraphAddKernelNode(&e->rg_dfs, e->rg_graph, &e->rg_seed1, 1, &pd));
+    HIPCHK(hipGraphAddKernelNode(&e->rg_seed, e->rg_graph, &e->rg_reset, 1, &ps));
+    HIPCHK(hipGraphAddKernelNode(&e->rg_dfs, e->rg_graph, &e->rg_seed, 1, &pd));
     HIPCHK(hipGraphInstantiate(&e->rg_exec, e->rg_graph, nullptr, nullptr, 0));
     e->rg_key = key;
   } else {
-    HIPCHK(hipGraphExecKernelNodeSetParams(e->rg_exec, e->rg_seed0, &p0));
-    HIPCHK(hipGraphExecKernelNodeSetParams(e->rg_exec, e->rg_seed1, &p1));
+    HIPCHK(hipGraphExecKernelNodeSetParams(e->rg_exec, e->rg_reset, &pr));
+    HIPCHK(hipGraphExecKernelNodeSetParams(e->rg_exec, e->rg_seed, &ps));
     HIPCHK(hipGraphExecKernelNodeSetParams(e->rg_exec, e->rg_dfs, &pd));
   }
   HIPCHK(hipGraphLaunch(e->rg_exec, e->stream));
@@ -917,25 +933,39 @@ int graph_round(dsm_engine *e, const RoundPart *parts, int nparts, uint32_t nrec
 // the end of seeding (eager only; a graph round records ev1 at its start) and
 // its end.
 int dfs_round(dsm_engine *e, const RoundPart *parts, int nparts, hipEvent_t ev0, hipEvent_t ev1,
-              hipEvent_t ev2) {
+              hipEvent_t ev2, ClearSpan clear = {}) {
   uint32_t nrec = 0;
   for (int i = 0; i < nparts; i++) nrec += parts[i].n;
+  if (e->counts_stale) {
+    clear = ClearSpan{e->tuple_count(), e->counts(), (uint32_t)e->queries.size() * 2};
+    e->counts_stale = false;
+  }
   if (ev0) HIPCHK(hipEventRecord(ev0, e->stream));
   if (e->graph_rounds) {
     if (ev1) HIPCHK(hipEventRecord(ev1, e->stream));
-    int rc = graph_round(e, parts, nparts, nrec);
+    int rc = graph_round(e, parts, nparts, nrec, clear);
     if (rc) return rc;
   } else {
-    HIPCHK(launch_ctl_reset(e->ctl.p, nullptr, nullptr, nullptr, 0, e->idle.p, idle_words(e->wave_slots), e->stream));
-    for (int i = 0; i < nparts; i++)
-      if (parts[i].n) HIPCHK(launch_seed(seed_args(e, parts[i]), e->stream));
-    if (ev1) HIPCHK(hipEventRecord(ev1, e->stream));
     DfsArgs da = dfs_args(e);
     const uint32_t blocks = dfs_grid(e, nrec);
     cap_donations(e, da);
+    HIPCHK(launch_ctl_reset(e->ctl.p, clear.tuple_count, clear.counts, clear.ncounts, e->idle.p,
+                            idle_words(e->last_blocks * e->last_wpb), e->stream));
+    HIPCHK(launch_seed(seed_args(e, parts, nparts), e->stream));
+    if (ev1) HIPCHK(hipEventRecord(ev1, e->stream));
     HIPCHK(launch_dfs(da, blocks, e->dfs_wpb, e->max_qn, e->stream));
   }
   if (ev2) HIPCHK(hipEventRecord(ev2, e->stream));
+  return DSM_OK;
+}
+
+// The tuple counter and the counts of slot 0 to the host; waits for the stream.
+int fetch_results(dsm_engine *e) {
+  const uint32_t n = (uint32_t)e->queries.size() * 2;
+  if (e->counts_stale) HIPCHK(launch_ctl_reset(nullptr, e->tuple_count(), e->counts(), n, nullptr, 0, e->stream));
+  e->counts_stale = false;
+  HIPCHK(hipMemcpyAsync(e->h_results.p, e->results.p, (size_t)(n + 1) * 8, hipMemcpyDeviceToHost, e->stream));
+  HIPCHK(hipStreamSynchronize(e->stream));
   return DSM_OK;
 }
 
@@ -1044,44 +1074,57 @@ void host_delta(const dsm_engine *e, const dsm_change *ch, uint32_t k, HostDelta
   }
 }
 
-// Uploads one apply round (a slice of every touched vertex's lists) and runs
-// merge + commit. Grows the pool when a commit found no room.
 int grow_pool(dsm_engine *e, unsigned long long extra);
 
-int apply_round(dsm_engine *e, const HostDelta &d, const std::vector<uint32_t> &tv,
-                const std::vector<uint32_t> &ioff, const std::vector<uint32_t> &doff,
-                const std::vector<uint32_t> &ins, const std::vector<uint32_t> &del) {
-  const uint32_t T = (uint32_t)tv.size();
-  if (T == 0) return DSM_OK;
-  (void)d;
-  // layout: tv | ioff | doff | ins | del
-  const size_t o_tv = 0, o_io = o_tv + T, o_do = o_io + T + 1, o_in = o_do + T + 1, o_de = o_in + ins.size();
-  const size_t total = o_de + del.size();
-  // device-only space after the uploaded part: prefix counts and big-list
-  // indices of the hub lists that the whole grid copies
-  const size_t o_gi = total, o_gd = o_gi + ins.size() + T, o_bm = o_gd + del.size() + T, o_bc = o_bm + T;
-  const size_t dtotal = o_bc + T;
-  // queued work must be done with the staging and device buffers before they are reused
-  HIPCHK(hipStreamSynchronize(e->stream));
+// One round of merges and commits: at most kMaxVertexChanges inserts and deletes
+// per vertex. An update with more on one vertex takes several.
+struct Slice {
+  std::vector<uint32_t> tv, ioff, doff, ins, del;
+};
+
+// The arrays of an update's round on the device: what the host sends (b's const
+// members, the relabels, and for a catch-up the last update's touched and
+// relabelled vertices), then what only kernels write.
+struct RoundArrays {
+  BatchDev b;
+  const uint32_t *last_touched, *last_relabel;
+};
+
+// Sends a round's arrays in one copy.
+int upload_round(dsm_engine *e, const Slice &sl, const HostDelta *relabels, bool last, RoundArrays &out) {
+  static const std::vector<uint32_t> none;
+  const uint32_t T = (uint32_t)sl.tv.size();
+  const std::vector<uint32_t> &rl_v = relabels ? relabels->rl_v : none, &rl_l = relabels ? relabels->rl_l : none;
+  const std::vector<uint32_t> &lt = last ? e->last_touched : none, &lr = last ? e->last_relabel : none;
+  const std::vector<uint32_t> *parts[] = {&sl.tv, &sl.ioff, &sl.doff, &sl.ins, &sl.del, &rl_v, &rl_l, &lt, &lr};
+  size_t off[10] = {};
+  for (int i = 0; i < 9; i++) off[i + 1] = off[i] + parts[i]->size();
+  const size_t total = off[9], R = rl_v.size();
+  // prefix counts and big-list indices of the hub lists that the whole grid copies
+  const size_t o_gi = total, o_gd = o_gi + sl.ins.size() + T, o_bm = o_gd + sl.del.size() + T, o_bc = o_bm + T,
+               o_rb = o_bc + T, dtotal = o_rb + R;
+  // an earlier round may still read the arrays, its copy the staging buffer
+  if (dtotal > e->bbuf.n) HIPCHK(hipStreamSynchronize(e->stream));
+  HIPCHK(hipEventSynchronize(e->ev_hbuf));
   HIPCHK(e->hbuf.ensure(total));
   HIPCHK(e->bbuf.ensure(dtotal));
-  uint32_t *h = e->hbuf.p;
-  std::copy(tv.begin(), tv.end(), h + o_tv);
-  std::copy(ioff.begin(), ioff.end(), h + o_io);
-  std::copy(doff.begin(), doff.end(), h + o_do);
-  std::copy(ins.begin(), ins.end(), h + o_in);
-  std::copy(del.begin(), del.end(), h + o_de);
-  HIPCHK(hipMemcpyAsync(e->bbuf.p, h, total * 4, hipMemcpyHostToDevice, e->stream));
+  for (int i = 0; i < 9; i++) std::copy(parts[i]->begin(), parts[i]->end(), e->hbuf.p + off[i]);
+  if (total) HIPCHK(hipMemcpyAsync(e->bbuf.p, e->hbuf.p, total * 4, hipMemcpyHostToDevice, e->stream));
+  HIPCHK(hipEventRecord(e->ev_hbuf, e->stream));
   HIPCHK(e->ndeg.ensure(T));
   HIPCHK(e->fail.ensure(T));
   HIPCHK(e->soff.ensure(T));
   BatchDev b{};
   b.ntouched = T;
-  b.tv = e->bbuf.p + o_tv;
-  b.ioff = e->bbuf.p + o_io;
-  b.doff = e->bbuf.p + o_do;
-  b.ins = e->bbuf.p + o_in;
-  b.del = e->bbuf.p + o_de;
+  b.tv = e->bbuf.p + off[0];
+  b.ioff = e->bbuf.p + off[1];
+  b.doff = e->bbuf.p + off[2];
+  b.ins = e->bbuf.p + off[3];
+  b.del = e->bbuf.p + off[4];
+  b.nrelabel = (uint32_t)R;
+  b.rl_v = e->bbuf.p + off[5];
+  b.rl_l = e->bbuf.p + off[6];
+  b.rl_big = e->bbuf.p + o_rb;
   b.ndeg = e->ndeg.p;
   b.soff = e->soff.p;
   b.fail = e->fail.p;
@@ -1089,30 +1132,49 @@ int apply_round(dsm_engine *e, const HostDelta &d, const std::vector<uint32_t> &
   b.gdcum = e->bbuf.p + o_gd;
   b.big_merge = e->bbuf.p + o_bm;
   b.big_commit = e->bbuf.p + o_bc;
-  // scratch must hold every touched list once plus the inserts: at most the
-  // pool's entries plus this round's inserts (the stream is idle here, so a
-  // larger scratch replaces the old one without copying)
-  const unsigned long long need = e->pool_cap + ins.size() + (1ull << 20);
-  if (need > e->scratch_cap) {
-    HIPCHK(e->scratch.alloc(need + need / 4));
-    e->scratch_cap = need + need / 4;
-  }
-  HIPCHK(launch_scratch_reset(e->actl.p, e->stream));
-  HIPCHK(launch_apply_merge(e->dev_graph(), b, e->scratch_cap, e->scratch.p, e->actl.p, e->stream));
-  HIPCHK(launch_apply_commit(e->dev_graph(), b, e->scratch.p, e->pool_cap, e->actl.p, e->dirty(), e->stream));
+  out.b = b;
+  out.last_touched = e->bbuf.p + off[7];
+  out.last_relabel = e->bbuf.p + off[8];
+  return DSM_OK;
+}
+
+// Room in the scratch for every touched list once plus the inserts: at most the
+// pool's entries plus the round's inserts.
+int ensure_scratch(dsm_engine *e, size_t inserts) {
+  const unsigned long long need = e->pool_cap + inserts + (1ull << 20);
+  if (need <= e->scratch_cap) return DSM_OK;
+  HIPCHK(hipStreamSynchronize(e->stream));  // an earlier round may still use it
+  HIPCHK(e->scratch.alloc(need + need / 4));
+  e->scratch_cap = need + need / 4;
+  return DSM_OK;
+}
+
+int enqueue_apply(dsm_engine *e, const BatchDev &b, uint32_t longest) {
+  HIPCHK(launch_apply_merge(e->dev_graph(), b, e->scratch_cap, e->scratch.p, e->actl.p, longest, e->stream));
+  HIPCHK(launch_apply_commit(e->dev_graph(), b, e->scratch.p, e->pool_cap, e->actl.p, e->dirty(), false, longest,
+                             e->stream));
+  return DSM_OK;
+}
+
+// Waits for the update's status.
+int take_status(dsm_engine *e) {
   HIPCHK(hipMemcpyAsync(e->h_actl.p, e->actl.p, sizeof(ApplyCtl), hipMemcpyDeviceToHost, e->stream));
   HIPCHK(hipStreamSynchronize(e->stream));
   if (e->h_actl.p->merge_overflow)
     return e->fail_msg(DSM_ELIMIT, "update: %u merged lists found no room in the merge scratch",
                        e->h_actl.p->merge_overflow);
+  return DSM_OK;
+}
+
+// Grows the pool for the commits that found no room and tries them again (the
+// status has been taken; their merged lists are in the scratch).
+int retry_commits(dsm_engine *e, const BatchDev &b, uint32_t longest) {
   for (int attempt = 0; e->h_actl.p->overflow && attempt < 4; attempt++) {
-    int rc = grow_pool(e, e->pool_cap / 2 + (1ull << 22));
-    if (rc) return rc;
-    // the merge itself overflowing scratch is impossible by sizing; only commits retry
-    HIPCHK(launch_apply_commit_failed(e->dev_graph(), b, e->scratch.p, e->pool_cap, e->actl.p, e->dirty(),
-                                      e->stream));
-    HIPCHK(hipMemcpyAsync(e->h_actl.p, e->actl.p, sizeof(ApplyCtl), hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
+    if (int rc = grow_pool(e, e->pool_cap / 2 + (1ull << 22))) return rc;
+    HIPCHK(launch_round_begin(e->actl.p, false, e->stream));
+    HIPCHK(launch_apply_commit(e->dev_graph(), b, e->scratch.p, e->pool_cap, e->actl.p, e->dirty(), true, longest,
+                               e->stream));
+    if (int rc = take_status(e)) return rc;
   }
   if (e->h_actl.p->overflow) return e->fail_msg(DSM_ENOMEM, "neighbour pool could not be grown");
   return DSM_OK;
@@ -1174,60 +1236,18 @@ int grow_pool(dsm_engine *e, unsigned long long extra) {
   return DSM_OK;
 }
 
-int do_apply_delta(dsm_engine *e, const HostDelta &d) {
-  const uint32_t T = (uint32_t)d.tv.size();
-  // split into rounds of at most kMaxVertexChanges inserts and deletes per vertex
-  uint32_t rounds = 1;
-  for (uint32_t t = 0; t < T; t++) {
-    uint32_t m = std::max(d.ioff[t + 1] - d.ioff[t], d.doff[t + 1] - d.doff[t]);
-    rounds = std::max(rounds, (m + kMaxVertexChanges - 1) / kMaxVertexChanges);
-  }
-  for (uint32_t rd = 0; rd < rounds; rd++) {
-    std::vector<uint32_t> tv, ioff{0}, doff{0}, ins, del;
-    for (uint32_t t = 0; t < T; t++) {
-      uint32_t i0 = d.ioff[t] + rd * kMaxVertexChanges, i1 = std::min(d.ioff[t + 1], i0 + kMaxVertexChanges);
-      uint32_t d0 = d.doff[t] + rd * kMaxVertexChanges, d1 = std::min(d.doff[t + 1], d0 + kMaxVertexChanges);
-      if (i0 >= i1 && d0 >= d1 && rd > 0) continue;
-      tv.push_back(d.tv[t]);
-      if (i0 < i1) ins.insert(ins.end(), d.ins.begin() + i0, d.ins.begin() + i1);
-      if (d0 < d1) del.insert(del.end(), d.del.begin() + d0, d.del.begin() + d1);
-      ioff.push_back((uint32_t)ins.size());
-      doff.push_back((uint32_t)del.size());
-    }
-    int rc = apply_round(e, d, tv, ioff, doff, ins, del);
-    if (rc) return rc;
-  }
-  e->stats.touched_vertices = T;
-  e->stats.relocated_vertices = e->h_actl.p->relocated;
-  // relabels
-  BatchDev b{};
-  const uint32_t R = (uint32_t)d.rl_v.size();
-  if (R) {
-    HIPCHK(hipStreamSynchronize(e->stream));
-    HIPCHK(e->hbuf.ensure(2 * (size_t)R));
-    HIPCHK(e->bbuf.ensure(3 * (size_t)R));
-    std::copy(d.rl_v.begin(), d.rl_v.end(), e->hbuf.p);
-    std::copy(d.rl_l.begin(), d.rl_l.end(), e->hbuf.p + R);
-    HIPCHK(hipMemcpyAsync(e->bbuf.p, e->hbuf.p, 2 * (size_t)R * 4, hipMemcpyHostToDevice, e->stream));
-    b.nrelabel = R;
-    b.rl_v = e->bbuf.p;
-    b.rl_l = e->bbuf.p + R;
-    b.rl_big = e->bbuf.p + 2 * (size_t)R;
-    HIPCHK(launch_relabel(e->dev_graph(), b, e->tables(), e->dirty(), e->stream));
-  }
-  return DSM_OK;
-}
-
+// Records on the device, src[k] | dst[k].
 int upload_records(dsm_engine *e, const std::vector<uint32_t> &s, const std::vector<uint32_t> &d,
                    DevBuf<uint32_t> &dev) {
   const size_t k = s.size();
-  PinnedBuf<uint32_t> &h = e->hbuf;
-  HIPCHK(hipStreamSynchronize(e->stream));
-  HIPCHK(dev.ensure(2 * k + 2));
-  HIPCHK(h.ensure(2 * k + 2));
-  std::copy(s.begin(), s.end(), h.p);
-  std::copy(d.begin(), d.end(), h.p + k);
-  HIPCHK(hipMemcpyAsync(dev.p, h.p, 2 * k * 4 + 4, hipMemcpyHostToDevice, e->stream));
+  if (2 * k > dev.n) HIPCHK(hipStreamSynchronize(e->stream));
+  HIPCHK(dev.ensure(2 * k));
+  HIPCHK(hipEventSynchronize(e->ev_hrec));
+  HIPCHK(e->hrec.ensure(2 * k));
+  std::copy(s.begin(), s.end(), e->hrec.p);
+  std::copy(d.begin(), d.end(), e->hrec.p + k);
+  HIPCHK(hipMemcpyAsync(dev.p, e->hrec.p, 2 * k * 4, hipMemcpyHostToDevice, e->stream));
+  HIPCHK(hipEventRecord(e->ev_hrec, e->stream));
   return DSM_OK;
 }
 
@@ -1277,52 +1297,119 @@ void take_refine_time(dsm_engine *e) {
   if (hipEventElapsedTime(&ms, e->ev_ref[0], e->ev_ref[1]) == hipSuccess) e->stats.ms_refine += ms;
 }
 
-// The label-sorted copies that a catch-up leaves to the update that follows
-// it: those of the last update's dirty vertices (the shared dirty list still
-// holds them until the next compaction), copied from `from` once the new
-// update has marked its own dirty vertices, skipping those, whose copies it
-// rebuilds from their lists anyway.
-struct SortedSync {
-  DevGraph from;
-  const uint32_t *ndirty;
-};
-
-// One batch's update and candidate refresh from its host delta, enqueued on
-// the engine's stream: reset the per-batch apply counters, apply (device
-// merge/commit, which waits for the commit's status), relabel, make a
-// catch-up's deferred label-sorted copies (sorted_sync), rebuild the dirty
-// vertices' label-sorted copies, then refilter the dirty vertices (long lists
-// take their neighbour-label counts from those copies). No wait at the end.
-int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const SortedSync *sorted_sync = nullptr) {
-  int rc;
-  e->shadow_delta_ok = false;
-  e->grew = false;
-  HIPCHK(launch_ctl_reset(nullptr, e->actl.p, nullptr, nullptr, 0, nullptr, 0, e->stream));
-  if ((rc = do_apply_delta(e, d))) return rc;
-  // the catch-up's deferred label-sorted copies: this update's dirty bits are
-  // all set and the dirty list still holds the last update's vertices. After
-  // a pool growth the slots moved and every copy is rebuilt instead.
-  if (sorted_sync && !e->grew && !e->lpool_stale)
-    HIPCHK(launch_sync_sorted(sorted_sync->from, e->dev_graph(), e->dirty_list.p, sorted_sync->ndirty,
-                              e->dirty_bits.p, e->sync_q.p, (uint32_t)e->sync_q.n, e->sync_ctl.p, e->stream));
-  HIPCHK(launch_dirty_compact(e->dirty(), e->n, e->stream));
-  // the dirty list (touched vertices, relabelled ones and their neighbours) is
-  // exactly the set whose label-sorted copies changed, unless the pool grew
-  if (e->lpool_stale) {
-    HIPCHK(launch_lbuild(e->dev_graph(), e->d_lmap.p, nullptr, nullptr, e->huge_sort(), e->stream));
-    e->lpool_stale = false;
-  } else {
-    HIPCHK(launch_lbuild(e->dev_graph(), e->d_lmap.p, e->dirty_list.p, &e->actl.p->ndirty, e->huge_sort(),
-                         e->stream));
-  }
-  HIPCHK(launch_filter_dirty(e->dev_graph(), e->tables(), e->dirty(), e->stream));
-  return cluster_refine(e);
+DevGraph graph_of(const dsm_engine *e, const dsm_engine::GraphCopy &c) {
+  DevGraph g;
+  g.n = e->n;
+  g.pool = c.pool.p;
+  g.start = c.start.p;
+  g.deg = c.deg.p;
+  g.cap = c.cap.p;
+  g.lab = c.lab.p;
+  g.lpool = c.lpool.p;
+  g.loff = c.loff.p;
+  g.nbuckets = e->nbuckets;
+  return g;
 }
 
-int apply_and_refresh(dsm_engine *e, const dsm_change *changes, uint32_t k) {
-  HostDelta d;
-  host_delta(e, changes, k, d);
-  return apply_delta_and_refresh(e, d);
+// One batch's update and candidate refresh from its host delta, on the engine's
+// stream: merge and commit the lists, relabel, rebuild the dirty vertices'
+// label-sorted copies, then refilter the dirty vertices (long lists take their
+// neighbour-label counts from those copies). Everything is enqueued at once;
+// kernels after the commit do nothing when a commit found no room, and are
+// launched again once the pool has grown. The update is done when this returns,
+// and *h_actl is its status; `done` (may be null) is recorded at its end.
+//
+// With `from`, the engine's graph lags behind that copy by exactly the last
+// update (shadow_delta_ok) and catches up first, by what that update touched and
+// relabelled and the signature rows. The label-sorted copies of its dirty
+// vertices (the shared dirty list holds them until the next compaction) follow
+// once the new update has marked its own, whose copies are rebuilt anyway.
+int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine::GraphCopy *from = nullptr,
+                            hipEvent_t done = nullptr) {
+  const uint32_t T = (uint32_t)d.tv.size();
+  e->shadow_delta_ok = false;
+  e->grew = false;
+  uint32_t rounds = 1, most_ins = 0;
+  for (uint32_t t = 0; t < T; t++) {
+    const uint32_t ni = d.ioff[t + 1] - d.ioff[t], m = std::max(ni, d.doff[t + 1] - d.doff[t]);
+    rounds = std::max(rounds, (m + kMaxVertexChanges - 1) / kMaxVertexChanges);
+    most_ins = std::max(most_ins, ni);
+  }
+  // no list is longer before the update, or after it
+  const uint32_t before = e->h_actl.p->max_deg;
+  const uint32_t longest = (uint32_t)std::min<uint64_t>((uint64_t)before + most_ins, 0xFFFFFFFFull);
+  Slice sl;
+  RoundArrays ra{};
+  for (uint32_t rd = 0; rd < rounds; rd++) {
+    if (rounds == 1) {
+      sl = Slice{d.tv, d.ioff, d.doff, d.ins, d.del};
+    } else {
+      sl = Slice{{}, {0}, {0}, {}, {}};
+      for (uint32_t t = 0; t < T; t++) {
+        const uint32_t i0 = d.ioff[t] + rd * kMaxVertexChanges, i1 = std::min(d.ioff[t + 1], i0 + kMaxVertexChanges);
+        const uint32_t d0 = d.doff[t] + rd * kMaxVertexChanges, d1 = std::min(d.doff[t + 1], d0 + kMaxVertexChanges);
+        if (i0 >= i1 && d0 >= d1 && rd > 0) continue;
+        sl.tv.push_back(d.tv[t]);
+        if (i0 < i1) sl.ins.insert(sl.ins.end(), d.ins.begin() + i0, d.ins.begin() + i1);
+        if (d0 < d1) sl.del.insert(sl.del.end(), d.del.begin() + d0, d.del.begin() + d1);
+        sl.ioff.push_back((uint32_t)sl.ins.size());
+        sl.doff.push_back((uint32_t)sl.del.size());
+      }
+    }
+    const bool final_round = rd + 1 == rounds;
+    if (int rc = upload_round(e, sl, final_round ? &d : nullptr, from && rd == 0, ra)) return rc;
+    if (rd == 0) {
+      HIPCHK(launch_update_begin(e->actl.p, from ? from->actl.p : nullptr, e->huge_ctl.p, e->stream));
+      if (from) {
+        CatchUp c;
+        c.x = graph_of(e, *from);
+        c.y = e->dev_graph();
+        c.touched = ra.last_touched;
+        c.ntouched = (uint32_t)e->last_touched.size();
+        c.relabeled = ra.last_relabel;
+        c.nrelabeled = (uint32_t)e->last_relabel.size();
+        c.bm_x = from->bm.p;
+        c.bm_y = e->bm.p;
+        c.nbm = (size_t)e->nsig_rows * e->words;
+        c.q = e->sync_q.p;
+        c.qcap = (uint32_t)e->sync_q.n;
+        c.actl = e->actl.p;
+        HIPCHK(launch_catch_up(c, before, e->stream));
+      }
+    } else {
+      HIPCHK(launch_round_begin(e->actl.p, true, e->stream));
+    }
+    if (int rc = ensure_scratch(e, sl.ins.size())) return rc;
+    if (int rc = enqueue_apply(e, ra.b, longest)) return rc;
+    if (!final_round) {
+      if (int rc = take_status(e)) return rc;
+      if (int rc = retry_commits(e, ra.b, longest)) return rc;
+    }
+  }
+  e->stats.touched_vertices = T;
+  for (int attempt = 0;; attempt++) {
+    HIPCHK(launch_relabel(e->dev_graph(), ra.b, e->tables(), e->dirty(), longest, e->stream));
+    // after a pool growth the slots moved and every copy is rebuilt instead
+    if (from && !e->grew && !e->lpool_stale)
+      HIPCHK(launch_sync_sorted(graph_of(e, *from), e->dev_graph(), e->dirty_list.p, &from->actl.p->ndirty,
+                                e->dirty_bits.p, e->sync_q.p, (uint32_t)e->sync_q.n, e->actl.p, before, e->stream));
+    HIPCHK(launch_dirty_compact(e->dirty(), e->n, e->stream));
+    // the dirty list (touched vertices, relabelled ones and their neighbours) is
+    // exactly the set whose label-sorted copies changed, unless the pool grew
+    const uint32_t *list = e->lpool_stale ? nullptr : e->dirty_list.p;
+    HIPCHK(launch_lbuild(e->dev_graph(), e->d_lmap.p, list, list ? &e->actl.p->ndirty : nullptr, e->huge_sort(), longest,
+                         e->stream));
+    HIPCHK(launch_filter_dirty(e->dev_graph(), e->tables(), e->dirty(), longest, e->stream));
+    if (int rc = cluster_refine(e)) return rc;
+    if (done) HIPCHK(hipEventRecord(done, e->stream));
+    if (int rc = take_status(e)) return rc;
+    if (!e->h_actl.p->overflow) break;
+    // the kernels above waited for this
+    if (int rc = retry_commits(e, ra.b, longest)) return rc;
+  }
+  e->lpool_stale = false;
+  e->stats.relocated_vertices = e->h_actl.p->relocated;
+  return DSM_OK;
 }
 
 // Blocks per CU of a DFS shape: the occupancy limit and, with overlap_apply,
@@ -1345,7 +1432,8 @@ int create_impl(dsm_engine *e, const dsm_graph_desc *graph, const dsm_query_desc
   int rc = 0;
   HIPCHK(hipSetDevice(e->opt.device));
   HIPCHK(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
-  HIPCHK(hipEventCreateWithFlags(&e->ev_pre, hipEventDisableTiming));
+  for (hipEvent_t *x : {&e->ev_pre, &e->ev_hbuf, &e->ev_hrec})
+    HIPCHK(hipEventCreateWithFlags(x, hipEventDisableTiming));
   HIPCHK(hipDeviceGetAttribute(&e->num_cu, hipDeviceAttributeMultiprocessorCount, e->opt.device));
   HIPCHK(hipDeviceGetAttribute(&e->wall_khz, hipDeviceAttributeWallClockRate, e->opt.device));
   {
@@ -1400,7 +1488,8 @@ int create_impl(dsm_engine *e, const dsm_graph_desc *graph, const dsm_query_desc
   e->leaf_segments = e->opt.leaf_segments != 0;
   e->poll_max = e->opt.poll_max ? std::min<uint32_t>(e->opt.poll_max, 16u) : 16u;
   HIPCHK(launch_filter_full(e->dev_graph(), e->tables(), e->stream));
-  HIPCHK(launch_lbuild(e->dev_graph(), e->d_lmap.p, nullptr, nullptr, e->huge_sort(), e->stream));
+  HIPCHK(launch_huge_reset(e->huge_sort(), e->stream));
+  HIPCHK(launch_lbuild(e->dev_graph(), e->d_lmap.p, nullptr, nullptr, e->huge_sort(), e->h_actl.p->max_deg, e->stream));
   if ((rc = cluster_refine(e))) return rc;
   HIPCHK(hipStreamSynchronize(e->stream));
   e->refine_timed = false;
@@ -1476,63 +1565,17 @@ int copy_graph(dsm_engine *e, const dsm_engine::GraphCopy &c) {
   return DSM_OK;
 }
 
+// The second copy lags by exactly the last update, in slots of the same places.
+bool catch_up_by_delta(const dsm_engine *e, const dsm_engine::GraphCopy &c) {
+  return kDeltaSync && e->shadow_delta_ok && e->pool_cap == c.pool_cap && e->n < (1u << 31);
+}
+
 // Applies one batch to the second copy of the graph while a round that was
 // enqueued on `stream` matches on the first: the copies swap, the new current
 // one becomes a copy of the old one (after ev_pre, i.e. after every update
 // enqueued before the round) and takes the batch, all on stream2. Returns
 // once the update is done; the copies stay swapped, or with keep = false
 // swap back (the update is dropped: the tuner's load).
-DevGraph graph_of(const dsm_engine *e, const dsm_engine::GraphCopy &c) {
-  DevGraph g;
-  g.n = e->n;
-  g.pool = c.pool.p;
-  g.start = c.start.p;
-  g.deg = c.deg.p;
-  g.cap = c.cap.p;
-  g.lab = c.lab.p;
-  g.lpool = c.lpool.p;
-  g.loff = c.loff.p;
-  g.nbuckets = e->nbuckets;
-  return g;
-}
-
-// Makes the engine's graph equal to `c` when it lags by exactly the last
-// update (shadow_delta_ok): only that update's touched, dirty and relabelled
-// vertices are copied (launch_sync), plus the signature rows and the apply
-// status; otherwise the whole graph (copy_graph). With `deferred`, the dirty
-// vertices' label-sorted copies are left to the update that follows: when the
-// copy is by the last update only, *deferred describes them and *has_deferred
-// is set (see SortedSync).
-int catch_up(dsm_engine *e, const dsm_engine::GraphCopy &c, SortedSync *deferred = nullptr,
-             bool *has_deferred = nullptr) {
-  if (has_deferred) *has_deferred = false;
-  if (!kDeltaSync || !e->shadow_delta_ok || e->pool_cap != c.pool_cap || e->n >= (1u << 31))
-    return copy_graph(e, c);
-  const uint32_t nt = (uint32_t)e->last_touched.size(), nr = (uint32_t)e->last_relabel.size();
-  HIPCHK(e->d_last_touched.ensure(std::max<uint32_t>(nt, 1)));
-  HIPCHK(e->d_last_relabel.ensure(std::max<uint32_t>(nr, 1)));
-  if (nt)
-    HIPCHK(hipMemcpyAsync(e->d_last_touched.p, e->last_touched.data(), (size_t)nt * 4, hipMemcpyHostToDevice,
-                          e->stream));
-  if (nr)
-    HIPCHK(hipMemcpyAsync(e->d_last_relabel.p, e->last_relabel.data(), (size_t)nr * 4, hipMemcpyHostToDevice,
-                          e->stream));
-  // long lists queued: at most one per touched and one per dirty vertex
-  HIPCHK(e->sync_q.ensure(2 * (size_t)e->n));
-  HIPCHK(e->sync_ctl.ensure(2));
-  const bool defer = deferred && has_deferred;
-  HIPCHK(launch_sync(graph_of(e, c), e->dev_graph(), e->d_last_touched.p, nt, defer ? nullptr : e->dirty_list.p,
-                     &c.actl.p->ndirty, e->d_last_relabel.p, nr, e->sync_q.p, (uint32_t)e->sync_q.n, e->sync_ctl.p,
-                     e->stream));
-  if (defer) {
-    *deferred = SortedSync{graph_of(e, c), &c.actl.p->ndirty};
-    *has_deferred = true;
-  }
-  HIPCHK(copy_buf(e->bm, c.bm, (size_t)e->nsig_rows * e->words, e->stream));
-  HIPCHK(copy_buf(e->actl, c.actl, 1, e->stream));
-  return DSM_OK;
-}
-
 int overlap_apply(dsm_engine *e, const HostDelta &d, bool stats, bool keep = true) {
   const ApplyCtl mirror = *e->h_actl.p;
   std::swap(e->stream, e->stream2);
@@ -1541,13 +1584,11 @@ int overlap_apply(dsm_engine *e, const HostDelta &d, bool stats, bool keep = tru
   auto run = [&]() -> int {
     HIPCHK(hipStreamWaitEvent(e->stream, e->ev_pre, 0));
     if (stats) HIPCHK(hipEventRecord(e->ev[0], e->stream));
-    SortedSync ss;
-    bool deferred = false;
-    if (int r = catch_up(e, e->shadow, &ss, &deferred)) return r;
-    if (int r = apply_delta_and_refresh(e, d, deferred ? &ss : nullptr)) return r;
-    if (stats) HIPCHK(hipEventRecord(e->ev[2], e->stream));
-    HIPCHK(hipMemcpyAsync(e->h_actl.p, e->actl.p, sizeof(ApplyCtl), hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
+    const bool by_delta = catch_up_by_delta(e, e->shadow);
+    // long lists queued: at most one per touched and one per dirty vertex
+    if (by_delta) HIPCHK(e->sync_q.ensure(2 * (size_t)e->n));
+    else if (int r = copy_graph(e, e->shadow)) return r;
+    if (int r = apply_delta_and_refresh(e, d, by_delta ? &e->shadow : nullptr, stats ? e->ev[2] : nullptr)) return r;
     if (stats) {
       e->stats.filter_entries += e->h_actl.p->filter_entries;
       e->stats.dirty_groups += e->h_actl.p->ndirty;
@@ -1662,7 +1703,7 @@ int dsm_apply_batch(dsm_engine *e, const dsm_change *changes, uint32_t k) {
     }
   }
   const uint32_t nq = (uint32_t)e->queries.size();
-  HIPCHK(launch_ctl_reset(nullptr, nullptr, e->tuple_count.p, e->counts.p, nq * 2, nullptr, 0, e->stream));
+  e->counts_stale = true;
   int rc;
   bool applied = false;
   // 1. negatives in the pre-batch graph; with overlap_apply the batch is
@@ -1672,12 +1713,8 @@ int dsm_apply_batch(dsm_engine *e, const dsm_change *changes, uint32_t k) {
     if ((rc = ensure_seed_cap(e, nn))) return rc;
     DevBuf<uint32_t> &rb = e->rec_neg;
     if ((rc = upload_records(e, e->neg_s, e->neg_d, rb))) return rc;
-    if (e->overlap_apply) {
-      // the update refills the staging buffer the records came from
-      HIPCHK(hipStreamSynchronize(e->stream));
-      HIPCHK(hipEventRecord(e->ev_pre, e->stream));
-    }
-    if ((rc = run_round(e, rb.p, rb.p + nn, nn, 0, e->ev[6], e->ev[7], e->ev[8]))) return rc;
+    if (e->overlap_apply) HIPCHK(hipEventRecord(e->ev_pre, e->stream));
+    if ((rc = run_round(e, rb.p, rb.p + nn, nn, 0, nullptr, e->ev[7], e->ev[8]))) return rc;
     if (e->overlap_apply) {
       HostDelta d;
       host_delta(e, changes, k, d);
@@ -1693,13 +1730,10 @@ int dsm_apply_batch(dsm_engine *e, const dsm_change *changes, uint32_t k) {
   // 2-3. apply + relabel + filter (update, relabel, refilter and
   // label-sorted copies; already done beside the negatives with overlap)
   if (!applied) {
+    HostDelta d;
+    host_delta(e, changes, k, d);
     HIPCHK(hipEventRecord(e->ev[0], e->stream));
-    if ((rc = apply_and_refresh(e, changes, k))) return rc;
-    HIPCHK(hipEventRecord(e->ev[2], e->stream));
-  }
-  HIPCHK(hipMemcpyAsync(e->h_actl.p, e->actl.p, sizeof(ApplyCtl), hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(hipStreamSynchronize(e->stream));
-  if (!applied) {
+    if ((rc = apply_delta_and_refresh(e, d, nullptr, e->ev[2]))) return rc;
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, e->ev[0], e->ev[2]));
     e->stats.ms_apply = ms;
@@ -1722,30 +1756,31 @@ int dsm_match_batch(dsm_engine *e, uint64_t *pos, uint64_t *neg) {
   if (!e) return DSM_EINVAL;
   HIPCHK(hipSetDevice(e->opt.device));
   int rc;
+  bool fetched = false;
   const uint32_t nq = (uint32_t)e->queries.size();
   if (e->batch_pending && !e->pos_s.empty()) {
     const uint32_t np = (uint32_t)e->pos_s.size();
     if ((rc = ensure_seed_cap(e, np))) return rc;
     DevBuf<uint32_t> &rb = e->rec_pos;
     if ((rc = upload_records(e, e->pos_s, e->pos_d, rb))) return rc;
-    if ((rc = run_round(e, rb.p, rb.p + np, np, 1, e->ev[3], e->ev[4], e->ev[5]))) return rc;
-    HIPCHK(hipStreamSynchronize(e->stream));
+    // a graph round's seeding is part of its DFS time
+    hipEvent_t seeding = e->graph_rounds ? nullptr : e->ev[3];
+    if ((rc = run_round(e, rb.p, rb.p + np, np, 1, seeding, e->ev[4], e->ev[5]))) return rc;
+    if ((rc = fetch_results(e))) return rc;
+    fetched = true;
     if ((rc = check_round(e, &e->stats.seeds_pos))) return rc;
     float ms = 0;
-    HIPCHK(hipEventElapsedTime(&ms, e->ev[3], e->ev[4]));
+    if (seeding) HIPCHK(hipEventElapsedTime(&ms, seeding, e->ev[4]));
     e->stats.ms_seed = ms;
     HIPCHK(hipEventElapsedTime(&ms, e->ev[4], e->ev[5]));
     e->stats.ms_dfs_pos = ms;
   }
   e->batch_pending = false;
-  HIPCHK(hipMemcpyAsync(e->h_counts.p, e->counts.p, (size_t)nq * 2 * 8, hipMemcpyDeviceToHost, e->stream));
-  unsigned long long tc = 0;
-  HIPCHK(hipMemcpyAsync(&tc, e->tuple_count.p, 8, hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(hipStreamSynchronize(e->stream));
-  e->stats.tuples = tc;
+  if (!fetched && (rc = fetch_results(e))) return rc;
+  e->stats.tuples = *e->h_results.p;
   for (uint32_t q = 0; q < nq; q++) {
-    if (pos) pos[q] = e->h_counts.p[2 * q + 1];
-    if (neg) neg[q] = e->h_counts.p[2 * q + 0];
+    if (pos) pos[q] = e->h_counts()[2 * q + 1];
+    if (neg) neg[q] = e->h_counts()[2 * q + 0];
   }
   return DSM_OK;
 }
@@ -1915,12 +1950,11 @@ int dsm_autotune(dsm_engine *e, const dsm_change *sample, uint32_t k, dsm_tune_r
     e->donate_every = c.dev;
     e->bit_probe_last = c.pl;
     if (loaded) HIPCHK(hipEventRecord(e->ev_pre, e->stream));
-    HIPCHK(launch_ctl_reset(nullptr, nullptr, e->tuple_count.p, e->counts.p, nq * 2, nullptr, 0, e->stream));
+    e->counts_stale = true;
     int rc2 = run_round(e, rb.p, rb.p + k, k, 0, e->ev[9], e->ev[10], e->ev[11]);
     if (rc2) return rc2;
     if (loaded && (rc2 = overlap_apply(e, load, true, false))) return rc2;
-    HIPCHK(hipMemcpyAsync(e->h_counts.p, e->counts.p, (size_t)nq * 2 * 8, hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
+    if ((rc2 = fetch_results(e))) return rc2;
     uint64_t seeds = 0;
     if ((rc2 = check_round(e, &seeds))) return rc2;
     HIPCHK(hipEventElapsedTime(&ms, e->ev[10], e->ev[11]));
@@ -1931,7 +1965,7 @@ int dsm_autotune(dsm_engine *e, const dsm_change *sample, uint32_t k, dsm_tune_r
       HIPCHK(hipEventElapsedTime(&ua, e->ev[10], e->ev[2]));
       ms = std::max(ms, ua);
     }
-    std::vector<unsigned long long> cnt(e->h_counts.p, e->h_counts.p + 2 * (size_t)nq);
+    std::vector<unsigned long long> cnt(e->h_counts(), e->h_counts() + 2 * (size_t)nq);
     if (ref_counts.empty()) ref_counts = cnt;
     else if (cnt != ref_counts)
       return e->fail_msg(DSM_EDEVICE, "autotune: launch configurations disagree on the counts");
@@ -2241,8 +2275,9 @@ int pipe_round(dsm_engine *e, PinnedBuf<uint32_t> &h_rec, DevBuf<uint32_t> &d_re
   const bool overlap = applied && R && d && e->overlap_apply;
   if (applied) *applied = false;
   if (overlap) HIPCHK(hipEventRecord(e->ev_pre, e->stream));
-  if (R) HIPCHK(launch_ctl_reset(nullptr, nullptr, nullptr, e->counts.p + (size_t)R->slot * nq * 2, nq * 2,
-                                 nullptr, 0, e->stream));
+  e->counts_stale = false;  // a slot of this round's is cleared instead
+  ClearSpan clear{};
+  if (R) clear = ClearSpan{nullptr, e->counts() + (size_t)R->slot * nq * 2, nq * 2};
   if (np + nn) {
     if ((rc = ensure_seed_cap(e, np + nn))) return rc;
     HIPCHK(h_rec.ensure(2 * (size_t)(np + nn) + 2));
@@ -2261,12 +2296,13 @@ int pipe_round(dsm_engine *e, PinnedBuf<uint32_t> &h_rec, DevBuf<uint32_t> &d_re
     int nparts = 0;
     if (np) parts[nparts++] = RoundPart{d_rec.p, d_rec.p + np, np, (P->slot << 1) | 1u};
     if (nn) parts[nparts++] = RoundPart{d_rec.p + 2 * np, d_rec.p + 2 * np + nn, nn, R->slot << 1};
-    if ((rc = dfs_round(e, parts, nparts, stats ? e->ev[9] : nullptr, stats ? e->ev[10] : nullptr,
-                        stats ? e->ev[11] : nullptr)))
+    if ((rc = dfs_round(e, parts, nparts, stats ? e->ev[9] : nullptr, nullptr, stats ? e->ev[11] : nullptr, clear)))
       return rc;
+  } else if (R) {
+    HIPCHK(launch_ctl_reset(nullptr, nullptr, clear.counts, clear.ncounts, nullptr, 0, e->stream));
   }
   if (P)
-    HIPCHK(hipMemcpyAsync(e->h_counts.p + (size_t)P->slot * nq * 2, e->counts.p + (size_t)P->slot * nq * 2,
+    HIPCHK(hipMemcpyAsync(e->h_counts() + (size_t)P->slot * nq * 2, e->counts() + (size_t)P->slot * nq * 2,
                           (size_t)nq * 2 * 8, hipMemcpyDeviceToHost, e->stream));
   if (R && d && !have_delta) host_delta(e, R->rec, R->nrec, *d);
   if (overlap) {
@@ -2288,7 +2324,7 @@ int pipe_round(dsm_engine *e, PinnedBuf<uint32_t> &h_rec, DevBuf<uint32_t> &d_re
   if (P) {
     P->pos.assign(nq, 0);
     P->neg.assign(nq, 0);
-    const unsigned long long *c = e->h_counts.p + (size_t)P->slot * nq * 2;
+    const unsigned long long *c = e->h_counts() + (size_t)P->slot * nq * 2;
     for (uint32_t q = 0; q < nq; q++) {
       P->pos[q] = c[2 * q + 1];
       P->neg[q] = c[2 * q + 0];
@@ -2543,8 +2579,7 @@ int dsm_process_batches(dsm_engine *e, const dsm_change *changes, const uint32_t
     if (P) publish_item(b - 1);
     if (!applied) {
       HIPCHK(hipEventRecord(e->ev[0], e->stream));
-      if ((rc = apply_delta_and_refresh(e, d))) return rc;
-      HIPCHK(hipEventRecord(e->ev[2], e->stream));
+      if ((rc = apply_delta_and_refresh(e, d, nullptr, e->ev[2]))) return rc;
       apply_timed = true;
     }
     P = R;

@@ -125,7 +125,9 @@ struct alignas(64) ApplyCtl {
   uint32_t nrelabel_huge;
   uint32_t nmerge_huge;
   uint32_t ncommit_huge;
-  uint32_t pad[13];
+  uint32_t max_deg;                 // no list has been longer (never lowered): kernels of longer lists are skipped
+  uint32_t sync_queued[4];          // long lists queued by the catch-up (block, grid) and the sorted catch-up
+  uint32_t pad[8];
 };
 static_assert(sizeof(ApplyCtl) == 128, "apply status layout");
 
@@ -220,15 +222,16 @@ struct SeedArgs {
   const Plan *plans;
   const uint32_t *plan_key;   // sorted (label0 << 8 | label1) of each plan
   uint32_t nplans;
-  const uint32_t *rs;
-  const uint32_t *rd;
-  uint32_t nrec;
+  // two record lists, each with the tag written to its seeds
+  const uint32_t *rs[2];
+  const uint32_t *rd[2];
+  uint32_t nrec[2];
+  uint32_t tag[2];
   uint32_t *seed_plan;
   uint32_t *seed_s;
   uint32_t *seed_d;
   uint32_t *seed_tag;
   uint32_t seed_cap;
-  uint32_t tag;               // written to every seed of these records
   DfsCtl *ctl;
 };
 
@@ -338,31 +341,54 @@ hipError_t launch_cluster_pass(const ClusterArgs &a, uint32_t max_blocks, hipStr
 hipError_t launch_cluster_heavy(const ClusterArgs &a, uint32_t blocks, hipStream_t s);
 
 // ---- launchers (dsm_kernels.hip) -------------------------------------------
+// Launches of an update. Every kernel after the commit does nothing once a
+// commit found no room (ApplyCtl::overflow) or a merge none (merge_overflow), so
+// that the whole update is enqueued at once and the host looks at the status
+// when it is done. `longest` is a length no list exceeds: kernels that only work
+// on longer lists are not launched.
+constexpr uint32_t kApplyWave = 8192;    // longer lists are merged and committed by the whole grid
+constexpr uint32_t kRelabelWave = 2048;  // neighbours of longer lists are marked by the whole grid
+constexpr uint32_t kSyncWave = 4096;     // longer lists are brought up to date by the whole grid
+constexpr uint32_t kLbuildBlock = 4096;  // label-sorted copies of longer lists are built by a block
+constexpr uint32_t kLight = 64;          // dirty vertices of higher degree are re-filtered by a wave
+
+// Takes over the status `from` (null: keeps its own) and clears what an update
+// counts, also hctl[4] (HugeSort::ctl).
+hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *hctl, hipStream_t s);
+// Another round of merges and commits of one update (first: before its merges;
+// else before commits that are tried again).
+hipError_t launch_round_begin(ApplyCtl *actl, bool first, hipStream_t s);
 hipError_t launch_apply_merge(const DevGraph &g, const BatchDev &b, unsigned long long scratch_cap,
-                              uint32_t *scratch, ApplyCtl *actl, hipStream_t s);
+                              uint32_t *scratch, ApplyCtl *actl, uint32_t longest, hipStream_t s);
 hipError_t launch_apply_commit(const DevGraph &g, const BatchDev &b, const uint32_t *scratch,
-                               unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d,
-                               hipStream_t s);
-hipError_t launch_apply_commit_failed(const DevGraph &g, const BatchDev &b, const uint32_t *scratch,
-                                      unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d,
-                                      hipStream_t s);
+                               unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d, bool only_failed,
+                               uint32_t longest, hipStream_t s);
 // The dirty list (d.list, its length added to d.actl->ndirty) from the dirty
 // bits of the update's n vertices.
 hipError_t launch_dirty_compact(const DirtyArgs &d, uint32_t n, hipStream_t s);
-// Copies what the last update changed from graph copy x to the stale copy y:
-// the touched vertices' slots and lists, the dirty vertices' label-sorted
-// copies (ndirty on the device; none when dirty is null), the relabelled
-// vertices' labels. q (qcap entries) and qctl[2] are scratch for the long
+// What the last update changed, from graph copy x to the stale copy y: the
+// touched vertices' slots and lists, the relabelled vertices' labels and the
+// nbm words of the signature rows. q (qcap entries) is scratch for the long
 // lists.
-hipError_t launch_sync(const DevGraph &x, const DevGraph &y, const uint32_t *touched, uint32_t ntouched,
-                       const uint32_t *dirty, const uint32_t *ndirty, const uint32_t *relabeled, uint32_t nrelabeled,
-                       uint32_t *q, uint32_t qcap, uint32_t *qctl, hipStream_t s);
+struct CatchUp {
+  DevGraph x, y;
+  const uint32_t *touched, *relabeled;
+  uint32_t ntouched, nrelabeled;
+  const uint64_t *bm_x;
+  uint64_t *bm_y;
+  size_t nbm;
+  uint32_t *q;
+  uint32_t qcap;
+  ApplyCtl *actl;  // y's
+};
+hipError_t launch_catch_up(const CatchUp &c, uint32_t longest, hipStream_t s);
 // The label-sorted copies and bucket offsets of the listed (dirty) vertices
 // from x to y, except those whose bit is set in skip.
 hipError_t launch_sync_sorted(const DevGraph &x, const DevGraph &y, const uint32_t *dirty, const uint32_t *ndirty,
-                              const uint32_t *skip, uint32_t *q, uint32_t qcap, uint32_t *qctl, hipStream_t s);
+                              const uint32_t *skip, uint32_t *q, uint32_t qcap, ApplyCtl *actl, uint32_t longest,
+                              hipStream_t s);
 hipError_t launch_relabel(const DevGraph &g, const BatchDev &b, const FilterTables &ft,
-                          const DirtyArgs &d, hipStream_t s);
+                          const DirtyArgs &d, uint32_t longest, hipStream_t s);
 hipError_t launch_filter_full(const DevGraph &g, const FilterTables &ft, hipStream_t s);
 // Label-sorted copies of lists longer than kHugeList entries are built in
 // segments of kHugeSeg entries spread over the grid: the vertices are queued
@@ -383,52 +409,49 @@ struct HugeSort {
   // written by the counting pass so that the scatter pass reads it back
   // instead of gathering the neighbour's label again (null: gather twice)
   uint8_t *bucket_bytes;
+  const ApplyCtl *actl;  // the update's status (null: a full build)
 };
 
 // Rebuilds the label-sorted copies of the listed vertices (list + count on the
-// device), or of every vertex when list is null.
+// device), or of every vertex when list is null. hs.ctl must be clear.
 hipError_t launch_lbuild(const DevGraph &g, const uint8_t *lmap, const uint32_t *list, const uint32_t *count,
-                         const HugeSort &hs, hipStream_t s);
-hipError_t launch_filter_dirty(const DevGraph &g, const FilterTables &ft, const DirtyArgs &d,
+                         const HugeSort &hs, uint32_t longest, hipStream_t s);
+hipError_t launch_huge_reset(const HugeSort &hs, hipStream_t s);
+hipError_t launch_filter_dirty(const DevGraph &g, const FilterTables &ft, const DirtyArgs &d, uint32_t longest,
                                hipStream_t s);
 hipError_t launch_seed(const SeedArgs &a, hipStream_t s);
 hipError_t launch_dfs(const DfsArgs &a, uint32_t blocks, uint32_t waves_per_block, uint32_t max_query_vertices,
                       hipStream_t s);
-// Resets the DFS control block (ctl) with the nidle waiting words and/or the
-// per-batch state (actl's counters, the tuple counter and the nq*2 match
-// counts); null pointers are skipped.
-hipError_t launch_ctl_reset(DfsCtl *ctl, ApplyCtl *actl, unsigned long long *tuple_count,
-                            unsigned long long *counts, uint32_t ncounts, IdleWord *idle, uint32_t nidle,
-                            hipStream_t s);
-hipError_t launch_scratch_reset(ApplyCtl *actl, hipStream_t s);
+// Resets the DFS control block (ctl) with the nidle waiting words, the tuple
+// counter and ncounts match counts; null pointers are skipped.
+hipError_t launch_ctl_reset(DfsCtl *ctl, unsigned long long *tuple_count, unsigned long long *counts,
+                            uint32_t ncounts, IdleWord *idle, uint32_t nidle, hipStream_t s);
 hipError_t launch_pool_move(const uint32_t *old_pool, uint32_t *new_pool, const uint32_t *old_start,
                             const uint32_t *new_start, const uint32_t *deg, uint32_t n,
                             hipStream_t s);
 int dfs_max_blocks_per_cu(uint32_t waves_per_block, uint32_t max_query_vertices);
 
-// Kernel-node parameters of one DFS round for a HIP graph (ctl reset, two seed
-// lists, the DFS), the same launches launch_ctl_reset / launch_seed /
-// launch_dfs make. The node's kernelParams point into `st`, which must stay
-// valid until the node is added or updated (the values are copied then). A
-// seed list with no records still gets one block, which does nothing.
+// Kernel-node parameters of one DFS round for a HIP graph (reset, seeding, the
+// DFS), the same launches launch_ctl_reset / launch_seed / launch_dfs make. The
+// node's kernelParams point into `st`, which must stay valid until the node is
+// added or updated (the values are copied then). A seeding with no records still
+// gets one block, which does nothing.
 struct RoundNodeArgs {
   DfsCtl *ctl;
-  ApplyCtl *no_actl;
-  unsigned long long *no_tc;
-  unsigned long long *no_counts;
-  uint32_t no_ncounts;
+  unsigned long long *tuple_count, *counts;  // cleared by the reset (null: kept)
+  uint32_t ncounts;
   IdleWord *idle;
   uint32_t nidle;
-  SeedArgs seed[2];
+  SeedArgs seed;
   DfsArgs dfs;
   uint32_t chunk_levels;
-  void *reset_params[7];
-  void *seed_params[2][1];
+  void *reset_params[6];
+  void *seed_params[1];
   void *dfs_params[2];
 };
 void round_node_params(RoundNodeArgs &st, uint32_t blocks, uint32_t waves_per_block,
-                       uint32_t max_query_vertices, hipKernelNodeParams *reset, hipKernelNodeParams *seed0,
-                       hipKernelNodeParams *seed1, hipKernelNodeParams *dfs);
+                       uint32_t max_query_vertices, hipKernelNodeParams *reset, hipKernelNodeParams *seed,
+                       hipKernelNodeParams *dfs);
 uint32_t dfs_lds_bytes_per_wave(uint32_t max_query_vertices);
 
 }  // namespace dsm

@@ -19,6 +19,7 @@
 //   k_dfs                           persistent wave64 DFS with per-wave LDS
 //                                   stacks, work donation and shared leaf sets
 //                                   (gpu_match.cu:96-876 restated for CDNA)
+#include <algorithm>
 #include <cstddef>
 
 #include "dsm_device.h"
@@ -28,8 +29,10 @@ namespace dsm {
 namespace {
 
 constexpr int kApplyWaves = 4;
-constexpr uint32_t kApplyWave = 8192;  // longer lists are copied by the whole grid
-constexpr int kLight = 64;          // dirty vertices up to this degree: one lane each
+
+// A commit or merge of this update found no room: the kernels after it wait for
+// the host, which makes room, tries again and launches them anew.
+__device__ __forceinline__ bool held_up(const ApplyCtl *actl) { return actl->overflow | actl->merge_overflow; }
 
 __device__ __forceinline__ bool bit_of(const uint64_t *bm, uint32_t words, uint32_t sig, uint32_t v) {
   return (bm[(size_t)sig * words + (v >> 6)] >> (v & 63)) & 1ull;
@@ -69,6 +72,7 @@ __global__ __launch_bounds__(256) void k_dirty_compact(DirtyArgs d, uint32_t nwo
   __shared__ uint32_t s_sum[256];
   __shared__ uint32_t s_base;
   const uint32_t tid = threadIdx.x;
+  if (held_up(d.actl)) return;
   for (uint32_t w0 = blockIdx.x * 256u; w0 < nwords; w0 += gridDim.x * 256u) {
     const uint32_t wi = w0 + tid;
     const uint32_t bits = wi < nwords ? d.bits[wi] : 0u;
@@ -370,6 +374,7 @@ __global__ __launch_bounds__(kApplyWaves * 64) void k_apply_commit(DevGraph g, B
     if (lane == 0) {
       g.deg[x] = nd;
       b.fail[t] = 0;
+      if (nd > ld_relaxed(&actl->max_deg)) atomicMax(&actl->max_deg, nd);
       mark_dirty_used(g, d, x);
     }
   }
@@ -388,20 +393,40 @@ __global__ __launch_bounds__(256) void k_apply_commit_big(DevGraph g, BatchDev b
   });
 }
 
-__global__ void k_big_reset(ApplyCtl *actl, int merge, int commit) {
-  if (threadIdx.x == 0) {
-    if (merge) actl->nmerge_big = actl->nmerge_huge = 0;
-    if (commit) actl->ncommit_big = actl->ncommit_huge = 0;
+// The start of an update: its status from another graph copy's, its counters
+// cleared.
+__global__ void k_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *hctl) {
+  if (threadIdx.x != 0) return;
+  if (from) {
+    actl->pool_used = from->pool_used;
+    actl->max_deg = from->max_deg;
   }
+  actl->scratch_used = 0;
+  actl->overflow = actl->merge_overflow = 0;
+  actl->relocated = actl->relabeled = 0;
+  actl->ndirty = actl->nheavy = 0;
+  actl->filter_entries = 0;
+  actl->filter_bits = 0;
+  actl->nmerge_big = actl->nmerge_huge = actl->ncommit_big = actl->ncommit_huge = 0;
+  actl->nrelabel_big = actl->nrelabel_huge = 0;
+  for (int i = 0; i < 4; i++) actl->sync_queued[i] = hctl[i] = 0;
+}
+
+__global__ void k_round_begin(ApplyCtl *actl, int first) {
+  if (threadIdx.x != 0) return;
+  if (first) {
+    actl->scratch_used = 0;
+    actl->nmerge_big = actl->nmerge_huge = 0;
+  }
+  actl->ncommit_big = actl->ncommit_huge = 0;
 }
 
 // One wave per relabel entry: set the label; when it changed, clear the
 // vertex's bits in every bitmap of its old label and mark it and all its
 // (post-update) neighbours dirty, since their neighbour-label counts changed.
-constexpr uint32_t kRelabelWave = 2048;  // longer lists are marked by the whole grid (k_relabel_big)
-
 __global__ __launch_bounds__(256) void k_relabel(DevGraph g, BatchDev b, FilterTables ft, DirtyArgs d) {
   const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
+  if (held_up(d.actl)) return;
   for (uint32_t r = blockIdx.x * 4 + wv; r < b.nrelabel; r += gridDim.x * 4) {
     const uint32_t x = b.rl_v[r];
     const uint32_t L = b.rl_l[r];
@@ -528,6 +553,7 @@ __global__ __launch_bounds__(256) void k_filter_light(DevGraph g, FilterTables f
   __shared__ uint8_t s_lmap[256];
   for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_lmap[i] = ft.lmap[i];
   __syncthreads();
+  if (held_up(d.actl)) return;
   const uint32_t nd = d.actl->ndirty < d.list_cap ? d.actl->ndirty : d.list_cap;
   uint8_t *cnt = s_cnt[threadIdx.x];
   unsigned long long entries = 0;  // list entries of the vertices this thread re-filters
@@ -543,7 +569,7 @@ __global__ __launch_bounds__(256) void k_filter_light(DevGraph g, FilterTables f
       bits += ft.sig_hi[L] - ft.sig_lo[L];
     }
     // long lists go to the heavy list, one counter add per wave
-    const bool heavy = has && dv > (uint32_t)kLight;
+    const bool heavy = has && dv > kLight;
     const uint64_t hm = ballot(heavy);
     if (hm) {
       const uint32_t leader = (uint32_t)__builtin_ctzll(hm);
@@ -707,7 +733,6 @@ __device__ __forceinline__ void bucket_scatter(const DevGraph &g, const uint8_t 
   }
 }
 
-constexpr uint32_t kLbuildBlock = 4096;  // lists longer than this are sorted by a whole block
 constexpr uint32_t kLbuildWaves = 16;    // waves of that block
 
 // The label-sorted copy of v (degree d) by one wave: bucket histogram,
@@ -755,6 +780,7 @@ __device__ __forceinline__ void queue_wave(uint32_t *q, uint32_t cap, uint32_t *
 __global__ __launch_bounds__(256) void k_lbuild_pick(DevGraph g, const uint32_t *list, const uint32_t *count,
                                                      HugeSort hs) {
   const uint32_t nb = g.nbuckets;
+  if (hs.actl && held_up(hs.actl)) return;
   const uint32_t total = list ? (*count < g.n ? *count : g.n) : g.n;
   for (uint32_t base = (blockIdx.x * blockDim.x + threadIdx.x) & ~63u; base < total;
        base += gridDim.x * blockDim.x) {
@@ -1003,8 +1029,11 @@ __global__ void k_huge_reset(HugeSort hs) {
 // s in C(u0) and d in C(u1) becomes a DFS root, provided (s,d) is an edge of
 // the graph being matched.
 __global__ __launch_bounds__(256) void k_seed(SeedArgs a) {
-  for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < a.nrec; r += gridDim.x * blockDim.x) {
-    const uint32_t s = a.rs[r], d = a.rd[r];
+  const uint32_t total = a.nrec[0] + a.nrec[1];
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x) {
+    const uint32_t which = i < a.nrec[0] ? 0u : 1u;
+    const uint32_t r = which ? i - a.nrec[0] : i;
+    const uint32_t s = a.rs[which][r], d = a.rd[which][r];
     if (s == d || s >= a.g.n || d >= a.g.n) continue;
     const uint32_t ls = a.g.lab[s], ld = a.g.lab[d];
     if (ls == kNoLabel || ld == kNoLabel) continue;
@@ -1033,43 +1062,26 @@ __global__ __launch_bounds__(256) void k_seed(SeedArgs a) {
         a.seed_plan[o] = p;
         a.seed_s[o] = s;
         a.seed_d[o] = d;
-        a.seed_tag[o] = a.tag;
+        a.seed_tag[o] = a.tag[which];
         o++;
       }
     }
   }
 }
 
-__global__ void k_ctl_reset(DfsCtl *ctl, ApplyCtl *actl, unsigned long long *tuple_count,
-                            unsigned long long *counts, uint32_t ncounts, IdleWord *idle, uint32_t nidle) {
+__global__ void k_ctl_reset(DfsCtl *ctl, unsigned long long *tuple_count, unsigned long long *counts,
+                            uint32_t ncounts, IdleWord *idle, uint32_t nidle) {
   for (uint32_t i = threadIdx.x; counts && i < ncounts; i += blockDim.x) counts[i] = 0;
   for (uint32_t i = threadIdx.x; i < nidle; i += blockDim.x) idle[i].v = 0;
+  if (ctl && threadIdx.x < kSeedHeads) ctl->seed_head[threadIdx.x].v = 0;
   if (threadIdx.x == 0) {
     if (tuple_count) *tuple_count = 0;
     if (ctl) {
       ctl->nseeds.v = 0;
-      for (uint32_t h = 0; h < kSeedHeads; h++) ctl->seed_head[h].v = 0;
       ctl->seed_overflow.v = 0;
       ctl->abort.v = 0;
     }
-    if (actl) {
-      actl->scratch_used = 0;
-      actl->overflow = 0;
-      actl->merge_overflow = 0;
-      actl->filter_entries = 0;
-      actl->filter_bits = 0;
-      actl->relocated = 0;
-      actl->ndirty = 0;
-      actl->nheavy = 0;
-      actl->relabeled = 0;
-      actl->nrelabel_big = 0;
-      actl->nrelabel_huge = 0;
-    }
   }
-}
-
-__global__ void k_scratch_reset(ApplyCtl *actl) {
-  if (threadIdx.x == 0) actl->scratch_used = 0;
 }
 
 // -------------------------------------------------------------------- DFS
@@ -2210,157 +2222,144 @@ int max_blocks(uint32_t chunk_levels) {
 // Bringing the second copy of the graph up to date before an overlapped
 // update: instead of copying the whole graph, only what the previous update
 // changed is copied from the up-to-date copy `x` to the stale one `y`: the
-// touched vertices' slots, degrees and lists, the dirty vertices' label-sorted
-// copies and bucket offsets, and the relabelled vertices' labels. Ranges of up
-// to kSyncWave entries are copied by one wave; longer ones are queued
-// (queue_big: a block each up to kBlockList entries, the whole grid beyond)
-// for k_sync_big. A queue entry is the vertex with bit 31 set for a
-// label-sorted copy.
-constexpr uint32_t kSyncWave = 4096;
-
-// mode 0: touched vertices (start, deg, cap and the pool slot); mode 1: dirty
-// vertices (bucket offsets and the label-sorted copy of lists longer than
-// kLabelSorted), except those whose bit is set in `skip`; mode 2: relabelled
-// vertices (label).
-__global__ __launch_bounds__(256) void k_sync_small(DevGraph x, DevGraph y, const uint32_t *list, const uint32_t *count,
-                                                    uint32_t n_host, uint32_t mode, const uint32_t *skip, uint32_t *q,
-                                                    uint32_t qcap, uint32_t *qctl) {
+// touched vertices' slots, degrees and lists, the relabelled vertices' labels and
+// the signature rows (k_catch_up), then, once the update has marked its own dirty
+// vertices, the other dirty vertices' label-sorted copies and bucket offsets
+// (k_sync_sorted). Lists of up to kSyncWave entries are copied by one wave;
+// longer ones are queued (queue_big: a block each up to kBlockList entries, the
+// whole grid beyond) for k_sync_big.
+__global__ __launch_bounds__(256) void k_catch_up(CatchUp c) {
   const uint32_t lane = lane_id();
-  const uint32_t total = count ? (*count < x.n ? *count : x.n) : n_host;
+  const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x, nth = (size_t)gridDim.x * blockDim.x;
+  for (size_t t = tid >> 6; t < c.ntouched; t += nth >> 6) {
+    const uint32_t v = c.touched[t];
+    const uint32_t st = c.x.start[v], d = c.x.deg[v];
+    if (lane == 0) {
+      c.y.start[v] = st;
+      c.y.deg[v] = d;
+      c.y.cap[v] = c.x.cap[v];
+    }
+    if (d <= kSyncWave) copy_range(c.x.pool + st, c.y.pool + st, lane, 64, d);
+    else if (lane == 0) queue_big(c.q, c.qcap, &c.actl->sync_queued[0], &c.actl->sync_queued[1], d, v);
+  }
+  for (size_t r = tid; r < c.nrelabeled; r += nth) {
+    const uint32_t v = c.relabeled[r];
+    c.y.lab[v] = c.x.lab[v];
+  }
+  size_t i = tid;
+  for (; i + 3 * nth < c.nbm; i += 4 * nth) {
+    const uint64_t w0 = c.bm_x[i], w1 = c.bm_x[i + nth], w2 = c.bm_x[i + 2 * nth], w3 = c.bm_x[i + 3 * nth];
+    c.bm_y[i] = w0;
+    c.bm_y[i + nth] = w1;
+    c.bm_y[i + 2 * nth] = w2;
+    c.bm_y[i + 3 * nth] = w3;
+  }
+  for (; i < c.nbm; i += nth) c.bm_y[i] = c.bm_x[i];
+}
+
+__global__ __launch_bounds__(256) void k_sync_sorted(DevGraph x, DevGraph y, const uint32_t *list,
+                                                     const uint32_t *count, const uint32_t *skip, uint32_t *q,
+                                                     uint32_t qcap, ApplyCtl *actl) {
+  const uint32_t lane = lane_id();
+  if (held_up(actl)) return;
+  const uint32_t total = *count < x.n ? *count : x.n;
   for (uint32_t t = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; t < total; t += (gridDim.x * blockDim.x) >> 6) {
     const uint32_t v = list[t];
-    if (mode == 2) {
-      if (lane == 0) y.lab[v] = x.lab[v];
-      continue;
-    }
-    if (skip && ((skip[v >> 5] >> (v & 31)) & 1u)) continue;
+    if ((skip[v >> 5] >> (v & 31)) & 1u) continue;
     const uint32_t st = x.start[v], d = x.deg[v];
-    if (mode == 0) {
-      if (lane == 0) {
-        y.start[v] = st;
-        y.deg[v] = d;
-        y.cap[v] = x.cap[v];
-      }
-    } else {
-      if (d <= kLabelSorted) continue;
-      const uint32_t nb = x.nbuckets + 1;
-      if (lane < nb) y.loff[(size_t)v * nb + lane] = x.loff[(size_t)v * nb + lane];
-    }
-    const uint32_t *from = (mode == 0 ? x.pool : x.lpool) + st;
-    uint32_t *to = (mode == 0 ? y.pool : y.lpool) + st;
-    if (d <= kSyncWave) {
-      copy_range(from, to, lane, 64, d);
-    } else if (lane == 0) {
-      queue_big(q, qcap, &qctl[0], &qctl[1], d, v | (mode << 31));
-    }
+    if (d <= kLabelSorted) continue;
+    const uint32_t nb = x.nbuckets + 1;
+    if (lane < nb) y.loff[(size_t)v * nb + lane] = x.loff[(size_t)v * nb + lane];
+    if (d <= kSyncWave) copy_range(x.lpool + st, y.lpool + st, lane, 64, d);
+    else if (lane == 0) queue_big(q, qcap, &actl->sync_queued[2], &actl->sync_queued[3], d, v);
   }
 }
 
-__global__ __launch_bounds__(256) void k_sync_big(DevGraph x, DevGraph y, const uint32_t *q, uint32_t qcap,
-                                                  const uint32_t *qctl) {
-  for_big_lists(q, qcap, qctl[0], qctl[1], [&](uint32_t e, uint32_t first, uint32_t stride) {
-    const uint32_t v = e & 0x7FFFFFFFu;
-    const bool sorted = e >> 31;
+__global__ __launch_bounds__(256) void k_sync_big(DevGraph x, const uint32_t *from, uint32_t *to, const uint32_t *q,
+                                                  uint32_t qcap, const uint32_t *queued) {
+  for_big_lists(q, qcap, queued[0], queued[1], [&](uint32_t v, uint32_t first, uint32_t stride) {
     const uint32_t st = x.start[v];
-    copy_range((sorted ? x.lpool : x.pool) + st, (sorted ? y.lpool : y.pool) + st, first, stride, x.deg[v]);
+    copy_range(from + st, to + st, first, stride, x.deg[v]);
   });
 }
 
-__global__ void k_sync_reset(uint32_t *qctl) {
-  if (threadIdx.x < 2) qctl[threadIdx.x] = 0;
+// Blocks for n items, so many a block.
+uint32_t blocks_for(size_t n, uint32_t per_block, uint32_t most) {
+  const size_t b = (n + per_block - 1) / per_block;
+  return b == 0 ? 1u : b < most ? (uint32_t)b : most;
 }
 
 }  // namespace
 
+hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *hctl, hipStream_t s) {
+  hipLaunchKernelGGL(k_update_begin, dim3(1), dim3(64), 0, s, actl, from, hctl);
+  return hipGetLastError();
+}
+
+hipError_t launch_round_begin(ApplyCtl *actl, bool first, hipStream_t s) {
+  hipLaunchKernelGGL(k_round_begin, dim3(1), dim3(64), 0, s, actl, first ? 1 : 0);
+  return hipGetLastError();
+}
+
 hipError_t launch_apply_merge(const DevGraph &g, const BatchDev &b, unsigned long long scratch_cap,
-                              uint32_t *scratch, ApplyCtl *actl, hipStream_t s) {
+                              uint32_t *scratch, ApplyCtl *actl, uint32_t longest, hipStream_t s) {
   if (b.ntouched == 0) return hipSuccess;
-  const uint32_t blocks = (b.ntouched + kApplyWaves - 1) / kApplyWaves;
-  hipLaunchKernelGGL(k_big_reset, dim3(1), dim3(64), 0, s, actl, 1, 0);
-  hipLaunchKernelGGL(k_apply_merge, dim3(blocks < 4096 ? blocks : 4096), dim3(kApplyWaves * 64), 0, s, g, b,
-                     scratch_cap, scratch, actl);
+  hipLaunchKernelGGL(k_apply_merge, dim3(blocks_for(b.ntouched, kApplyWaves, 4096)), dim3(kApplyWaves * 64), 0, s, g,
+                     b, scratch_cap, scratch, actl);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess || longest <= kApplyWave) return e;
   hipLaunchKernelGGL(k_apply_merge_big, dim3(1024), dim3(256), 0, s, g, b, scratch, actl);
   return hipGetLastError();
 }
 
 hipError_t launch_apply_commit(const DevGraph &g, const BatchDev &b, const uint32_t *scratch,
-                               unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d,
-                               hipStream_t s, int only_failed) {
+                               unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d, bool only_failed,
+                               uint32_t longest, hipStream_t s) {
   if (b.ntouched == 0) return hipSuccess;
-  const uint32_t blocks = (b.ntouched + kApplyWaves - 1) / kApplyWaves;
-  hipLaunchKernelGGL(k_big_reset, dim3(1), dim3(64), 0, s, actl, 0, 1);
-  hipLaunchKernelGGL(k_apply_commit, dim3(blocks < 4096 ? blocks : 4096), dim3(kApplyWaves * 64), 0, s, g,
-                     b, scratch, pool_cap, actl, d, only_failed);
+  hipLaunchKernelGGL(k_apply_commit, dim3(blocks_for(b.ntouched, kApplyWaves, 4096)), dim3(kApplyWaves * 64), 0, s, g,
+                     b, scratch, pool_cap, actl, d, only_failed ? 1 : 0);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess || longest <= kApplyWave) return e;
   hipLaunchKernelGGL(k_apply_commit_big, dim3(1024), dim3(256), 0, s, g, b, scratch, actl);
   return hipGetLastError();
 }
 
-hipError_t launch_apply_commit(const DevGraph &g, const BatchDev &b, const uint32_t *scratch,
-                               unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d,
-                               hipStream_t s) {
-  return launch_apply_commit(g, b, scratch, pool_cap, actl, d, s, 0);
-}
-
-hipError_t launch_apply_commit_failed(const DevGraph &g, const BatchDev &b, const uint32_t *scratch,
-                                      unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d,
-                                      hipStream_t s) {
-  return launch_apply_commit(g, b, scratch, pool_cap, actl, d, s, 1);
-}
-
 hipError_t launch_dirty_compact(const DirtyArgs &d, uint32_t n, hipStream_t s) {
   const uint32_t nwords = (n + 31) / 32;
-  const uint32_t blocks = (nwords + 255) / 256 < 4096 ? (nwords + 255) / 256 : 4096;
-  hipLaunchKernelGGL(k_dirty_compact, dim3(blocks ? blocks : 1), dim3(256), 0, s, d, nwords);
+  hipLaunchKernelGGL(k_dirty_compact, dim3(blocks_for(nwords, 256, 4096)), dim3(256), 0, s, d, nwords);
   return hipGetLastError();
 }
 
-hipError_t launch_sync(const DevGraph &x, const DevGraph &y, const uint32_t *touched, uint32_t ntouched,
-                       const uint32_t *dirty, const uint32_t *ndirty, const uint32_t *relabeled, uint32_t nrelabeled,
-                       uint32_t *q, uint32_t qcap, uint32_t *qctl, hipStream_t s) {
-  hipLaunchKernelGGL(k_sync_reset, dim3(1), dim3(64), 0, s, qctl);
+hipError_t launch_catch_up(const CatchUp &c, uint32_t longest, hipStream_t s) {
+  const uint32_t blocks = std::max(blocks_for(c.ntouched, 4, 4096), std::max(blocks_for(c.nrelabeled, 256, 4096),
+                                                                            blocks_for(c.nbm, 1024, 4096)));
+  hipLaunchKernelGGL(k_catch_up, dim3(blocks), dim3(256), 0, s, c);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const uint32_t *no_skip = nullptr;
-  if (ntouched) {
-    hipLaunchKernelGGL(k_sync_small, dim3((ntouched + 3) / 4 < 4096 ? (ntouched + 3) / 4 : 4096), dim3(256), 0, s, x, y,
-                       touched, (const uint32_t *)nullptr, ntouched, 0u, no_skip, q, qcap, qctl);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
-  if (dirty) {
-    hipLaunchKernelGGL(k_sync_small, dim3(4096), dim3(256), 0, s, x, y, dirty, ndirty, 0u, 1u, no_skip, q, qcap, qctl);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
-  if (nrelabeled) {
-    hipLaunchKernelGGL(k_sync_small, dim3((nrelabeled + 3) / 4 < 4096 ? (nrelabeled + 3) / 4 : 4096), dim3(256), 0, s, x, y,
-                       relabeled, (const uint32_t *)nullptr, nrelabeled, 2u, no_skip, q, qcap, qctl);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
-  hipLaunchKernelGGL(k_sync_big, dim3(1024), dim3(256), 0, s, x, y, q, qcap, qctl);
+  if (e != hipSuccess || longest <= kSyncWave) return e;
+  hipLaunchKernelGGL(k_sync_big, dim3(1024), dim3(256), 0, s, c.x, (const uint32_t *)c.x.pool, c.y.pool,
+                     (const uint32_t *)c.q, c.qcap, (const uint32_t *)&c.actl->sync_queued[0]);
   return hipGetLastError();
 }
 
 hipError_t launch_sync_sorted(const DevGraph &x, const DevGraph &y, const uint32_t *dirty, const uint32_t *ndirty,
-                              const uint32_t *skip, uint32_t *q, uint32_t qcap, uint32_t *qctl, hipStream_t s) {
-  hipLaunchKernelGGL(k_sync_reset, dim3(1), dim3(64), 0, s, qctl);
+                              const uint32_t *skip, uint32_t *q, uint32_t qcap, ApplyCtl *actl, uint32_t longest,
+                              hipStream_t s) {
+  if (longest <= kLabelSorted) return hipSuccess;
+  hipLaunchKernelGGL(k_sync_sorted, dim3(blocks_for(x.n, 4, 4096)), dim3(256), 0, s, x, y, dirty, ndirty, skip, q, qcap,
+                     actl);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_sync_small, dim3(4096), dim3(256), 0, s, x, y, dirty, ndirty, 0u, 1u, skip, q, qcap, qctl);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_sync_big, dim3(1024), dim3(256), 0, s, x, y, q, qcap, qctl);
+  if (e != hipSuccess || longest <= kSyncWave) return e;
+  hipLaunchKernelGGL(k_sync_big, dim3(1024), dim3(256), 0, s, x, (const uint32_t *)x.lpool, y.lpool,
+                     (const uint32_t *)q, qcap, (const uint32_t *)&actl->sync_queued[2]);
   return hipGetLastError();
 }
 
 hipError_t launch_relabel(const DevGraph &g, const BatchDev &b, const FilterTables &ft,
-                          const DirtyArgs &d, hipStream_t s) {
+                          const DirtyArgs &d, uint32_t longest, hipStream_t s) {
   if (b.nrelabel == 0) return hipSuccess;
-  const uint32_t blocks = (b.nrelabel + 3) / 4;
-  hipLaunchKernelGGL(k_relabel, dim3(blocks < 4096 ? blocks : 4096), dim3(256), 0, s, g, b, ft, d);
+  hipLaunchKernelGGL(k_relabel, dim3(blocks_for(b.nrelabel, 4, 4096)), dim3(256), 0, s, g, b, ft, d);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess || longest <= kRelabelWave) return e;
   hipLaunchKernelGGL(k_relabel_big, dim3(1024), dim3(256), 0, s, g, b, d);
   return hipGetLastError();
 }
@@ -2372,27 +2371,32 @@ hipError_t launch_filter_full(const DevGraph &g, const FilterTables &ft, hipStre
   return hipGetLastError();
 }
 
-hipError_t launch_filter_dirty(const DevGraph &g, const FilterTables &ft, const DirtyArgs &d,
+hipError_t launch_filter_dirty(const DevGraph &g, const FilterTables &ft, const DirtyArgs &d, uint32_t longest,
                                hipStream_t s) {
-  hipLaunchKernelGGL(k_filter_light, dim3(1024), dim3(256), 0, s, g, ft, d);
+  hipLaunchKernelGGL(k_filter_light, dim3(blocks_for(g.n, 256, 1024)), dim3(256), 0, s, g, ft, d);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_filter_heavy, dim3(1024), dim3(256), 0, s, g, ft, d);
+  if (e != hipSuccess || longest <= kLight) return e;
+  hipLaunchKernelGGL(k_filter_heavy, dim3(blocks_for(g.n, 4, 1024)), dim3(256), 0, s, g, ft, d);
+  return hipGetLastError();
+}
+
+hipError_t launch_huge_reset(const HugeSort &hs, hipStream_t s) {
+  hipLaunchKernelGGL(k_huge_reset, dim3(1), dim3(64), 0, s, hs);
   return hipGetLastError();
 }
 
 hipError_t launch_lbuild(const DevGraph &g, const uint8_t *lmap, const uint32_t *list, const uint32_t *count,
-                         const HugeSort &hs, hipStream_t s) {
-  const uint32_t blocks = list ? 2048u : ((g.n + 3) / 4 < 8192 ? (g.n + 3) / 4 : 8192u);
-  hipLaunchKernelGGL(k_huge_reset, dim3(1), dim3(64), 0, s, hs);
-  hipLaunchKernelGGL(k_lbuild_pick, dim3(blocks), dim3(256), 0, s, g, list, count, hs);
+                         const HugeSort &hs, uint32_t longest, hipStream_t s) {
+  if (longest <= kLabelSorted) return hipSuccess;
+  hipLaunchKernelGGL(k_lbuild_pick, dim3(blocks_for(g.n, list ? 256 : 4, list ? 2048 : 8192)), dim3(256), 0, s, g, list,
+                     count, hs);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_lbuild, dim3(2048), dim3(256), 0, s, g, lmap, hs);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
+  hipLaunchKernelGGL(k_lbuild, dim3(blocks_for(g.n, 4, 2048)), dim3(256), 0, s, g, lmap, hs);
+  if ((e = hipGetLastError()) != hipSuccess || longest <= kLbuildBlock) return e;
   hipLaunchKernelGGL(k_lbuild_big, dim3(list ? 256u : 1024u), dim3(kLbuildWaves * 64), 0, s, g, lmap, list, count,
                      hs);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if ((e = hipGetLastError()) != hipSuccess || longest <= kHugeList) return e;
   hipLaunchKernelGGL(k_lbuild_huge_count, dim3(512), dim3(kLbuildWaves * 64), 0, s, g, lmap, hs);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL(k_lbuild_huge_scatter, dim3(512), dim3(kLbuildWaves * 64), 0, s, g, lmap, hs);
@@ -2400,9 +2404,9 @@ hipError_t launch_lbuild(const DevGraph &g, const uint8_t *lmap, const uint32_t 
 }
 
 hipError_t launch_seed(const SeedArgs &a, hipStream_t s) {
-  if (a.nrec == 0 || a.nplans == 0) return hipSuccess;
-  const uint32_t blocks = (a.nrec + 255) / 256;
-  hipLaunchKernelGGL(k_seed, dim3(blocks < 4096 ? blocks : 4096), dim3(256), 0, s, a);
+  const uint32_t nrec = a.nrec[0] + a.nrec[1];
+  if (nrec == 0 || a.nplans == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_seed, dim3(blocks_for(nrec, 256, 4096)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -2424,19 +2428,14 @@ hipError_t launch_dfs(const DfsArgs &a, uint32_t blocks, uint32_t waves_per_bloc
 }
 
 void round_node_params(RoundNodeArgs &st, uint32_t blocks, uint32_t waves_per_block,
-                       uint32_t max_query_vertices, hipKernelNodeParams *reset, hipKernelNodeParams *seed0,
-                       hipKernelNodeParams *seed1, hipKernelNodeParams *dfs) {
-  st.no_actl = nullptr;
-  st.no_tc = nullptr;
-  st.no_counts = nullptr;
-  st.no_ncounts = 0;
+                       uint32_t max_query_vertices, hipKernelNodeParams *reset, hipKernelNodeParams *seed,
+                       hipKernelNodeParams *dfs) {
   st.reset_params[0] = &st.ctl;
-  st.reset_params[1] = &st.no_actl;
-  st.reset_params[2] = &st.no_tc;
-  st.reset_params[3] = &st.no_counts;
-  st.reset_params[4] = &st.no_ncounts;
-  st.reset_params[5] = &st.idle;
-  st.reset_params[6] = &st.nidle;
+  st.reset_params[1] = &st.tuple_count;
+  st.reset_params[2] = &st.counts;
+  st.reset_params[3] = &st.ncounts;
+  st.reset_params[4] = &st.idle;
+  st.reset_params[5] = &st.nidle;
   *reset = hipKernelNodeParams{};
   reset->func = reinterpret_cast<void *>(&k_ctl_reset);
   reset->gridDim = dim3(1);
@@ -2444,18 +2443,14 @@ void round_node_params(RoundNodeArgs &st, uint32_t blocks, uint32_t waves_per_bl
   reset->sharedMemBytes = 0;
   reset->kernelParams = st.reset_params;
   reset->extra = nullptr;
-  hipKernelNodeParams *sp[2] = {seed0, seed1};
-  for (int i = 0; i < 2; i++) {
-    st.seed_params[i][0] = &st.seed[i];
-    const uint32_t b = st.seed[i].nrec ? (st.seed[i].nrec + 255) / 256 : 1u;
-    *sp[i] = hipKernelNodeParams{};
-    sp[i]->func = reinterpret_cast<void *>(&k_seed);
-    sp[i]->gridDim = dim3(b < 4096 ? b : 4096);
-    sp[i]->blockDim = dim3(256);
-    sp[i]->sharedMemBytes = 0;
-    sp[i]->kernelParams = st.seed_params[i];
-    sp[i]->extra = nullptr;
-  }
+  st.seed_params[0] = &st.seed;
+  *seed = hipKernelNodeParams{};
+  seed->func = reinterpret_cast<void *>(&k_seed);
+  seed->gridDim = dim3(blocks_for(st.seed.nrec[0] + st.seed.nrec[1], 256, 4096));
+  seed->blockDim = dim3(256);
+  seed->sharedMemBytes = 0;
+  seed->kernelParams = st.seed_params;
+  seed->extra = nullptr;
   st.chunk_levels = max_query_vertices > 3 ? max_query_vertices - 3 : 1;
   st.dfs_params[0] = &st.dfs;
   st.dfs_params[1] = &st.chunk_levels;
@@ -2493,15 +2488,9 @@ int dfs_max_blocks_per_cu(uint32_t waves_per_block, uint32_t max_query_vertices)
   }
 }
 
-hipError_t launch_ctl_reset(DfsCtl *ctl, ApplyCtl *actl, unsigned long long *tuple_count,
-                            unsigned long long *counts, uint32_t ncounts, IdleWord *idle, uint32_t nidle,
-                            hipStream_t s) {
-  hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(256), 0, s, ctl, actl, tuple_count, counts, ncounts, idle, nidle);
-  return hipGetLastError();
-}
-
-hipError_t launch_scratch_reset(ApplyCtl *actl, hipStream_t s) {
-  hipLaunchKernelGGL(k_scratch_reset, dim3(1), dim3(64), 0, s, actl);
+hipError_t launch_ctl_reset(DfsCtl *ctl, unsigned long long *tuple_count, unsigned long long *counts,
+                            uint32_t ncounts, IdleWord *idle, uint32_t nidle, hipStream_t s) {
+  hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(256), 0, s, ctl, tuple_count, counts, ncounts, idle, nidle);
   return hipGetLastError();
 }
 

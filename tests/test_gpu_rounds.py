@@ -97,3 +97,46 @@ def test_leaf_sets_at_their_limits(da, db, labels):
             assert pos.tolist() == want["pos"] and neg.tolist() == want["neg"], kw
         finally:
             eng.close()
+
+
+@pytest.mark.parametrize("limit", [64, 2048, 4096, 8192, 65536])
+def test_lists_that_grow_past_a_kernel_limit(limit):
+    """A hub's list grows by one entry at a time from just below a length at which
+    an update needs one more kernel to just above it, and shrinks again, one batch
+    per call and pipelined: counts, graph and candidate bitmaps against the oracle."""
+    n = limit + 40
+    rng = np.random.default_rng(limit)
+    lab = rng.integers(0, 3, n).astype(np.uint32)
+    k = limit - 2
+    u = np.concatenate([np.zeros(k, np.uint32), rng.integers(1, n, 300).astype(np.uint32)])
+    v = np.concatenate([np.arange(1, k + 1, dtype=np.uint32), rng.integers(1, n, 300).astype(np.uint32)])
+    keep = u != v
+    u, v = u[keep], v[keep]
+    tri = np.array([(0, 1), (1, 2), (0, 2)], np.uint32)
+    queries = [(3, np.array([0, 1, 2], np.uint32), tri[:, 0].copy(), tri[:, 1].copy()), one_label("path3")]
+    new = np.arange(k + 1, k + 7, dtype=np.uint32)
+    batches = [(np.ones(1, np.uint8), np.zeros(1, np.uint32), x[None], lab[x][None]) for x in new]
+    # delete one and insert one (the hub changes its label), so that the update runs beside a round
+    batches += [(np.array([0, 1], np.uint8), np.array([0, x], np.uint32), np.array([x, x + 9], np.uint32),
+                 np.full(2, (b + 1) % 3, np.uint32)) for b, x in enumerate(new[:3])]
+    batches += [(np.array([1, 0], np.uint8), np.array([0, 0], np.uint32), np.array([x, x + 3], np.uint32),
+                 np.full(2, b, np.uint32)) for b, x in enumerate(new[:3])]
+    want = O.run_stream(O.Graph(n, lab, u, v), [O.Query(*q) for q in queries], batches)
+    one, many = (E.Engine((n, lab, u, v), queries) for _ in range(2))
+    try:
+        pos, neg, _ = many.process_batches(batches)
+        for i, b in enumerate(batches):
+            p, m = one.process_batch(*b)
+            assert p.tolist() == want[i]["pos"] == pos[i].tolist() and m.tolist() == want[i]["neg"] == neg[i].tolist(), i
+        g = O.Graph(n, lab, u, v)
+        O.run_stream(g, [O.Query(*queries[0])], batches)
+        off, nb, dl = g.export()
+        cand = g.candidates(O.Query(*queries[0]))
+        for eng in (one, many):
+            o2, n2, l2 = eng.graph()
+            assert np.array_equal(off, o2) and np.array_equal(nb, n2) and np.array_equal(dl, l2)
+            for q in range(3):
+                assert np.array_equal(eng.candidates(0, q), cand[q].astype(bool)), q
+    finally:
+        one.close()
+        many.close()
