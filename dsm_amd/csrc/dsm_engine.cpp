@@ -186,8 +186,9 @@ struct dsm_engine {
   PinnedBuf<uint32_t> hrec;           // a round's records (pinned staging)
   // the copies out of hbuf / hrec: done before either is filled again
   hipEvent_t ev_hbuf = nullptr, ev_hrec = nullptr;
-  DevBuf<uint32_t> ndeg, fail;
+  DevBuf<uint32_t> tinfo;             // per touched vertex: new degree, new inserts, slot, state
   DevBuf<unsigned long long> soff;
+  DevBuf<uint2> segs;                 // pieces of the touched lists
   DevBuf<ApplyCtl> actl;
   PinnedBuf<ApplyCtl> h_actl;
   // DFS
@@ -770,9 +771,6 @@ int upload_tables(dsm_engine *e) {
       HIPCHK(hipMalloc((void **)&e->tuples, bytes));
     }
   }
-  HIPCHK(e->ndeg.alloc(1024));
-  HIPCHK(e->fail.alloc(1024));
-  HIPCHK(e->soff.alloc(1024));
   return DSM_OK;
 }
 
@@ -1090,6 +1088,11 @@ struct RoundArrays {
   const uint32_t *last_touched, *last_relabel;
 };
 
+// A bound on the pieces of T touched lists and their inserts.
+size_t max_segs(const dsm_engine *e, size_t T, size_t inserts) {
+  return T + (size_t)((e->pool_cap + inserts) / kApplySeg);
+}
+
 // Sends a round's arrays in one copy.
 int upload_round(dsm_engine *e, const Slice &sl, const HostDelta *relabels, bool last, RoundArrays &out) {
   static const std::vector<uint32_t> none;
@@ -1100,9 +1103,8 @@ int upload_round(dsm_engine *e, const Slice &sl, const HostDelta *relabels, bool
   size_t off[10] = {};
   for (int i = 0; i < 9; i++) off[i + 1] = off[i] + parts[i]->size();
   const size_t total = off[9], R = rl_v.size();
-  // prefix counts and big-list indices of the hub lists that the whole grid copies
-  const size_t o_gi = total, o_gd = o_gi + sl.ins.size() + T, o_bm = o_gd + sl.del.size() + T, o_bc = o_bm + T,
-               o_rb = o_bc + T, dtotal = o_rb + R;
+  // the changes' positions, and the relabelled vertices with long lists
+  const size_t o_ri = total, o_rd = o_ri + sl.ins.size(), o_rb = o_rd + sl.del.size(), dtotal = o_rb + R;
   // an earlier round may still read the arrays, its copy the staging buffer
   if (dtotal > e->bbuf.n) HIPCHK(hipStreamSynchronize(e->stream));
   HIPCHK(hipEventSynchronize(e->ev_hbuf));
@@ -1111,9 +1113,10 @@ int upload_round(dsm_engine *e, const Slice &sl, const HostDelta *relabels, bool
   for (int i = 0; i < 9; i++) std::copy(parts[i]->begin(), parts[i]->end(), e->hbuf.p + off[i]);
   if (total) HIPCHK(hipMemcpyAsync(e->bbuf.p, e->hbuf.p, total * 4, hipMemcpyHostToDevice, e->stream));
   HIPCHK(hipEventRecord(e->ev_hbuf, e->stream));
-  HIPCHK(e->ndeg.ensure(T));
-  HIPCHK(e->fail.ensure(T));
+  if (T > e->soff.n || max_segs(e, T, sl.ins.size()) > e->segs.n) HIPCHK(hipStreamSynchronize(e->stream));
   HIPCHK(e->soff.ensure(T));
+  HIPCHK(e->tinfo.ensure(4 * e->soff.n));
+  HIPCHK(e->segs.ensure(max_segs(e, T, sl.ins.size())));
   BatchDev b{};
   b.ntouched = T;
   b.tv = e->bbuf.p + off[0];
@@ -1125,13 +1128,14 @@ int upload_round(dsm_engine *e, const Slice &sl, const HostDelta *relabels, bool
   b.rl_v = e->bbuf.p + off[5];
   b.rl_l = e->bbuf.p + off[6];
   b.rl_big = e->bbuf.p + o_rb;
-  b.ndeg = e->ndeg.p;
+  b.ndeg = e->tinfo.p;
+  b.nnew = e->tinfo.p + e->soff.n;
+  b.dst = e->tinfo.p + 2 * e->soff.n;
+  b.state = e->tinfo.p + 3 * e->soff.n;
   b.soff = e->soff.p;
-  b.fail = e->fail.p;
-  b.gicum = e->bbuf.p + o_gi;
-  b.gdcum = e->bbuf.p + o_gd;
-  b.big_merge = e->bbuf.p + o_bm;
-  b.big_commit = e->bbuf.p + o_bc;
+  b.ri = e->bbuf.p + o_ri;
+  b.rd = e->bbuf.p + o_rd;
+  b.segs = e->segs.p;
   out.b = b;
   out.last_touched = e->bbuf.p + off[7];
   out.last_relabel = e->bbuf.p + off[8];
@@ -1149,13 +1153,6 @@ int ensure_scratch(dsm_engine *e, size_t inserts) {
   return DSM_OK;
 }
 
-int enqueue_apply(dsm_engine *e, const BatchDev &b, uint32_t longest) {
-  HIPCHK(launch_apply_merge(e->dev_graph(), b, e->scratch_cap, e->scratch.p, e->actl.p, longest, e->stream));
-  HIPCHK(launch_apply_commit(e->dev_graph(), b, e->scratch.p, e->pool_cap, e->actl.p, e->dirty(), false, longest,
-                             e->stream));
-  return DSM_OK;
-}
-
 // Waits for the update's status.
 int take_status(dsm_engine *e) {
   HIPCHK(hipMemcpyAsync(e->h_actl.p, e->actl.p, sizeof(ApplyCtl), hipMemcpyDeviceToHost, e->stream));
@@ -1168,12 +1165,11 @@ int take_status(dsm_engine *e) {
 
 // Grows the pool for the commits that found no room and tries them again (the
 // status has been taken; their merged lists are in the scratch).
-int retry_commits(dsm_engine *e, const BatchDev &b, uint32_t longest) {
+int retry_commits(dsm_engine *e, const BatchDev &b) {
   for (int attempt = 0; e->h_actl.p->overflow && attempt < 4; attempt++) {
     if (int rc = grow_pool(e, e->pool_cap / 2 + (1ull << 22))) return rc;
-    HIPCHK(launch_round_begin(e->actl.p, false, e->stream));
-    HIPCHK(launch_apply_commit(e->dev_graph(), b, e->scratch.p, e->pool_cap, e->actl.p, e->dirty(), true, longest,
-                               e->stream));
+    HIPCHK(launch_commit_again(e->dev_graph(), b, e->scratch.p, e->pool_cap, e->actl.p, e->dirty(),
+                               e->h_actl.p->nsegs, e->stream));
     if (int rc = take_status(e)) return rc;
   }
   if (e->h_actl.p->overflow) return e->fail_msg(DSM_ENOMEM, "neighbour pool could not be grown");
@@ -1377,13 +1373,17 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine:
         HIPCHK(launch_catch_up(c, before, e->stream));
       }
     } else {
-      HIPCHK(launch_round_begin(e->actl.p, true, e->stream));
+      HIPCHK(launch_round_begin(e->actl.p, e->stream));
     }
     if (int rc = ensure_scratch(e, sl.ins.size())) return rc;
-    if (int rc = enqueue_apply(e, ra.b, longest)) return rc;
+    // pieces: one a list, and what no list can go past
+    const size_t segs = std::min<size_t>(max_segs(e, sl.tv.size(), sl.ins.size()),
+                                         sl.tv.size() * (1 + (size_t)(longest / kApplySeg)));
+    HIPCHK(launch_apply(e->dev_graph(), ra.b, e->scratch.p, e->scratch_cap, e->pool_cap, e->actl.p, e->dirty(), segs,
+                        e->stream));
     if (!final_round) {
       if (int rc = take_status(e)) return rc;
-      if (int rc = retry_commits(e, ra.b, longest)) return rc;
+      if (int rc = retry_commits(e, ra.b)) return rc;
     }
   }
   e->stats.touched_vertices = T;
@@ -1405,7 +1405,7 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine:
     if (int rc = take_status(e)) return rc;
     if (!e->h_actl.p->overflow) break;
     // the kernels above waited for this
-    if (int rc = retry_commits(e, ra.b, longest)) return rc;
+    if (int rc = retry_commits(e, ra.b)) return rc;
   }
   e->lpool_stale = false;
   e->stats.relocated_vertices = e->h_actl.p->relocated;
@@ -1414,7 +1414,7 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine:
 
 // Blocks per CU of a DFS shape: the occupancy limit and, with overlap_apply,
 // at most what leaves 32 KB of the CU's LDS to the update kernels that run
-// beside a pipelined round (k_apply_merge takes 16 KB per block). A shape
+// beside a pipelined round (k_apply_rank takes 16 KB per block). A shape
 // that fills the LDS makes them wait for the round.
 uint32_t dfs_bpc(const dsm_engine *e, uint32_t wpb) {
   uint32_t b = (uint32_t)std::max(1, dfs_max_blocks_per_cu(wpb, e->max_qn));

@@ -115,19 +115,16 @@ struct alignas(64) ApplyCtl {
   uint32_t nheavy;                  // dirty vertices re-filtered by a whole wave
   uint32_t relabeled;
   uint32_t nrelabel_big;            // relabelled vertices whose neighbours the whole grid marks
-  uint32_t nmerge_big;              // touched vertices whose merge the whole grid copies
-  uint32_t ncommit_big;             // touched vertices whose commit the whole grid copies
+  uint32_t nsegs;                   // pieces of the touched lists (kApplySeg entries) on BatchDev::segs
   uint32_t merge_overflow;          // merges that found no room in the scratch (must stay 0)
   uint32_t filter_bits;             // candidate bits the re-filter writes (work measure)
   unsigned long long filter_entries;  // list entries of the vertices re-filtered (work measure)
   // of the big lists above, those longer than kBlockList (split over the whole
   // grid; queued from the back of the same arrays, the rest from the front)
   uint32_t nrelabel_huge;
-  uint32_t nmerge_huge;
-  uint32_t ncommit_huge;
   uint32_t max_deg;                 // no list has been longer (never lowered): kernels of longer lists are skipped
   uint32_t sync_queued[4];          // long lists queued by the catch-up (block, grid) and the sorted catch-up
-  uint32_t pad[8];
+  uint32_t pad[10];
 };
 static_assert(sizeof(ApplyCtl) == 128, "apply status layout");
 
@@ -165,16 +162,14 @@ struct BatchDev {
   const uint32_t *doff;     // [ntouched+1] into del
   const uint32_t *ins;
   const uint32_t *del;
-  uint32_t *ndeg;           // [ntouched] new degree (merge -> commit)
-  unsigned long long *soff; // [ntouched] scratch offset
-  uint32_t *fail;           // [ntouched] commit found no room
-  // lists longer than kApplyWave: their merge and commit copies are split over
-  // the whole grid. icum/dcum of touched vertex t live at ioff[t] + t and
-  // doff[t] + t; big_merge / big_commit list the vertices (indices t).
-  uint32_t *gicum;          // [ins + ntouched]
-  uint32_t *gdcum;          // [del + ntouched]
-  uint32_t *big_merge;      // [ntouched]
-  uint32_t *big_commit;     // [ntouched]
+  // what the kernels of the round pass on, per touched vertex: the new degree,
+  // how many of its inserts are new, where its merged list goes in the scratch
+  // and where it ends up in the pool, and how far it is
+  uint32_t *ndeg, *nnew, *dst, *state;
+  unsigned long long *soff;
+  uint32_t *ri;             // [ins] positions in the old list of t's new inserts, ascending, from ioff[t]
+  uint32_t *rd;             // [del] positions of its deletes that are there, ascending, from doff[t]
+  uint2 *segs;              // (t, piece): the touched lists in pieces of kApplySeg entries
   uint32_t nrelabel;
   const uint32_t *rl_v;
   const uint32_t *rl_l;     // device label (already clamped)
@@ -346,7 +341,13 @@ hipError_t launch_cluster_heavy(const ClusterArgs &a, uint32_t blocks, hipStream
 // that the whole update is enqueued at once and the host looks at the status
 // when it is done. `longest` is a length no list exceeds: kernels that only work
 // on longer lists are not launched.
-constexpr uint32_t kApplyWave = 8192;    // longer lists are merged and committed by the whole grid
+constexpr uint32_t kApplySeg = 1024;     // entries of a touched list a wave merges or commits at a time
+// states of a touched vertex
+constexpr uint32_t kInPlace = 0;   // its list fits its slot: merged into the scratch, then committed
+constexpr uint32_t kDirect = 1;    // merged into a new slot
+constexpr uint32_t kNoRoom = 2;    // merged into the scratch, needs a slot the pool has no room for
+constexpr uint32_t kRetried = 3;   // has one now: to be committed
+constexpr uint32_t kDone = 4;      // committed by an earlier try
 constexpr uint32_t kRelabelWave = 2048;  // neighbours of longer lists are marked by the whole grid
 constexpr uint32_t kSyncWave = 4096;     // longer lists are brought up to date by the whole grid
 constexpr uint32_t kLbuildBlock = 4096;  // label-sorted copies of longer lists are built by a block
@@ -355,14 +356,16 @@ constexpr uint32_t kLight = 64;          // dirty vertices of higher degree are 
 // Takes over the status `from` (null: keeps its own) and clears what an update
 // counts, also hctl[4] (HugeSort::ctl).
 hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *hctl, hipStream_t s);
-// Another round of merges and commits of one update (first: before its merges;
-// else before commits that are tried again).
-hipError_t launch_round_begin(ApplyCtl *actl, bool first, hipStream_t s);
-hipError_t launch_apply_merge(const DevGraph &g, const BatchDev &b, unsigned long long scratch_cap,
-                              uint32_t *scratch, ApplyCtl *actl, uint32_t longest, hipStream_t s);
-hipError_t launch_apply_commit(const DevGraph &g, const BatchDev &b, const uint32_t *scratch,
-                               unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d, bool only_failed,
-                               uint32_t longest, hipStream_t s);
+// Clears what the merges of one round count (updates with more than one).
+hipError_t launch_round_begin(ApplyCtl *actl, hipStream_t s);
+// The merges and commits of a round; max_segs bounds the pieces.
+hipError_t launch_apply(const DevGraph &g, const BatchDev &b, uint32_t *scratch, unsigned long long scratch_cap,
+                        unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d, size_t max_segs,
+                        hipStream_t s);
+// The commits that found no room, again.
+hipError_t launch_commit_again(const DevGraph &g, const BatchDev &b, const uint32_t *scratch,
+                               unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d, size_t max_segs,
+                               hipStream_t s);
 // The dirty list (d.list, its length added to d.actl->ndirty) from the dirty
 // bits of the update's n vertices.
 hipError_t launch_dirty_compact(const DirtyArgs &d, uint32_t n, hipStream_t s);

@@ -1,7 +1,7 @@
 // HIP kernels of the MI355X continuous subgraph matching engine (gfx950,
 // wave64). Integer work only; no MFMA.
 //
-//   k_apply_merge / k_apply_commit (+ _big for hub lists)
+//   k_apply_plan / k_apply_rank / k_apply_merge / k_apply_commit
 //                                   in-place batch update of the slack CSR
 //                                   (the reference rebuilds the whole graph on
 //                                   the host, cpuGraph.cpp:521-607, and
@@ -164,233 +164,220 @@ __device__ __forceinline__ void copy_range(const uint32_t *__restrict__ from, ui
   if (first < len - done) to[done + first] = from[done + first];
 }
 
-// One wave per touched vertex: new list = (A \ D) u I written to scratch.
-// I and D are sorted and hold at most kMaxVertexChanges entries each; every
-// key has a single final operation, so I and D are disjoint.
-__global__ __launch_bounds__(kApplyWaves * 64) void k_apply_merge(DevGraph g, BatchDev b,
-                                                                  unsigned long long scratch_cap,
-                                                                  uint32_t *scratch, ApplyCtl *actl) {
-  __shared__ uint16_t s_icum[kApplyWaves][kMaxVertexChanges + 1];
-  __shared__ uint16_t s_dcum[kApplyWaves][kMaxVertexChanges + 1];
-  // up to kStageChanges inserts and deletes of the wave's vertex, staged in
-  // LDS for the per-entry searches (more are searched in global memory)
-  constexpr uint32_t kStageChanges = 128;
-  __shared__ uint32_t s_I[kApplyWaves][kStageChanges], s_D[kApplyWaves][kStageChanges];
-  const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
-  uint16_t *icum = s_icum[wv];
-  uint16_t *dcum = s_dcum[wv];
-  for (uint32_t t = blockIdx.x * kApplyWaves + wv; t < b.ntouched; t += gridDim.x * kApplyWaves) {
-    const uint32_t x = b.tv[t];
-    const uint32_t *A = g.pool + g.start[x];
-    const uint32_t na = g.deg[x];
-    const uint32_t i0 = b.ioff[t], ni = b.ioff[t + 1] - i0;
-    const uint32_t d0 = b.doff[t], nd = b.doff[t + 1] - d0;
-    const uint32_t *I = b.ins + i0;
-    const uint32_t *D = b.del + d0;
-    wave_sync();  // the previous vertex's stage is no longer read
-    if (ni <= kStageChanges && nd <= kStageChanges) {
-      for (uint32_t j = lane; j < ni; j += 64) s_I[wv][j] = I[j];
-      for (uint32_t j = lane; j < nd; j += 64) s_D[wv][j] = D[j];
-      wave_sync();
-      I = s_I[wv];
-      D = s_D[wv];
+// An update of the lists, new list = (A \ D) u I per touched vertex, in four
+// kernels. I and D are sorted and hold at most kMaxVertexChanges entries each;
+// every key has a single final operation, so I and D are disjoint.
+//
+//   k_apply_plan    a lane per vertex: room in the scratch for its merged list and
+//                   its pieces of kApplySeg entries, one counter add per wave
+//   k_apply_rank    a wave per vertex: where its changes fall in the old list, its
+//                   new degree and, when it outgrows its slot, a new one; writes
+//                   the new inserts to their places
+//   k_apply_merge   a wave per piece of the old lists: copies it, shifted by the
+//                   changes before it
+//   k_apply_commit  a wave per piece of the new lists: back into the slots of the
+//                   lists that stay in place; a lane sets the vertex's record
+//
+// The lists are long and their changes few (500,000 vertices, 8 M edges, batches
+// of 32,768 records: 31,000 lists of 1,100 entries in the mean, two changes each),
+// so the pieces nearly all are plain copies; what counts is that they are many and
+// alike, and that no counter is added to once per vertex. With a wave per list (a
+// block or the grid for long ones), changes searched for every entry and a
+// counter add per list, merge and commit of such a batch took 870 us.
+
+// The number of p[0, n) below x, for the whole wave; p ascends.
+__device__ __forceinline__ uint32_t wave_count_below(const uint32_t *p, uint32_t n, uint32_t x) {
+  if (n <= 64) return (uint32_t)__popcll(ballot(lane_id() < n && p[min(lane_id(), n - 1)] < x));
+  return lower_bound(p, n, x);
+}
+
+__global__ __launch_bounds__(256) void k_apply_plan(DevGraph g, BatchDev b, unsigned long long scratch_cap,
+                                                    ApplyCtl *actl) {
+  for (uint32_t t0 = (blockIdx.x * blockDim.x + threadIdx.x) & ~63u; t0 < b.ntouched; t0 += gridDim.x * blockDim.x) {
+    const uint32_t t = t0 + lane_id();
+    uint32_t len = 0;  // of the merged list, at most
+    if (t < b.ntouched) len = g.deg[b.tv[t]] + b.ioff[t + 1] - b.ioff[t];
+    const uint32_t ns = t < b.ntouched ? max(1u, (len + kApplySeg - 1) / kApplySeg) : 0u;
+    uint32_t most = len;
+    for (int o = 32; o >= 1; o >>= 1) most = max(most, (uint32_t)__shfl_xor(most, o));
+    // the sum of 64 lists may pass 32 bits
+    unsigned long long end = len;
+    for (int o = 1; o < 64; o <<= 1) {
+      const unsigned long long y = __shfl_up(end, o);
+      if (lane_id() >= (uint32_t)o) end += y;
     }
-    // exclusive prefix of "insert is new" and "delete hits"
-    uint32_t run = 0;
-    for (uint32_t c = 0; c < ni; c += 64) {
-      const uint32_t j = c + lane;
-      const bool fl = j < ni && !contains(A, na, I[j]);
-      const uint64_t m = ballot(fl);
-      if (j < ni) icum[j] = (uint16_t)(run + mbcnt(m));
-      run += __popcll(m);
-    }
-    const uint32_t nnew = run;
-    run = 0;
-    for (uint32_t c = 0; c < nd; c += 64) {
-      const uint32_t j = c + lane;
-      const bool fl = j < nd && contains(A, na, D[j]);
-      const uint64_t m = ballot(fl);
-      if (j < nd) dcum[j] = (uint16_t)(run + mbcnt(m));
-      run += __popcll(m);
-    }
-    const uint32_t nhit = run;
-    if (lane == 0) {
-      icum[ni] = (uint16_t)nnew;
-      dcum[nd] = (uint16_t)nhit;
-    }
-    wave_sync();
-    const uint32_t newdeg = na - nhit + nnew;
-    if (na > kApplyWave) {
-      // the prefix counts go to global memory; k_apply_merge_big copies
-      for (uint32_t j = lane; j <= ni; j += 64) b.gicum[i0 + t + j] = icum[j];
-      for (uint32_t j = lane; j <= nd; j += 64) b.gdcum[d0 + t + j] = dcum[j];
-    }
+    uint32_t nsegs;
+    const uint32_t before = wave_excl_sum(ns, &nsegs);
+    const unsigned long long all = bcast64(__shfl(end, 63));
     unsigned long long so = 0;
-    if (lane == 0) so = atomicAdd(&actl->scratch_used, (unsigned long long)(na + nnew));
+    uint32_t at = 0;
+    if (lane_id() == 0) {
+      so = atomicAdd(&actl->scratch_used, all);
+      at = atomicAdd(&actl->nsegs, nsegs);
+      if (most > ld_relaxed(&actl->max_deg)) atomicMax(&actl->max_deg, most);
+      if (so + all > scratch_cap) atomicAdd(&actl->merge_overflow, 1u);  // sized by the host so that this cannot happen
+    }
     so = bcast64(so);
-    if (so + na + nnew > scratch_cap) {  // sized by the host so that this cannot happen
-      if (lane == 0) {
-        b.ndeg[t] = na;
-        b.soff[t] = ~0ull;
-        atomicAdd(&actl->merge_overflow, 1u);
-      }
-      continue;
-    }
-    uint32_t *out = scratch + so;
-    if (na > kApplyWave) {
-      if (lane == 0) {
-        b.ndeg[t] = newdeg;
-        b.soff[t] = so;
-        queue_big(b.big_merge, b.ntouched, &actl->nmerge_big, &actl->nmerge_huge, na, t);
-      }
-      wave_sync();
-      continue;
-    }
-    for (uint32_t j = lane; j < na; j += 64) {
-      const uint32_t a = A[j];
-      const uint32_t p = lower_bound(D, nd, a);
-      if (p < nd && D[p] == a) continue;
-      const uint32_t q = lower_bound(I, ni, a);
-      out[j - dcum[p] + icum[q]] = a;
-    }
-    for (uint32_t j = lane; j < ni; j += 64) {
-      if (icum[j + 1] == icum[j]) continue;  // already present
-      const uint32_t i = I[j];
-      const uint32_t r = lower_bound(A, na, i);
-      const uint32_t p = lower_bound(D, nd, i);
-      out[r - dcum[p] + icum[j]] = i;
-    }
-    if (lane == 0) {
-      b.ndeg[t] = newdeg;
-      b.soff[t] = so;
-    }
-    wave_sync();
+    at = bcast(at) + before;
+    if (t >= b.ntouched) continue;
+    b.soff[t] = so + end - len;
+    for (uint32_t k = 0; k < ns; k++) b.segs[at + k] = uint2{t, k};
   }
 }
 
-// The merge copies of the lists longer than kApplyWave (for_big_lists splits
-// them), with the prefix counts k_apply_merge stored.
-__global__ __launch_bounds__(256) void k_apply_merge_big(DevGraph g, BatchDev b, uint32_t *scratch,
-                                                         const ApplyCtl *actl) {
-  // the list's inserts and deletes with their prefix counts, staged in LDS:
-  // every chunk of the list searches them
-  __shared__ uint32_t s_I[kMaxVertexChanges], s_D[kMaxVertexChanges];
-  __shared__ uint32_t s_icum[kMaxVertexChanges + 1], s_dcum[kMaxVertexChanges + 1];
-  const uint32_t lane = lane_id();
-  for_big_lists(b.big_merge, b.ntouched, actl->nmerge_big, actl->nmerge_huge, [&](uint32_t t, uint32_t tid,
-                                                                                   uint32_t nth) {
-    const uint32_t x = b.tv[t];
-    const uint32_t na = g.deg[x];
-    // waves of the share: the thread's wave index and the number of waves
-    const uint32_t gw = tid >> 6, nw = nth >> 6;
-    const uint32_t *A = g.pool + g.start[x];
-    const uint32_t i0 = b.ioff[t], ni = b.ioff[t + 1] - i0;
-    const uint32_t d0 = b.doff[t], nd = b.doff[t + 1] - d0;
-    __syncthreads();  // the previous list's stage is no longer read
-    for (uint32_t j = threadIdx.x; j <= ni; j += blockDim.x) {
-      if (j < ni) s_I[j] = b.ins[i0 + j];
-      s_icum[j] = b.gicum[i0 + t + j];
-    }
-    for (uint32_t j = threadIdx.x; j <= nd; j += blockDim.x) {
-      if (j < nd) s_D[j] = b.del[d0 + j];
-      s_dcum[j] = b.gdcum[d0 + t + j];
-    }
-    __syncthreads();
-    const uint32_t *I = s_I;
-    const uint32_t *D = s_D;
-    const uint32_t *icum = s_icum;
-    const uint32_t *dcum = s_dcum;
-    uint32_t *out = scratch + b.soff[t];
-    // waves take 64-entry chunks of A in turn; the deletes and inserts that
-    // fall inside a chunk's key range are found once per chunk, so each entry
-    // searches only that (usually empty) range
-    for (uint32_t c0 = gw * 64; c0 < na; c0 += nw * 64) {
-      const uint32_t c1 = c0 + 64 < na ? c0 + 64 : na;
-      const uint32_t lo_key = A[c0], hi_key = A[c1 - 1];
-      const uint32_t p0 = lower_bound(D, nd, lo_key), p1 = lower_bound(D, nd, hi_key + 1);
-      const uint32_t q0 = lower_bound(I, ni, lo_key), q1 = lower_bound(I, ni, hi_key + 1);
-      const uint32_t j = c0 + lane;
-      if (j < c1) {
-        const uint32_t a = A[j];
-        const uint32_t p = p0 + lower_bound(D + p0, p1 - p0, a);
-        if (!(p < nd && D[p] == a)) {
-          const uint32_t q = q0 + lower_bound(I + q0, q1 - q0, a);
-          out[j - dcum[p] + icum[q]] = a;
-        }
-      }
-    }
-    for (uint32_t j = tid; j < ni; j += nth) {
-      if (icum[j + 1] == icum[j]) continue;
-      const uint32_t i = I[j];
-      const uint32_t rr = lower_bound(A, na, i);
-      const uint32_t p = lower_bound(D, nd, i);
-      out[rr - dcum[p] + icum[j]] = i;
-    }
-  });
+// A slot for t's merged list of nd entries: its own, a new one from the pool's
+// bump pointer, or none.
+__device__ __forceinline__ uint32_t take_slot(const DevGraph &g, const BatchDev &b, uint32_t t, uint32_t x, uint32_t nd,
+                                              unsigned long long pool_cap, ApplyCtl *actl, uint32_t fits,
+                                              uint32_t moves) {
+  if (nd <= g.cap[x]) {
+    b.dst[t] = g.start[x];
+    return fits;
+  }
+  const uint32_t newcap = nd + nd / 4 + 8;
+  const unsigned long long base = atomicAdd(&actl->pool_used, (unsigned long long)newcap);
+  if (base + newcap > pool_cap) {
+    atomicAdd(&actl->overflow, 1u);
+    return kNoRoom;
+  }
+  atomicAdd(&actl->relocated, 1u);
+  b.dst[t] = (uint32_t)base;
+  return moves;
 }
 
-// One wave per touched vertex: copy the merged list back into its slot, or
-// into a new, larger slot taken from the pool's bump pointer. A vertex that
-// finds no room keeps its old list and is flagged for a retry after the host
-// grows the pool. With only_failed, only flagged vertices are processed.
-__global__ __launch_bounds__(kApplyWaves * 64) void k_apply_commit(DevGraph g, BatchDev b,
-                                                                   const uint32_t *scratch,
-                                                                   unsigned long long pool_cap,
-                                                                   ApplyCtl *actl, DirtyArgs d,
-                                                                   int only_failed) {
+__global__ __launch_bounds__(kApplyWaves * 64) void k_apply_rank(DevGraph g, BatchDev b, uint32_t *scratch,
+                                                                 unsigned long long pool_cap, ApplyCtl *actl) {
+  __shared__ uint32_t s_rd[kApplyWaves][kMaxVertexChanges];
+  if (actl->merge_overflow) return;
   const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
+  uint32_t *rd = s_rd[wv];
   for (uint32_t t = blockIdx.x * kApplyWaves + wv; t < b.ntouched; t += gridDim.x * kApplyWaves) {
-    if (only_failed && b.fail[t] == 0) continue;
     const uint32_t x = b.tv[t];
-    const uint32_t nd = b.ndeg[t];
-    const unsigned long long so = b.soff[t];
-    if (so == ~0ull) continue;
-    uint32_t dst = g.start[x];
-    if (nd > g.cap[x]) {
-      const uint32_t newcap = nd + nd / 4 + 8;
-      unsigned long long base = 0;
-      if (lane == 0) base = atomicAdd(&actl->pool_used, (unsigned long long)newcap);
-      base = bcast64(base);
-      if (base + newcap > pool_cap) {
-        if (lane == 0) {
-          b.fail[t] = 1;
-          atomicAdd(&actl->overflow, 1u);
-        }
-        continue;
+    const uint32_t *A = g.pool + g.start[x];
+    const uint32_t na = g.deg[x];
+    const uint32_t i0 = b.ioff[t], ni = b.ioff[t + 1] - i0;
+    const uint32_t d0 = b.doff[t], nd = b.doff[t + 1] - d0;
+    // changes 0 .. ni-1 are the inserts, the rest the deletes
+    uint32_t nnew = 0, nhit = 0, key = 0, r = 0;
+    bool fresh = false;
+    wave_sync();  // the previous vertex's positions are no longer read
+    for (uint32_t c = 0; c < ni + nd; c += 64) {
+      const uint32_t j = c + lane;
+      const bool ins = j < ni, del = !ins && j < ni + nd;
+      key = ins ? b.ins[i0 + j] : del ? b.del[d0 + j - ni] : 0u;
+      if (ni + nd <= 2) {
+        // the whole wave searches for the one or two keys
+        uint32_t r0, r1, loads = 0;
+        bounds2(A, na, __builtin_amdgcn_readlane(key, 0), __builtin_amdgcn_readlane(key, 1), r0, r1, loads);
+        r = lane == 0 ? r0 : r1;
+      } else if (ins || del) {
+        r = lower_bound(A, na, key);
       }
-      dst = (uint32_t)base;
-      if (lane == 0) {
-        g.start[x] = dst;
-        g.cap[x] = newcap;
-        atomicAdd(&actl->relocated, 1u);
+      const bool there = (ins || del) && r < na && A[r] == key;
+      fresh = ins && !there;
+      const uint64_t mi = ballot(fresh), md = ballot(del && there);
+      if (fresh) b.ri[i0 + nnew + mbcnt(mi)] = r;
+      if (del && there) {
+        const uint32_t k = nhit + mbcnt(md);
+        b.rd[d0 + k] = r;
+        rd[k] = r;
       }
+      nnew += (uint32_t)__popcll(mi);
+      nhit += (uint32_t)__popcll(md);
     }
-    if (nd > kApplyWave) {
-      // k_apply_commit_big copies; the new degree is only read by later kernels
-      if (lane == 0) queue_big(b.big_commit, b.ntouched, &actl->ncommit_big, &actl->ncommit_huge, nd, t);
-    } else {
-      copy_range(scratch + so, g.pool + dst, lane, 64, nd);
-    }
+    wave_sync();
+    const uint32_t ndeg = na - nhit + nnew;
+    uint32_t state = 0, dst = 0;
     if (lane == 0) {
+      state = take_slot(g, b, t, x, ndeg, pool_cap, actl, kInPlace, kDirect);
+      if (state == kDirect) dst = b.dst[t];
+      b.ndeg[t] = ndeg;
+      b.nnew[t] = nnew;
+      b.state[t] = state;
+    }
+    state = bcast(state);
+    dst = bcast(dst);
+    // the new inserts to their places, now that all deletes are known
+    uint32_t *out = state == kDirect ? g.pool + dst : scratch + b.soff[t];
+    for (uint32_t c = 0, seen = 0; c < ni; c += 64) {
+      if (ni + nd > 64) {
+        const uint32_t j = c + lane;
+        key = j < ni ? b.ins[i0 + j] : 0u;
+        r = j < ni ? lower_bound(A, na, key) : 0u;
+        fresh = j < ni && !(r < na && A[r] == key);
+      }
+      const uint64_t m = ballot(fresh);
+      if (fresh) out[r - lower_bound(rd, nhit, r) + seen + mbcnt(m)] = key;
+      seen += (uint32_t)__popcll(m);
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void k_apply_merge(DevGraph g, BatchDev b, uint32_t *scratch, const ApplyCtl *actl) {
+  if (actl->merge_overflow) return;
+  const uint32_t lane = lane_id(), nsegs = actl->nsegs;
+  for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < nsegs; i += (gridDim.x * blockDim.x) >> 6) {
+    const uint2 sg = b.segs[i];
+    const uint32_t t = bcast(sg.x), s0 = bcast(sg.y) * kApplySeg;
+    const uint32_t x = b.tv[t];
+    const uint32_t na = g.deg[x];
+    if (s0 >= na) continue;
+    const uint32_t s1 = min(s0 + kApplySeg, na);
+    const uint32_t nnew = b.nnew[t], nhit = na + nnew - b.ndeg[t];
+    const uint32_t *ri = b.ri + b.ioff[t], *rd = b.rd + b.doff[t];
+    const uint32_t *A = g.pool + g.start[x];
+    uint32_t *out = b.state[t] == kDirect ? g.pool + b.dst[t] : scratch + b.soff[t];
+    // new inserts at or before the piece's first and last entry, deletes before
+    // its first entry and its end
+    const uint32_t q0 = wave_count_below(ri, nnew, s0 + 1), q1 = wave_count_below(ri, nnew, s1);
+    const uint32_t p0 = wave_count_below(rd, nhit, s0), p1 = wave_count_below(rd, nhit, s1);
+    if (q0 == q1 && p0 == p1) {
+      copy_range(A + s0, out + s0 + q0 - p0, lane, 64, s1 - s0);
+      continue;
+    }
+    for (uint32_t j = s0 + lane; j < s1; j += 64) {
+      const uint32_t a = A[j];
+      const uint32_t p = p0 + lower_bound(rd + p0, p1 - p0, j);
+      if (p < p1 && rd[p] == j) continue;
+      const uint32_t q = q0 + lower_bound(ri + q0, q1 - q0, j + 1);
+      out[j - p + q] = a;
+    }
+  }
+}
+
+// With `again`, the commits that found no room the first time.
+__global__ __launch_bounds__(256) void k_apply_commit(DevGraph g, BatchDev b, const uint32_t *scratch,
+                                                      const ApplyCtl *actl, DirtyArgs d, int again) {
+  if (actl->merge_overflow) return;
+  const uint32_t lane = lane_id(), nsegs = actl->nsegs;
+  for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < nsegs; i += (gridDim.x * blockDim.x) >> 6) {
+    const uint2 sg = b.segs[i];
+    const uint32_t t = bcast(sg.x), s0 = bcast(sg.y) * kApplySeg;
+    const uint32_t state = b.state[t], nd = b.ndeg[t], dst = b.dst[t];
+    if (again ? state != kRetried : state == kNoRoom) continue;
+    if (state != kDirect && s0 < nd)
+      copy_range(scratch + b.soff[t] + s0, g.pool + dst + s0, lane, 64, min(kApplySeg, nd - s0));
+    if (s0 == 0 && lane == 0) {
+      const uint32_t x = b.tv[t];
+      if (g.start[x] != dst) {
+        g.start[x] = dst;
+        g.cap[x] = nd + nd / 4 + 8;
+      }
       g.deg[x] = nd;
-      b.fail[t] = 0;
-      if (nd > ld_relaxed(&actl->max_deg)) atomicMax(&actl->max_deg, nd);
       mark_dirty_used(g, d, x);
     }
   }
 }
 
-// The commit copies of the lists longer than kApplyWave (for_big_lists splits
-// them).
-__global__ __launch_bounds__(256) void k_apply_commit_big(DevGraph g, BatchDev b, const uint32_t *scratch,
-                                                          const ApplyCtl *actl) {
-  for_big_lists(b.big_commit, b.ntouched, actl->ncommit_big, actl->ncommit_huge, [&](uint32_t t, uint32_t first,
-                                                                                     uint32_t stride) {
-    const uint32_t nd = b.ndeg[t];
-    const uint32_t dst = g.start[b.tv[t]];
-    const unsigned long long so = b.soff[t];
-    copy_range(scratch + so, g.pool + dst, first, stride, nd);
-  });
+// After the pool has grown: slots for the merged lists that found none.
+__global__ __launch_bounds__(256) void k_apply_slots(DevGraph g, BatchDev b, unsigned long long pool_cap,
+                                                     ApplyCtl *actl) {
+  for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < b.ntouched; t += gridDim.x * blockDim.x) {
+    const uint32_t was = b.state[t];
+    uint32_t state = kDone;
+    if (was == kNoRoom) state = take_slot(g, b, t, b.tv[t], b.ndeg[t], pool_cap, actl, kRetried, kRetried);
+    b.state[t] = state;
+  }
 }
 
 // The start of an update: its status from another graph copy's, its counters
@@ -407,18 +394,15 @@ __global__ void k_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *h
   actl->ndirty = actl->nheavy = 0;
   actl->filter_entries = 0;
   actl->filter_bits = 0;
-  actl->nmerge_big = actl->nmerge_huge = actl->ncommit_big = actl->ncommit_huge = 0;
+  actl->nsegs = 0;
   actl->nrelabel_big = actl->nrelabel_huge = 0;
   for (int i = 0; i < 4; i++) actl->sync_queued[i] = hctl[i] = 0;
 }
 
-__global__ void k_round_begin(ApplyCtl *actl, int first) {
+__global__ void k_round_begin(ApplyCtl *actl) {
   if (threadIdx.x != 0) return;
-  if (first) {
-    actl->scratch_used = 0;
-    actl->nmerge_big = actl->nmerge_huge = 0;
-  }
-  actl->ncommit_big = actl->ncommit_huge = 0;
+  actl->scratch_used = 0;
+  actl->nsegs = 0;
 }
 
 // One wave per relabel entry: set the label; when it changed, clear the
@@ -2296,31 +2280,38 @@ hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *h
   return hipGetLastError();
 }
 
-hipError_t launch_round_begin(ApplyCtl *actl, bool first, hipStream_t s) {
-  hipLaunchKernelGGL(k_round_begin, dim3(1), dim3(64), 0, s, actl, first ? 1 : 0);
+hipError_t launch_round_begin(ApplyCtl *actl, hipStream_t s) {
+  hipLaunchKernelGGL(k_round_begin, dim3(1), dim3(64), 0, s, actl);
   return hipGetLastError();
 }
 
-hipError_t launch_apply_merge(const DevGraph &g, const BatchDev &b, unsigned long long scratch_cap,
-                              uint32_t *scratch, ApplyCtl *actl, uint32_t longest, hipStream_t s) {
+hipError_t launch_apply(const DevGraph &g, const BatchDev &b, uint32_t *scratch, unsigned long long scratch_cap,
+                        unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d, size_t max_segs,
+                        hipStream_t s) {
   if (b.ntouched == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_apply_merge, dim3(blocks_for(b.ntouched, kApplyWaves, 4096)), dim3(kApplyWaves * 64), 0, s, g,
-                     b, scratch_cap, scratch, actl);
+  const dim3 seg_blocks(blocks_for(max_segs, 4, 4096));
+  hipLaunchKernelGGL(k_apply_plan, dim3(blocks_for(b.ntouched, 256, 4096)), dim3(256), 0, s, g, b, scratch_cap, actl);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || longest <= kApplyWave) return e;
-  hipLaunchKernelGGL(k_apply_merge_big, dim3(1024), dim3(256), 0, s, g, b, scratch, actl);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_apply_rank, dim3(blocks_for(b.ntouched, kApplyWaves, 4096)), dim3(kApplyWaves * 64), 0, s, g, b,
+                     scratch, pool_cap, actl);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  hipLaunchKernelGGL(k_apply_merge, seg_blocks, dim3(256), 0, s, g, b, scratch, (const ApplyCtl *)actl);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  hipLaunchKernelGGL(k_apply_commit, seg_blocks, dim3(256), 0, s, g, b, (const uint32_t *)scratch,
+                     (const ApplyCtl *)actl, d, 0);
   return hipGetLastError();
 }
 
-hipError_t launch_apply_commit(const DevGraph &g, const BatchDev &b, const uint32_t *scratch,
-                               unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d, bool only_failed,
-                               uint32_t longest, hipStream_t s) {
+hipError_t launch_commit_again(const DevGraph &g, const BatchDev &b, const uint32_t *scratch,
+                               unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d, size_t max_segs,
+                               hipStream_t s) {
   if (b.ntouched == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_apply_commit, dim3(blocks_for(b.ntouched, kApplyWaves, 4096)), dim3(kApplyWaves * 64), 0, s, g,
-                     b, scratch, pool_cap, actl, d, only_failed ? 1 : 0);
+  hipLaunchKernelGGL(k_apply_slots, dim3(blocks_for(b.ntouched, 256, 4096)), dim3(256), 0, s, g, b, pool_cap, actl);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || longest <= kApplyWave) return e;
-  hipLaunchKernelGGL(k_apply_commit_big, dim3(1024), dim3(256), 0, s, g, b, scratch, actl);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_apply_commit, dim3(blocks_for(max_segs, 4, 4096)), dim3(256), 0, s, g, b, scratch,
+                     (const ApplyCtl *)actl, d, 1);
   return hipGetLastError();
 }
 
