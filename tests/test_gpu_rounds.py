@@ -140,3 +140,36 @@ def test_lists_that_grow_past_a_kernel_limit(limit):
     finally:
         one.close()
         many.close()
+
+
+@pytest.mark.parametrize("n", [2, 3, 65, 2048, 2049, 70000])
+@pytest.mark.parametrize("records", [255, 256, 2500])
+def test_update_rule_on_conflicting_batches(n, records):
+    """Batches just below and above the length sorted by counting passes, full of
+    repeated and contradicting records of the same edges in both directions: the
+    graph and labels after the update rule equal the oracle's."""
+    rng = np.random.default_rng(n * 7 + records)
+    lab = rng.integers(0, 4, n).astype(np.uint32)
+    u, v = np.zeros(1, np.uint32), np.ones(1, np.uint32)
+    pairs = rng.integers(0, n, (max(1, records // 6), 2)).astype(np.uint32)
+    pairs[pairs[:, 0] == pairs[:, 1], 1] = 0
+    pairs = pairs[pairs[:, 0] != pairs[:, 1]]
+    if not len(pairs):
+        pairs = np.array([[0, 1]], np.uint32)
+    queries = [one_label("path3"), (2, np.array([1, 2], np.uint32), np.zeros(1, np.uint32), np.ones(1, np.uint32))]
+    g = O.Graph(n, lab, u, v)
+    eng = E.Engine((n, lab, u, v), queries)
+    try:
+        for _ in range(2):
+            p = pairs[rng.integers(0, len(pairs), records)]
+            turn = rng.random(records) < 0.5
+            b = ((rng.random(records) < 0.6).astype(np.uint8), np.where(turn, p[:, 1], p[:, 0]),
+                 np.where(turn, p[:, 0], p[:, 1]), rng.integers(0, 4, records).astype(np.uint32))
+            O.run_stream(g, [], [b])
+            eng.process_batch(*b)
+            off, nb, dl = g.export()
+            o2, n2, l2 = eng.graph()
+            assert np.array_equal(off, o2) and np.array_equal(nb, n2)
+            assert np.array_equal(np.where(dl > 2, 255, dl), l2)
+    finally:
+        eng.close()
