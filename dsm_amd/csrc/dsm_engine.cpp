@@ -169,10 +169,9 @@ struct dsm_engine {
   DevBuf<uint32_t> pool, start, deg, cap;
   DevBuf<uint8_t> lab;
   DevBuf<uint32_t> lpool, loff;  // label-sorted copies of long lists
-  DevBuf<uint32_t> huge_list, huge_ctl, huge_hist;  // segmented builds of the longest lists
-  DevBuf<uint32_t> big_list;                         // vertices whose copy a whole block builds
-  DevBuf<uint32_t> mid_list;                         // vertices whose copy one wave builds
-  uint32_t huge_segs = 0;
+  // builds of the label-sorted copies (SortedBuild)
+  DevBuf<uint32_t> build_ctl, build_mid, build_hist;
+  DevBuf<uint2> build_big, build_pieces;
   uint32_t nbuckets = 1;
   unsigned long long pool_cap = 0;
   // filter
@@ -186,7 +185,8 @@ struct dsm_engine {
   // batch
   DevBuf<uint32_t> scratch;
   unsigned long long scratch_cap = 0;
-  DevBuf<uint32_t> dirty_bits, dirty_list, heavy_list;
+  DevBuf<uint8_t> dirty_marks;
+  DevBuf<uint32_t> dirty_list;
   DevBuf<uint32_t> bbuf;              // an update's arrays (device)
   PinnedBuf<uint32_t> hbuf;           // the same (pinned staging)
   PinnedBuf<uint32_t> hrec;           // a round's records (pinned staging)
@@ -331,17 +331,13 @@ struct dsm_engine {
     t.words = words;
     return t;
   }
-  HugeSort huge_sort() {
-    HugeSort h;
-    h.list = huge_list.p;
-    h.cap = (uint32_t)(huge_list.n / 2);
-    h.ctl = huge_ctl.p;
-    h.big = big_list.p;
-    h.big_cap = (uint32_t)big_list.n;
-    h.mid = mid_list.p;
-    h.mid_cap = (uint32_t)mid_list.n;
-    h.hist = huge_hist.p;
-    h.segs = huge_segs;
+  SortedBuild sorted_build() {
+    SortedBuild h;
+    h.ctl = build_ctl.p;
+    h.mid = build_mid.p;
+    h.big = build_big.p;
+    h.pieces = build_pieces.p;
+    h.hist = build_hist.p;
     // the merge scratch (at least one entry per pool entry) is idle while the
     // label-sorted copies are rebuilt
     h.bucket_bytes = scratch_cap >= pool_cap ? reinterpret_cast<uint8_t *>(scratch.p) : nullptr;
@@ -350,9 +346,8 @@ struct dsm_engine {
   }
   DirtyArgs dirty() {
     DirtyArgs d;
-    d.bits = dirty_bits.p;
+    d.marks = dirty_marks.p;
     d.list = dirty_list.p;
-    d.heavy = heavy_list.p;
     d.list_cap = n;
     d.actl = actl.p;
     return d;
@@ -653,22 +648,18 @@ int build_queries(dsm_engine *e, const dsm_query_desc *qs, uint32_t nq, const st
 
 // ------------------------------------------------------------- graph set-up
 
-// Segment slots for the segmented label sort: enough for every list of the
-// pool to be split into kHugeSeg-entry segments, plus a margin.
-int size_huge_sort(dsm_engine *e) {
-  const uint32_t segs = (uint32_t)(e->pool_cap / kHugeSeg + 1024);
-  if (segs > e->huge_segs) {
-    HIPCHK(e->huge_hist.alloc((size_t)segs * (kMaxRel + 2)));
-    e->huge_segs = segs;
+// Queues of the label-sorted builds: every vertex once among the short lists; at
+// most pool / kBuildSeg lists are longer, in at most twice as many pieces.
+int size_sorted_build(dsm_engine *e) {
+  const size_t lists = (size_t)(e->pool_cap / kBuildSeg) + 1;
+  if (lists > e->build_big.n) {
+    HIPCHK(e->build_big.alloc(lists));
+    HIPCHK(e->build_pieces.alloc(2 * lists));
+    HIPCHK(e->build_hist.alloc(2 * lists * (kMaxRel + 2)));
   }
-  if (!e->huge_list.p) {
-    HIPCHK(e->huge_list.alloc(2 * 4096));
-    HIPCHK(e->huge_ctl.alloc(4));
-    // every vertex at most once (a dirty list holds each vertex once)
-    HIPCHK(e->mid_list.alloc(e->n));
-    // at most 2 m / 4,097 vertices have a degree above 4,096; a longer queue
-    // makes k_lbuild_big look at every listed vertex instead
-    HIPCHK(e->big_list.alloc((size_t)e->n / 64 + 4096));
+  if (!e->build_ctl.p) {
+    HIPCHK(e->build_ctl.alloc(4));
+    HIPCHK(e->build_mid.alloc(e->n));
   }
   return DSM_OK;
 }
@@ -714,14 +705,14 @@ int upload_graph(dsm_engine *e, const dsm_graph_desc *g) {
   HIPCHK(e->start.alloc(n));
   HIPCHK(e->deg.alloc(n));
   HIPCHK(e->cap.alloc(n));
-  HIPCHK(e->lab.alloc(n));
+  HIPCHK(e->lab.alloc(((size_t)n + 15) / 16 * 16));  // read 16 at a time
   HIPCHK(e->lpool.alloc(pcap));
   e->nbuckets = 1;
   for (int l = 0; l < 255; l++)
     if (e->lmap[l] != 0xFF) e->nbuckets = std::max<uint32_t>(e->nbuckets, e->lmap[l] + 2u);
   HIPCHK(e->loff.alloc((size_t)n * (e->nbuckets + 1)));
   e->pool_cap = pcap;
-  if (int rc = size_huge_sort(e)) return rc;
+  if (int rc = size_sorted_build(e)) return rc;
   HIPCHK(hipMemcpy(e->pool.p, hp.data(), total * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(e->start.p, st.data(), (size_t)n * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(e->deg.p, dg.data(), (size_t)n * 4, hipMemcpyHostToDevice));
@@ -737,10 +728,9 @@ int upload_graph(dsm_engine *e, const dsm_graph_desc *g) {
   a0.max_deg = n ? *std::max_element(dg.begin(), dg.end()) : 0;
   HIPCHK(hipMemcpy(e->actl.p, &a0, sizeof a0, hipMemcpyHostToDevice));
   *e->h_actl.p = a0;
-  HIPCHK(e->dirty_bits.alloc((n + 31) / 32));
-  HIPCHK(hipMemset(e->dirty_bits.p, 0, ((n + 31) / 32) * 4));
+  HIPCHK(e->dirty_marks.alloc(((size_t)n + 15) / 16 * 16));
+  HIPCHK(hipMemset(e->dirty_marks.p, 0, e->dirty_marks.n));
   HIPCHK(e->dirty_list.alloc(n));
-  HIPCHK(e->heavy_list.alloc(n));
   return DSM_OK;
 }
 
@@ -1161,8 +1151,8 @@ int upload_round(dsm_engine *e, const Slice &sl, const HostDelta *relabels, bool
   size_t off[10] = {};
   for (int i = 0; i < 9; i++) off[i + 1] = off[i] + parts[i]->size();
   const size_t total = off[9], R = rl_v.size();
-  // the changes' positions, and the relabelled vertices with long lists
-  const size_t o_ri = total, o_rd = o_ri + sl.ins.size(), o_rb = o_rd + sl.del.size(), dtotal = o_rb + R;
+  // the changes' positions
+  const size_t o_ri = total, o_rd = o_ri + sl.ins.size(), dtotal = o_rd + sl.del.size();
   // an earlier round may still read the arrays, its copy the staging buffer
   if (dtotal > e->bbuf.n) HIPCHK(hipStreamSynchronize(e->stream));
   HIPCHK(hipEventSynchronize(e->ev_hbuf));
@@ -1171,10 +1161,12 @@ int upload_round(dsm_engine *e, const Slice &sl, const HostDelta *relabels, bool
   for (int i = 0; i < 9; i++) std::copy(parts[i]->begin(), parts[i]->end(), e->hbuf.p + off[i]);
   if (total) HIPCHK(hipMemcpyAsync(e->bbuf.p, e->hbuf.p, total * 4, hipMemcpyHostToDevice, e->stream));
   HIPCHK(hipEventRecord(e->ev_hbuf, e->stream));
-  if (T > e->soff.n || max_segs(e, T, sl.ins.size()) > e->segs.n) HIPCHK(hipStreamSynchronize(e->stream));
+  // first the touched lists' pieces, then the relabelled vertices'
+  const size_t segs = max_segs(e, std::max<size_t>(T, R), sl.ins.size());
+  if (T > e->soff.n || segs > e->segs.n) HIPCHK(hipStreamSynchronize(e->stream));
   HIPCHK(e->soff.ensure(T));
   HIPCHK(e->tinfo.ensure(4 * e->soff.n));
-  HIPCHK(e->segs.ensure(max_segs(e, T, sl.ins.size())));
+  HIPCHK(e->segs.ensure(segs));
   BatchDev b{};
   b.ntouched = T;
   b.tv = e->bbuf.p + off[0];
@@ -1185,7 +1177,6 @@ int upload_round(dsm_engine *e, const Slice &sl, const HostDelta *relabels, bool
   b.nrelabel = (uint32_t)R;
   b.rl_v = e->bbuf.p + off[5];
   b.rl_l = e->bbuf.p + off[6];
-  b.rl_big = e->bbuf.p + o_rb;
   b.ndeg = e->tinfo.p;
   b.nnew = e->tinfo.p + e->soff.n;
   b.dst = e->tinfo.p + 2 * e->soff.n;
@@ -1261,7 +1252,7 @@ int grow_pool(dsm_engine *e, unsigned long long extra) {
   std::swap(e->start.p, nst.p);
   std::swap(e->start.n, nst.n);
   e->pool_cap = ncap;
-  if (int rc = size_huge_sort(e)) return rc;
+  if (int rc = size_sorted_build(e)) return rc;
   // every label-sorted copy moves with the pool: the update that grew it
   // rebuilds them all once its commits are done (the rebuild uses the merge
   // scratch, which still holds the lists of the commits that failed)
@@ -1412,7 +1403,7 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine:
     const bool final_round = rd + 1 == rounds;
     if (int rc = upload_round(e, sl, final_round ? &d : nullptr, from && rd == 0, ra)) return rc;
     if (rd == 0) {
-      HIPCHK(launch_update_begin(e->actl.p, from ? from->actl.p : nullptr, e->huge_ctl.p, e->stream));
+      HIPCHK(launch_update_begin(e->actl.p, from ? from->actl.p : nullptr, e->build_ctl.p, e->stream));
       if (from) {
         CatchUp c;
         c.x = graph_of(e, *from);
@@ -1445,18 +1436,20 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine:
   }
   e->stats.touched_vertices = T;
   for (;;) {
-    HIPCHK(launch_relabel(e->dev_graph(), ra.b, e->tables(), e->dirty(), longest, e->stream));
+    const size_t R = ra.b.nrelabel;
+    HIPCHK(launch_relabel(e->dev_graph(), ra.b, e->tables(), e->dirty(),
+                          std::min(max_segs(e, R, 0), R * (1 + (size_t)(longest / kApplySeg))), e->stream));
     // after a pool growth the slots moved and every copy is rebuilt instead
     if (from && !e->grew && !e->lpool_stale)
       HIPCHK(launch_sync_sorted(graph_of(e, *from), e->dev_graph(), e->dirty_list.p, &from->actl.p->ndirty,
-                                e->dirty_bits.p, e->sync_q.p, (uint32_t)e->sync_q.n, e->actl.p, before, e->stream));
-    HIPCHK(launch_dirty_compact(e->dirty(), e->n, e->stream));
+                                e->dirty_marks.p, e->sync_q.p, (uint32_t)e->sync_q.n, e->actl.p, before, e->stream));
+    HIPCHK(launch_dirty_compact(e->dev_graph(), e->dirty(), e->stream));
     // the dirty list (touched vertices, relabelled ones and their neighbours) is
     // exactly the set whose label-sorted copies changed, unless the pool grew
     const uint32_t *list = e->lpool_stale ? nullptr : e->dirty_list.p;
-    HIPCHK(launch_lbuild(e->dev_graph(), e->d_lmap.p, list, list ? &e->actl.p->ndirty : nullptr, e->huge_sort(), longest,
-                         e->stream));
-    HIPCHK(launch_filter_dirty(e->dev_graph(), e->tables(), e->dirty(), longest, e->stream));
+    HIPCHK(launch_lbuild(e->dev_graph(), e->tables(), list, list ? &e->actl.p->ndirty : nullptr, e->sorted_build(),
+                         longest, true, e->stream));
+    HIPCHK(launch_filter_dirty(e->dev_graph(), e->tables(), e->dirty(), e->stream));
     if (int rc = cluster_refine(e)) return rc;
     if (done) HIPCHK(hipEventRecord(done, e->stream));
     if (int rc = take_status(e)) return rc;
@@ -1545,8 +1538,9 @@ int create_impl(dsm_engine *e, const dsm_graph_desc *graph, const dsm_query_desc
   e->leaf_segments = e->opt.leaf_segments != 0;
   e->poll_max = e->opt.poll_max ? std::min<uint32_t>(e->opt.poll_max, 16u) : 16u;
   HIPCHK(launch_filter_full(e->dev_graph(), e->tables(), e->stream));
-  HIPCHK(launch_huge_reset(e->huge_sort(), e->stream));
-  HIPCHK(launch_lbuild(e->dev_graph(), e->d_lmap.p, nullptr, nullptr, e->huge_sort(), e->h_actl.p->max_deg, e->stream));
+  HIPCHK(launch_build_reset(e->sorted_build(), e->stream));
+  HIPCHK(launch_lbuild(e->dev_graph(), e->tables(), nullptr, nullptr, e->sorted_build(), e->h_actl.p->max_deg, false,
+                       e->stream));
   if ((rc = cluster_refine(e))) return rc;
   HIPCHK(hipStreamSynchronize(e->stream));
   e->refine_timed = false;

@@ -19,7 +19,7 @@ constexpr uint8_t kNoLabel = 255;  // device label of vertices whose label no qu
 #define DSM_LABEL_SORTED 64
 #endif
 constexpr uint32_t kLabelSorted = DSM_LABEL_SORTED;  // vertices of higher degree keep a label-sorted list copy
-static_assert(kLabelSorted <= 64, "the heavy refilter reads the label-sorted copies of lists longer than 64");
+static_assert(kLabelSorted <= 64, "k_filter_light counts the entries of shorter lists in bytes");
 
 // Matching plan of one (query, ordered query edge (u0,u1)) pair: positions 0
 // and 1 hold the seeded edge, later positions follow a greedy order in which
@@ -112,19 +112,15 @@ struct alignas(64) ApplyCtl {
   uint32_t overflow;                // commits that found no room (host grows the pool)
   uint32_t relocated;
   uint32_t ndirty;                  // vertices on the dirty list
-  uint32_t nheavy;                  // dirty vertices re-filtered by a whole wave
   uint32_t relabeled;
-  uint32_t nrelabel_big;            // relabelled vertices whose neighbours the whole grid marks
+  uint32_t nrelabel_segs;           // pieces of the relabelled vertices' lists on BatchDev::segs
   uint32_t nsegs;                   // pieces of the touched lists (kApplySeg entries) on BatchDev::segs
   uint32_t merge_overflow;          // merges that found no room in the scratch (must stay 0)
   uint32_t filter_bits;             // candidate bits the re-filter writes (work measure)
   unsigned long long filter_entries;  // list entries of the vertices re-filtered (work measure)
-  // of the big lists above, those longer than kBlockList (split over the whole
-  // grid; queued from the back of the same arrays, the rest from the front)
-  uint32_t nrelabel_huge;
   uint32_t max_deg;                 // no list has been longer (never lowered): kernels of longer lists are skipped
   uint32_t sync_queued[4];          // long lists queued by the catch-up (block, grid) and the sorted catch-up
-  uint32_t pad[10];
+  uint32_t pad[12];
 };
 static_assert(sizeof(ApplyCtl) == 128, "apply status layout");
 
@@ -169,11 +165,11 @@ struct BatchDev {
   unsigned long long *soff;
   uint32_t *ri;             // [ins] positions in the old list of t's new inserts, ascending, from ioff[t]
   uint32_t *rd;             // [del] positions of its deletes that are there, ascending, from doff[t]
-  uint2 *segs;              // (t, piece): the touched lists in pieces of kApplySeg entries
+  uint2 *segs;              // (t, piece): the touched lists in pieces of kApplySeg entries; once they are
+                            // committed (vertex, piece | old label << 24): the relabelled vertices' lists
   uint32_t nrelabel;
   const uint32_t *rl_v;
   const uint32_t *rl_l;     // device label (already clamped)
-  uint32_t *rl_big;         // [nrelabel] relabelled vertices of degree > kRelabelWave
 };
 
 struct DfsArgs {
@@ -231,9 +227,8 @@ struct SeedArgs {
 };
 
 struct DirtyArgs {
-  uint32_t *bits;      // [ceil(n/32)] dirty flags
+  uint8_t *marks;      // [n rounded up to 16] dirty marks
   uint32_t *list;      // dirty vertices
-  uint32_t *heavy;     // dirty vertices with a long list
   uint32_t list_cap;
   ApplyCtl *actl;
 };
@@ -348,14 +343,12 @@ constexpr uint32_t kDirect = 1;    // merged into a new slot
 constexpr uint32_t kNoRoom = 2;    // merged into the scratch, needs a slot the pool has no room for
 constexpr uint32_t kRetried = 3;   // has one now: to be committed
 constexpr uint32_t kDone = 4;      // committed by an earlier try
-constexpr uint32_t kRelabelWave = 2048;  // neighbours of longer lists are marked by the whole grid
 constexpr uint32_t kSyncWave = 4096;     // longer lists are brought up to date by the whole grid
-constexpr uint32_t kLbuildBlock = 4096;  // label-sorted copies of longer lists are built by a block
-constexpr uint32_t kLight = 64;          // dirty vertices of higher degree are re-filtered by a wave
+constexpr uint32_t kBuildSeg = 1024;     // label-sorted copies of longer lists are built in pieces
 
 // Takes over the status `from` (null: keeps its own) and clears what an update
-// counts, also hctl[4] (HugeSort::ctl).
-hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *hctl, hipStream_t s);
+// counts, also bctl[4] (SortedBuild::ctl).
+hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl, hipStream_t s);
 // Clears what the merges of one round count (updates with more than one).
 hipError_t launch_round_begin(ApplyCtl *actl, hipStream_t s);
 // The merges and commits of a round; max_segs bounds the pieces.
@@ -368,7 +361,7 @@ hipError_t launch_commit_again(const DevGraph &g, const BatchDev &b, const uint3
                                hipStream_t s);
 // The dirty list (d.list, its length added to d.actl->ndirty) from the dirty
 // bits of the update's n vertices.
-hipError_t launch_dirty_compact(const DirtyArgs &d, uint32_t n, hipStream_t s);
+hipError_t launch_dirty_compact(const DevGraph &g, const DirtyArgs &d, hipStream_t s);
 // What the last update changed, from graph copy x to the stale copy y: the
 // touched vertices' slots and lists, the relabelled vertices' labels and the
 // nbm words of the signature rows. q (qcap entries) is scratch for the long
@@ -388,26 +381,21 @@ hipError_t launch_catch_up(const CatchUp &c, uint32_t longest, hipStream_t s);
 // The label-sorted copies and bucket offsets of the listed (dirty) vertices
 // from x to y, except those whose bit is set in skip.
 hipError_t launch_sync_sorted(const DevGraph &x, const DevGraph &y, const uint32_t *dirty, const uint32_t *ndirty,
-                              const uint32_t *skip, uint32_t *q, uint32_t qcap, ApplyCtl *actl, uint32_t longest,
+                              const uint8_t *skip, uint32_t *q, uint32_t qcap, ApplyCtl *actl, uint32_t longest,
                               hipStream_t s);
 hipError_t launch_relabel(const DevGraph &g, const BatchDev &b, const FilterTables &ft,
-                          const DirtyArgs &d, uint32_t longest, hipStream_t s);
+                          const DirtyArgs &d, size_t max_segs, hipStream_t s);
 hipError_t launch_filter_full(const DevGraph &g, const FilterTables &ft, hipStream_t s);
-// Label-sorted copies of lists longer than kHugeList entries are built in
-// segments of kHugeSeg entries spread over the grid: the vertices are queued
-// here with their first segment slot, and per-segment bucket counts go to hist.
-constexpr uint32_t kHugeList = 65536;
-constexpr uint32_t kHugeSeg = 65536;
-struct HugeSort {
-  uint32_t *list;      // [cap][2]: vertex, first segment slot
-  uint32_t cap;
-  uint32_t *ctl;       // [4]: queued vertices, segment slots taken, vertices on big, on mid
-  uint32_t *big;       // [big_cap]: vertices of degree > 4,096 for the block-per-list build
-  uint32_t big_cap;
-  uint32_t *mid;       // [mid_cap]: vertices of degree 65..4,096 for the wave-per-list build
-  uint32_t mid_cap;
-  uint32_t *hist;      // [segs][kMaxRel + 2]
-  uint32_t segs;
+// Label-sorted copies: lists of up to kBuildSeg entries are built by a wave each,
+// longer ones in pieces (at most kBuildPieces a list), whose bucket counts go to
+// hist.
+constexpr uint32_t kBuildPieces = 512;
+struct SortedBuild {
+  uint32_t *ctl;       // [4]: short lists queued, long ones queued, pieces dealt
+  uint32_t *mid;       // [n]: vertices with short lists
+  uint2 *big;          // [pool / kBuildSeg]: (vertex with a long list, its first piece)
+  uint2 *pieces;       // [2 pool / kBuildSeg]: (vertex, piece)
+  uint32_t *hist;      // [pieces][kMaxRel + 2]
   // one byte per pool entry (indexed like the pool): the bucket of each entry,
   // written by the counting pass so that the scatter pass reads it back
   // instead of gathering the neighbour's label again (null: gather twice)
@@ -416,12 +404,13 @@ struct HugeSort {
 };
 
 // Rebuilds the label-sorted copies of the listed vertices (list + count on the
-// device), or of every vertex when list is null. hs.ctl must be clear.
-hipError_t launch_lbuild(const DevGraph &g, const uint8_t *lmap, const uint32_t *list, const uint32_t *count,
-                         const HugeSort &hs, uint32_t longest, hipStream_t s);
-hipError_t launch_huge_reset(const HugeSort &hs, hipStream_t s);
-hipError_t launch_filter_dirty(const DevGraph &g, const FilterTables &ft, const DirtyArgs &d, uint32_t longest,
-                               hipStream_t s);
+// device), or of every vertex when list is null, and, if asked, sets those
+// vertices' candidate bits. hs.ctl must be clear.
+hipError_t launch_lbuild(const DevGraph &g, const FilterTables &ft, const uint32_t *list, const uint32_t *count,
+                         const SortedBuild &hs, uint32_t longest, bool filter, hipStream_t s);
+hipError_t launch_build_reset(const SortedBuild &hs, hipStream_t s);
+// The candidate bits of the dirty vertices without a label-sorted copy.
+hipError_t launch_filter_dirty(const DevGraph &g, const FilterTables &ft, const DirtyArgs &d, hipStream_t s);
 hipError_t launch_seed(const SeedArgs &a, hipStream_t s);
 hipError_t launch_dfs(const DfsArgs &a, uint32_t blocks, uint32_t waves_per_block, uint32_t max_query_vertices,
                       hipStream_t s);

@@ -6,12 +6,12 @@
 //                                   (the reference rebuilds the whole graph on
 //                                   the host, cpuGraph.cpp:521-607, and
 //                                   re-uploads it, io.cu:279-302)
-//   k_relabel (+ _big)              label changes of the update rule
+//   k_relabel / k_relabel_marks     label changes of the update rule
 //                                   (cpuGraph.cpp:564) + dirty marking
-//   k_lbuild / k_lbuild_big / k_lbuild_huge_*
+//   k_lbuild_pick / k_lbuild / k_lbuild_starts / k_lbuild_place
 //                                   label-sorted copies of lists longer than
 //                                   64 entries, rebuilt for the dirty set
-//   k_filter_full / k_filter_light / k_filter_heavy
+//   k_filter_full / k_filter_light
 //                                   LDF/NLF candidate bitmaps
 //                                   (filter.cu:394-566, compact filter.cu:1692)
 //   k_seed                          device edge seeding (main.cu:268-329;
@@ -38,64 +38,83 @@ __device__ __forceinline__ bool bit_of(const uint64_t *bm, uint32_t words, uint3
   return (bm[(size_t)sig * words + (v >> 6)] >> (v & 63)) & 1ull;
 }
 
-// all 8 byte fields of x >= those of y (fields hold 0..15)
+// all 8 byte fields of x >= those of y (fields hold 0..127)
 __device__ __forceinline__ bool ge_bytes(uint64_t x, uint64_t y) {
   constexpr uint64_t H = 0x8080808080808080ull;
   return (((x | H) - y) & H) == H;
 }
 
-// Marks x dirty in the update being applied: its bit only. The dirty list is
-// compacted from the bits once all marks are in (k_dirty_compact), so that
-// the marks of a hub's neighbours do not contend on a shared list counter. A
-// set bit stays set for the update: read first, so that marking an already
-// dirty vertex (the common case around hubs) costs a load, not an atomic.
-__device__ __forceinline__ void mark_dirty(const DirtyArgs &d, uint32_t x) {
-  const uint32_t bit = 1u << (x & 31);
-  if (ld_relaxed(&d.bits[x >> 5]) & bit) return;
-  atomicOr(&d.bits[x >> 5], bit);
-}
+// Marks x dirty in the update being applied. A byte a vertex, so that a mark is a
+// plain store (every marker stores the same 1): bits took an atomic each, and the
+// marks of 19,000 relabelled vertices' neighbours queued up for the few lines that
+// hold the bits of 500,000 vertices (157 us, a third of it now). The dirty list is
+// made from the marks once all are in (k_dirty_compact).
+__device__ __forceinline__ void mark_dirty(const DirtyArgs &d, uint32_t x) { d.marks[x] = 1; }
 
-// Only vertices with a label some query uses need their candidacy and their
-// label-sorted copy kept current: no seed, DFS level or refilter reads the
-// copy or the bits of any other vertex. A vertex that takes such a label later
-// is marked by its own relabel, so a stale copy never gets read. (A label read
-// here can race with the vertex's own relabel in the same kernel; either
-// order marks what the relabel needs.)
-__device__ __forceinline__ void mark_dirty_used(const DevGraph &g, const DirtyArgs &d, uint32_t x) {
-  if (g.lab[x] != kNoLabel) mark_dirty(d, x);
-}
-
-// The dirty list from the dirty bits: a thread per bit word, a block prefix
-// sum of the words' counts and one counter add per block; the list comes out
-// in id order within each block's words.
-__global__ __launch_bounds__(256) void k_dirty_compact(DirtyArgs d, uint32_t nwords) {
-  __shared__ uint32_t s_sum[256];
-  __shared__ uint32_t s_base;
-  const uint32_t tid = threadIdx.x;
-  if (held_up(d.actl)) return;
-  for (uint32_t w0 = blockIdx.x * 256u; w0 < nwords; w0 += gridDim.x * 256u) {
-    const uint32_t wi = w0 + tid;
-    const uint32_t bits = wi < nwords ? d.bits[wi] : 0u;
-    const uint32_t c = (uint32_t)__popc(bits);
-    s_sum[tid] = c;
-    __syncthreads();
-    for (uint32_t off = 1; off < 256; off <<= 1) {
-      const uint32_t y = tid >= off ? s_sum[tid - off] : 0u;
-      __syncthreads();
-      s_sum[tid] += y;
-      __syncthreads();
+// The caller's place among the block's c entries each, taken from *count with one
+// add for the block: adds of every wave to one counter follow each other at some
+// 20 ns. sums holds a word per wave and one more; all threads call it together.
+template <typename T>
+__device__ __forceinline__ T block_take(T c, T *count, T *sums) {
+  const uint32_t wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  T incl = c;
+  if constexpr (sizeof(T) == 4) {
+    incl = wave_incl_sum(c);
+  } else {
+    for (int o = 1; o < 64; o <<= 1) {
+      const T y = __shfl_up(incl, o);
+      if (lane_id() >= (uint32_t)o) incl += y;
     }
-    if (tid == 255) s_base = s_sum[255] ? atomicAdd(&d.actl->ndirty, s_sum[255]) : 0u;
-    __syncthreads();
-    uint32_t p = s_base + s_sum[tid] - c;
-    uint32_t b = bits;
-    while (b) {
-      const uint32_t k = (uint32_t)__builtin_ctz(b);
-      b &= b - 1;
-      if (p < d.list_cap) d.list[p] = wi * 32u + k;
+  }
+  __syncthreads();  // the previous call's sums are no longer read
+  if (lane_id() == 63) sums[wv] = incl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    T all = 0;
+    for (uint32_t w = 0; w < nw; w++) {
+      const T y = sums[w];
+      sums[w] = all;
+      all += y;
+    }
+    sums[nw] = all ? atomicAdd(count, all) : (T)0;
+  }
+  __syncthreads();
+  return sums[nw] + sums[wv] + incl - c;
+}
+
+// The dirty list from the marks, which are cleared: 16 vertices a thread, a block
+// prefix sum and one counter add per block; the list comes out in id order within
+// each block's vertices. Only vertices with a label some query uses are listed:
+// no seed, DFS level or refilter reads the label-sorted copy or the candidate bits
+// of any other vertex, and one that takes such a label later is marked by its own
+// relabel, so a stale copy never gets read.
+constexpr uint32_t kCompactBlock = 512;
+__global__ __launch_bounds__(kCompactBlock) void k_dirty_compact(DevGraph g, DirtyArgs d) {
+  __shared__ uint32_t s_sum[kCompactBlock / 64 + 1];
+  const uint32_t ngroups = (g.n + 15) / 16;
+  if (held_up(d.actl)) return;
+  for (uint32_t w0 = blockIdx.x * kCompactBlock; w0 < ngroups; w0 += gridDim.x * kCompactBlock) {
+    const uint32_t wi = w0 + threadIdx.x;
+    uint4 *at = reinterpret_cast<uint4 *>(d.marks) + wi;
+    uint4 m = wi < ngroups ? *at : uint4{0, 0, 0, 0};
+    uint32_t take = 0;  // bit k: vertex 16 wi + k is listed
+    if (m.x | m.y | m.z | m.w) {
+      *at = uint4{0, 0, 0, 0};
+      const uint4 l = reinterpret_cast<const uint4 *>(g.lab)[wi];
+      const uint32_t mk[4] = {m.x, m.y, m.z, m.w}, lb[4] = {l.x, l.y, l.z, l.w};
+#pragma unroll
+      for (uint32_t k = 0; k < 16; k++) {
+        const uint32_t sh = k % 4 * 8;
+        if ((mk[k / 4] >> sh & 0xFF) && (lb[k / 4] >> sh & 0xFF) != kNoLabel) take |= 1u << k;
+      }
+    }
+    uint32_t p = block_take((uint32_t)__popc(take), &d.actl->ndirty, s_sum);
+    while (take) {
+      const uint32_t k = (uint32_t)__builtin_ctz(take);
+      take &= take - 1;
+      if (p < d.list_cap) d.list[p] = wi * 16u + k;
       p++;
     }
-    __syncthreads();
   }
 }
 
@@ -185,44 +204,49 @@ __device__ __forceinline__ void copy_range(const uint32_t *__restrict__ from, ui
 // block or the grid for long ones), changes searched for every entry and a
 // counter add per list, merge and commit of such a batch took 870 us.
 
+// Deals out the lanes' lists in pieces: a lane's list `id` has ns of them, queued
+// as (id, piece | tag); one counter add for the wave. Returns where the lane's
+// first one went. All lanes must be active.
+__device__ __forceinline__ uint32_t deal_pieces(uint2 *q, uint32_t *count, uint32_t id, uint32_t ns, uint32_t tag) {
+  uint32_t all;
+  const uint32_t before = wave_excl_sum(ns, &all);
+  uint32_t at = 0;
+  if (all && lane_id() == 0) at = atomicAdd(count, all);
+  at = bcast(at) + before;
+  for (uint32_t k = 0; k < ns; k++) q[at + k] = uint2{id, k | tag};
+  return at;
+}
+
 // The number of p[0, n) below x, for the whole wave; p ascends.
 __device__ __forceinline__ uint32_t wave_count_below(const uint32_t *p, uint32_t n, uint32_t x) {
   if (n <= 64) return (uint32_t)__popcll(ballot(lane_id() < n && p[min(lane_id(), n - 1)] < x));
   return lower_bound(p, n, x);
 }
 
-__global__ __launch_bounds__(256) void k_apply_plan(DevGraph g, BatchDev b, unsigned long long scratch_cap,
-                                                    ApplyCtl *actl) {
-  for (uint32_t t0 = (blockIdx.x * blockDim.x + threadIdx.x) & ~63u; t0 < b.ntouched; t0 += gridDim.x * blockDim.x) {
-    const uint32_t t = t0 + lane_id();
+constexpr uint32_t kPlanBlock = 512;
+__global__ __launch_bounds__(kPlanBlock) void k_apply_plan(DevGraph g, BatchDev b, unsigned long long scratch_cap,
+                                                           ApplyCtl *actl) {
+  __shared__ unsigned long long s_len[kPlanBlock / 64 + 1];
+  __shared__ uint32_t s_segs[kPlanBlock / 64 + 1], s_most;
+  if (threadIdx.x == 0) s_most = 0;
+  for (uint32_t t0 = blockIdx.x * kPlanBlock; t0 < b.ntouched; t0 += gridDim.x * kPlanBlock) {
+    const uint32_t t = t0 + threadIdx.x;
     uint32_t len = 0;  // of the merged list, at most
     if (t < b.ntouched) len = g.deg[b.tv[t]] + b.ioff[t + 1] - b.ioff[t];
     const uint32_t ns = t < b.ntouched ? max(1u, (len + kApplySeg - 1) / kApplySeg) : 0u;
-    uint32_t most = len;
-    for (int o = 32; o >= 1; o >>= 1) most = max(most, (uint32_t)__shfl_xor(most, o));
-    // the sum of 64 lists may pass 32 bits
-    unsigned long long end = len;
-    for (int o = 1; o < 64; o <<= 1) {
-      const unsigned long long y = __shfl_up(end, o);
-      if (lane_id() >= (uint32_t)o) end += y;
+    // (the sum of a block's lists may pass 32 bits)
+    const unsigned long long so = block_take((unsigned long long)len, &actl->scratch_used, s_len);
+    const uint32_t at = block_take(ns, &actl->nsegs, s_segs);
+    atomicMax(&s_most, len);
+    if (t < b.ntouched) {
+      b.soff[t] = so;
+      for (uint32_t k = 0; k < ns; k++) b.segs[at + k] = uint2{t, k};
     }
-    uint32_t nsegs;
-    const uint32_t before = wave_excl_sum(ns, &nsegs);
-    const unsigned long long all = bcast64(__shfl(end, 63));
-    unsigned long long so = 0;
-    uint32_t at = 0;
-    if (lane_id() == 0) {
-      so = atomicAdd(&actl->scratch_used, all);
-      at = atomicAdd(&actl->nsegs, nsegs);
-      if (most > ld_relaxed(&actl->max_deg)) atomicMax(&actl->max_deg, most);
-      if (so + all > scratch_cap) atomicAdd(&actl->merge_overflow, 1u);  // sized by the host so that this cannot happen
-    }
-    so = bcast64(so);
-    at = bcast(at) + before;
-    if (t >= b.ntouched) continue;
-    b.soff[t] = so + end - len;
-    for (uint32_t k = 0; k < ns; k++) b.segs[at + k] = uint2{t, k};
+    // sized by the host so that this cannot happen
+    if (so + len > scratch_cap) atomicAdd(&actl->merge_overflow, 1u);
   }
+  __syncthreads();
+  if (threadIdx.x == 0 && s_most > ld_relaxed(&actl->max_deg)) atomicMax(&actl->max_deg, s_most);
 }
 
 // A slot for t's merged list of nd entries: its own, a new one from the pool's
@@ -364,7 +388,7 @@ __global__ __launch_bounds__(256) void k_apply_commit(DevGraph g, BatchDev b, co
         g.cap[x] = nd + nd / 4 + 8;
       }
       g.deg[x] = nd;
-      mark_dirty_used(g, d, x);
+      mark_dirty(d, x);
     }
   }
 }
@@ -382,7 +406,7 @@ __global__ __launch_bounds__(256) void k_apply_slots(DevGraph g, BatchDev b, uns
 
 // The start of an update: its status from another graph copy's, its counters
 // cleared.
-__global__ void k_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *hctl) {
+__global__ void k_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl) {
   if (threadIdx.x != 0) return;
   if (from) {
     actl->pool_used = from->pool_used;
@@ -391,12 +415,12 @@ __global__ void k_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *h
   actl->scratch_used = 0;
   actl->overflow = actl->merge_overflow = 0;
   actl->relocated = actl->relabeled = 0;
-  actl->ndirty = actl->nheavy = 0;
+  actl->ndirty = 0;
   actl->filter_entries = 0;
   actl->filter_bits = 0;
   actl->nsegs = 0;
-  actl->nrelabel_big = actl->nrelabel_huge = 0;
-  for (int i = 0; i < 4; i++) actl->sync_queued[i] = hctl[i] = 0;
+  actl->nrelabel_segs = 0;
+  for (int i = 0; i < 4; i++) actl->sync_queued[i] = bctl[i] = 0;
 }
 
 __global__ void k_round_begin(ApplyCtl *actl) {
@@ -405,60 +429,62 @@ __global__ void k_round_begin(ApplyCtl *actl) {
   actl->nsegs = 0;
 }
 
-// One wave per relabel entry: set the label; when it changed, clear the
-// vertex's bits in every bitmap of its old label and mark it and all its
-// (post-update) neighbours dirty, since their neighbour-label counts changed.
-__global__ __launch_bounds__(256) void k_relabel(DevGraph g, BatchDev b, FilterTables ft, DirtyArgs d) {
-  const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
+// The relabels, a lane each: set the label; when it changed, mark the vertex
+// dirty and deal out its (post-update) list in pieces for k_relabel_marks, with
+// its old label.
+__global__ __launch_bounds__(256) void k_relabel(DevGraph g, BatchDev b, DirtyArgs d) {
   if (held_up(d.actl)) return;
-  for (uint32_t r = blockIdx.x * 4 + wv; r < b.nrelabel; r += gridDim.x * 4) {
-    const uint32_t x = b.rl_v[r];
-    const uint32_t L = b.rl_l[r];
-    const uint32_t old = g.lab[x];
-    if (old == L) continue;
-    if (lane == 0) {
-      g.lab[x] = (uint8_t)L;
-      atomicAdd(&d.actl->relabeled, 1u);
-      if (L != kNoLabel) mark_dirty(d, x);
+  for (uint32_t r0 = (blockIdx.x * blockDim.x + threadIdx.x) & ~63u; r0 < b.nrelabel; r0 += gridDim.x * blockDim.x) {
+    const uint32_t r = r0 + lane_id();
+    uint32_t x = 0, old = 0, L = 0;
+    bool changed = false;
+    if (r < b.nrelabel) {
+      x = b.rl_v[r];
+      L = b.rl_l[r];
+      old = g.lab[x];
+      changed = old != L;
     }
-    if (old != kNoLabel) {
+    uint32_t ns = 0;
+    if (changed) {
+      g.lab[x] = (uint8_t)L;
+      mark_dirty(d, x);
+      ns = max(1u, (g.deg[x] + kApplySeg - 1) / kApplySeg);
+    }
+    const uint32_t n = (uint32_t)__popcll(ballot(changed));
+    if (n && lane_id() == 0) atomicAdd(&d.actl->relabeled, n);
+    deal_pieces(b.segs, &d.actl->nrelabel_segs, x, ns, old << 24);
+  }
+}
+
+// A wave per piece of a relabelled vertex's list: its neighbours' neighbour-label
+// counts changed, so they are marked dirty; with the first piece the vertex's bits
+// go from every bitmap of its old label.
+__global__ __launch_bounds__(256) void k_relabel_marks(DevGraph g, BatchDev b, FilterTables ft, DirtyArgs d) {
+  const uint32_t lane = lane_id(), nsegs = d.actl->nrelabel_segs;
+  for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < nsegs; i += (gridDim.x * blockDim.x) >> 6) {
+    const uint2 sg = b.segs[i];
+    const uint32_t x = bcast(sg.x), s0 = bcast(sg.y & 0xFFFFFFu) * kApplySeg, old = bcast(sg.y >> 24);
+    if (s0 == 0 && old != kNoLabel) {
       const uint64_t clr = ~(1ull << (x & 63));
       for (uint32_t s = ft.sig_lo[old] + lane; s < ft.sig_hi[old]; s += 64)
         atomicAnd((unsigned long long *)&ft.bm[(size_t)s * ft.words + (x >> 6)], (unsigned long long)clr);
     }
     const uint32_t *A = g.pool + g.start[x];
-    const uint32_t na = g.deg[x];
-    if (na > kRelabelWave) {
-      if (lane == 0) queue_big(b.rl_big, b.nrelabel, &d.actl->nrelabel_big, &d.actl->nrelabel_huge, na, x);
-      continue;
+    const uint32_t s1 = min(s0 + kApplySeg, g.deg[x]);
+    constexpr uint32_t kU = 4;  // entries a lane in flight
+    for (uint32_t j0 = s0; j0 < s1; j0 += 64 * kU) {
+      uint32_t w[kU];
+#pragma unroll
+      for (uint32_t u = 0; u < kU; u++) w[u] = A[min(j0 + u * 64 + lane, s1 - 1)];
+#pragma unroll
+      for (uint32_t u = 0; u < kU; u++) mark_dirty(d, w[u]);
     }
-    for (uint32_t j = lane; j < na; j += 64) mark_dirty_used(g, d, A[j]);
   }
-}
-
-// The neighbours of every relabelled vertex of degree > kRelabelWave, marked
-// dirty (for_big_lists splits the lists).
-__global__ __launch_bounds__(256) void k_relabel_big(DevGraph g, BatchDev b, DirtyArgs d) {
-  for_big_lists(b.rl_big, b.nrelabel, d.actl->nrelabel_big, d.actl->nrelabel_huge, [&](uint32_t x, uint32_t first,
-                                                                                         uint32_t stride) {
-    const uint32_t na = g.deg[x];
-    const uint32_t *A = g.pool + g.start[x];
-    // four entries per thread in flight before their marks
-    uint32_t j = first;
-    for (; j + 3 * stride < na; j += 4 * stride) {
-      const uint32_t x0 = A[j], x1 = A[j + stride], x2 = A[j + 2 * stride], x3 = A[j + 3 * stride];
-      mark_dirty_used(g, d, x0);
-      mark_dirty_used(g, d, x1);
-      mark_dirty_used(g, d, x2);
-      mark_dirty_used(g, d, x3);
-    }
-    for (; j < na; j += stride) mark_dirty_used(g, d, A[j]);
-  });
 }
 
 // ----------------------------------------------------------------- filter
 
-__device__ __forceinline__ bool sig_pass(const SigReq &r, uint32_t deg, const uint64_t c[4]) {
+__device__ __forceinline__ bool sig_pass(const SigReq &r, uint32_t deg, const uint64_t *c) {
   return deg >= r.deg && ge_bytes(c[0], r.nlc[0]) && ge_bytes(c[1], r.nlc[1]) &&
          ge_bytes(c[2], r.nlc[2]) && ge_bytes(c[3], r.nlc[3]);
 }
@@ -523,109 +549,123 @@ __global__ __launch_bounds__(256) void k_filter_full(DevGraph g, FilterTables ft
   }
 }
 
-__device__ __forceinline__ void set_bit(uint64_t *w, uint32_t v, bool on) {
+// Sets v's bit in its bitmap word w, which read `cur` before: only this lane
+// changes this bit in this kernel.
+__device__ __forceinline__ void set_bit_from(uint64_t *w, uint64_t cur, uint32_t v, bool on) {
   const uint64_t bit = 1ull << (v & 63);
-  const bool cur = (*w & bit) != 0;  // only this thread changes this bit in this kernel
-  if (cur == on) return;
+  if (((cur & bit) != 0) == on) return;
   if (on) atomicOr((unsigned long long *)w, (unsigned long long)bit);
   else atomicAnd((unsigned long long *)w, (unsigned long long)~bit);
 }
 
-// Dirty vertices, one lane each; lists longer than kLight go to the heavy list.
+// The lane's K places k among ranges whose ends are pre[1 .. 64] (LDS, ascending;
+// pre[0] = 0): the last range that starts at or before each.
+template <int K>
+__device__ __forceinline__ void ranges_of(const uint32_t *pre, const uint32_t (&k)[K], uint32_t (&o)[K]) {
+#pragma unroll
+  for (int u = 0; u < K; u++) o[u] = 0;
+  for (uint32_t half = 32; half; half >>= 1) {
+#pragma unroll
+    for (int u = 0; u < K; u++) o[u] = pre[o[u] + half] <= k[u] ? o[u] + half : o[u];
+  }
+}
+
+// The dirty vertices, up to 64 to a wave, but those with a label-sorted copy, which
+// were filtered from its bucket sizes (filter_buckets). The lists of a wave's vertices are read as one array, as many lanes
+// to a list as it has entries, and so are their (vertex, signature) pairs, four
+// entries and two pairs a lane in flight. Bound by the scattered label and bitmap
+// reads. With a lane per vertex, its list and its signatures one after the other,
+// 25 us for 4,900 dirty vertices of 100,000 (the longest chain of a wave).
 __global__ __launch_bounds__(256) void k_filter_light(DevGraph g, FilterTables ft, DirtyArgs d) {
-  __shared__ uint8_t s_cnt[256][kMaxRel];
+  // counts of the wave's vertices: a byte per label (at most kLabelSorted), 32 of them
+  // (a 64-bit word of padding keeps the vertices apart in the banks)
+  __shared__ uint64_t s_cnt[4][64][kMaxRel / 8 + 1];
+  __shared__ uint32_t s_pre[4][65], s_from[4][64], s_v[4][64], s_deg[4][64];
+  __shared__ unsigned long long s_sum[2];
   __shared__ uint8_t s_lmap[256];
   for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_lmap[i] = ft.lmap[i];
   __syncthreads();
   if (held_up(d.actl)) return;
+  const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
   const uint32_t nd = d.actl->ndirty < d.list_cap ? d.actl->ndirty : d.list_cap;
-  uint8_t *cnt = s_cnt[threadIdx.x];
-  unsigned long long entries = 0;  // list entries of the vertices this thread re-filters
+  uint32_t *pre = s_pre[wv], *from = s_from[wv];
+  unsigned long long entries = 0;  // list entries of the vertices this lane re-filters
   uint32_t bits = 0;               // candidate bits they receive (one per signature of the label)
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nd; i += gridDim.x * blockDim.x) {
-    const uint32_t v = d.list[i];
-    atomicAnd(&d.bits[v >> 5], ~(1u << (v & 31)));
-    const uint32_t L = g.lab[v];
-    const bool has = L != kNoLabel && ft.sig_lo[L] != ft.sig_hi[L];
-    const uint32_t dv = has ? g.deg[v] : 0u;
-    if (has) {
+  if (lane == 0) pre[0] = 0;
+  if (threadIdx.x < 2) s_sum[threadIdx.x] = 0;
+  __syncthreads();
+  // fewer vertices a wave where there are waves enough: shorter chains
+  uint32_t per = 64;
+  while (per > 8 && nd <= per / 2 * gridDim.x * 4) per >>= 1;
+  for (uint32_t i0 = (blockIdx.x * 4 + wv) * per; i0 < nd; i0 += gridDim.x * 4 * per) {
+    const uint32_t i = i0 + lane;
+    uint32_t v = 0, L = kNoLabel, dv = 0, lo = 0, ns = 0;
+    if (lane < per && i < nd) {
+      v = d.list[i];
+      L = g.lab[v];
+    }
+    if (L != kNoLabel) {
+      lo = ft.sig_lo[L];
+      ns = ft.sig_hi[L] - lo;
+    }
+    if (ns) {
+      dv = g.deg[v];
       entries += dv;
-      bits += ft.sig_hi[L] - ft.sig_lo[L];
+      bits += ns;
     }
-    // long lists go to the heavy list, one counter add per wave
-    const bool heavy = has && dv > kLight;
-    const uint64_t hm = ballot(heavy);
-    if (hm) {
-      const uint32_t leader = (uint32_t)__builtin_ctzll(hm);
-      uint32_t base = 0;
-      if (lane_id() == leader) base = atomicAdd(&d.actl->nheavy, (uint32_t)__popcll(hm));
-      base = __shfl(base, (int)leader);
-      const uint32_t p = base + mbcnt(hm);
-      if (heavy && p < d.list_cap) d.heavy[p] = v;
-    }
-    if (!has || heavy) continue;
-    for (int l = 0; l < kMaxRel; l++) cnt[l] = 0;
-    const uint32_t *A = g.pool + g.start[v];
-    // four entries, then their four label reads, in flight before the counts
-    uint32_t j = 0;
-    for (; j + 4 <= dv; j += 4) {
-      const uint32_t x0 = A[j], x1 = A[j + 1], x2 = A[j + 2], x3 = A[j + 3];
-      const uint32_t l0 = g.lab[x0], l1 = g.lab[x1], l2 = g.lab[x2], l3 = g.lab[x3];
-      const uint32_t li[4] = {s_lmap[l0], s_lmap[l1], s_lmap[l2], s_lmap[l3]};
+    if (dv > kLabelSorted) dv = ns = 0;
+    wave_sync();  // the previous vertices' arrays are no longer read
+    pre[lane + 1] = wave_incl_sum(dv);
+    from[lane] = ns ? g.start[v] : 0;
+    s_v[wv][lane] = v;
+    s_deg[wv][lane] = dv;
+    for (int k = 0; k < kMaxRel / 8; k++) s_cnt[wv][lane][k] = 0;
+    wave_sync();
+    const uint32_t total = pre[64];
+    for (uint32_t e = 0; e < total; e += 256) {
+      uint32_t k[4], o[4], w[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) k[u] = min(e + u * 64 + lane, total - 1);
+      ranges_of(pre, k, o);
+#pragma unroll
+      for (int u = 0; u < 4; u++) w[u] = g.pool[from[o[u]] + (k[u] - pre[o[u]])];
+#pragma unroll
+      for (int u = 0; u < 4; u++) w[u] = s_lmap[g.lab[w[u]]];
 #pragma unroll
       for (int u = 0; u < 4; u++)
-        if (li[u] != 0xFF && cnt[li[u]] < 15) cnt[li[u]]++;
+        if (e + u * 64 + lane < total && w[u] != 0xFF)
+          atomicAdd(reinterpret_cast<uint32_t *>(s_cnt[wv][o[u]]) + (w[u] >> 2), 1u << (w[u] & 3) * 8);
     }
-    for (; j < dv; j++) {
-      const uint32_t li = s_lmap[g.lab[A[j]]];
-      if (li != 0xFF && cnt[li] < 15) cnt[li]++;
-    }
-    uint64_t c[4];
-    for (int k = 0; k < 4; k++) {
-      uint64_t x = 0;
-      for (int b = 0; b < 8; b++) x |= (uint64_t)cnt[k * 8 + b] << (b * 8);
-      c[k] = x;
-    }
-    for (uint32_t s = ft.sig_lo[L]; s < ft.sig_hi[L]; s++)
-      set_bit(&ft.bm[(size_t)s * ft.words + (v >> 6)], v, sig_pass(ft.sigs[s], dv, c));
-  }
-  for (int o = 32; o >= 1; o >>= 1) {
-    entries += __shfl_xor(entries, o);
-    bits += __shfl_xor(bits, o);
-  }
-  if (lane_id() == 0 && entries) atomicAdd(&d.actl->filter_entries, entries);
-  if (lane_id() == 0 && bits) atomicAdd(&d.actl->filter_bits, bits);
-}
-
-// Dirty vertices with long lists (every one has a label-sorted copy, rebuilt
-// for this batch before this kernel runs): the neighbour count of query label
-// index li is the size of label group li, so no list is scanned. One wave per
-// vertex; lanes test the bitmaps in parallel.
-__global__ __launch_bounds__(256) void k_filter_heavy(DevGraph g, FilterTables ft, DirtyArgs d) {
-  __shared__ uint64_t s_pack[4][4];
-  const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
-  const uint32_t nh = d.actl->nheavy < d.list_cap ? d.actl->nheavy : d.list_cap;
-  for (uint32_t h = blockIdx.x * 4 + wv; h < nh; h += gridDim.x * 4) {
-    const uint32_t v = d.heavy[h];
-    const uint32_t L = g.lab[v];
-    const uint32_t dv = g.deg[v];
-    const uint32_t *row = g.loff + (size_t)v * (g.nbuckets + 1);
-    if (lane < 4) {
-      uint64_t x = 0;
-      for (int b = 0; b < 8; b++) {
-        // groups 0 .. nbuckets-2 are the query labels; the last one, the rest
-        const uint32_t li = lane * 8 + b;
-        const uint32_t y = li + 1 < g.nbuckets ? row[li + 1] - row[li] : 0u;
-        x |= (uint64_t)(y < 15 ? y : 15) << (b * 8);
+    // the pairs take the lists' place in the arrays
+    wave_sync();
+    pre[lane + 1] = wave_incl_sum(ns);
+    from[lane] = lo;
+    wave_sync();
+    const uint32_t pairs = pre[64];
+    for (uint32_t e = 0; e < pairs; e += 128) {
+      uint32_t k[2], o[2];
+      uint64_t *word[2], cur[2];
+      bool pass[2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) k[u] = min(e + u * 64 + lane, pairs - 1);
+      ranges_of(pre, k, o);
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const uint32_t s = from[o[u]] + (k[u] - pre[o[u]]);
+        word[u] = &ft.bm[(size_t)s * ft.words + (s_v[wv][o[u]] >> 6)];
+        cur[u] = ld_relaxed(word[u]);
+        pass[u] = sig_pass(ft.sigs[s], s_deg[wv][o[u]], s_cnt[wv][o[u]]);
       }
-      s_pack[wv][lane] = x;
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+        if (e + u * 64 + lane < pairs) set_bit_from(word[u], cur[u], s_v[wv][o[u]], pass[u]);
     }
-    wave_sync();
-    const uint64_t c[4] = {s_pack[wv][0], s_pack[wv][1], s_pack[wv][2], s_pack[wv][3]};
-    for (uint32_t s = ft.sig_lo[L] + lane; s < ft.sig_hi[L]; s += 64)
-      set_bit(&ft.bm[(size_t)s * ft.words + (v >> 6)], v, sig_pass(ft.sigs[s], dv, c));
-    wave_sync();
   }
+  if (entries) atomicAdd(&s_sum[0], entries);
+  if (bits) atomicAdd(&s_sum[1], (unsigned long long)bits);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_sum[0]) atomicAdd(&d.actl->filter_entries, s_sum[0]);
+  if (threadIdx.x == 1 && s_sum[1]) atomicAdd(&d.actl->filter_bits, (uint32_t)s_sum[1]);
 }
 
 // ---------------------------------------------------- label-sorted copies
@@ -652,7 +692,7 @@ __device__ __forceinline__ uint32_t bucket_of(const DevGraph &g, const uint8_t *
 // lowest lane of each peer group adds the group's size).
 __device__ __forceinline__ void bucket_count(const DevGraph &g, const uint8_t *s_lmap, const uint32_t *A,
                                              uint32_t lo, uint32_t hi, uint32_t bits, uint32_t *cnt,
-                                             const uint8_t *bk_in, uint8_t *bk_out) {
+                                             uint8_t *bk_out) {
   const uint32_t lane = lane_id();
   // four chunks at a time: their entries, then their label reads, are all in
   // flight before the first chunk's counts are taken
@@ -662,12 +702,12 @@ __device__ __forceinline__ void bucket_count(const DevGraph &g, const uint8_t *s
 #pragma unroll
     for (uint32_t u = 0; u < kU; u++) {
       const uint32_t j = c0 + u * 64 + lane;
-      x[u] = j < hi && !bk_in ? A[j] : 0u;
+      x[u] = j < hi ? A[j] : 0u;
     }
 #pragma unroll
     for (uint32_t u = 0; u < kU; u++) {
       const uint32_t j = c0 + u * 64 + lane;
-      b[u] = j < hi ? (bk_in ? (uint32_t)bk_in[j] : bucket_of(g, s_lmap, x[u])) : 0u;
+      b[u] = j < hi ? bucket_of(g, s_lmap, x[u]) : 0u;
     }
 #pragma unroll
     for (uint32_t u = 0; u < kU; u++) {
@@ -717,294 +757,220 @@ __device__ __forceinline__ void bucket_scatter(const DevGraph &g, const uint8_t 
   }
 }
 
-constexpr uint32_t kLbuildWaves = 16;    // waves of that block
 
-// The label-sorted copy of v (degree d) by one wave: bucket histogram,
-// offsets, then a stable scatter of the id-sorted list into lpool bucket by
-// bucket.
-__device__ __forceinline__ void build_one(const DevGraph &g, const uint8_t *s_lmap, uint32_t v, uint32_t d,
-                                          uint32_t nb, uint32_t bits, uint32_t *cnt, uint8_t *bucket_bytes) {
-  const uint32_t lane = lane_id();
-  const uint32_t *A = g.pool + g.start[v];
+// The candidate bits of a dirty vertex with a label-sorted copy: its neighbour
+// count of query label li is the size of bucket li, so no list is read again. One
+// wave; `size` is the lane's bucket's, of nb (the last one holds the other labels);
+// pack is the wave's.
+__device__ __forceinline__ void filter_buckets(const DevGraph &g, const FilterTables &ft, uint32_t v, uint32_t d,
+                                               uint32_t size, uint32_t nb, uint64_t *pack) {
+  const uint32_t lane = lane_id(), L = g.lab[v];
+  if (L == kNoLabel) return;
+  if (lane < kMaxRel) reinterpret_cast<uint8_t *>(pack)[lane] = (uint8_t)(lane + 1 < nb ? min(size, 15u) : 0u);
+  wave_sync();
+  for (uint32_t s = ft.sig_lo[L] + lane; s < ft.sig_hi[L]; s += 64) {
+    uint64_t *word = &ft.bm[(size_t)s * ft.words + (v >> 6)];
+    const uint64_t cur = ld_relaxed(word);
+    set_bit_from(word, cur, v, sig_pass(ft.sigs[s], d, pack));
+  }
+  wave_sync();
+}
+
+// The label-sorted copy of v (degree d, at most 64 U) by one wave, which holds the
+// whole list in registers: each entry's place among its bucket's, the buckets'
+// starts, then the entries to their places (in id order inside a bucket). Returns
+// the size of the lane's bucket. Bound by the chain of reads (list, labels) and the
+// ballots per entry: with the list read and its buckets matched twice 62 us for the
+// 12,000 such lists of a 32,768-record batch.
+template <uint32_t U>
+__device__ __forceinline__ uint32_t build_one(const DevGraph &g, const uint8_t *s_lmap, uint32_t v, uint32_t d,
+                                              uint32_t nb, uint32_t bits, uint32_t *cnt) {
+  const uint32_t lane = lane_id(), st = g.start[v];
+  const uint32_t *A = g.pool + st;
   uint32_t *row = g.loff + (size_t)v * (nb + 1);
   if (lane < nb) cnt[lane] = 0;
+  uint32_t x[U], b[U];
+#pragma unroll
+  for (uint32_t u = 0; u < U; u++) x[u] = u * 64 < d ? A[min(u * 64 + lane, d - 1)] : 0u;
+#pragma unroll
+  for (uint32_t u = 0; u < U; u++) b[u] = u * 64 < d ? bucket_of(g, s_lmap, x[u]) : 0u;
   wave_sync();
-  uint8_t *bk = bucket_bytes ? bucket_bytes + g.start[v] : nullptr;
-  bucket_count(g, s_lmap, A, 0, d, bits, cnt, nullptr, bk);
+#pragma unroll
+  for (uint32_t u = 0; u < U; u++) {
+    if (u * 64 >= d) break;
+    const bool valid = u * 64 + lane < d;
+    const uint64_t pm = bucket_peers(b[u], valid, bits);
+    const uint32_t rank = mbcnt(pm), before = cnt[b[u]];
+    wave_sync();
+    if (valid && rank == 0) cnt[b[u]] = before + (uint32_t)__popcll(pm);
+    wave_sync();
+    b[u] |= (before + rank) << 8;
+  }
   // bucket starts: an exclusive scan with a lane per bucket (nb <= kMaxRel + 1 < 64)
   uint32_t total;
   const uint32_t c = lane < nb ? cnt[lane] : 0u;
   const uint32_t first = wave_excl_sum(c, &total);
-  if (lane < nb) {
-    cnt[lane] = first;
-    row[lane] = first;
-  }
+  if (lane < nb) row[lane] = cnt[lane] = first;
   if (lane == 0) row[nb] = total;
   wave_sync();
-  bucket_scatter(g, s_lmap, A, 0, d, bits, cnt, g.lpool + g.start[v], bk);
+  uint32_t *out = g.lpool + st;
+#pragma unroll
+  for (uint32_t u = 0; u < U; u++)
+    if (u * 64 + lane < d) out[cnt[b[u] & 0xFF] + (b[u] >> 8)] = x[u];
+  wave_sync();
+  return c;
 }
 
-// Appends the lanes' vertices with `take` to q (count at *cnt, room for cap),
-// one counter add per wave.
-__device__ __forceinline__ void queue_wave(uint32_t *q, uint32_t cap, uint32_t *cnt, uint32_t v, bool take) {
-  const uint64_t m = ballot(take);
-  if (m == 0) return;
-  const uint32_t leader = (uint32_t)__builtin_ctzll(m);
-  uint32_t at = 0;
-  if (lane_id() == leader) at = atomicAdd(cnt, (uint32_t)__popcll(m));
-  at = __shfl(at, (int)leader) + mbcnt(m);
-  if (take && at < cap) q[at] = v;
+// Entries per piece of a long list: kBuildSeg, more where the list would have over
+// kBuildPieces pieces; a multiple of 64.
+__device__ __forceinline__ uint32_t build_piece(uint32_t d) {
+  return max(kBuildSeg, ((d + kBuildPieces - 1) / kBuildPieces + 63) & ~63u);
 }
 
-// The listed vertices (or all), a lane each, sorted into the two build
-// kernels' queues: degree in (kLabelSorted, kLbuildBlock] on hs.mid for
-// k_lbuild (a wave each), longer on hs.big for k_lbuild_big (a block each).
+// The listed vertices (or all), four a lane: those of degree in (kLabelSorted,
+// kBuildSeg] to hs.mid, longer ones to hs.big and in pieces to hs.pieces.
 // Vertices whose label no query uses are skipped (never read, see
-// mark_dirty_used); a full build leaves their groups empty.
+// k_dirty_compact); a full build leaves their groups empty.
 __global__ __launch_bounds__(256) void k_lbuild_pick(DevGraph g, const uint32_t *list, const uint32_t *count,
-                                                     HugeSort hs) {
+                                                     SortedBuild hs) {
+  __shared__ uint32_t s_sum[5];
   const uint32_t nb = g.nbuckets;
   if (hs.actl && held_up(hs.actl)) return;
   const uint32_t total = list ? (*count < g.n ? *count : g.n) : g.n;
-  for (uint32_t base = (blockIdx.x * blockDim.x + threadIdx.x) & ~63u; base < total;
-       base += gridDim.x * blockDim.x) {
-    const uint32_t t = base + lane_id();
-    uint32_t v = 0, d = 0;
-    bool used = false;
-    if (t < total) {
-      v = list ? list[t] : t;
-      d = g.deg[v];
-      used = g.lab[v] != kNoLabel;
-      if (!used && !list && d > kLabelSorted)
-        for (uint32_t k = 0; k <= nb; k++) g.loff[(size_t)v * (nb + 1) + k] = 0;
+  constexpr uint32_t kU = 4;
+  for (uint32_t base = blockIdx.x * 256 * kU; base < total; base += gridDim.x * 256 * kU) {
+    uint32_t v[kU], d[kU], l[kU], nmid = 0, nbig = 0, npieces = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kU; u++) {
+      const uint32_t t = min(base + u * 256 + threadIdx.x, total - 1);
+      v[u] = list ? list[t] : t;
     }
-    queue_wave(hs.mid, hs.mid_cap, &hs.ctl[3], v, used && d > kLabelSorted && d <= kLbuildBlock);
-    queue_wave(hs.big, hs.big_cap, &hs.ctl[2], v, used && d > kLbuildBlock);
+#pragma unroll
+    for (uint32_t u = 0; u < kU; u++) {
+      d[u] = base + u * 256 + threadIdx.x < total ? g.deg[v[u]] : 0u;
+      l[u] = g.lab[v[u]];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kU; u++) {
+      if (d[u] <= kLabelSorted) continue;
+      if (l[u] == kNoLabel) {
+        if (!list)
+          for (uint32_t k = 0; k <= nb; k++) g.loff[(size_t)v[u] * (nb + 1) + k] = 0;
+        d[u] = 0;
+      } else if (d[u] <= kBuildSeg) {
+        nmid++;
+      } else {
+        const uint32_t sz = build_piece(d[u]);
+        nbig++;
+        npieces += (d[u] + sz - 1) / sz;
+      }
+    }
+    uint32_t at = block_take(nmid, &hs.ctl[0], s_sum);
+#pragma unroll
+    for (uint32_t u = 0; u < kU; u++)
+      if (d[u] > kLabelSorted && d[u] <= kBuildSeg) hs.mid[at++] = v[u];
+    if (!__syncthreads_or(nbig != 0)) continue;
+    at = block_take(nbig, &hs.ctl[1], s_sum);
+    uint32_t first = block_take(npieces, &hs.ctl[2], s_sum);
+#pragma unroll
+    for (uint32_t u = 0; u < kU; u++) {
+      if (d[u] <= kBuildSeg) continue;
+      const uint32_t sz = build_piece(d[u]), np = (d[u] + sz - 1) / sz;
+      hs.big[at++] = uint2{v[u], first};
+      for (uint32_t k = 0; k < np; k++) hs.pieces[first + k] = uint2{v[u], k};
+      first += np;
+    }
   }
 }
 
-// A wave per vertex queued on hs.mid: its label-sorted copy (build_one).
-__global__ __launch_bounds__(256) void k_lbuild(DevGraph g, const uint8_t *lmap, HugeSort hs) {
+// A wave per piece of a long list: its bucket counts; then a wave per short list:
+// its label-sorted copy and, if asked, its vertex's candidate bits.
+__global__ __launch_bounds__(256) void k_lbuild(DevGraph g, FilterTables ft, SortedBuild hs, bool filter) {
+  __shared__ uint8_t s_lmap[256];
+  __shared__ uint32_t s_cnt[4][kMaxRel + 2];
+  __shared__ uint64_t s_pack[4][kMaxRel / 8];
+  for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_lmap[i] = ft.lmap[i];
+  __syncthreads();
+  const uint32_t wv = bcast(threadIdx.x >> 6), lane = lane_id();
+  const uint32_t nb = g.nbuckets;
+  const uint32_t bits = 32u - (uint32_t)__builtin_clz(nb > 1 ? nb - 1 : 1u);
+  const uint32_t npieces = hs.ctl[2], total = npieces + hs.ctl[0];
+  uint32_t *cnt = s_cnt[wv];
+  for (uint32_t t = blockIdx.x * 4 + wv; t < total; t += gridDim.x * 4) {
+    if (t >= npieces) {
+      const uint32_t v = bcast(hs.mid[t - npieces]), d = bcast(g.deg[v]);
+      const uint32_t size = d <= 256 ? build_one<4>(g, s_lmap, v, d, nb, bits, cnt)
+                                     : build_one<kBuildSeg / 64>(g, s_lmap, v, d, nb, bits, cnt);
+      if (filter) filter_buckets(g, ft, v, d, size, nb, s_pack[wv]);
+      continue;
+    }
+    const uint2 pc = hs.pieces[t];
+    const uint32_t v = bcast(pc.x), d = g.deg[v], sz = build_piece(d);
+    const uint32_t lo = bcast(pc.y) * sz, hi = min(lo + sz, d);
+    if (lane < nb) cnt[lane] = 0;
+    wave_sync();
+    bucket_count(g, s_lmap, g.pool + g.start[v], lo, hi, bits, cnt,
+                 hs.bucket_bytes ? hs.bucket_bytes + g.start[v] : nullptr);
+    if (lane < nb) hs.hist[(size_t)t * (kMaxRel + 2) + lane] = cnt[lane];
+    wave_sync();
+  }
+}
+
+// A wave per long list, a lane per bucket (nb <= kMaxRel + 1 < 64): the buckets'
+// starts, and each piece's start inside every bucket in place of its counts; if
+// asked, its vertex's candidate bits.
+__global__ __launch_bounds__(256) void k_lbuild_starts(DevGraph g, FilterTables ft, SortedBuild hs, bool filter) {
+  __shared__ uint64_t s_pack[4][kMaxRel / 8];
+  const uint32_t lane = lane_id(), nb = g.nbuckets, nbig = hs.ctl[1];
+  for (uint32_t t = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; t < nbig; t += (gridDim.x * blockDim.x) >> 6) {
+    const uint2 bg = hs.big[t];
+    const uint32_t v = bcast(bg.x), d = g.deg[v], sz = build_piece(d), np = (d + sz - 1) / sz;
+    uint32_t *hist = hs.hist + (size_t)bcast(bg.y) * (kMaxRel + 2) + lane;
+    uint32_t sum = 0, total;
+    if (lane < nb)
+#pragma unroll 8
+      for (uint32_t p = 0; p < np; p++) sum += hist[(size_t)p * (kMaxRel + 2)];
+    uint32_t run = wave_excl_sum(sum, &total);
+    uint32_t *row = g.loff + (size_t)v * (nb + 1);
+    if (lane < nb) {
+      row[lane] = run;
+#pragma unroll 8
+      for (uint32_t p = 0; p < np; p++) {
+        const uint32_t c = hist[(size_t)p * (kMaxRel + 2)];
+        hist[(size_t)p * (kMaxRel + 2)] = run;
+        run += c;
+      }
+    }
+    if (lane == 0) row[nb] = total;
+    if (filter) filter_buckets(g, ft, v, d, sum, nb, s_pack[threadIdx.x >> 6]);
+  }
+}
+
+// A wave per piece of a long list: its entries to their buckets, in id order.
+__global__ __launch_bounds__(256) void k_lbuild_place(DevGraph g, const uint8_t *lmap, SortedBuild hs) {
   __shared__ uint8_t s_lmap[256];
   __shared__ uint32_t s_cnt[4][kMaxRel + 2];
   for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_lmap[i] = lmap[i];
   __syncthreads();
-  const uint32_t wv = threadIdx.x >> 6;
-  const uint32_t nb = g.nbuckets;
-  const uint32_t bits = 32u - (uint32_t)__builtin_clz(nb > 1 ? nb - 1 : 1u);
-  const uint32_t total = hs.ctl[3] < hs.mid_cap ? hs.ctl[3] : hs.mid_cap;
-  for (uint32_t t = blockIdx.x * 4 + wv; t < total; t += gridDim.x * 4) {
-    const uint32_t v = hs.mid[t];
-    build_one(g, s_lmap, v, g.deg[v], nb, bits, s_cnt[wv], hs.bucket_bytes);
-  }
-}
-
-// One block of kLbuildWaves waves per vertex of degree > kLbuildBlock: each
-// wave takes a contiguous segment of the list; per-wave histograms give every
-// wave its starting position inside every bucket, so the block-wide scatter
-// stays stable (id order inside each bucket). Control flow around the block
-// barriers depends only on the block's vertex, so it is uniform.
-__global__ __launch_bounds__(kLbuildWaves * 64) void k_lbuild_big(DevGraph g, const uint8_t *lmap,
-                                                                  const uint32_t *list, const uint32_t *count,
-                                                                  HugeSort hs) {
-  __shared__ uint8_t s_lmap[256];
-  __shared__ uint32_t s_cnt[kLbuildWaves][kMaxRel + 2];
-  __shared__ uint32_t s_queued;
-  for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_lmap[i] = lmap[i];
-  __syncthreads();
   const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
   const uint32_t nb = g.nbuckets;
   const uint32_t bits = 32u - (uint32_t)__builtin_clz(nb > 1 ? nb - 1 : 1u);
-  // the vertices k_lbuild queued; past the queue's capacity, every listed
-  // vertex is looked at again
-  const uint32_t queued = hs.ctl[2];
-  const bool from_queue = queued <= hs.big_cap;
-  const uint32_t total = from_queue ? queued : list ? (*count < g.n ? *count : g.n) : g.n;
-  for (uint32_t t = blockIdx.x; t < total; t += gridDim.x) {
-    const uint32_t v = from_queue ? hs.big[t] : list ? list[t] : t;
-    const uint32_t d = g.deg[v];
-    if (d <= kLbuildBlock || g.lab[v] == kNoLabel) continue;
-    if (d > kHugeList) {
-      // queue it for the segmented build when its slots fit, else sort here
-      if (threadIdx.x == 0) {
-        const uint32_t nseg = (d + kHugeSeg - 1) / kHugeSeg;
-        uint32_t ok = 0;
-        const uint32_t i = atomicAdd(&hs.ctl[0], 1u);
-        if (i < hs.cap) {
-          const uint32_t sb = atomicAdd(&hs.ctl[1], nseg);
-          if (sb + nseg <= hs.segs) {
-            hs.list[2 * i] = v;
-            hs.list[2 * i + 1] = sb;
-            ok = 1;
-          } else {
-            hs.list[2 * i] = 0xFFFFFFFFu;  // slot taken but unused
-          }
-        }
-        s_queued = ok;
-      }
-      __syncthreads();
-      const uint32_t queued = s_queued;
-      __syncthreads();
-      if (queued) continue;
-    }
-    const uint32_t *A = g.pool + g.start[v];
-    uint32_t *row = g.loff + (size_t)v * (nb + 1);
-    const uint32_t seg = (d + kLbuildWaves - 1) / kLbuildWaves;
-    const uint32_t lo = wv * seg < d ? wv * seg : d;
-    const uint32_t hi = lo + seg < d ? lo + seg : d;
-    uint32_t *cnt = s_cnt[wv];
-    uint8_t *bk = hs.bucket_bytes ? hs.bucket_bytes + g.start[v] : nullptr;
-    if (lane < nb) cnt[lane] = 0;
+  const uint32_t npieces = hs.ctl[2];
+  uint32_t *cnt = s_cnt[wv];
+  for (uint32_t t = blockIdx.x * 4 + wv; t < npieces; t += gridDim.x * 4) {
+    const uint2 pc = hs.pieces[t];
+    const uint32_t v = bcast(pc.x), d = g.deg[v], sz = build_piece(d);
+    const uint32_t lo = bcast(pc.y) * sz, hi = min(lo + sz, d);
+    if (lane < nb) cnt[lane] = hs.hist[(size_t)t * (kMaxRel + 2) + lane];
     wave_sync();
-    bucket_count(g, s_lmap, A, lo, hi, bits, cnt, nullptr, bk);
-    __syncthreads();
-    if (wv == 0) {
-      // wave 0, a lane per bucket (nb <= kMaxRel + 1 < 64): the bucket's total
-      // over the waves, the bucket starts by a scan over the lanes, then each
-      // wave's start inside the bucket
-      uint32_t tot = 0;
-      if (lane < nb)
-        for (uint32_t w = 0; w < kLbuildWaves; w++) tot += s_cnt[w][lane];
-      uint32_t total;
-      uint32_t run = wave_excl_sum(tot, &total);
-      if (lane < nb) {
-        row[lane] = run;
-        for (uint32_t w = 0; w < kLbuildWaves; w++) {
-          const uint32_t c = s_cnt[w][lane];
-          s_cnt[w][lane] = run;
-          run += c;
-        }
-      }
-      if (lane == 0) row[nb] = total;
-    }
-    __syncthreads();
-    bucket_scatter(g, s_lmap, A, lo, hi, bits, cnt, g.lpool + g.start[v], bk);
-    __syncthreads();
+    bucket_scatter(g, s_lmap, g.pool + g.start[v], lo, hi, bits, cnt, g.lpool + g.start[v],
+                   hs.bucket_bytes ? hs.bucket_bytes + g.start[v] : nullptr);
+    wave_sync();
   }
 }
 
-// Segmented build of the queued lists (longer than kHugeList): segment k of a
-// list is handled by block (slot + k) mod gridDim. Pass 1 stores each
-// segment's bucket counts; pass 2 derives every segment's start inside every
-// bucket from them and scatters the segment (per-wave histograms order the
-// waves inside the segment), so the copy stays stable.
-__device__ __forceinline__ void huge_entry(const HugeSort &hs, uint32_t i, uint32_t &v, uint32_t &sb) {
-  v = hs.list[2 * i];
-  sb = hs.list[2 * i + 1];
-}
-
-__global__ __launch_bounds__(kLbuildWaves * 64) void k_lbuild_huge_count(DevGraph g, const uint8_t *lmap,
-                                                                         HugeSort hs) {
-  __shared__ uint8_t s_lmap[256];
-  __shared__ uint32_t s_cnt[kLbuildWaves][kMaxRel + 2];
-  for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_lmap[i] = lmap[i];
-  __syncthreads();
-  const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
-  const uint32_t nb = g.nbuckets;
-  const uint32_t bits = 32u - (uint32_t)__builtin_clz(nb > 1 ? nb - 1 : 1u);
-  const uint32_t nq = hs.ctl[0] < hs.cap ? hs.ctl[0] : hs.cap;
-  for (uint32_t i = 0; i < nq; i++) {
-    uint32_t v, sb;
-    huge_entry(hs, i, v, sb);
-    if (v == 0xFFFFFFFFu) continue;
-    const uint32_t d = g.deg[v];
-    const uint32_t nseg = (d + kHugeSeg - 1) / kHugeSeg;
-    const uint32_t *A = g.pool + g.start[v];
-    for (uint32_t k = 0; k < nseg; k++) {
-      if ((sb + k) % gridDim.x != blockIdx.x) continue;
-      const uint32_t s0 = k * kHugeSeg, s1 = s0 + kHugeSeg < d ? s0 + kHugeSeg : d;
-      const uint32_t sub = (s1 - s0 + kLbuildWaves - 1) / kLbuildWaves;
-      const uint32_t lo = s0 + wv * sub < s1 ? s0 + wv * sub : s1;
-      const uint32_t hi = lo + sub < s1 ? lo + sub : s1;
-      uint8_t *bk = hs.bucket_bytes ? hs.bucket_bytes + g.start[v] : nullptr;
-      if (lane < nb) s_cnt[wv][lane] = 0;
-      wave_sync();
-      bucket_count(g, s_lmap, A, lo, hi, bits, s_cnt[wv], nullptr, bk);
-      __syncthreads();
-      if (threadIdx.x < nb) {
-        uint32_t tot = 0;
-        for (uint32_t w = 0; w < kLbuildWaves; w++) tot += s_cnt[w][threadIdx.x];
-        hs.hist[(size_t)(sb + k) * (kMaxRel + 2) + threadIdx.x] = tot;
-      }
-      __syncthreads();
-    }
-  }
-}
-
-__global__ __launch_bounds__(kLbuildWaves * 64) void k_lbuild_huge_scatter(DevGraph g, const uint8_t *lmap,
-                                                                           HugeSort hs) {
-  __shared__ uint8_t s_lmap[256];
-  __shared__ uint32_t s_cnt[kLbuildWaves][kMaxRel + 2];
-  __shared__ uint32_t s_tot[kMaxRel + 2], s_before[kMaxRel + 2];
-  for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_lmap[i] = lmap[i];
-  __syncthreads();
-  const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
-  const uint32_t nb = g.nbuckets;
-  const uint32_t bits = 32u - (uint32_t)__builtin_clz(nb > 1 ? nb - 1 : 1u);
-  const uint32_t nq = hs.ctl[0] < hs.cap ? hs.ctl[0] : hs.cap;
-  for (uint32_t i = 0; i < nq; i++) {
-    uint32_t v, sb;
-    huge_entry(hs, i, v, sb);
-    if (v == 0xFFFFFFFFu) continue;
-    const uint32_t d = g.deg[v];
-    const uint32_t nseg = (d + kHugeSeg - 1) / kHugeSeg;
-    const uint32_t *A = g.pool + g.start[v];
-    uint32_t *row = g.loff + (size_t)v * (nb + 1);
-    for (uint32_t k = 0; k < nseg; k++) {
-      if ((sb + k) % gridDim.x != blockIdx.x) continue;
-      // bucket totals over all segments, and this segment's share before it
-      if (threadIdx.x < nb) {
-        uint32_t tot = 0, before = 0;
-        for (uint32_t k2 = 0; k2 < nseg; k2++) {
-          const uint32_t c = hs.hist[(size_t)(sb + k2) * (kMaxRel + 2) + threadIdx.x];
-          tot += c;
-          if (k2 < k) before += c;
-        }
-        s_tot[threadIdx.x] = tot;
-        s_before[threadIdx.x] = before;
-      }
-      const uint32_t s0 = k * kHugeSeg, s1 = s0 + kHugeSeg < d ? s0 + kHugeSeg : d;
-      const uint32_t sub = (s1 - s0 + kLbuildWaves - 1) / kLbuildWaves;
-      const uint32_t lo = s0 + wv * sub < s1 ? s0 + wv * sub : s1;
-      const uint32_t hi = lo + sub < s1 ? lo + sub : s1;
-      const uint8_t *bk = hs.bucket_bytes ? hs.bucket_bytes + g.start[v] : nullptr;
-      if (lane < nb) s_cnt[wv][lane] = 0;
-      wave_sync();
-      bucket_count(g, s_lmap, A, lo, hi, bits, s_cnt[wv], bk, nullptr);
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        uint32_t run = 0;
-        for (uint32_t b = 0; b < nb; b++) {
-          const uint32_t c = s_tot[b];
-          s_tot[b] = run;  // bucket start
-          if (k == 0) row[b] = run;
-          run += c;
-        }
-        if (k == 0) row[nb] = run;
-      }
-      __syncthreads();
-      if (threadIdx.x < nb) {
-        uint32_t run = s_tot[threadIdx.x] + s_before[threadIdx.x];
-        for (uint32_t w = 0; w < kLbuildWaves; w++) {
-          const uint32_t c = s_cnt[w][threadIdx.x];
-          s_cnt[w][threadIdx.x] = run;
-          run += c;
-        }
-      }
-      __syncthreads();
-      bucket_scatter(g, s_lmap, A, lo, hi, bits, s_cnt[wv], g.lpool + g.start[v], bk);
-      __syncthreads();
-    }
-  }
-}
-
-__global__ void k_huge_reset(HugeSort hs) {
-  if (threadIdx.x == 0) {
-    hs.ctl[0] = 0;
-    hs.ctl[1] = 0;
-    hs.ctl[2] = 0;
-    hs.ctl[3] = 0;
-  }
+__global__ void k_build_reset(SortedBuild hs) {
+  if (threadIdx.x < 4) hs.ctl[threadIdx.x] = 0;
 }
 
 // ------------------------------------------------------------------- seed
@@ -2242,14 +2208,14 @@ __global__ __launch_bounds__(256) void k_catch_up(CatchUp c) {
 }
 
 __global__ __launch_bounds__(256) void k_sync_sorted(DevGraph x, DevGraph y, const uint32_t *list,
-                                                     const uint32_t *count, const uint32_t *skip, uint32_t *q,
+                                                     const uint32_t *count, const uint8_t *skip, uint32_t *q,
                                                      uint32_t qcap, ApplyCtl *actl) {
   const uint32_t lane = lane_id();
   if (held_up(actl)) return;
   const uint32_t total = *count < x.n ? *count : x.n;
   for (uint32_t t = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; t < total; t += (gridDim.x * blockDim.x) >> 6) {
     const uint32_t v = list[t];
-    if ((skip[v >> 5] >> (v & 31)) & 1u) continue;
+    if (skip[v]) continue;
     const uint32_t st = x.start[v], d = x.deg[v];
     if (d <= kLabelSorted) continue;
     const uint32_t nb = x.nbuckets + 1;
@@ -2275,8 +2241,8 @@ uint32_t blocks_for(size_t n, uint32_t per_block, uint32_t most) {
 
 }  // namespace
 
-hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *hctl, hipStream_t s) {
-  hipLaunchKernelGGL(k_update_begin, dim3(1), dim3(64), 0, s, actl, from, hctl);
+hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl, hipStream_t s) {
+  hipLaunchKernelGGL(k_update_begin, dim3(1), dim3(64), 0, s, actl, from, bctl);
   return hipGetLastError();
 }
 
@@ -2290,7 +2256,7 @@ hipError_t launch_apply(const DevGraph &g, const BatchDev &b, uint32_t *scratch,
                         hipStream_t s) {
   if (b.ntouched == 0) return hipSuccess;
   const dim3 seg_blocks(blocks_for(max_segs, 4, 4096));
-  hipLaunchKernelGGL(k_apply_plan, dim3(blocks_for(b.ntouched, 256, 4096)), dim3(256), 0, s, g, b, scratch_cap, actl);
+  hipLaunchKernelGGL(k_apply_plan, dim3(blocks_for(b.ntouched, kPlanBlock, 4096)), dim3(kPlanBlock), 0, s, g, b, scratch_cap, actl);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_apply_rank, dim3(blocks_for(b.ntouched, kApplyWaves, 4096)), dim3(kApplyWaves * 64), 0, s, g, b,
@@ -2315,9 +2281,8 @@ hipError_t launch_commit_again(const DevGraph &g, const BatchDev &b, const uint3
   return hipGetLastError();
 }
 
-hipError_t launch_dirty_compact(const DirtyArgs &d, uint32_t n, hipStream_t s) {
-  const uint32_t nwords = (n + 31) / 32;
-  hipLaunchKernelGGL(k_dirty_compact, dim3(blocks_for(nwords, 256, 4096)), dim3(256), 0, s, d, nwords);
+hipError_t launch_dirty_compact(const DevGraph &g, const DirtyArgs &d, hipStream_t s) {
+  hipLaunchKernelGGL(k_dirty_compact, dim3(blocks_for(g.n, 16 * kCompactBlock, 4096)), dim3(kCompactBlock), 0, s, g, d);
   return hipGetLastError();
 }
 
@@ -2333,7 +2298,7 @@ hipError_t launch_catch_up(const CatchUp &c, uint32_t longest, hipStream_t s) {
 }
 
 hipError_t launch_sync_sorted(const DevGraph &x, const DevGraph &y, const uint32_t *dirty, const uint32_t *ndirty,
-                              const uint32_t *skip, uint32_t *q, uint32_t qcap, ApplyCtl *actl, uint32_t longest,
+                              const uint8_t *skip, uint32_t *q, uint32_t qcap, ApplyCtl *actl, uint32_t longest,
                               hipStream_t s) {
   if (longest <= kLabelSorted) return hipSuccess;
   hipLaunchKernelGGL(k_sync_sorted, dim3(blocks_for(x.n, 4, 4096)), dim3(256), 0, s, x, y, dirty, ndirty, skip, q, qcap,
@@ -2346,12 +2311,12 @@ hipError_t launch_sync_sorted(const DevGraph &x, const DevGraph &y, const uint32
 }
 
 hipError_t launch_relabel(const DevGraph &g, const BatchDev &b, const FilterTables &ft,
-                          const DirtyArgs &d, uint32_t longest, hipStream_t s) {
+                          const DirtyArgs &d, size_t max_segs, hipStream_t s) {
   if (b.nrelabel == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_relabel, dim3(blocks_for(b.nrelabel, 4, 4096)), dim3(256), 0, s, g, b, ft, d);
+  hipLaunchKernelGGL(k_relabel, dim3(blocks_for(b.nrelabel, 256, 4096)), dim3(256), 0, s, g, b, d);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || longest <= kRelabelWave) return e;
-  hipLaunchKernelGGL(k_relabel_big, dim3(1024), dim3(256), 0, s, g, b, d);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_relabel_marks, dim3(blocks_for(max_segs, 4, 4096)), dim3(256), 0, s, g, b, ft, d);
   return hipGetLastError();
 }
 
@@ -2362,35 +2327,27 @@ hipError_t launch_filter_full(const DevGraph &g, const FilterTables &ft, hipStre
   return hipGetLastError();
 }
 
-hipError_t launch_filter_dirty(const DevGraph &g, const FilterTables &ft, const DirtyArgs &d, uint32_t longest,
-                               hipStream_t s) {
+hipError_t launch_filter_dirty(const DevGraph &g, const FilterTables &ft, const DirtyArgs &d, hipStream_t s) {
   hipLaunchKernelGGL(k_filter_light, dim3(blocks_for(g.n, 256, 1024)), dim3(256), 0, s, g, ft, d);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || longest <= kLight) return e;
-  hipLaunchKernelGGL(k_filter_heavy, dim3(blocks_for(g.n, 4, 1024)), dim3(256), 0, s, g, ft, d);
   return hipGetLastError();
 }
 
-hipError_t launch_huge_reset(const HugeSort &hs, hipStream_t s) {
-  hipLaunchKernelGGL(k_huge_reset, dim3(1), dim3(64), 0, s, hs);
+hipError_t launch_build_reset(const SortedBuild &hs, hipStream_t s) {
+  hipLaunchKernelGGL(k_build_reset, dim3(1), dim3(64), 0, s, hs);
   return hipGetLastError();
 }
 
-hipError_t launch_lbuild(const DevGraph &g, const uint8_t *lmap, const uint32_t *list, const uint32_t *count,
-                         const HugeSort &hs, uint32_t longest, hipStream_t s) {
+hipError_t launch_lbuild(const DevGraph &g, const FilterTables &ft, const uint32_t *list, const uint32_t *count,
+                         const SortedBuild &hs, uint32_t longest, bool filter, hipStream_t s) {
   if (longest <= kLabelSorted) return hipSuccess;
-  hipLaunchKernelGGL(k_lbuild_pick, dim3(blocks_for(g.n, list ? 256 : 4, list ? 2048 : 8192)), dim3(256), 0, s, g, list,
-                     count, hs);
+  hipLaunchKernelGGL(k_lbuild_pick, dim3(blocks_for(g.n, 1024, 2048)), dim3(256), 0, s, g, list, count, hs);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_lbuild, dim3(blocks_for(g.n, 4, 2048)), dim3(256), 0, s, g, lmap, hs);
-  if ((e = hipGetLastError()) != hipSuccess || longest <= kLbuildBlock) return e;
-  hipLaunchKernelGGL(k_lbuild_big, dim3(list ? 256u : 1024u), dim3(kLbuildWaves * 64), 0, s, g, lmap, list, count,
-                     hs);
-  if ((e = hipGetLastError()) != hipSuccess || longest <= kHugeList) return e;
-  hipLaunchKernelGGL(k_lbuild_huge_count, dim3(512), dim3(kLbuildWaves * 64), 0, s, g, lmap, hs);
+  hipLaunchKernelGGL(k_lbuild, dim3(blocks_for(g.n, 4, 2048)), dim3(256), 0, s, g, ft, hs, filter);
+  if ((e = hipGetLastError()) != hipSuccess || longest <= kBuildSeg) return e;
+  hipLaunchKernelGGL(k_lbuild_starts, dim3(blocks_for(g.n, 4, 1024)), dim3(256), 0, s, g, ft, hs, filter);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_lbuild_huge_scatter, dim3(512), dim3(kLbuildWaves * 64), 0, s, g, lmap, hs);
+  hipLaunchKernelGGL(k_lbuild_place, dim3(blocks_for(g.n, 4, 2048)), dim3(256), 0, s, g, ft.lmap, hs);
   return hipGetLastError();
 }
 

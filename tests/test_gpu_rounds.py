@@ -99,7 +99,7 @@ def test_leaf_sets_at_their_limits(da, db, labels):
             eng.close()
 
 
-@pytest.mark.parametrize("limit", [64, 2048, 4096, 8192, 65536])
+@pytest.mark.parametrize("limit", [64, 1024, 2048, 4096, 8192, 65536, 524288])
 def test_lists_that_grow_past_a_kernel_limit(limit):
     """A hub's list grows by one entry at a time from just below a length at which
     an update needs one more kernel to just above it, and shrinks again, one batch
