@@ -666,45 +666,53 @@ int size_sorted_build(dsm_engine *e) {
 
 int upload_graph(dsm_engine *e, const dsm_graph_desc *g) {
   const uint32_t n = g->num_vertices;
-  // sorted, deduplicated CSR
-  std::vector<uint64_t> off(n + 1, 0);
-  for (uint64_t i = 0; i < g->num_edges; i++) {
-    uint32_t a = g->edge_src[i], b = g->edge_dst[i];
-    if (a >= n || b >= n) return e->fail_msg(DSM_EINVAL, "edge %llu: endpoint out of range", (unsigned long long)i);
-    off[a + 1]++;
-    off[b + 1]++;
+  const uint64_t m = g->num_edges;
+  const size_t count = 2 * m;
+  const uint32_t bits = n > 1 ? 32u - (uint32_t)__builtin_clz(n - 1) : 1u;
+  // the sort's buffers go before the pool's copies come, which are larger
+  DevBuf<unsigned long long> keys[2], hist, sums, slot;
+  DevBuf<uint32_t> begin;
+  DevBuf<CsrCtl> ctl;
+  CsrCtl c0{~0ull, 0, 0, 0, 0};
+  HIPCHK(ctl.alloc(1));
+  HIPCHK(hipMemcpy(ctl.p, &c0, sizeof c0, hipMemcpyHostToDevice));
+  HIPCHK(sums.alloc(csr_sum_words(std::max<size_t>(csr_scan_words(count), n))));
+  uint32_t cur = 0;
+  if (m) {
+    for (auto &k : keys) HIPCHK(k.alloc(count));
+    HIPCHK(hist.alloc(csr_scan_words(count)));
+    // the edges lie in the buffer that the first pass fills
+    uint32_t *edges = reinterpret_cast<uint32_t *>(keys[1].p);
+    HIPCHK(hipMemcpyAsync(edges, g->edge_src, m * 4, hipMemcpyHostToDevice, e->stream));
+    HIPCHK(hipMemcpyAsync(edges + m, g->edge_dst, m * 4, hipMemcpyHostToDevice, e->stream));
+    HIPCHK(launch_csr_keys(edges, edges + m, m, n, bits, keys[0].p, ctl.p, e->stream));
+    for (uint32_t shift = 0; shift < 2 * bits; shift += 8, cur ^= 1)
+      HIPCHK(launch_radix_pass(keys[cur].p, keys[cur ^ 1].p, count, shift, hist.p, sums.p, e->stream));
+    HIPCHK(launch_csr_unique(keys[cur].p, keys[cur ^ 1].p, count, hist.p, sums.p, ctl.p, e->stream));
+    cur ^= 1;
   }
-  for (uint32_t v = 0; v < n; v++) off[v + 1] += off[v];
-  std::vector<uint32_t> nb(off[n]);
-  {
-    std::vector<uint64_t> pos(off.begin(), off.end() - 1);
-    for (uint64_t i = 0; i < g->num_edges; i++) {
-      uint32_t a = g->edge_src[i], b = g->edge_dst[i];
-      nb[pos[a]++] = b;
-      nb[pos[b]++] = a;
-    }
-  }
-  std::vector<uint32_t> dg(n), cp(n), st(n);
-  unsigned long long total = 0;
-  for (uint32_t v = 0; v < n; v++) {
-    auto b = nb.begin() + off[v], en = nb.begin() + off[v + 1];
-    std::sort(b, en);
-    dg[v] = (uint32_t)(std::unique(b, en) - b);
-    cp[v] = dg[v] + dg[v] / 4 + 4;
-    st[v] = (uint32_t)total;
-    total += cp[v];
-  }
-  const unsigned long long pcap = total + total / 2 + (1ull << 20);
-  if (pcap >= (1ull << 32)) return e->fail_msg(DSM_ELIMIT, "graph too large for 32-bit pool offsets");
-  std::vector<uint32_t> hp(total, 0xFFFFFFFFu);
-  for (uint32_t v = 0; v < n; v++) std::copy(nb.begin() + off[v], nb.begin() + off[v] + dg[v], hp.begin() + st[v]);
-  std::vector<uint8_t> hl(n);
-  for (uint32_t v = 0; v < n; v++) hl[v] = clamp_label(g->labels[v], e->label_used);
-
-  HIPCHK(e->pool.alloc(pcap));
   HIPCHK(e->start.alloc(n));
   HIPCHK(e->deg.alloc(n));
   HIPCHK(e->cap.alloc(n));
+  HIPCHK(begin.alloc(n));
+  HIPCHK(slot.alloc(n));
+  HIPCHK(hipMemsetAsync(e->deg.p, 0, (size_t)n * 4, e->stream));
+  HIPCHK(launch_csr_slots(keys[cur].p, count, n, bits, begin.p, e->deg.p, e->cap.p, e->start.p, slot.p, sums.p, ctl.p,
+                          e->stream));
+  std::vector<uint8_t> hl(n);
+  for (uint32_t v = 0; v < n; v++) hl[v] = clamp_label(g->labels[v], e->label_used);
+  HIPCHK(hipStreamSynchronize(e->stream));
+  HIPCHK(hipMemcpy(&c0, ctl.p, sizeof c0, hipMemcpyDeviceToHost));
+  if (c0.bad != ~0ull) return e->fail_msg(DSM_EINVAL, "edge %llu: endpoint out of range", c0.bad);
+  const unsigned long long total = c0.total, pcap = total + total / 2 + (1ull << 20);
+  if (c0.unique >= (1ull << 32) || pcap >= (1ull << 32))
+    return e->fail_msg(DSM_ELIMIT, "graph too large for 32-bit pool offsets");
+  keys[cur ^ 1].reset();
+  hist.reset();
+  HIPCHK(e->pool.alloc(pcap));
+  HIPCHK(launch_csr_fill(keys[cur].p, count, bits, begin.p, e->start.p, e->pool.p, ctl.p, e->stream));
+  HIPCHK(hipStreamSynchronize(e->stream));
+  keys[cur].reset();
   HIPCHK(e->lab.alloc(((size_t)n + 15) / 16 * 16));  // read 16 at a time
   HIPCHK(e->lpool.alloc(pcap));
   e->nbuckets = 1;
@@ -713,10 +721,6 @@ int upload_graph(dsm_engine *e, const dsm_graph_desc *g) {
   HIPCHK(e->loff.alloc((size_t)n * (e->nbuckets + 1)));
   e->pool_cap = pcap;
   if (int rc = size_sorted_build(e)) return rc;
-  HIPCHK(hipMemcpy(e->pool.p, hp.data(), total * 4, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(e->start.p, st.data(), (size_t)n * 4, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(e->deg.p, dg.data(), (size_t)n * 4, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(e->cap.p, cp.data(), (size_t)n * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(e->lab.p, hl.data(), n, hipMemcpyHostToDevice));
   // scratch holds one merged copy of every touched list
   e->scratch_cap = pcap + (1ull << 20);
@@ -725,7 +729,7 @@ int upload_graph(dsm_engine *e, const dsm_graph_desc *g) {
   HIPCHK(e->h_actl.ensure(1));
   ApplyCtl a0{};
   a0.pool_used = total;
-  a0.max_deg = n ? *std::max_element(dg.begin(), dg.end()) : 0;
+  a0.max_deg = c0.max_deg;
   HIPCHK(hipMemcpy(e->actl.p, &a0, sizeof a0, hipMemcpyHostToDevice));
   *e->h_actl.p = a0;
   HIPCHK(e->dirty_marks.alloc(((size_t)n + 15) / 16 * 16));

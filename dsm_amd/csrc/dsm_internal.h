@@ -236,6 +236,32 @@ struct DirtyArgs {
 // Message of the last failed call that has no engine (dsm_last_error(NULL)).
 void set_global_error(const char *fmt, ...);
 
+// The adjacency of an edge list (dsm_build.hip). Keys are source << bits | target,
+// two an edge (count = 2 m); hist has csr_scan_words(count) words, sums
+// csr_sum_words of what is scanned (hist, or n slots).
+struct CsrCtl {
+  unsigned long long bad;     // the first edge with an endpoint out of range (set to ~0 before)
+  unsigned long long unique;  // keys left once equal ones are dropped
+  unsigned long long total;   // pool entries the slots take
+  uint32_t max_deg;
+  uint32_t pad;
+};
+size_t csr_scan_words(size_t count);
+size_t csr_sum_words(size_t items);
+hipError_t launch_csr_keys(const uint32_t *src, const uint32_t *dst, size_t m, uint32_t n, uint32_t bits,
+                           unsigned long long *keys, CsrCtl *ctl, hipStream_t s);
+// One stable pass of the sort over the 8 bits from shift up.
+hipError_t launch_radix_pass(const unsigned long long *from, unsigned long long *to, size_t count, uint32_t shift,
+                             unsigned long long *hist, unsigned long long *sums, hipStream_t s);
+hipError_t launch_csr_unique(const unsigned long long *from, unsigned long long *to, size_t count,
+                             unsigned long long *hist, unsigned long long *sums, CsrCtl *ctl, hipStream_t s);
+// Degrees, capacities and slot starts of ctl->unique keys; deg must be clear.
+hipError_t launch_csr_slots(const unsigned long long *keys, size_t count, uint32_t n, uint32_t bits, uint32_t *begin,
+                            uint32_t *deg, uint32_t *cap, uint32_t *start, unsigned long long *slot,
+                            unsigned long long *sums, CsrCtl *ctl, hipStream_t s);
+hipError_t launch_csr_fill(const unsigned long long *keys, size_t count, uint32_t bits, const uint32_t *begin,
+                           const uint32_t *start, uint32_t *pool, const CsrCtl *ctl, hipStream_t s);
+
 // Sorted-set intersection (dsm_intersect.hip): k_intersect writes chunk c's
 // members of B at hits[c * 64 ..] and their number at cnt[c].
 uint32_t intersect_chunks(uint32_t na);
