@@ -1872,24 +1872,25 @@ int dsm_get_graph(dsm_engine *e, uint64_t *offsets, uint32_t *neighbours, uint64
   HIPCHK(hipSetDevice(e->opt.device));
   HIPCHK(hipStreamSynchronize(e->stream));
   const uint32_t n = e->n;
-  std::vector<uint32_t> st(n), dg(n);
-  std::vector<uint8_t> lb(n);
-  HIPCHK(hipMemcpy(st.data(), e->start.p, (size_t)n * 4, hipMemcpyDeviceToHost));
-  HIPCHK(hipMemcpy(dg.data(), e->deg.p, (size_t)n * 4, hipMemcpyDeviceToHost));
-  HIPCHK(hipMemcpy(lb.data(), e->lab.p, n, hipMemcpyDeviceToHost));
-  uint64_t o = 0;
-  for (uint32_t v = 0; v < n; v++) {
-    offsets[v] = o;
-    o += dg[v];
-  }
-  offsets[n] = o;
+  // packed in the merge scratch, which is idle between updates and has room for
+  // the offsets: it is as large as a pool with at least four entries a vertex
+  unsigned long long *off = reinterpret_cast<unsigned long long *>(e->scratch.p);
+  const size_t sums = csr_sum_words(n + 1ull), head = 2 * (n + 1ull + sums);
+  HIPCHK(launch_graph_offsets(n, e->deg.p, off, off + n + 1, e->stream));
+  HIPCHK(hipMemcpyAsync(offsets, off, (n + 1ull) * 8, hipMemcpyDeviceToHost, e->stream));
+  std::vector<uint8_t> lb(labels ? n : 0);
+  if (labels) HIPCHK(hipMemcpyAsync(lb.data(), e->lab.p, n, hipMemcpyDeviceToHost, e->stream));
+  HIPCHK(hipStreamSynchronize(e->stream));
+  const uint64_t o = offsets[n];
   *num_entries = o;
-  if (labels)
-    for (uint32_t v = 0; v < n; v++) labels[v] = lb[v];
+  for (uint32_t v = 0; labels && v < n; v++) labels[v] = lb[v];
   if (o > cap || !neighbours) return o > cap ? e->fail_msg(DSM_ETRUNC, "neighbour buffer too small") : DSM_OK;
-  std::vector<uint32_t> hp((size_t)e->pool_cap);
-  HIPCHK(hipMemcpy(hp.data(), e->pool.p, (size_t)e->pool_cap * 4, hipMemcpyDeviceToHost));
-  for (uint32_t v = 0; v < n; v++) std::copy(hp.begin() + st[v], hp.begin() + st[v] + dg[v], neighbours + offsets[v]);
+  DevBuf<uint32_t> own;  // where the lists do not fit behind the offsets
+  if (head + o > e->scratch_cap) HIPCHK(own.alloc(o));
+  uint32_t *lists = own.p ? own.p : e->scratch.p + head;
+  HIPCHK(launch_graph_lists(n, off, e->start.p, e->pool.p, o, lists, e->stream));
+  HIPCHK(hipMemcpyAsync(neighbours, lists, o * 4, hipMemcpyDeviceToHost, e->stream));
+  HIPCHK(hipStreamSynchronize(e->stream));
   return DSM_OK;
 }
 

@@ -262,6 +262,13 @@ hipError_t launch_csr_slots(const unsigned long long *keys, size_t count, uint32
 hipError_t launch_csr_fill(const unsigned long long *keys, size_t count, uint32_t bits, const uint32_t *begin,
                            const uint32_t *start, uint32_t *pool, const CsrCtl *ctl, hipStream_t s);
 
+// The lists of a graph packed: off[0, n] from the degrees (sums: csr_sum_words(n + 1)
+// words), then the total = off[n] entries.
+hipError_t launch_graph_offsets(uint32_t n, const uint32_t *deg, unsigned long long *off, unsigned long long *sums,
+                                hipStream_t s);
+hipError_t launch_graph_lists(uint32_t n, const unsigned long long *off, const uint32_t *start, const uint32_t *pool,
+                              size_t total, uint32_t *out, hipStream_t s);
+
 // Sorted-set intersection (dsm_intersect.hip): k_intersect writes chunk c's
 // members of B at hits[c * 64 ..] and their number at cnt[c].
 uint32_t intersect_chunks(uint32_t na);
