@@ -269,12 +269,6 @@ hipError_t launch_graph_offsets(uint32_t n, const uint32_t *deg, unsigned long l
 hipError_t launch_graph_lists(uint32_t n, const unsigned long long *off, const uint32_t *start, const uint32_t *pool,
                               size_t total, uint32_t *out, hipStream_t s);
 
-// Sorted-set intersection (dsm_intersect.hip): k_intersect writes chunk c's
-// members of B at hits[c * 64 ..] and their number at cnt[c].
-uint32_t intersect_chunks(uint32_t na);
-hipError_t launch_intersect(const uint32_t *A, uint32_t na, const uint32_t *B, uint32_t nb, uint32_t *hits,
-                            uint32_t *cnt, hipStream_t s);
-
 // ---- cluster-encoding refinement (dsm_cluster_plan.cpp, dsm_cluster.hip) ---
 
 constexpr uint32_t kNone = 0xFFFFFFFFu;

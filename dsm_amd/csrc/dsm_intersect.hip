@@ -7,7 +7,6 @@
 // its own, outside the DFS.
 #include <algorithm>
 #include <mutex>
-#include <vector>
 
 #include "../../include/dsm.h"
 #include "dsm_device.h"
@@ -17,14 +16,35 @@ namespace dsm {
 namespace {
 
 constexpr int kIntersectWaves = 4;
+constexpr uint32_t kBadInput = 0xFFFFFFFFu;  // in place of the result's size: inputs not in order
+
+// *bad = 1 unless both inputs are strictly ascending and end below 0xFFFFFFFF; it
+// must be clear. (The host's loop over 5,000,000 entries took half of the 2.0 ms of
+// 1,000,000 x 4,000,003; 1.0 ms this way.)
+__global__ void k_check_clear(uint32_t *bad) { *bad = 0; }
+__global__ __launch_bounds__(256) void k_check_sorted(const uint32_t *A, uint32_t na, const uint32_t *B, uint32_t nb,
+                                                      uint32_t *bad) {
+  const uint64_t total = (uint64_t)na + nb;
+  bool wrong = false;
+  for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < total; i += gridDim.x * 256ull) {
+    const bool first = i < na;
+    const uint32_t *p = first ? A + i : B + (i - na);
+    const bool last = first ? i + 1 == na : i + 1 == total;
+    wrong |= last ? *p == 0xFFFFFFFFu : p[0] >= p[1];
+  }
+  if (ballot(wrong) && lane_id() == 0) *bad = 1;
+}
 
 // A wave per 64-entry chunk of A: the chunk's members of B, in order, at
-// hits[chunk * 64 ..] and their number at cnt[chunk].
+// hits[chunk * 64 ..] and their number at cnt[chunk]; none of it if the inputs are
+// bad.
 __global__ __launch_bounds__(kIntersectWaves * 64) void k_intersect(const uint32_t *A, uint32_t na, const uint32_t *B,
-                                                                    uint32_t nb, uint32_t *hits, uint32_t *cnt) {
+                                                                    uint32_t nb, uint32_t *hits, uint32_t *cnt,
+                                                                    const uint32_t *bad) {
   __shared__ uint32_t win[kIntersectWaves][kWin];
   const uint32_t lane = lane_id(), wv = threadIdx.x >> 6;
   const uint32_t nch = (na + 63) / 64;
+  if (*bad) return;
   for (uint32_t c = blockIdx.x * kIntersectWaves + wv; c < nch; c += gridDim.x * kIntersectWaves) {
     const uint32_t i = c * 64 + lane;
     const bool in = i < na;
@@ -37,18 +57,76 @@ __global__ __launch_bounds__(kIntersectWaves * 64) void k_intersect(const uint32
   }
 }
 
-}  // namespace
-
-uint32_t intersect_chunks(uint32_t na) { return (na + 63) / 64; }
-
-hipError_t launch_intersect(const uint32_t *A, uint32_t na, const uint32_t *B, uint32_t nb, uint32_t *hits,
-                            uint32_t *cnt, hipStream_t s) {
-  const uint32_t nch = intersect_chunks(na);
-  if (nch == 0) return hipSuccess;
-  const uint32_t blocks = std::min<uint32_t>((nch + kIntersectWaves - 1) / kIntersectWaves, 2048);
-  hipLaunchKernelGGL(k_intersect, dim3(blocks), dim3(kIntersectWaves * 64), 0, s, A, na, B, nb, hits, cnt);
-  return hipGetLastError();
+// Exclusive prefix of cnt[0, nch) into off, the total at *total (one block), which
+// said before whether the inputs are bad: kBadInput then.
+__global__ __launch_bounds__(1024) void k_chunk_offsets(const uint32_t *cnt, uint32_t nch, uint32_t *off,
+                                                        uint32_t *total) {
+  __shared__ uint32_t s_sum[16];
+  uint32_t run = 0;
+  const bool bad = *total != 0;
+  if (bad) nch = 0;
+  __syncthreads();
+  for (uint32_t base = 0; base < nch; base += 1024) {
+    const uint32_t i = base + threadIdx.x;
+    const uint32_t x = i < nch ? cnt[i] : 0u, incl = wave_incl_sum(x);
+    __syncthreads();  // the previous sums are no longer read
+    if (lane_id() == 63) s_sum[threadIdx.x >> 6] = incl;
+    __syncthreads();
+    uint32_t before = run;
+    for (uint32_t w = 0; w < 16; w++) {
+      if (w < threadIdx.x >> 6) before += s_sum[w];
+      run += s_sum[w];
+    }
+    if (i < nch) off[i] = before + incl - x;
+  }
+  if (threadIdx.x == 0) *total = bad ? kBadInput : run;
 }
+
+// Chunk c's members (hits[c * 64 ..], cnt[c] of them) to res[off[c] ..].
+__global__ __launch_bounds__(256) void k_chunk_gather(const uint32_t *hits, const uint32_t *cnt,
+                                                      const uint32_t *off, uint32_t nch, const uint32_t *total,
+                                                      uint32_t *res) {
+  const uint32_t lane = lane_id();
+  if (*total == kBadInput) return;
+  for (uint32_t c = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; c < nch; c += (gridDim.x * blockDim.x) >> 6)
+    if (lane < cnt[c]) res[off[c] + lane] = hits[(size_t)c * 64 + lane];
+}
+
+// The whole intersection by one block, a wave per chunk, 16 chunks at a time:
+// their number to *total, the members to res. For a short A, where the two
+// launches and the trip through memory between them cost more than the search.
+// With `checked`, *total says before whether the inputs are bad: kBadInput then.
+constexpr uint32_t kShortWaves = 16;
+__global__ __launch_bounds__(kShortWaves * 64) void k_intersect_short(const uint32_t *A, uint32_t na,
+                                                                      const uint32_t *B, uint32_t nb, bool checked,
+                                                                      uint32_t *total, uint32_t *res) {
+  __shared__ uint32_t win[kShortWaves][kWin], s_cnt[kShortWaves];
+  const uint32_t lane = lane_id(), wv = bcast(threadIdx.x >> 6);
+  uint32_t run = 0;
+  const bool bad = checked && *total != 0;
+  if (bad) na = 0;
+  __syncthreads();
+  for (uint32_t base = 0; base < na; base += kShortWaves * 64) {
+    const uint32_t i = base + threadIdx.x;
+    const bool in = i < na;
+    const uint32_t w = in ? A[i] : 0xFFFFFFFFu;
+    uint32_t loads = 0;
+    const bool ok = window_member(B, nb, w, in, win[wv], loads);
+    const uint64_t m = ballot(ok);
+    __syncthreads();  // the previous counts are no longer read
+    if (lane == 0) s_cnt[wv] = (uint32_t)__popcll(m);
+    __syncthreads();
+    uint32_t at = run;
+    for (uint32_t k = 0; k < kShortWaves; k++) {
+      if (k < wv) at += s_cnt[k];
+      run += s_cnt[k];
+    }
+    if (ok) res[at + mbcnt(m)] = w;
+  }
+  if (threadIdx.x == 0) *total = bad ? kBadInput : run;
+}
+
+}  // namespace
 
 // Inputs of the intersection entry points: strictly ascending, no 0xFFFFFFFF.
 bool sorted_set(const uint32_t *a, uint32_t n) {
@@ -59,59 +137,129 @@ bool sorted_set(const uint32_t *a, uint32_t n) {
   return true;
 }
 
-// hits/cnt (device results of k_intersect, copied to the host) -> out.
-uint32_t gather_hits(const std::vector<uint32_t> &hits, const std::vector<uint32_t> &cnt, uint32_t *out) {
-  uint32_t k = 0;
-  for (size_t c = 0; c < cnt.size(); c++)
-    for (uint32_t j = 0; j < cnt[c]; j++) out[k++] = hits[c * 64 + j];
-  return k;
+namespace {
+
+// Short calls. At most kShortA entries of A go to k_intersect_short (two rounds of
+// its block); inputs of at most kShortCopy entries together are uploaded in one
+// copy, and results of at most as many come back in one with their number: a copy
+// costs some 8 us, however small. 1,000 x 3,000 entries: 67 us with a copy per array
+// and three launches, 36 with one of each.
+constexpr uint32_t kShortA = 2048, kShortCopy = 8192;
+
+uint32_t chunks_of(uint32_t na) { return (na + 63) / 64; }
+
+// Words of device memory: a | b | hits (64 per chunk) | cnt | off | total | result
+size_t words_of(uint32_t na, uint32_t nb) {
+  const size_t nch = chunks_of(na);
+  return (size_t)na + nb + nch * 64 + 2 * nch + 1 + std::min(na, nb);
 }
 
+// a and b, not empty, intersected in the words_of(na, nb) words at base; kBadInput
+// as the size if they are not in order, which the device checks with `check`.
+hipError_t intersect_in(uint32_t *base, const uint32_t *a, uint32_t na, const uint32_t *b, uint32_t nb, bool check,
+                        uint32_t *out, uint32_t *num_out) {
+  const uint32_t nch = chunks_of(na), most = std::min(na, nb);
+  uint32_t *dA = base, *dB = dA + na, *dH = dB + nb, *dC = dH + (size_t)nch * 64, *dO = dC + nch, *dT = dO + nch,
+           *dR = dT + 1;
+  uint32_t buf[kShortCopy + 1];
+  hipError_t e;
+  if ((size_t)na + nb <= kShortCopy) {
+    std::copy(a, a + na, buf);
+    std::copy(b, b + nb, buf + na);
+    if ((e = hipMemcpy(dA, buf, ((size_t)na + nb) * 4, hipMemcpyHostToDevice)) != hipSuccess) return e;
+  } else {
+    if ((e = hipMemcpy(dA, a, (size_t)na * 4, hipMemcpyHostToDevice)) != hipSuccess) return e;
+    if ((e = hipMemcpy(dB, b, (size_t)nb * 4, hipMemcpyHostToDevice)) != hipSuccess) return e;
+  }
+  if (check || na > kShortA) {
+    hipLaunchKernelGGL(k_check_clear, dim3(1), dim3(1), 0, nullptr, dT);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  if (check) {
+    const uint32_t blocks = (uint32_t)std::min<size_t>(((size_t)na + nb + 255) / 256, 2048);
+    hipLaunchKernelGGL(k_check_sorted, dim3(blocks), dim3(256), 0, nullptr, dA, na, dB, nb, dT);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  if (na <= kShortA) {
+    hipLaunchKernelGGL(k_intersect_short, dim3(1), dim3(kShortWaves * 64), 0, nullptr, dA, na, dB, nb, check, dT, dR);
+  } else {
+    const uint32_t blocks = (nch + kIntersectWaves - 1) / kIntersectWaves;
+    hipLaunchKernelGGL(k_intersect, dim3(std::min(blocks, 2048u)), dim3(kIntersectWaves * 64), 0, nullptr, dA, na, dB,
+                       nb, dH, dC, dT);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_chunk_offsets, dim3(1), dim3(1024), 0, nullptr, dC, nch, dO, dT);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_chunk_gather, dim3(std::min((nch + 3) / 4, 2048u)), dim3(256), 0, nullptr, dH, dC, dO, nch,
+                       dT, dR);
+  }
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if (most <= kShortCopy) {
+    if ((e = hipMemcpy(buf, dT, ((size_t)most + 1) * 4, hipMemcpyDeviceToHost)) != hipSuccess) return e;
+    *num_out = buf[0];
+    if (buf[0] != kBadInput) std::copy(buf + 1, buf + 1 + buf[0], out);
+    return hipSuccess;
+  }
+  uint32_t total = 0;
+  if ((e = hipMemcpy(&total, dT, 4, hipMemcpyDeviceToHost)) != hipSuccess) return e;
+  if (total && total != kBadInput &&
+      (e = hipMemcpy(out, dR, (size_t)total * 4, hipMemcpyDeviceToHost)) != hipSuccess)
+    return e;
+  *num_out = total;
+  return hipSuccess;
+}
+
+}  // namespace
 }  // namespace dsm
 
 using namespace dsm;
 
-#define ICHK(expr)                                                                                  \
-  do {                                                                                              \
-    hipError_t _e = (expr);                                                                         \
-    if (_e != hipSuccess) {                                                                         \
-      set_global_error("%s failed: %s (%s:%d)", #expr, hipGetErrorString(_e), __FILE__, __LINE__); \
-      rc = DSM_EDEVICE;                                                                             \
-      goto done;                                                                                    \
-    }                                                                                               \
-  } while (0)
+namespace {
+
+int not_sorted(const char *who) {
+  set_global_error("%s: inputs must be strictly ascending and below 0xFFFFFFFF", who);
+  return DSM_EINVAL;
+}
+
+// Arguments that settle the call: DSM_EINVAL, or DSM_OK with *num_out = 0; else 1.
+// Inputs that need the device's check are looked at here only if `all`.
+int settled(const char *who, const uint32_t *a, uint32_t na, const uint32_t *b, uint32_t nb, const uint32_t *out,
+            uint32_t *num_out, bool all) {
+  if (!num_out || (na && !a) || (nb && !b) || (na && nb && !out)) {
+    set_global_error("%s: null argument", who);
+    return DSM_EINVAL;
+  }
+  const bool none = na == 0 || nb == 0;
+  if ((none || all || (size_t)na + nb <= kShortCopy) && (!sorted_set(a, na) || !sorted_set(b, nb)))
+    return not_sorted(who);
+  if (!none) return 1;
+  *num_out = 0;
+  return DSM_OK;
+}
+
+// The call's end: what intersect_in (or an allocation before it) gave.
+int finished(const char *who, hipError_t e, const uint32_t *a, uint32_t na, const uint32_t *b, uint32_t nb,
+             uint32_t size, uint32_t *num_out) {
+  if (e == hipSuccess && size == kBadInput) return not_sorted(who);
+  // bad inputs are bad inputs, also where there is no device to say so
+  if (e != hipSuccess && (!sorted_set(a, na) || !sorted_set(b, nb))) return not_sorted(who);
+  *num_out = e == hipSuccess ? size : 0;
+  if (e == hipSuccess) return DSM_OK;
+  set_global_error("%s failed: %s", who, hipGetErrorString(e));
+  return DSM_EDEVICE;
+}
+
+}  // namespace
 
 extern "C" int dsm_intersect_sorted(int device, const uint32_t *a, uint32_t na, const uint32_t *b, uint32_t nb,
                                     uint32_t *out, uint32_t *num_out) {
-  if (!num_out || (na && !a) || (nb && !b) || (na && nb && !out)) {
-    set_global_error("dsm_intersect_sorted: null argument");
-    return DSM_EINVAL;
-  }
-  if (!sorted_set(a, na) || !sorted_set(b, nb)) {
-    set_global_error("dsm_intersect_sorted: inputs must be strictly ascending and below 0xFFFFFFFF");
-    return DSM_EINVAL;
-  }
-  *num_out = 0;
-  if (na == 0 || nb == 0) return DSM_OK;
-  int rc = DSM_OK;
-  const uint32_t nch = intersect_chunks(na);
-  std::vector<uint32_t> hits((size_t)nch * 64), cnt(nch);
-  uint32_t *dA = nullptr, *dB = nullptr, *dH = nullptr, *dC = nullptr;
-  ICHK(hipSetDevice(device));
-  ICHK(hipMalloc(&dA, (size_t)na * 4));
-  ICHK(hipMalloc(&dB, (size_t)nb * 4));
-  ICHK(hipMalloc(&dH, (size_t)nch * 64 * 4));
-  ICHK(hipMalloc(&dC, (size_t)nch * 4));
-  ICHK(hipMemcpy(dA, a, (size_t)na * 4, hipMemcpyHostToDevice));
-  ICHK(hipMemcpy(dB, b, (size_t)nb * 4, hipMemcpyHostToDevice));
-  ICHK(launch_intersect(dA, na, dB, nb, dH, dC, nullptr));
-  ICHK(hipMemcpy(cnt.data(), dC, (size_t)nch * 4, hipMemcpyDeviceToHost));
-  ICHK(hipMemcpy(hits.data(), dH, (size_t)nch * 64 * 4, hipMemcpyDeviceToHost));
-  *num_out = gather_hits(hits, cnt, out);
-done:
-  for (uint32_t *p : {dA, dB, dH, dC})
-    if (p) (void)hipFree(p);
-  return rc;
+  const char *who = "dsm_intersect_sorted";
+  if (int rc = settled(who, a, na, b, nb, out, num_out, false); rc <= 0) return rc;
+  uint32_t *base = nullptr, size = 0;
+  hipError_t e = hipSetDevice(device);
+  if (e == hipSuccess) e = hipMalloc(&base, words_of(na, nb) * 4);
+  if (e == hipSuccess) e = intersect_in(base, a, na, b, nb, (size_t)na + nb > kShortCopy, out, &size);
+  if (base) (void)hipFree(base);
+  return finished(who, e, a, na, b, nb, size, num_out);
 }
 
 // ------------------------------------------------------------------------
@@ -136,40 +284,6 @@ uint32_t *g_scratch[kMaxDevices] = {};
 std::once_flag g_scratch_once[kMaxDevices];
 hipError_t g_scratch_rc[kMaxDevices] = {};
 
-// Exclusive prefix of cnt[0, nch) into off, the total at *total (one block).
-__global__ __launch_bounds__(1024) void k_chunk_offsets(const uint32_t *cnt, uint32_t nch, uint32_t *off,
-                                                        uint32_t *total) {
-  __shared__ uint32_t part[1024];
-  __shared__ uint32_t carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (uint32_t base = 0; base < nch; base += 1024) {
-    const uint32_t i = base + threadIdx.x;
-    const uint32_t x = i < nch ? cnt[i] : 0u;
-    part[threadIdx.x] = x;
-    __syncthreads();
-    for (uint32_t d = 1; d < 1024; d <<= 1) {
-      const uint32_t y = threadIdx.x >= d ? part[threadIdx.x - d] : 0u;
-      __syncthreads();
-      part[threadIdx.x] += y;
-      __syncthreads();
-    }
-    if (i < nch) off[i] = carry + part[threadIdx.x] - x;
-    __syncthreads();
-    if (threadIdx.x == 1023) carry += part[1023];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *total = carry;
-}
-
-// Chunk c's members (hits[c * 64 ..], cnt[c] of them) to res[off[c] ..].
-__global__ __launch_bounds__(256) void k_chunk_gather(const uint32_t *hits, const uint32_t *cnt,
-                                                      const uint32_t *off, uint32_t nch, uint32_t *res) {
-  const uint32_t lane = lane_id();
-  for (uint32_t c = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; c < nch; c += (gridDim.x * blockDim.x) >> 6)
-    if (lane < cnt[c]) res[off[c] + lane] = hits[(size_t)c * 64 + lane];
-}
-
 // The array's address on `device` (current), looked up once per device.
 hipError_t scratch_of(int device, uint32_t **out) {
   if (device < 0 || device >= kMaxDevices) return hipErrorInvalidDevice;
@@ -187,43 +301,18 @@ hipError_t scratch_of(int device, uint32_t **out) {
 
 extern "C" int dsm_intersect_sorted_noalloc(int device, const uint32_t *a, uint32_t na, const uint32_t *b,
                                             uint32_t nb, uint32_t *out, uint32_t *num_out) {
-  if (!num_out || (na && !a) || (nb && !b) || (na && nb && !out)) {
-    set_global_error("dsm_intersect_sorted_noalloc: null argument");
-    return DSM_EINVAL;
-  }
-  if (!sorted_set(a, na) || !sorted_set(b, nb)) {
-    set_global_error("dsm_intersect_sorted_noalloc: inputs must be strictly ascending and below 0xFFFFFFFF");
-    return DSM_EINVAL;
-  }
-  *num_out = 0;
-  if (na == 0 || nb == 0) return DSM_OK;
-  const size_t nch = intersect_chunks(na);
-  // layout: a | b | hits (64 per chunk) | cnt | off | total | result
-  const size_t need = (size_t)na + nb + nch * 64 + 2 * nch + 1 + std::min(na, nb);
+  const char *who = "dsm_intersect_sorted_noalloc";
+  const size_t need = words_of(na, nb);
+  if (int rc = settled(who, a, na, b, nb, out, num_out, need > kScratchWords); rc <= 0) return rc;
   if (need > kScratchWords) {
+    *num_out = 0;
     set_global_error("dsm_intersect_sorted_noalloc: %zu scratch words needed, %zu available (na + nb + 66 per "
                      "64 entries of a + min(na, nb) + 1)", need, kScratchWords);
     return DSM_ELIMIT;
   }
-  int rc = DSM_OK;
-  uint32_t *base = nullptr, total = 0;
-  ICHK(hipSetDevice(device));
-  ICHK(scratch_of(device, &base));
-  {
-    uint32_t *dA = base, *dB = dA + na, *dH = dB + nb, *dC = dH + nch * 64, *dO = dC + nch, *dT = dO + nch,
-             *dR = dT + 1;
-    ICHK(hipMemcpy(dA, a, (size_t)na * 4, hipMemcpyHostToDevice));
-    ICHK(hipMemcpy(dB, b, (size_t)nb * 4, hipMemcpyHostToDevice));
-    ICHK(launch_intersect(dA, na, dB, nb, dH, dC, nullptr));
-    hipLaunchKernelGGL(k_chunk_offsets, dim3(1), dim3(1024), 0, nullptr, dC, (uint32_t)nch, dO, dT);
-    ICHK(hipGetLastError());
-    hipLaunchKernelGGL(k_chunk_gather, dim3((uint32_t)std::min<size_t>((nch + 3) / 4, 2048)), dim3(256), 0,
-                       nullptr, dH, dC, dO, (uint32_t)nch, dR);
-    ICHK(hipGetLastError());
-    ICHK(hipMemcpy(&total, dT, 4, hipMemcpyDeviceToHost));
-    if (total) ICHK(hipMemcpy(out, dR, (size_t)total * 4, hipMemcpyDeviceToHost));
-    *num_out = total;
-  }
-done:
-  return rc;
+  uint32_t *base = nullptr, size = 0;
+  hipError_t e = hipSetDevice(device);
+  if (e == hipSuccess) e = scratch_of(device, &base);
+  if (e == hipSuccess) e = intersect_in(base, a, na, b, nb, (size_t)na + nb > kShortCopy, out, &size);
+  return finished(who, e, a, na, b, nb, size, num_out);
 }
