@@ -75,6 +75,18 @@ __device__ __forceinline__ uint64_t wave_sum(uint64_t x) {
   return x;
 }
 
+// The lane's K places k among ranges whose ends are pre[1 .. 64] (LDS, ascending;
+// pre[0] = 0): the last range that starts at or before each.
+template <int K>
+__device__ __forceinline__ void ranges_of(const uint32_t *pre, const uint32_t (&k)[K], uint32_t (&o)[K]) {
+#pragma unroll
+  for (int u = 0; u < K; u++) o[u] = 0;
+  for (uint32_t half = 32; half; half >>= 1) {
+#pragma unroll
+    for (int u = 0; u < K; u++) o[u] = pre[o[u] + half] <= k[u] ? o[u] + half : o[u];
+  }
+}
+
 template <typename T>
 __device__ __forceinline__ T ld_relaxed(T *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -484,7 +484,7 @@ int build_cluster_ops(dsm_engine *e, const dsm_query_desc *qs, uint32_t nq) {
   if (!crow.empty()) HIPCHK(hipMemcpy(e->d_crow.p, crow.data(), crow.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(e->d_alive_src.alloc(asrc.size()));
   if (!asrc.empty()) HIPCHK(hipMemcpy(e->d_alive_src.p, asrc.data(), asrc.size() * 4, hipMemcpyHostToDevice));
-  HIPCHK(e->cctl.alloc(2 * (size_t)std::max<uint32_t>(nsteps, 1)));
+  HIPCHK(e->cctl.alloc(std::max<uint32_t>(nsteps, 1)));
   for (auto &x : e->ev_ref) HIPCHK(hipEventCreate(&x));
   return DSM_OK;
 }
@@ -1307,7 +1307,7 @@ int upload_records(dsm_engine *e, const std::vector<uint32_t> &s, const std::vec
 // every query runs as one k_cluster_pass launch plus one k_cluster_heavy
 // launch for the chunks of candidates with long lists (filter.cu:936-1177 runs
 // one kernel and one device synchronisation per cluster of one query).
-int cluster_refine(dsm_engine *e) {
+int cluster_refine(dsm_engine *e, uint32_t longest) {
   if (!e->cluster) return DSM_OK;
   const uint32_t nsteps = (uint32_t)e->cstep_off.size() - 1;
   // heavy chunks of one pass: at most 2 x (list entries) / kClusterChunk
@@ -1316,7 +1316,7 @@ int cluster_refine(dsm_engine *e) {
   if (need > e->cheavy.n) HIPCHK(e->cheavy.alloc(need));
   HIPCHK(hipEventRecord(e->ev_ref[0], e->stream));
   HIPCHK(launch_cluster_init(e->bm.p, e->words, e->nsig_rows, e->npos_rows, e->calive.p, e->d_alive_src.p,
-                             e->nalive_src, e->cctl.p, 2 * nsteps, e->stream));
+                             e->nalive_src, e->cctl.p, nsteps, e->stream));
   ClusterArgs a{};
   a.g = e->dev_graph();
   a.bm = e->bm.p;
@@ -1328,9 +1328,9 @@ int cluster_refine(dsm_engine *e) {
   for (uint32_t st = 0; st < nsteps; st++) {
     a.ops = e->d_cops.p + e->cstep_off[st];
     a.nops = e->cstep_off[st + 1] - e->cstep_off[st];
-    a.ctl = e->cctl.p + 2 * st;
+    a.ctl = e->cctl.p + st;
     HIPCHK(launch_cluster_pass(a, (uint32_t)e->num_cu * 8, e->stream));
-    HIPCHK(launch_cluster_heavy(a, (uint32_t)e->num_cu * 4, e->stream));
+    if (longest > kClusterChunk) HIPCHK(launch_cluster_heavy(a, (uint32_t)e->num_cu * 4, e->stream));
   }
   HIPCHK(hipEventRecord(e->ev_ref[1], e->stream));
   e->refine_timed = true;
@@ -1454,7 +1454,7 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine:
     HIPCHK(launch_lbuild(e->dev_graph(), e->tables(), list, list ? &e->actl.p->ndirty : nullptr, e->sorted_build(),
                          longest, true, e->stream));
     HIPCHK(launch_filter_dirty(e->dev_graph(), e->tables(), e->dirty(), e->stream));
-    if (int rc = cluster_refine(e)) return rc;
+    if (int rc = cluster_refine(e, longest)) return rc;
     if (done) HIPCHK(hipEventRecord(done, e->stream));
     if (int rc = take_status(e)) return rc;
     if (!e->h_actl.p->overflow) break;
@@ -1545,7 +1545,7 @@ int create_impl(dsm_engine *e, const dsm_graph_desc *graph, const dsm_query_desc
   HIPCHK(launch_build_reset(e->sorted_build(), e->stream));
   HIPCHK(launch_lbuild(e->dev_graph(), e->tables(), nullptr, nullptr, e->sorted_build(), e->h_actl.p->max_deg, false,
                        e->stream));
-  if ((rc = cluster_refine(e))) return rc;
+  if ((rc = cluster_refine(e, e->h_actl.p->max_deg))) return rc;
   HIPCHK(hipStreamSynchronize(e->stream));
   e->refine_timed = false;
   return DSM_OK;

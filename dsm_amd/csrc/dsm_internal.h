@@ -346,7 +346,7 @@ struct ClusterArgs {
   const uint32_t *crow;
   ClusterHeavy *heavy;
   uint32_t heavy_cap;
-  uint32_t *ctl;        // [2]: heavy entries queued, heavy entries claimed
+  uint32_t *ctl;        // [1]: heavy entries queued
 };
 
 // Zeroes bm rows [first_row, first_row + nrows), copies the listed (alive row,

@@ -558,18 +558,6 @@ __device__ __forceinline__ void set_bit_from(uint64_t *w, uint64_t cur, uint32_t
   else atomicAnd((unsigned long long *)w, (unsigned long long)~bit);
 }
 
-// The lane's K places k among ranges whose ends are pre[1 .. 64] (LDS, ascending;
-// pre[0] = 0): the last range that starts at or before each.
-template <int K>
-__device__ __forceinline__ void ranges_of(const uint32_t *pre, const uint32_t (&k)[K], uint32_t (&o)[K]) {
-#pragma unroll
-  for (int u = 0; u < K; u++) o[u] = 0;
-  for (uint32_t half = 32; half; half >>= 1) {
-#pragma unroll
-    for (int u = 0; u < K; u++) o[u] = pre[o[u] + half] <= k[u] ? o[u] + half : o[u];
-  }
-}
-
 // The dirty vertices, up to 64 to a wave, but those with a label-sorted copy, which
 // were filtered from its bucket sizes (filter_buckets). The lists of a wave's vertices are read as one array, as many lanes
 // to a list as it has entries, and so are their (vertex, signature) pairs, four
