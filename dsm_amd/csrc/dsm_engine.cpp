@@ -181,7 +181,7 @@ struct dsm_engine {
   DevBuf<uint32_t> d_sig_lo, d_sig_hi;
   DevBuf<uint8_t> d_lmap;
   DevBuf<Plan> d_plans;
-  DevBuf<uint32_t> d_plan_key;
+  DevBuf<uint2> d_plan_of;
   // batch
   DevBuf<uint32_t> scratch;
   unsigned long long scratch_cap = 0;
@@ -754,8 +754,14 @@ int upload_tables(dsm_engine *e) {
   HIPCHK(hipMemcpy(e->d_lmap.p, e->lmap.data(), 256, hipMemcpyHostToDevice));
   HIPCHK(e->d_plans.alloc(e->plans.size()));
   HIPCHK(hipMemcpy(e->d_plans.p, e->plans.data(), e->plans.size() * sizeof(Plan), hipMemcpyHostToDevice));
-  HIPCHK(e->d_plan_key.alloc(e->plan_key.size()));
-  HIPCHK(hipMemcpy(e->d_plan_key.p, e->plan_key.data(), e->plan_key.size() * 4, hipMemcpyHostToDevice));
+  std::vector<uint2> plan_of(kMaxRel * kMaxRel, uint2{0, 0});
+  for (size_t i = 0; i < e->plan_key.size(); i++) {
+    const uint32_t l0 = e->lmap[e->plan_key[i] >> 8], l1 = e->lmap[e->plan_key[i] & 0xFF];
+    uint2 &x = plan_of[l0 * kMaxRel + l1];
+    if (x.y++ == 0) x.x = (uint32_t)i;
+  }
+  HIPCHK(e->d_plan_of.alloc(plan_of.size()));
+  HIPCHK(hipMemcpy(e->d_plan_of.p, plan_of.data(), plan_of.size() * sizeof(uint2), hipMemcpyHostToDevice));
   const uint32_t nq = (uint32_t)e->queries.size();
   HIPCHK(e->results.alloc((size_t)nq * 2 * kMaxSlots + 1));
   HIPCHK(e->query_busy.alloc(nq));
@@ -810,7 +816,8 @@ SeedArgs seed_args(dsm_engine *e, const RoundPart *parts, int nparts) {
   sa.bm = e->bm.p;
   sa.words = e->words;
   sa.plans = e->d_plans.p;
-  sa.plan_key = e->d_plan_key.p;
+  sa.lmap = e->d_lmap.p;
+  sa.plan_of = e->d_plan_of.p;
   sa.nplans = (uint32_t)e->plans.size();
   for (int i = 0; i < 2; i++) {
     sa.rs[i] = i < nparts ? parts[i].rs : nullptr;

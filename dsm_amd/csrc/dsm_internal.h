@@ -211,7 +211,8 @@ struct SeedArgs {
   const uint64_t *bm;
   uint32_t words;
   const Plan *plans;
-  const uint32_t *plan_key;   // sorted (label0 << 8 | label1) of each plan
+  const uint8_t *lmap;        // device label -> dense index of the query labels (0xFF: none)
+  const uint2 *plan_of;       // [kMaxRel][kMaxRel]: first plan and number of plans of a pair of them
   uint32_t nplans;
   // two record lists, each with the tag written to its seeds
   const uint32_t *rs[2];
