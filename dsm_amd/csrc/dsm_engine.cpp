@@ -220,7 +220,7 @@ struct dsm_engine {
   uint32_t donate_min = 256, lane_work = 16, donate_every = 4, donate_min_n2 = 64, leaf_budget = 8192;
   bool leaf_sets = true;
   bool bit_probe_last = false;
-  bool graph_rounds = true;
+  bool seeding_timed = false;
   PinnedBuf<uint32_t> pipe_h_rec;  // records of a pipelined round (dsm_process_batches)
   DevBuf<uint32_t> pipe_d_rec;
   bool leaf_segments = true;
@@ -250,11 +250,7 @@ struct dsm_engine {
   DevBuf<unsigned long long> query_busy;  // per query: DFS task ticks since the last read
   uint32_t wave_slots = 0;       // waves of the largest grid
   uint32_t last_blocks = 0, last_wpb = 0;  // grid of the last DFS launch
-  // the DFS round as a HIP graph (graph_round)
-  hipGraph_t rg_graph = nullptr;
-  hipGraphExec_t rg_exec = nullptr;
-  hipGraphNode_t rg_reset = nullptr, rg_seed = nullptr, rg_dfs = nullptr;
-  uint32_t rg_key = 0;
+  bool results_here = false;  // h_results holds the counts of the batch applied last
   uint32_t watchdog_ms = 60000;
   int wall_khz = 100000;
   DeltaSort delta_sort;  // used by one thread at a time: the caller, or the worker it waits for
@@ -283,8 +279,6 @@ struct dsm_engine {
   ~dsm_engine() {
     for (auto &x : ev_ref)
       if (x) (void)hipEventDestroy(x);
-    if (rg_exec) (void)hipGraphExecDestroy(rg_exec);
-    if (rg_graph) (void)hipGraphDestroy(rg_graph);
     for (auto &e : ev)
       if (e) (void)hipEventDestroy(e);
     if (tuples) {
@@ -871,12 +865,15 @@ DfsArgs dfs_args(dsm_engine *e) {
   return da;
 }
 
-// The grid: a round over a handful of records gets one block per CU, so that
-// few waves pay the start-up and termination atomics.
+// The grid: a round over a handful of records gets one block per CU, so that few
+// waves pay the start-up and termination atomics, and fewer where no list is long
+// enough to give a CU's waves anything to share (a record of a graph whose lists have
+// 30 entries is matched by a few waves; 256 blocks' records cost more than that).
 uint32_t dfs_grid(dsm_engine *e, uint32_t nrec) {
   const uint64_t want =
       ((uint64_t)nrec * std::max<uint32_t>(e->max_plans_per_key, 1) * 8 + e->dfs_wpb - 1) / e->dfs_wpb;
-  uint32_t b = (uint32_t)std::min<uint64_t>(e->dfs_blocks, std::max<uint64_t>(want, (uint64_t)e->num_cu));
+  const uint64_t least = std::min<uint64_t>((uint64_t)e->num_cu, want * std::max(1u, e->h_actl.p->max_deg / 16));
+  uint32_t b = (uint32_t)std::min<uint64_t>(e->dfs_blocks, std::max<uint64_t>(want, least));
   e->last_wpb = e->tuples ? 4u : e->dfs_wpb;
   b = std::min(b, e->wave_slots / e->last_wpb);  // a mailbox for every wave
   e->last_blocks = b;
@@ -886,60 +883,19 @@ uint32_t dfs_grid(dsm_engine *e, uint32_t nrec) {
 // The waiting words of a grid.
 uint32_t idle_words(uint32_t waves) { return (waves + kIdleGroup - 1) / kIdleGroup; }
 
-void drop_round_graph(dsm_engine *e) {
-  if (e->rg_exec) (void)hipGraphExecDestroy(e->rg_exec);
-  if (e->rg_graph) (void)hipGraphDestroy(e->rg_graph);
-  e->rg_exec = nullptr;
-  e->rg_graph = nullptr;
-}
-
 // queue_capacity bounds the tasks a round hands to waiting waves: an equal share
 // for every wave of the grid.
 void cap_donations(dsm_engine *e, DfsArgs &da) {
   if (e->opt.queue_capacity) da.donate_cap = e->opt.queue_capacity / (e->last_blocks * e->last_wpb);
 }
 
-// The round as one HIP graph: reset -> seeding -> DFS, whose blocks write their
-// records to pinned host memory. Built once per launch shape (waves per block,
-// tuples or not); every later round updates the kernel nodes' arguments and
-// grids in the executable graph and launches it.
-int graph_round(dsm_engine *e, const RoundPart *parts, int nparts, uint32_t nrec, const ClearSpan &clear) {
-  RoundNodeArgs st;
-  st.ctl = e->ctl.p;
-  st.tuple_count = clear.tuple_count;
-  st.counts = clear.counts;
-  st.ncounts = clear.ncounts;
-  st.seed = seed_args(e, parts, nparts);
-  st.dfs = dfs_args(e);
-  hipKernelNodeParams pr, ps, pd;
-  const uint32_t blocks = dfs_grid(e, nrec);
-  cap_donations(e, st.dfs);
-  st.idle = e->idle.p;
-  st.nidle = idle_words(e->last_blocks * e->last_wpb);
-  round_node_params(st, blocks, e->dfs_wpb, e->max_qn, &pr, &ps, &pd);
-  const uint32_t key = (e->tuples ? 16u : 0u) | e->dfs_wpb;
-  if (!e->rg_exec || e->rg_key != key) {
-    drop_round_graph(e);
-    HIPCHK(hipGraphCreate(&e->rg_graph, 0));
-    HIPCHK(hipGraphAddKernelNode(&e->rg_reset, e->rg_graph, nullptr, 0, &pr));
-    HIPCHK(hipGraphAddKernelNode(&e->rg_seed, e->rg_graph, &e->rg_reset, 1, &ps));
-    HIPCHK(hipGraphAddKernelNode(&e->rg_dfs, e->rg_graph, &e->rg_seed, 1, &pd));
-    HIPCHK(hipGraphInstantiate(&e->rg_exec, e->rg_graph, nullptr, nullptr, 0));
-    e->rg_key = key;
-  } else {
-    HIPCHK(hipGraphExecKernelNodeSetParams(e->rg_exec, e->rg_reset, &pr));
-    HIPCHK(hipGraphExecKernelNodeSetParams(e->rg_exec, e->rg_seed, &ps));
-    HIPCHK(hipGraphExecKernelNodeSetParams(e->rg_exec, e->rg_dfs, &pd));
-  }
-  HIPCHK(hipGraphLaunch(e->rg_exec, e->stream));
-  return DSM_OK;
-}
-
-// One round, eager or as a graph. ev0 / ev1 / ev2 (may be null) mark its start,
-// the end of seeding (eager only; a graph round records ev1 at its start) and
-// its end.
+// One round. ev0 / ev1 / ev2 (may be null) mark its start, the end of seeding (its
+// start, unless seeding is timed on its own) and its end; `up` brings the records,
+// where they have not been sent. Three launches: as one HIP graph with its nodes
+// updated for every round, a round of 11 us of kernels took 25 to 28 us on the
+// device (a call with 8 records on a dense graph: 165 us, with launches 117).
 int dfs_round(dsm_engine *e, const RoundPart *parts, int nparts, hipEvent_t ev0, hipEvent_t ev1,
-              hipEvent_t ev2, ClearSpan clear = {}) {
+              hipEvent_t ev2, const SmallCopy &up, ClearSpan clear = {}) {
   uint32_t nrec = 0;
   for (int i = 0; i < nparts; i++) nrec += parts[i].n;
   if (e->counts_stale) {
@@ -947,38 +903,46 @@ int dfs_round(dsm_engine *e, const RoundPart *parts, int nparts, hipEvent_t ev0,
     e->counts_stale = false;
   }
   if (ev0) HIPCHK(hipEventRecord(ev0, e->stream));
-  if (e->graph_rounds) {
-    if (ev1) HIPCHK(hipEventRecord(ev1, e->stream));
-    int rc = graph_round(e, parts, nparts, nrec, clear);
-    if (rc) return rc;
-  } else {
-    DfsArgs da = dfs_args(e);
-    const uint32_t blocks = dfs_grid(e, nrec);
-    cap_donations(e, da);
-    HIPCHK(launch_ctl_reset(e->ctl.p, clear.tuple_count, clear.counts, clear.ncounts, e->idle.p,
-                            idle_words(e->last_blocks * e->last_wpb), e->stream));
-    HIPCHK(launch_seed(seed_args(e, parts, nparts), e->stream));
-    if (ev1) HIPCHK(hipEventRecord(ev1, e->stream));
-    HIPCHK(launch_dfs(da, blocks, e->dfs_wpb, e->max_qn, e->stream));
-  }
+  e->results_here = false;
+  if (ev1 && !e->seeding_timed) HIPCHK(hipEventRecord(ev1, e->stream));
+  DfsArgs da = dfs_args(e);
+  const uint32_t blocks = dfs_grid(e, nrec);
+  cap_donations(e, da);
+  HIPCHK(launch_ctl_reset(e->ctl.p, clear.tuple_count, clear.counts, clear.ncounts, e->idle.p,
+                          idle_words(e->last_blocks * e->last_wpb), up, e->stream));
+  HIPCHK(launch_seed(seed_args(e, parts, nparts), e->stream));
+  if (ev1 && e->seeding_timed) HIPCHK(hipEventRecord(ev1, e->stream));
+  HIPCHK(launch_dfs(da, blocks, e->dfs_wpb, e->max_qn, e->stream));
   if (ev2) HIPCHK(hipEventRecord(ev2, e->stream));
   return DSM_OK;
+}
+
+// count values to pinned host memory.
+template <typename T>
+hipError_t to_host(T *to, const T *from, size_t count, hipStream_t s) {
+  const size_t words = count * sizeof(T) / 4;
+  if (words <= kSmallCopy && ((uintptr_t)from & 7) == 0 && ((uintptr_t)to & 7) == 0)
+    return launch_small_copy({reinterpret_cast<const uint32_t *>(from), reinterpret_cast<uint32_t *>(to),
+                              (uint32_t)words}, s);
+  return hipMemcpyAsync(to, from, count * sizeof(T), hipMemcpyDeviceToHost, s);
 }
 
 // The tuple counter and the counts of slot 0 to the host; waits for the stream.
 int fetch_results(dsm_engine *e) {
   const uint32_t n = (uint32_t)e->queries.size() * 2;
-  if (e->counts_stale) HIPCHK(launch_ctl_reset(nullptr, e->tuple_count(), e->counts(), n, nullptr, 0, e->stream));
+  if (e->counts_stale) HIPCHK(launch_ctl_reset(nullptr, e->tuple_count(), e->counts(), n, nullptr, 0, {}, e->stream));
   e->counts_stale = false;
-  HIPCHK(hipMemcpyAsync(e->h_results.p, e->results.p, (size_t)(n + 1) * 8, hipMemcpyDeviceToHost, e->stream));
+  HIPCHK(to_host(e->h_results.p, e->results.p, n + 1, e->stream));
   HIPCHK(hipStreamSynchronize(e->stream));
   return DSM_OK;
 }
 
 int run_round(dsm_engine *e, const uint32_t *rs, const uint32_t *rd, uint32_t nrec, uint32_t tag,
-              hipEvent_t ev0, hipEvent_t ev1, hipEvent_t ev2) {
+              hipEvent_t ev0, hipEvent_t ev1, hipEvent_t ev2, const SmallCopy &up = {}) {
   const RoundPart p{rs, rd, nrec, tag};
-  return dfs_round(e, &p, 1, ev0, ev1, ev2);
+  if (int rc = dfs_round(e, &p, 1, ev0, ev1, ev2, up)) return rc;
+  if (up.words) HIPCHK(hipEventRecord(e->ev_hrec, e->stream));
+  return DSM_OK;
 }
 
 // The last round's errors: the records of its blocks, which have ended.
@@ -1145,6 +1109,7 @@ int grow_pool(dsm_engine *e, unsigned long long extra);
 struct RoundArrays {
   BatchDev b;
   const uint32_t *last_touched, *last_relabel;
+  SmallCopy up;
 };
 
 // A bound on the pieces of T touched lists and their inserts.
@@ -1152,7 +1117,8 @@ size_t max_segs(const dsm_engine *e, size_t T, size_t inserts) {
   return T + (size_t)((e->pool_cap + inserts) / kApplySeg);
 }
 
-// Sends a round's arrays in one copy.
+// Sends a round's arrays in one copy, or leaves it to the kernel that begins the round
+// (out.up); the caller records ev_hbuf after that.
 int upload_round(dsm_engine *e, const Slice &sl, const HostDelta *relabels, bool last, RoundArrays &out) {
   static const std::vector<uint32_t> none;
   const uint32_t T = (uint32_t)sl.tv.size();
@@ -1170,8 +1136,9 @@ int upload_round(dsm_engine *e, const Slice &sl, const HostDelta *relabels, bool
   HIPCHK(e->hbuf.ensure(total));
   HIPCHK(e->bbuf.ensure(dtotal));
   for (int i = 0; i < 9; i++) std::copy(parts[i]->begin(), parts[i]->end(), e->hbuf.p + off[i]);
-  if (total) HIPCHK(hipMemcpyAsync(e->bbuf.p, e->hbuf.p, total * 4, hipMemcpyHostToDevice, e->stream));
-  HIPCHK(hipEventRecord(e->ev_hbuf, e->stream));
+  out.up = {};
+  if (total <= kSmallCopy) out.up = {e->hbuf.p, e->bbuf.p, (uint32_t)total};
+  else HIPCHK(hipMemcpyAsync(e->bbuf.p, e->hbuf.p, total * 4, hipMemcpyHostToDevice, e->stream));
   // first the touched lists' pieces, then the relabelled vertices'
   const size_t segs = max_segs(e, std::max<size_t>(T, R), sl.ins.size());
   if (T > e->soff.n || segs > e->segs.n) HIPCHK(hipStreamSynchronize(e->stream));
@@ -1215,7 +1182,7 @@ int ensure_scratch(dsm_engine *e, size_t inserts) {
 
 // Waits for the update's status.
 int take_status(dsm_engine *e) {
-  HIPCHK(hipMemcpyAsync(e->h_actl.p, e->actl.p, sizeof(ApplyCtl), hipMemcpyDeviceToHost, e->stream));
+  HIPCHK(to_host(e->h_actl.p, e->actl.p, 1, e->stream));
   HIPCHK(hipStreamSynchronize(e->stream));
   if (e->h_actl.p->merge_overflow)
     return e->fail_msg(DSM_ELIMIT, "update: %u merged lists found no room in the merge scratch",
@@ -1292,9 +1259,10 @@ int grow_pool(dsm_engine *e, unsigned long long extra) {
   return DSM_OK;
 }
 
-// Records on the device, src[k] | dst[k].
+// Records on the device, src[k] | dst[k]; few of them are left to the next round's
+// first kernel (up), where it is given.
 int upload_records(dsm_engine *e, const std::vector<uint32_t> &s, const std::vector<uint32_t> &d,
-                   DevBuf<uint32_t> &dev) {
+                   DevBuf<uint32_t> &dev, SmallCopy *up = nullptr) {
   const size_t k = s.size();
   if (2 * k > dev.n) HIPCHK(hipStreamSynchronize(e->stream));
   HIPCHK(dev.ensure(2 * k));
@@ -1302,6 +1270,10 @@ int upload_records(dsm_engine *e, const std::vector<uint32_t> &s, const std::vec
   HIPCHK(e->hrec.ensure(2 * k));
   std::copy(s.begin(), s.end(), e->hrec.p);
   std::copy(d.begin(), d.end(), e->hrec.p + k);
+  if (up && 2 * k <= kSmallCopy) {
+    *up = {e->hrec.p, dev.p, (uint32_t)(2 * k)};
+    return DSM_OK;
+  }
   HIPCHK(hipMemcpyAsync(dev.p, e->hrec.p, 2 * k * 4, hipMemcpyHostToDevice, e->stream));
   HIPCHK(hipEventRecord(e->ev_hrec, e->stream));
   return DSM_OK;
@@ -1414,7 +1386,8 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine:
     const bool final_round = rd + 1 == rounds;
     if (int rc = upload_round(e, sl, final_round ? &d : nullptr, from && rd == 0, ra)) return rc;
     if (rd == 0) {
-      HIPCHK(launch_update_begin(e->actl.p, from ? from->actl.p : nullptr, e->build_ctl.p, e->stream));
+      HIPCHK(launch_update_begin(e->actl.p, from ? from->actl.p : nullptr, e->build_ctl.p, ra.up, e->stream));
+      HIPCHK(hipEventRecord(e->ev_hbuf, e->stream));
       if (from) {
         CatchUp c;
         c.x = graph_of(e, *from);
@@ -1432,7 +1405,8 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine:
         HIPCHK(launch_catch_up(c, before, e->stream));
       }
     } else {
-      HIPCHK(launch_round_begin(e->actl.p, e->stream));
+      HIPCHK(launch_round_begin(e->actl.p, ra.up, e->stream));
+      HIPCHK(hipEventRecord(e->ev_hbuf, e->stream));
     }
     if (int rc = ensure_scratch(e, sl.ins.size())) return rc;
     // pieces: one a list, and what no list can go past
@@ -1545,7 +1519,7 @@ int create_impl(dsm_engine *e, const dsm_graph_desc *graph, const dsm_query_desc
   e->donate_min_n2 = e->opt.donate_min_n2 ? e->opt.donate_min_n2 : 64;
   e->leaf_sets = e->opt.leaf_sets != 0;
   e->bit_probe_last = e->opt.bit_probe_last != 0;
-  e->graph_rounds = e->opt.graph_rounds != 0;
+  e->seeding_timed = e->opt.graph_rounds == 0;
   e->leaf_segments = e->opt.leaf_segments != 0;
   e->poll_max = e->opt.poll_max ? std::min<uint32_t>(e->opt.poll_max, 16u) : 16u;
   HIPCHK(launch_filter_full(e->dev_graph(), e->tables(), e->stream));
@@ -1579,15 +1553,6 @@ void swap_graph(dsm_engine *e) {
   std::swap(e->pool_cap, c.pool_cap);
 }
 
-template <typename T>
-hipError_t copy_buf(DevBuf<T> &dst, const DevBuf<T> &src, size_t count, hipStream_t s) {
-  if (dst.n < src.n) {
-    hipError_t err = dst.alloc(src.n);
-    if (err != hipSuccess) return err;
-  }
-  return count ? hipMemcpyAsync(dst.p, src.p, count * sizeof(T), hipMemcpyDeviceToDevice, s) : hipSuccess;
-}
-
 // Allocates the second copy of the graph at the current sizes; its contents
 // are written by the first overlapped update.
 int reserve_shadow(dsm_engine *e) {
@@ -1613,16 +1578,25 @@ int reserve_shadow(dsm_engine *e) {
 int copy_graph(dsm_engine *e, const dsm_engine::GraphCopy &c) {
   unsigned long long used = e->h_actl.p->pool_used;
   if (used == 0 || used > c.pool_cap) used = c.pool_cap;
-  HIPCHK(copy_buf(e->pool, c.pool, used, e->stream));
-  HIPCHK(copy_buf(e->lpool, c.lpool, used, e->stream));
-  HIPCHK(copy_buf(e->start, c.start, c.start.n, e->stream));
-  HIPCHK(copy_buf(e->deg, c.deg, c.deg.n, e->stream));
-  HIPCHK(copy_buf(e->cap, c.cap, c.cap.n, e->stream));
-  HIPCHK(copy_buf(e->loff, c.loff, c.loff.n, e->stream));
-  HIPCHK(copy_buf(e->lab, c.lab, c.lab.n, e->stream));
+  ArrayCopies a{};
+  auto add = [&](auto &dst, const auto &src, size_t count) -> hipError_t {
+    a.from[a.n] = src.p;
+    a.bytes[a.n] = count * sizeof(*src.p);
+    const hipError_t err = dst.n < src.n ? dst.alloc(src.n) : hipSuccess;
+    a.to[a.n++] = dst.p;
+    return err;
+  };
+  HIPCHK(add(e->pool, c.pool, used));
+  HIPCHK(add(e->lpool, c.lpool, used));
+  HIPCHK(add(e->start, c.start, c.start.n));
+  HIPCHK(add(e->deg, c.deg, c.deg.n));
+  HIPCHK(add(e->cap, c.cap, c.cap.n));
+  HIPCHK(add(e->loff, c.loff, c.loff.n));
+  HIPCHK(add(e->lab, c.lab, c.lab.n));
   // the signature rows; the cluster position rows are recomputed by the update
-  HIPCHK(copy_buf(e->bm, c.bm, (size_t)e->nsig_rows * e->words, e->stream));
-  HIPCHK(copy_buf(e->actl, c.actl, 1, e->stream));
+  HIPCHK(add(e->bm, c.bm, (size_t)e->nsig_rows * e->words));
+  HIPCHK(add(e->actl, c.actl, 1));
+  HIPCHK(launch_array_copies(a, e->stream));
   e->pool_cap = c.pool_cap;
   return DSM_OK;
 }
@@ -1765,6 +1739,7 @@ int dsm_apply_batch(dsm_engine *e, const dsm_change *changes, uint32_t k) {
     }
   }
   e->counts_stale = true;
+  e->results_here = false;
   int rc;
   bool applied = false;
   // 1. negatives in the pre-batch graph; with overlap_apply the batch is
@@ -1773,9 +1748,12 @@ int dsm_apply_batch(dsm_engine *e, const dsm_change *changes, uint32_t k) {
     const uint32_t nn = (uint32_t)e->neg_s.size();
     if ((rc = ensure_seed_cap(e, nn))) return rc;
     DevBuf<uint32_t> &rb = e->rec_neg;
-    if ((rc = upload_records(e, e->neg_s, e->neg_d, rb))) return rc;
+    SmallCopy up{};
+    if ((rc = upload_records(e, e->neg_s, e->neg_d, rb, &up))) return rc;
     if (e->overlap_apply) HIPCHK(hipEventRecord(e->ev_pre, e->stream));
-    if ((rc = run_round(e, rb.p, rb.p + nn, nn, 0, nullptr, e->ev[7], e->ev[8]))) return rc;
+    if ((rc = run_round(e, rb.p, rb.p + nn, nn, 0, nullptr, e->ev[7], e->ev[8], up))) return rc;
+    // with no positives to come these are the batch's counts
+    if (e->pos_s.empty()) HIPCHK(to_host(e->h_results.p, e->results.p, 2 * e->queries.size() + 1, e->stream));
     if (e->overlap_apply) {
       HostDelta d;
       host_delta(e, changes, k, d);
@@ -1783,6 +1761,7 @@ int dsm_apply_batch(dsm_engine *e, const dsm_change *changes, uint32_t k) {
       applied = true;
     }
     HIPCHK(hipStreamSynchronize(e->stream));
+    e->results_here = e->pos_s.empty();
     if ((rc = check_round(e, &e->stats.seeds_neg))) return rc;
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, e->ev[7], e->ev[8]));
@@ -1823,10 +1802,10 @@ int dsm_match_batch(dsm_engine *e, uint64_t *pos, uint64_t *neg) {
     const uint32_t np = (uint32_t)e->pos_s.size();
     if ((rc = ensure_seed_cap(e, np))) return rc;
     DevBuf<uint32_t> &rb = e->rec_pos;
-    if ((rc = upload_records(e, e->pos_s, e->pos_d, rb))) return rc;
-    // a graph round's seeding is part of its DFS time
-    hipEvent_t seeding = e->graph_rounds ? nullptr : e->ev[3];
-    if ((rc = run_round(e, rb.p, rb.p + np, np, 1, seeding, e->ev[4], e->ev[5]))) return rc;
+    SmallCopy up{};
+    if ((rc = upload_records(e, e->pos_s, e->pos_d, rb, &up))) return rc;
+    hipEvent_t seeding = e->seeding_timed ? e->ev[3] : nullptr;  // else part of the DFS time
+    if ((rc = run_round(e, rb.p, rb.p + np, np, 1, seeding, e->ev[4], e->ev[5], up))) return rc;
     if ((rc = fetch_results(e))) return rc;
     fetched = true;
     if ((rc = check_round(e, &e->stats.seeds_pos))) return rc;
@@ -1837,7 +1816,7 @@ int dsm_match_batch(dsm_engine *e, uint64_t *pos, uint64_t *neg) {
     e->stats.ms_dfs_pos = ms;
   }
   e->batch_pending = false;
-  if (!fetched && (rc = fetch_results(e))) return rc;
+  if (!fetched && !e->results_here && (rc = fetch_results(e))) return rc;
   e->stats.tuples = *e->h_results.p;
   for (uint32_t q = 0; q < nq; q++) {
     if (pos) pos[q] = e->h_counts()[2 * q + 1];
@@ -2353,19 +2332,21 @@ int pipe_round(dsm_engine *e, PinnedBuf<uint32_t> &h_rec, DevBuf<uint32_t> &d_re
       std::copy(R->ns.begin(), R->ns.end(), h + 2 * np);
       std::copy(R->nd.begin(), R->nd.end(), h + 2 * np + nn);
     }
-    HIPCHK(hipMemcpyAsync(d_rec.p, h, 2 * (size_t)(np + nn) * 4, hipMemcpyHostToDevice, e->stream));
+    SmallCopy up{};
+    if (2 * (size_t)(np + nn) <= kSmallCopy) up = {h, d_rec.p, 2 * (np + nn)};
+    else HIPCHK(hipMemcpyAsync(d_rec.p, h, 2 * (size_t)(np + nn) * 4, hipMemcpyHostToDevice, e->stream));
     RoundPart parts[2];
     int nparts = 0;
     if (np) parts[nparts++] = RoundPart{d_rec.p, d_rec.p + np, np, (P->slot << 1) | 1u};
     if (nn) parts[nparts++] = RoundPart{d_rec.p + 2 * np, d_rec.p + 2 * np + nn, nn, R->slot << 1};
-    if ((rc = dfs_round(e, parts, nparts, stats ? e->ev[9] : nullptr, nullptr, stats ? e->ev[11] : nullptr, clear)))
+    if ((rc = dfs_round(e, parts, nparts, stats ? e->ev[9] : nullptr, nullptr, stats ? e->ev[11] : nullptr, up, clear)))
       return rc;
   } else if (R) {
-    HIPCHK(launch_ctl_reset(nullptr, nullptr, clear.counts, clear.ncounts, nullptr, 0, e->stream));
+    HIPCHK(launch_ctl_reset(nullptr, nullptr, clear.counts, clear.ncounts, nullptr, 0, {}, e->stream));
   }
   if (P)
-    HIPCHK(hipMemcpyAsync(e->h_counts() + (size_t)P->slot * nq * 2, e->counts() + (size_t)P->slot * nq * 2,
-                          (size_t)nq * 2 * 8, hipMemcpyDeviceToHost, e->stream));
+    HIPCHK(to_host(e->h_counts() + (size_t)P->slot * nq * 2, e->counts() + (size_t)P->slot * nq * 2, (size_t)nq * 2,
+                   e->stream));
   if (R && d && !have_delta) host_delta(e, R->rec, R->nrec, *d);
   if (overlap) {
     if ((rc = overlap_apply(e, *d, stats))) return rc;

@@ -237,6 +237,28 @@ struct DirtyArgs {
 // Message of the last failed call that has no engine (dsm_last_error(NULL)).
 void set_global_error(const char *fmt, ...);
 
+// Words that a kernel copies between pinned host memory and the device on its way
+// (none if words is 0). A copy of its own costs a launch, an API call and a blit
+// kernel, some 8 us in all; up to kSmallCopy words one block reads them over the
+// host link in 3 to 4 us.
+constexpr uint32_t kSmallCopy = 4096;
+struct SmallCopy {
+  const uint32_t *from;
+  uint32_t *to;
+  uint32_t words;
+};
+// A copy of at most kSmallCopy words.
+hipError_t launch_small_copy(const SmallCopy &c, hipStream_t s);
+// Several arrays copied by one launch (from and to aligned to 16 bytes).
+struct ArrayCopies {
+  static constexpr uint32_t kMost = 10;
+  const void *from[kMost];
+  void *to[kMost];
+  size_t bytes[kMost];  // multiples of 4
+  uint32_t n;
+};
+hipError_t launch_array_copies(const ArrayCopies &c, hipStream_t s);
+
 // The adjacency of an edge list (dsm_build.hip). Keys are source << bits | target,
 // two an edge (count = 2 m); hist has csr_scan_words(count) words, sums
 // csr_sum_words of what is scanned (hist, or n slots).
@@ -376,9 +398,10 @@ constexpr uint32_t kBuildSeg = 1024;     // label-sorted copies of longer lists 
 
 // Takes over the status `from` (null: keeps its own) and clears what an update
 // counts, also bctl[4] (SortedBuild::ctl).
-hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl, hipStream_t s);
+hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl, const SmallCopy &up,
+                               hipStream_t s);
 // Clears what the merges of one round count (updates with more than one).
-hipError_t launch_round_begin(ApplyCtl *actl, hipStream_t s);
+hipError_t launch_round_begin(ApplyCtl *actl, const SmallCopy &up, hipStream_t s);
 // The merges and commits of a round; max_segs bounds the pieces.
 hipError_t launch_apply(const DevGraph &g, const BatchDev &b, uint32_t *scratch, unsigned long long scratch_cap,
                         unsigned long long pool_cap, ApplyCtl *actl, const DirtyArgs &d, size_t max_segs,
@@ -443,35 +466,15 @@ hipError_t launch_seed(const SeedArgs &a, hipStream_t s);
 hipError_t launch_dfs(const DfsArgs &a, uint32_t blocks, uint32_t waves_per_block, uint32_t max_query_vertices,
                       hipStream_t s);
 // Resets the DFS control block (ctl) with the nidle waiting words, the tuple
-// counter and ncounts match counts; null pointers are skipped.
+// counter and ncounts match counts; null pointers are skipped. Also the copy `up`
+// (the round's records).
 hipError_t launch_ctl_reset(DfsCtl *ctl, unsigned long long *tuple_count, unsigned long long *counts,
-                            uint32_t ncounts, IdleWord *idle, uint32_t nidle, hipStream_t s);
+                            uint32_t ncounts, IdleWord *idle, uint32_t nidle, const SmallCopy &up, hipStream_t s);
 hipError_t launch_pool_move(const uint32_t *old_pool, uint32_t *new_pool, const uint32_t *old_start,
                             const uint32_t *new_start, const uint32_t *deg, uint32_t n,
                             hipStream_t s);
 int dfs_max_blocks_per_cu(uint32_t waves_per_block, uint32_t max_query_vertices);
 
-// Kernel-node parameters of one DFS round for a HIP graph (reset, seeding, the
-// DFS), the same launches launch_ctl_reset / launch_seed / launch_dfs make. The
-// node's kernelParams point into `st`, which must stay valid until the node is
-// added or updated (the values are copied then). A seeding with no records still
-// gets one block, which does nothing.
-struct RoundNodeArgs {
-  DfsCtl *ctl;
-  unsigned long long *tuple_count, *counts;  // cleared by the reset (null: kept)
-  uint32_t ncounts;
-  IdleWord *idle;
-  uint32_t nidle;
-  SeedArgs seed;
-  DfsArgs dfs;
-  uint32_t chunk_levels;
-  void *reset_params[6];
-  void *seed_params[1];
-  void *dfs_params[2];
-};
-void round_node_params(RoundNodeArgs &st, uint32_t blocks, uint32_t waves_per_block,
-                       uint32_t max_query_vertices, hipKernelNodeParams *reset, hipKernelNodeParams *seed,
-                       hipKernelNodeParams *dfs);
 uint32_t dfs_lds_bytes_per_wave(uint32_t max_query_vertices);
 
 }  // namespace dsm

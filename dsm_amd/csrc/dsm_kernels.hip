@@ -118,6 +118,32 @@ __global__ __launch_bounds__(kCompactBlock) void k_dirty_compact(DevGraph g, Dir
   }
 }
 
+// The block's part in a SmallCopy, 8 bytes a thread at a time (both sides are
+// aligned to that), eight in flight.
+__device__ __forceinline__ void small_copy(const SmallCopy &c) {
+  const uint2 *from = reinterpret_cast<const uint2 *>(c.from);
+  uint2 *to = reinterpret_cast<uint2 *>(c.to);
+  const uint32_t pairs = c.words / 2;
+#pragma unroll 8
+  for (uint32_t i = threadIdx.x; i < pairs; i += blockDim.x) to[i] = from[i];
+  if (threadIdx.x == 0 && c.words % 2) c.to[c.words - 1] = c.from[c.words - 1];
+}
+
+__global__ __launch_bounds__(256) void k_small_copy(SmallCopy c) { small_copy(c); }
+
+__global__ __launch_bounds__(256) void k_array_copies(ArrayCopies c) {
+  const size_t tid = (size_t)blockIdx.x * 256 + threadIdx.x, nth = (size_t)gridDim.x * 256;
+  for (uint32_t k = 0; k < c.n; k++) {
+    const uint4 *from = static_cast<const uint4 *>(c.from[k]);
+    uint4 *to = static_cast<uint4 *>(c.to[k]);
+    const size_t quads = c.bytes[k] / 16, words = c.bytes[k] / 4;
+#pragma unroll 4
+    for (size_t i = tid; i < quads; i += nth) to[i] = from[i];
+    const size_t w = quads * 4 + tid;
+    if (w < words) static_cast<uint32_t *>(c.to[k])[w] = static_cast<const uint32_t *>(c.from[k])[w];
+  }
+}
+
 // ------------------------------------------------------------------ apply
 
 constexpr uint32_t kBlockList = 65536;
@@ -406,7 +432,9 @@ __global__ __launch_bounds__(256) void k_apply_slots(DevGraph g, BatchDev b, uns
 
 // The start of an update: its status from another graph copy's, its counters
 // cleared.
-__global__ void k_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl) {
+__global__ __launch_bounds__(256) void k_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl,
+                                                       SmallCopy up) {
+  small_copy(up);
   if (threadIdx.x != 0) return;
   if (from) {
     actl->pool_used = from->pool_used;
@@ -423,7 +451,8 @@ __global__ void k_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *b
   for (int i = 0; i < 4; i++) actl->sync_queued[i] = bctl[i] = 0;
 }
 
-__global__ void k_round_begin(ApplyCtl *actl) {
+__global__ __launch_bounds__(256) void k_round_begin(ApplyCtl *actl, SmallCopy up) {
+  small_copy(up);
   if (threadIdx.x != 0) return;
   actl->scratch_used = 0;
   actl->nsegs = 0;
@@ -1096,8 +1125,10 @@ __global__ __launch_bounds__(256) void k_seed(SeedArgs a) {
   }
 }
 
-__global__ void k_ctl_reset(DfsCtl *ctl, unsigned long long *tuple_count, unsigned long long *counts,
-                            uint32_t ncounts, IdleWord *idle, uint32_t nidle) {
+__global__ __launch_bounds__(256) void k_ctl_reset(DfsCtl *ctl, unsigned long long *tuple_count,
+                                                    unsigned long long *counts, uint32_t ncounts, IdleWord *idle,
+                                                    uint32_t nidle, SmallCopy up) {
+  small_copy(up);
   for (uint32_t i = threadIdx.x; counts && i < ncounts; i += blockDim.x) counts[i] = 0;
   for (uint32_t i = threadIdx.x; i < nidle; i += blockDim.x) idle[i].v = 0;
   if (ctl && threadIdx.x < kSeedHeads) ctl->seed_head[threadIdx.x].v = 0;
@@ -2318,13 +2349,26 @@ uint32_t blocks_for(size_t n, uint32_t per_block, uint32_t most) {
 
 }  // namespace
 
-hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl, hipStream_t s) {
-  hipLaunchKernelGGL(k_update_begin, dim3(1), dim3(64), 0, s, actl, from, bctl);
+hipError_t launch_small_copy(const SmallCopy &c, hipStream_t s) {
+  if (c.words) hipLaunchKernelGGL(k_small_copy, dim3(1), dim3(256), 0, s, c);
   return hipGetLastError();
 }
 
-hipError_t launch_round_begin(ApplyCtl *actl, hipStream_t s) {
-  hipLaunchKernelGGL(k_round_begin, dim3(1), dim3(64), 0, s, actl);
+hipError_t launch_array_copies(const ArrayCopies &c, hipStream_t s) {
+  size_t most = 0;
+  for (uint32_t k = 0; k < c.n; k++) most = std::max(most, c.bytes[k]);
+  if (most) hipLaunchKernelGGL(k_array_copies, dim3(blocks_for(most, 4 * 256 * 16, 4096)), dim3(256), 0, s, c);
+  return hipGetLastError();
+}
+
+hipError_t launch_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl, const SmallCopy &up,
+                               hipStream_t s) {
+  hipLaunchKernelGGL(k_update_begin, dim3(1), dim3(256), 0, s, actl, from, bctl, up);
+  return hipGetLastError();
+}
+
+hipError_t launch_round_begin(ApplyCtl *actl, const SmallCopy &up, hipStream_t s) {
+  hipLaunchKernelGGL(k_round_begin, dim3(1), dim3(256), 0, s, actl, up);
   return hipGetLastError();
 }
 
@@ -2452,54 +2496,6 @@ hipError_t launch_dfs(const DfsArgs &a, uint32_t blocks, uint32_t waves_per_bloc
   return hipGetLastError();
 }
 
-void round_node_params(RoundNodeArgs &st, uint32_t blocks, uint32_t waves_per_block,
-                       uint32_t max_query_vertices, hipKernelNodeParams *reset, hipKernelNodeParams *seed,
-                       hipKernelNodeParams *dfs) {
-  st.reset_params[0] = &st.ctl;
-  st.reset_params[1] = &st.tuple_count;
-  st.reset_params[2] = &st.counts;
-  st.reset_params[3] = &st.ncounts;
-  st.reset_params[4] = &st.idle;
-  st.reset_params[5] = &st.nidle;
-  *reset = hipKernelNodeParams{};
-  reset->func = reinterpret_cast<void *>(&k_ctl_reset);
-  reset->gridDim = dim3(1);
-  reset->blockDim = dim3(256);
-  reset->sharedMemBytes = 0;
-  reset->kernelParams = st.reset_params;
-  reset->extra = nullptr;
-  st.seed_params[0] = &st.seed;
-  *seed = hipKernelNodeParams{};
-  seed->func = reinterpret_cast<void *>(&k_seed);
-  const uint32_t nrec = st.seed.nrec[0] + st.seed.nrec[1];
-  seed->gridDim = dim3(blocks_for(nrec, 4 * seed_share(nrec), 4096));
-  seed->blockDim = dim3(256);
-  seed->sharedMemBytes = 0;
-  seed->kernelParams = st.seed_params;
-  seed->extra = nullptr;
-  st.chunk_levels = max_query_vertices > 3 ? max_query_vertices - 3 : 1;
-  st.dfs_params[0] = &st.dfs;
-  st.dfs_params[1] = &st.chunk_levels;
-  const size_t per = wave_lds_bytes(st.chunk_levels);
-  uint32_t wpb = st.dfs.tuples ? 4u : waves_per_block;
-  void *fn;
-  if (st.dfs.tuples) fn = reinterpret_cast<void *>(&k_dfs<4, true>);
-  else if (wpb == 1) fn = reinterpret_cast<void *>(&k_dfs<1, false>);
-  else if (wpb == 2) fn = reinterpret_cast<void *>(&k_dfs<2, false>);
-  else if (wpb == 8) fn = reinterpret_cast<void *>(&k_dfs<8, false>);
-  else {
-    wpb = 4;
-    fn = reinterpret_cast<void *>(&k_dfs<4, false>);
-  }
-  *dfs = hipKernelNodeParams{};
-  dfs->func = fn;
-  dfs->gridDim = dim3(blocks);
-  dfs->blockDim = dim3(wpb * 64);
-  dfs->sharedMemBytes = (unsigned int)(wpb * per);
-  dfs->kernelParams = st.dfs_params;
-  dfs->extra = nullptr;
-}
-
 uint32_t dfs_lds_bytes_per_wave(uint32_t max_query_vertices) {
   return wave_lds_bytes(max_query_vertices > 3 ? max_query_vertices - 3 : 1);
 }
@@ -2515,8 +2511,8 @@ int dfs_max_blocks_per_cu(uint32_t waves_per_block, uint32_t max_query_vertices)
 }
 
 hipError_t launch_ctl_reset(DfsCtl *ctl, unsigned long long *tuple_count, unsigned long long *counts,
-                            uint32_t ncounts, IdleWord *idle, uint32_t nidle, hipStream_t s) {
-  hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(256), 0, s, ctl, tuple_count, counts, ncounts, idle, nidle);
+                            uint32_t ncounts, IdleWord *idle, uint32_t nidle, const SmallCopy &up, hipStream_t s) {
+  hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(256), 0, s, ctl, tuple_count, counts, ncounts, idle, nidle, up);
   return hipGetLastError();
 }
 

@@ -92,9 +92,10 @@ typedef struct {
                                 8-unit s_sleeps between polls (1..16; 0 = 16) */
   int leaf_segments;         /* 1: with leaf sets, the lanes' leaf lists are scanned as
                                 one segmented array; 0: each lane scans its own */
-  int graph_rounds;          /* 1: each DFS round (control reset, seeding, DFS, status
-                                copy) is one HIP graph launch, built once and updated
-                                per round; 0: separate launches */
+  int graph_rounds;          /* a DFS round is three launches (reset, seeding, DFS) either
+                                way, which take less than one HIP graph of them; 0: their
+                                seeding is timed on its own (dsm_stats.ms_seed), 1: as
+                                part of the DFS */
   int overlap_apply;         /* 1: the update is applied to a second copy of the graph
                                 while a round matches on the first: the next batch's
                                 during pipelined rounds (dsm_process_batches, the served
