@@ -460,6 +460,14 @@ struct SortedBuild {
 hipError_t launch_lbuild(const DevGraph &g, const FilterTables &ft, const uint32_t *list, const uint32_t *count,
                          const SortedBuild &hs, uint32_t longest, bool filter, hipStream_t s);
 hipError_t launch_build_reset(const SortedBuild &hs, hipStream_t s);
+// A whole update in one launch: begin, apply, relabel, builds and re-filter, with its
+// status written to pinned host memory. longest <= kBuildSeg, kSmallChanges changes,
+// the arrays small enough for `up`.
+constexpr uint32_t kSmallChanges = 128;
+hipError_t launch_update_small(const DevGraph &g, const BatchDev &b, const FilterTables &ft, const DirtyArgs &d,
+                               const SortedBuild &hs, uint32_t *scratch, unsigned long long scratch_cap,
+                               unsigned long long pool_cap, uint32_t longest, const SmallCopy &up, ApplyCtl *status,
+                               hipStream_t s);
 // The candidate bits of the dirty vertices without a label-sorted copy.
 hipError_t launch_filter_dirty(const DevGraph &g, const FilterTables &ft, const DirtyArgs &d, hipStream_t s);
 hipError_t launch_seed(const SeedArgs &a, hipStream_t s);

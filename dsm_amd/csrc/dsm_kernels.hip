@@ -14,6 +14,7 @@
 //   k_filter_full / k_filter_light
 //                                   LDF/NLF candidate bitmaps
 //                                   (filter.cu:394-566, compact filter.cu:1692)
+//   k_update_small                  all of the above for a small update, by one block
 //   k_seed                          device edge seeding (main.cu:268-329;
 //                                   replaces the host ResTable and join.cu)
 //   k_dfs                           persistent wave64 DFS with per-wave LDS
@@ -32,7 +33,15 @@ constexpr int kApplyWaves = 4;
 
 // A commit or merge of this update found no room: the kernels after it wait for
 // the host, which makes room, tries again and launches them anew.
-__device__ __forceinline__ bool held_up(const ApplyCtl *actl) { return actl->overflow | actl->merge_overflow; }
+// ONE: in the one-block update (k_update_small), whose own atomics wrote the words.
+template <bool ONE = false, typename T>
+__device__ __forceinline__ T ctl_word(const T &w) {
+  return ONE ? ld_relaxed(&w) : w;
+}
+template <bool ONE = false>
+__device__ __forceinline__ bool held_up(const ApplyCtl *actl) {
+  return ctl_word<ONE>(actl->overflow) | ctl_word<ONE>(actl->merge_overflow);
+}
 
 __device__ __forceinline__ bool bit_of(const uint64_t *bm, uint32_t words, uint32_t sig, uint32_t v) {
   return (bm[(size_t)sig * words + (v >> 6)] >> (v & 63)) & 1ull;
@@ -89,10 +98,11 @@ __device__ __forceinline__ T block_take(T c, T *count, T *sums) {
 // of any other vertex, and one that takes such a label later is marked by its own
 // relabel, so a stale copy never gets read.
 constexpr uint32_t kCompactBlock = 512;
-__global__ __launch_bounds__(kCompactBlock) void k_dirty_compact(DevGraph g, DirtyArgs d) {
+template <bool ONE>
+__device__ __forceinline__ void compact_dirty(DevGraph g, DirtyArgs d) {
   __shared__ uint32_t s_sum[kCompactBlock / 64 + 1];
   const uint32_t ngroups = (g.n + 15) / 16;
-  if (held_up(d.actl)) return;
+  if (held_up<ONE>(d.actl)) return;
   for (uint32_t w0 = blockIdx.x * kCompactBlock; w0 < ngroups; w0 += gridDim.x * kCompactBlock) {
     const uint32_t wi = w0 + threadIdx.x;
     uint4 *at = reinterpret_cast<uint4 *>(d.marks) + wi;
@@ -116,6 +126,9 @@ __global__ __launch_bounds__(kCompactBlock) void k_dirty_compact(DevGraph g, Dir
       p++;
     }
   }
+}
+__global__ __launch_bounds__(kCompactBlock) void k_dirty_compact(DevGraph g, DirtyArgs d) {
+  compact_dirty<false>(g, d);
 }
 
 // The block's part in a SmallCopy, 8 bytes a thread at a time (both sides are
@@ -250,8 +263,8 @@ __device__ __forceinline__ uint32_t wave_count_below(const uint32_t *p, uint32_t
 }
 
 constexpr uint32_t kPlanBlock = 512;
-__global__ __launch_bounds__(kPlanBlock) void k_apply_plan(DevGraph g, BatchDev b, unsigned long long scratch_cap,
-                                                           ApplyCtl *actl) {
+template <bool ONE>
+__device__ __forceinline__ void plan_lists(DevGraph g, BatchDev b, unsigned long long scratch_cap, ApplyCtl *actl) {
   __shared__ unsigned long long s_len[kPlanBlock / 64 + 1];
   __shared__ uint32_t s_segs[kPlanBlock / 64 + 1], s_most;
   if (threadIdx.x == 0) s_most = 0;
@@ -274,6 +287,9 @@ __global__ __launch_bounds__(kPlanBlock) void k_apply_plan(DevGraph g, BatchDev 
   __syncthreads();
   if (threadIdx.x == 0 && s_most > ld_relaxed(&actl->max_deg)) atomicMax(&actl->max_deg, s_most);
 }
+__global__ __launch_bounds__(kPlanBlock) void k_apply_plan(DevGraph g, BatchDev b, unsigned long long scratch_cap, ApplyCtl *actl) {
+  plan_lists<false>(g, b, scratch_cap, actl);
+}
 
 // A slot for t's merged list of nd entries: its own, a new one from the pool's
 // bump pointer, or none.
@@ -295,13 +311,13 @@ __device__ __forceinline__ uint32_t take_slot(const DevGraph &g, const BatchDev 
   return moves;
 }
 
-__global__ __launch_bounds__(kApplyWaves * 64) void k_apply_rank(DevGraph g, BatchDev b, uint32_t *scratch,
-                                                                 unsigned long long pool_cap, ApplyCtl *actl) {
-  __shared__ uint32_t s_rd[kApplyWaves][kMaxVertexChanges];
-  if (actl->merge_overflow) return;
+template <bool ONE, uint32_t WAVES, uint32_t CHANGES>
+__device__ __forceinline__ void rank_changes(DevGraph g, BatchDev b, uint32_t *scratch, unsigned long long pool_cap, ApplyCtl *actl) {
+  __shared__ uint32_t s_rd[WAVES][CHANGES];
+  if (ctl_word<ONE>(actl->merge_overflow)) return;
   const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
   uint32_t *rd = s_rd[wv];
-  for (uint32_t t = blockIdx.x * kApplyWaves + wv; t < b.ntouched; t += gridDim.x * kApplyWaves) {
+  for (uint32_t t = blockIdx.x * WAVES + wv; t < b.ntouched; t += gridDim.x * WAVES) {
     const uint32_t x = b.tv[t];
     const uint32_t *A = g.pool + g.start[x];
     const uint32_t na = g.deg[x];
@@ -362,10 +378,14 @@ __global__ __launch_bounds__(kApplyWaves * 64) void k_apply_rank(DevGraph g, Bat
     }
   }
 }
+__global__ __launch_bounds__(kApplyWaves * 64) void k_apply_rank(DevGraph g, BatchDev b, uint32_t *scratch, unsigned long long pool_cap, ApplyCtl *actl) {
+  rank_changes<false, kApplyWaves, kMaxVertexChanges>(g, b, scratch, pool_cap, actl);
+}
 
-__global__ __launch_bounds__(256) void k_apply_merge(DevGraph g, BatchDev b, uint32_t *scratch, const ApplyCtl *actl) {
-  if (actl->merge_overflow) return;
-  const uint32_t lane = lane_id(), nsegs = actl->nsegs;
+template <bool ONE>
+__device__ __forceinline__ void merge_lists(DevGraph g, BatchDev b, uint32_t *scratch, const ApplyCtl *actl) {
+  if (ctl_word<ONE>(actl->merge_overflow)) return;
+  const uint32_t lane = lane_id(), nsegs = ctl_word<ONE>(actl->nsegs);
   for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < nsegs; i += (gridDim.x * blockDim.x) >> 6) {
     const uint2 sg = b.segs[i];
     const uint32_t t = bcast(sg.x), s0 = bcast(sg.y) * kApplySeg;
@@ -394,12 +414,15 @@ __global__ __launch_bounds__(256) void k_apply_merge(DevGraph g, BatchDev b, uin
     }
   }
 }
+__global__ __launch_bounds__(256) void k_apply_merge(DevGraph g, BatchDev b, uint32_t *scratch, const ApplyCtl *actl) {
+  merge_lists<false>(g, b, scratch, actl);
+}
 
 // With `again`, the commits that found no room the first time.
-__global__ __launch_bounds__(256) void k_apply_commit(DevGraph g, BatchDev b, const uint32_t *scratch,
-                                                      const ApplyCtl *actl, DirtyArgs d, int again) {
-  if (actl->merge_overflow) return;
-  const uint32_t lane = lane_id(), nsegs = actl->nsegs;
+template <bool ONE>
+__device__ __forceinline__ void commit_lists(DevGraph g, BatchDev b, const uint32_t *scratch, const ApplyCtl *actl, DirtyArgs d, int again) {
+  if (ctl_word<ONE>(actl->merge_overflow)) return;
+  const uint32_t lane = lane_id(), nsegs = ctl_word<ONE>(actl->nsegs);
   for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < nsegs; i += (gridDim.x * blockDim.x) >> 6) {
     const uint2 sg = b.segs[i];
     const uint32_t t = bcast(sg.x), s0 = bcast(sg.y) * kApplySeg;
@@ -418,6 +441,9 @@ __global__ __launch_bounds__(256) void k_apply_commit(DevGraph g, BatchDev b, co
     }
   }
 }
+__global__ __launch_bounds__(256) void k_apply_commit(DevGraph g, BatchDev b, const uint32_t *scratch, const ApplyCtl *actl, DirtyArgs d, int again) {
+  commit_lists<false>(g, b, scratch, actl, d, again);
+}
 
 // After the pool has grown: slots for the merged lists that found none.
 __global__ __launch_bounds__(256) void k_apply_slots(DevGraph g, BatchDev b, unsigned long long pool_cap,
@@ -432,23 +458,36 @@ __global__ __launch_bounds__(256) void k_apply_slots(DevGraph g, BatchDev b, uns
 
 // The start of an update: its status from another graph copy's, its counters
 // cleared.
-__global__ __launch_bounds__(256) void k_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl,
-                                                       SmallCopy up) {
-  small_copy(up);
-  if (threadIdx.x != 0) return;
+template <bool ONE>
+__device__ __forceinline__ void begin_update(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl) {
+  const auto put = [](auto &w, auto x) {
+    if (ONE) __hip_atomic_store(&w, (std::remove_reference_t<decltype(w)>)x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else w = x;
+  };
   if (from) {
     actl->pool_used = from->pool_used;
     actl->max_deg = from->max_deg;
   }
-  actl->scratch_used = 0;
-  actl->overflow = actl->merge_overflow = 0;
-  actl->relocated = actl->relabeled = 0;
-  actl->ndirty = 0;
-  actl->filter_entries = 0;
-  actl->filter_bits = 0;
-  actl->nsegs = 0;
-  actl->nrelabel_segs = 0;
-  for (int i = 0; i < 4; i++) actl->sync_queued[i] = bctl[i] = 0;
+  put(actl->scratch_used, 0);
+  put(actl->overflow, 0);
+  put(actl->merge_overflow, 0);
+  put(actl->relocated, 0);
+  put(actl->relabeled, 0);
+  put(actl->ndirty, 0);
+  put(actl->filter_entries, 0);
+  put(actl->filter_bits, 0);
+  put(actl->nsegs, 0);
+  put(actl->nrelabel_segs, 0);
+  for (int i = 0; i < 4; i++) {
+    put(actl->sync_queued[i], 0);
+    put(bctl[i], 0);
+  }
+}
+
+__global__ __launch_bounds__(256) void k_update_begin(ApplyCtl *actl, const ApplyCtl *from, uint32_t *bctl,
+                                                       SmallCopy up) {
+  small_copy(up);
+  if (threadIdx.x == 0) begin_update<false>(actl, from, bctl);
 }
 
 __global__ __launch_bounds__(256) void k_round_begin(ApplyCtl *actl, SmallCopy up) {
@@ -461,8 +500,9 @@ __global__ __launch_bounds__(256) void k_round_begin(ApplyCtl *actl, SmallCopy u
 // The relabels, a lane each: set the label; when it changed, mark the vertex
 // dirty and deal out its (post-update) list in pieces for k_relabel_marks, with
 // its old label.
-__global__ __launch_bounds__(256) void k_relabel(DevGraph g, BatchDev b, DirtyArgs d) {
-  if (held_up(d.actl)) return;
+template <bool ONE>
+__device__ __forceinline__ void relabel(DevGraph g, BatchDev b, DirtyArgs d) {
+  if (held_up<ONE>(d.actl)) return;
   for (uint32_t r0 = (blockIdx.x * blockDim.x + threadIdx.x) & ~63u; r0 < b.nrelabel; r0 += gridDim.x * blockDim.x) {
     const uint32_t r = r0 + lane_id();
     uint32_t x = 0, old = 0, L = 0;
@@ -484,12 +524,16 @@ __global__ __launch_bounds__(256) void k_relabel(DevGraph g, BatchDev b, DirtyAr
     deal_pieces(b.segs, &d.actl->nrelabel_segs, x, ns, old << 24);
   }
 }
+__global__ __launch_bounds__(256) void k_relabel(DevGraph g, BatchDev b, DirtyArgs d) {
+  relabel<false>(g, b, d);
+}
 
 // A wave per piece of a relabelled vertex's list: its neighbours' neighbour-label
 // counts changed, so they are marked dirty; with the first piece the vertex's bits
 // go from every bitmap of its old label.
-__global__ __launch_bounds__(256) void k_relabel_marks(DevGraph g, BatchDev b, FilterTables ft, DirtyArgs d) {
-  const uint32_t lane = lane_id(), nsegs = d.actl->nrelabel_segs;
+template <bool ONE>
+__device__ __forceinline__ void relabel_marks(DevGraph g, BatchDev b, FilterTables ft, DirtyArgs d) {
+  const uint32_t lane = lane_id(), nsegs = ctl_word<ONE>(d.actl->nrelabel_segs);
   for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < nsegs; i += (gridDim.x * blockDim.x) >> 6) {
     const uint2 sg = b.segs[i];
     const uint32_t x = bcast(sg.x), s0 = bcast(sg.y & 0xFFFFFFu) * kApplySeg, old = bcast(sg.y >> 24);
@@ -509,6 +553,9 @@ __global__ __launch_bounds__(256) void k_relabel_marks(DevGraph g, BatchDev b, F
       for (uint32_t u = 0; u < kU; u++) mark_dirty(d, w[u]);
     }
   }
+}
+__global__ __launch_bounds__(256) void k_relabel_marks(DevGraph g, BatchDev b, FilterTables ft, DirtyArgs d) {
+  relabel_marks<false>(g, b, ft, d);
 }
 
 // ----------------------------------------------------------------- filter
@@ -593,18 +640,19 @@ __device__ __forceinline__ void set_bit_from(uint64_t *w, uint64_t cur, uint32_t
 // entries and two pairs a lane in flight. Bound by the scattered label and bitmap
 // reads. With a lane per vertex, its list and its signatures one after the other,
 // 25 us for 4,900 dirty vertices of 100,000 (the longest chain of a wave).
-__global__ __launch_bounds__(256) void k_filter_light(DevGraph g, FilterTables ft, DirtyArgs d) {
+template <bool ONE, uint32_t WAVES>
+__device__ __forceinline__ void filter_light(DevGraph g, FilterTables ft, DirtyArgs d) {
   // counts of the wave's vertices: a byte per label (at most kLabelSorted), 32 of them
   // (a 64-bit word of padding keeps the vertices apart in the banks)
-  __shared__ uint64_t s_cnt[4][64][kMaxRel / 8 + 1];
-  __shared__ uint32_t s_pre[4][65], s_from[4][64], s_v[4][64], s_deg[4][64];
+  __shared__ uint64_t s_cnt[WAVES][64][kMaxRel / 8 + 1];
+  __shared__ uint32_t s_pre[WAVES][65], s_from[WAVES][64], s_v[WAVES][64], s_deg[WAVES][64];
   __shared__ unsigned long long s_sum[2];
   __shared__ uint8_t s_lmap[256];
   for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_lmap[i] = ft.lmap[i];
   __syncthreads();
-  if (held_up(d.actl)) return;
+  if (held_up<ONE>(d.actl)) return;
   const uint32_t wv = threadIdx.x >> 6, lane = lane_id();
-  const uint32_t nd = d.actl->ndirty < d.list_cap ? d.actl->ndirty : d.list_cap;
+  const uint32_t nd = min(ctl_word<ONE>(d.actl->ndirty), d.list_cap);
   uint32_t *pre = s_pre[wv], *from = s_from[wv];
   unsigned long long entries = 0;  // list entries of the vertices this lane re-filters
   uint32_t bits = 0;               // candidate bits they receive (one per signature of the label)
@@ -613,8 +661,8 @@ __global__ __launch_bounds__(256) void k_filter_light(DevGraph g, FilterTables f
   __syncthreads();
   // fewer vertices a wave where there are waves enough: shorter chains
   uint32_t per = 64;
-  while (per > 8 && nd <= per / 2 * gridDim.x * 4) per >>= 1;
-  for (uint32_t i0 = (blockIdx.x * 4 + wv) * per; i0 < nd; i0 += gridDim.x * 4 * per) {
+  while (per > 8 && nd <= per / 2 * gridDim.x * WAVES) per >>= 1;
+  for (uint32_t i0 = (blockIdx.x * WAVES + wv) * per; i0 < nd; i0 += gridDim.x * WAVES * per) {
     const uint32_t i = i0 + lane;
     uint32_t v = 0, L = kNoLabel, dv = 0, lo = 0, ns = 0;
     if (lane < per && i < nd) {
@@ -640,7 +688,7 @@ __global__ __launch_bounds__(256) void k_filter_light(DevGraph g, FilterTables f
     wave_sync();
     const uint32_t total = pre[64];
     for (uint32_t e = 0; e < total; e += 256) {
-      uint32_t k[4], o[4], w[4];
+      uint32_t k[WAVES], o[WAVES], w[WAVES];
 #pragma unroll
       for (int u = 0; u < 4; u++) k[u] = min(e + u * 64 + lane, total - 1);
       ranges_of(pre, k, o);
@@ -683,6 +731,9 @@ __global__ __launch_bounds__(256) void k_filter_light(DevGraph g, FilterTables f
   __syncthreads();
   if (threadIdx.x == 0 && s_sum[0]) atomicAdd(&d.actl->filter_entries, s_sum[0]);
   if (threadIdx.x == 1 && s_sum[1]) atomicAdd(&d.actl->filter_bits, (uint32_t)s_sum[1]);
+}
+__global__ __launch_bounds__(256) void k_filter_light(DevGraph g, FilterTables ft, DirtyArgs d) {
+  filter_light<false, 4>(g, ft, d);
 }
 
 // ---------------------------------------------------- label-sorted copies
@@ -848,23 +899,23 @@ __device__ __forceinline__ uint32_t build_piece(uint32_t d) {
 // kBuildSeg] to hs.mid, longer ones to hs.big and in pieces to hs.pieces.
 // Vertices whose label no query uses are skipped (never read, see
 // k_dirty_compact); a full build leaves their groups empty.
-__global__ __launch_bounds__(256) void k_lbuild_pick(DevGraph g, const uint32_t *list, const uint32_t *count,
-                                                     SortedBuild hs) {
-  __shared__ uint32_t s_sum[5];
+template <bool ONE, uint32_t WAVES>
+__device__ __forceinline__ void pick_builds(DevGraph g, const uint32_t *list, const uint32_t *count, SortedBuild hs) {
+  __shared__ uint32_t s_sum[WAVES + 1];
   const uint32_t nb = g.nbuckets;
-  if (hs.actl && held_up(hs.actl)) return;
-  const uint32_t total = list ? (*count < g.n ? *count : g.n) : g.n;
+  if (hs.actl && held_up<ONE>(hs.actl)) return;
+  const uint32_t total = list ? min(ctl_word<ONE>(*count), g.n) : g.n;
   constexpr uint32_t kU = 4;
-  for (uint32_t base = blockIdx.x * 256 * kU; base < total; base += gridDim.x * 256 * kU) {
+  for (uint32_t base = blockIdx.x * (WAVES * 64) * kU; base < total; base += gridDim.x * (WAVES * 64) * kU) {
     uint32_t v[kU], d[kU], l[kU], nmid = 0, nbig = 0, npieces = 0;
 #pragma unroll
     for (uint32_t u = 0; u < kU; u++) {
-      const uint32_t t = min(base + u * 256 + threadIdx.x, total - 1);
+      const uint32_t t = min(base + u * (WAVES * 64) + threadIdx.x, total - 1);
       v[u] = list ? list[t] : t;
     }
 #pragma unroll
     for (uint32_t u = 0; u < kU; u++) {
-      d[u] = base + u * 256 + threadIdx.x < total ? g.deg[v[u]] : 0u;
+      d[u] = base + u * (WAVES * 64) + threadIdx.x < total ? g.deg[v[u]] : 0u;
       l[u] = g.lab[v[u]];
     }
 #pragma unroll
@@ -899,21 +950,25 @@ __global__ __launch_bounds__(256) void k_lbuild_pick(DevGraph g, const uint32_t 
     }
   }
 }
+__global__ __launch_bounds__(256) void k_lbuild_pick(DevGraph g, const uint32_t *list, const uint32_t *count, SortedBuild hs) {
+  pick_builds<false, 4>(g, list, count, hs);
+}
 
 // A wave per piece of a long list: its bucket counts; then a wave per short list:
 // its label-sorted copy and, if asked, its vertex's candidate bits.
-__global__ __launch_bounds__(256) void k_lbuild(DevGraph g, FilterTables ft, SortedBuild hs, bool filter) {
+template <bool ONE, uint32_t WAVES>
+__device__ __forceinline__ void sort_lists(DevGraph g, FilterTables ft, SortedBuild hs, bool filter) {
   __shared__ uint8_t s_lmap[256];
-  __shared__ uint32_t s_cnt[4][kMaxRel + 2];
-  __shared__ uint64_t s_pack[4][kMaxRel / 8];
+  __shared__ uint32_t s_cnt[WAVES][kMaxRel + 2];
+  __shared__ uint64_t s_pack[WAVES][kMaxRel / 8];
   for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_lmap[i] = ft.lmap[i];
   __syncthreads();
   const uint32_t wv = bcast(threadIdx.x >> 6), lane = lane_id();
   const uint32_t nb = g.nbuckets;
   const uint32_t bits = 32u - (uint32_t)__builtin_clz(nb > 1 ? nb - 1 : 1u);
-  const uint32_t npieces = hs.ctl[2], total = npieces + hs.ctl[0];
+  const uint32_t npieces = ctl_word<ONE>(hs.ctl[2]), total = npieces + ctl_word<ONE>(hs.ctl[0]);
   uint32_t *cnt = s_cnt[wv];
-  for (uint32_t t = blockIdx.x * 4 + wv; t < total; t += gridDim.x * 4) {
+  for (uint32_t t = blockIdx.x * WAVES + wv; t < total; t += gridDim.x * WAVES) {
     if (t >= npieces) {
       const uint32_t v = bcast(hs.mid[t - npieces]), d = bcast(g.deg[v]);
       const uint32_t size = d <= 256 ? build_one<4>(g, s_lmap, v, d, nb, bits, cnt)
@@ -931,6 +986,9 @@ __global__ __launch_bounds__(256) void k_lbuild(DevGraph g, FilterTables ft, Sor
     if (lane < nb) hs.hist[(size_t)t * (kMaxRel + 2) + lane] = cnt[lane];
     wave_sync();
   }
+}
+__global__ __launch_bounds__(256) void k_lbuild(DevGraph g, FilterTables ft, SortedBuild hs, bool filter) {
+  sort_lists<false, 4>(g, ft, hs, filter);
 }
 
 // A wave per long list, a lane per bucket (nb <= kMaxRel + 1 < 64): the buckets'
@@ -984,6 +1042,53 @@ __global__ __launch_bounds__(256) void k_lbuild_place(DevGraph g, const uint8_t 
                    hs.bucket_bytes ? hs.bucket_bytes + g.start[v] : nullptr);
     wave_sync();
   }
+}
+
+// A whole update by one block, its phases a block barrier apart instead of a launch:
+// for one record on lists of 30 entries the ten kernels took 37 us, most of it between
+// them, and this takes 25 to 28 in one launch. Lists of at most kBuildSeg entries (no pieces), at most kSmallChanges changes.
+// It ends with the update's status in pinned host memory.
+constexpr uint32_t kOneWaves = 8;
+static_assert(kOneWaves * 64 == kPlanBlock && kOneWaves * 64 == kCompactBlock, "the phases' strides");
+__global__ __launch_bounds__(kOneWaves * 64) void k_update_small(DevGraph g, BatchDev b, FilterTables ft, DirtyArgs d,
+                                                                 SortedBuild hs, uint32_t *scratch,
+                                                                 unsigned long long scratch_cap,
+                                                                 unsigned long long pool_cap, bool sorted, SmallCopy up,
+                                                                 uint32_t *status) {
+  ApplyCtl *actl = d.actl;
+  // a phase's stores and counter adds have been taken before the next begins
+  const auto next = [] {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+  };
+  small_copy(up);
+  if (threadIdx.x == 0) begin_update<true>(actl, nullptr, hs.ctl);
+  next();
+  plan_lists<true>(g, b, scratch_cap, actl);
+  next();
+  rank_changes<true, kOneWaves, kSmallChanges>(g, b, scratch, pool_cap, actl);
+  next();
+  merge_lists<true>(g, b, scratch, actl);
+  next();
+  commit_lists<true>(g, b, scratch, actl, d, 0);
+  next();
+  if (b.nrelabel) {
+    relabel<true>(g, b, d);
+    next();
+    relabel_marks<true>(g, b, ft, d);
+    next();
+  }
+  compact_dirty<true>(g, d);
+  next();
+  if (sorted) {
+    pick_builds<true, kOneWaves>(g, d.list, &actl->ndirty, hs);
+    next();
+    sort_lists<true, kOneWaves>(g, ft, hs, true);
+    next();
+  }
+  filter_light<true, kOneWaves>(g, ft, d);
+  next();
+  if (threadIdx.x < sizeof(ApplyCtl) / 4) status[threadIdx.x] = ld_relaxed(reinterpret_cast<uint32_t *>(actl) + threadIdx.x);
 }
 
 __global__ void k_build_reset(SortedBuild hs) {
@@ -2450,6 +2555,15 @@ hipError_t launch_filter_full(const DevGraph &g, const FilterTables &ft, hipStre
 
 hipError_t launch_filter_dirty(const DevGraph &g, const FilterTables &ft, const DirtyArgs &d, hipStream_t s) {
   hipLaunchKernelGGL(k_filter_light, dim3(blocks_for(g.n, 256, 1024)), dim3(256), 0, s, g, ft, d);
+  return hipGetLastError();
+}
+
+hipError_t launch_update_small(const DevGraph &g, const BatchDev &b, const FilterTables &ft, const DirtyArgs &d,
+                               const SortedBuild &hs, uint32_t *scratch, unsigned long long scratch_cap,
+                               unsigned long long pool_cap, uint32_t longest, const SmallCopy &up, ApplyCtl *status,
+                               hipStream_t s) {
+  hipLaunchKernelGGL(k_update_small, dim3(1), dim3(kOneWaves * 64), 0, s, g, b, ft, d, hs, scratch, scratch_cap,
+                     pool_cap, longest > kLabelSorted, up, reinterpret_cast<uint32_t *>(status));
   return hipGetLastError();
 }
 
