@@ -54,9 +54,11 @@ def test_small_updates(records, hub, n, relabel):
             eng.close()
 
 
-def test_the_pool_grows_in_a_small_update():
+@pytest.mark.parametrize("deletes", [0, 1])
+def test_the_pool_grows_in_a_small_update(deletes):
     """4,000 lists of 700 entries filled to the end of their slots (879) by one batch,
-    then moved to larger ones up to 32 a batch until there is no room for them."""
+    then moved to larger ones up to 32 a batch until there is no room for them; with a
+    delete in every batch its round runs beside the update, ahead of the inserts'."""
     n = 4000
     i = np.arange(n)
     ring = [(i, (i + k) % n) for k in range(1, 351)]
@@ -76,13 +78,18 @@ def test_the_pool_grows_in_a_small_update():
         before = eng.stats()["pool_entries_capacity"]
         src, dst = flat([over])
         for x in range(0, 2000, 16):
-            pos, _ = eng.process_batch(np.ones(16, np.uint8), src[x:x + 16], dst[x:x + 16], np.zeros(16, np.uint32))
-            assert pos.tolist() == [32], x
+            add = np.concatenate([np.ones(16, np.uint8), np.zeros(deletes, np.uint8)])
+            gone = np.full(deletes, 3000 + x // 16 * 4, np.uint32)
+            pos, neg = eng.process_batch(add, np.concatenate([src[x:x + 16], gone]),
+                                         np.concatenate([dst[x:x + 16], gone + 5]), np.zeros(16 + deletes, np.uint32))
+            assert pos.tolist() == [32] and neg.tolist() == [2 * deletes], x
         assert eng.stats()["pool_entries_capacity"] > before
         off, nb, _ = eng.graph()
     finally:
         eng.close()
     a, b = (x.astype(np.int64) for x in flat(ring + fill + [over]))
     key = np.unique(np.concatenate([a * n + b, b * n + a]))
+    gone = np.arange(3000, 3500, 4) if deletes else np.zeros(0, np.int64)
+    key = np.setdiff1d(key, np.concatenate([gone * n + gone + 5, (gone + 5) * n + gone]))
     assert np.array_equal(nb, (key % n).astype(np.uint32))
     assert np.array_equal(np.diff(off).astype(np.int64), np.bincount(key // n, minlength=n))
