@@ -1645,17 +1645,20 @@ __device__ __forceinline__ uint32_t leaf_count_lane(const WaveMem &M, const DfsA
 // consecutive entries of a list are read by consecutive lanes. Four steps are
 // taken at a time, their reads in flight together. The lists that are not empty
 // sit in the window buffer (where its entry 0 would be, and w); the list of an
-// entry is the number of list starts at or before it, from a bit mask of the
-// starts in its step. Returns this lane's share of the count (the task sums the
+// entry is the number of list starts at or before it, from the starts' bits, which
+// are set there for 2,048 entries at a time. Returns this lane's share of the count (the task sums the
 // wave).
 //
 // Bound by the latency of the reads and of the LDS steps between them: a step of
 // 64 entries took 2,460 cycles one at a time, with the list found by a binary
 // search over shuffles, and was 27% of the search (1M vertices, 64 queries). With
 // it, the hash sets, searches four at a time and the DPP scans, the waves' time
-// on tasks fell from 19.4 to 12.5 s per launch at 2,048 waves. Fetching the next
+// on tasks fell from 19.4 to 12.5 s per launch at 2,048 waves. With the starts' bits
+// put together from the lanes by two wave-wide ors a step, not set in LDS, the launch
+// takes 2% longer. Fetching the next
 // four steps ahead of the tests takes 14 more registers and gave 2%; the update
 // beside the round then waits for room, so it is not done.
+constexpr uint32_t kStartBits = 64 * 32;
 __device__ __forceinline__ uint32_t leaf_scan_segments(const WaveMem &M, const DfsArgs &a, uint32_t leaf, uint32_t w,
                                                        bool has, const LeafList &ll, uint32_t &scanned) {
   constexpr int K = 4;
@@ -1666,44 +1669,42 @@ __device__ __forceinline__ uint32_t leaf_scan_segments(const WaveMem &M, const D
   uint32_t total;
   const uint32_t excl = wave_excl_sum(n, &total);
   const LeafRule r = leaf_rule(*M.h, leaf);
-  uint4 *seg = reinterpret_cast<uint4 *>(M.win);  // [64]
+  // [64]: x, y a list's entry 0; z its w; the w words hold the bits of the starts
+  uint4 *seg = reinterpret_cast<uint4 *>(M.win);
   wave_sync();
   if (n > 0) {
     const unsigned long long p = (unsigned long long)ll.L - 4ull * excl;
     seg[mbcnt(lists)] = uint4{(uint32_t)p, (uint32_t)(p >> 32), w, 0};
   }
-  wave_sync();
-  uint32_t c = 0, before = 0;  // list starts before the step
-  for (uint32_t base = 0; base < total; base += 64 * K) {
-    uint32_t li[K], wo[K], y[K];
-    bool ok[K];
-    const uint32_t at = excl - base;
-    if (ballot(n > 0 && at < 64 * K) == 0) {
-      // one list goes through all steps
+  uint32_t c = 0;
+  for (uint32_t part = 0; part < total; part += kStartBits) {
+    // bit k: a list starts at entry part + k + 1
+    wave_sync();
+    seg[lane].w = 0;
+    wave_sync();
+    const uint32_t bit = excl - 1 - part;
+    if (n > 0 && excl > part && bit < kStartBits) atomicOr(&seg[bit >> 5].w, 1u << (bit & 31));
+    wave_sync();
+    uint32_t before = (uint32_t)__popcll(ballot(n > 0 && excl > 0 && excl <= part));
+    for (uint32_t at = 0; at < kStartBits && part + at < total; at += 64 * K) {
+      uint32_t wo[K], y[K];
+      uint64_t starts[K];
+      bool ok[K];
 #pragma unroll
-      for (int u = 0; u < K; u++) li[u] = before - 1;
-    } else {
+      for (int u = 0; u < K; u++)
+        starts[u] = (uint64_t)seg[at / 32 + 2 * u + 1].w << 32 | seg[at / 32 + 2 * u].w;
 #pragma unroll
       for (int u = 0; u < K; u++) {
-        const uint32_t q = at - 64 * u;
-        const uint32_t lo = wave_or(n > 0 && q < 32 ? 1u << q : 0u);
-        const uint32_t hi = wave_or(n > 0 && q >= 32 && q < 64 ? 1u << (q - 32) : 0u);
-        const uint64_t starts = (uint64_t)hi << 32 | lo;
-        // starts at or before this lane's entry
-        li[u] = before + mbcnt(starts) + (uint32_t)(starts >> lane & 1) - 1;
-        before += (uint32_t)__popcll(starts);
+        const uint32_t k = part + at + 64 * u + lane;
+        const uint4 s = seg[before + mbcnt(starts[u])];
+        before += (uint32_t)__popcll(bcast64(starts[u]));
+        const uint32_t *L = reinterpret_cast<const uint32_t *>((unsigned long long)s.y << 32 | s.x);
+        wo[u] = s.z;
+        ok[u] = k < total;
+        y[u] = L[ok[u] ? k : total - 1];
       }
+      c += leaf_accept(M, a, r, wo, y, ok);
     }
-#pragma unroll
-    for (int u = 0; u < K; u++) {
-      const uint32_t k = base + 64 * u + lane;
-      const uint4 s = seg[li[u]];
-      const uint32_t *L = reinterpret_cast<const uint32_t *>((unsigned long long)s.y << 32 | s.x);
-      wo[u] = s.z;
-      ok[u] = k < total;
-      y[u] = L[ok[u] ? k : total - 1];
-    }
-    c += leaf_accept(M, a, r, wo, y, ok);
   }
   scanned += n;
   wave_sync();  // the window buffer is free again
