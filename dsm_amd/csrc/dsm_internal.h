@@ -239,8 +239,8 @@ void set_global_error(const char *fmt, ...);
 
 // Words that a kernel copies between pinned host memory and the device on its way
 // (none if words is 0). A copy of its own costs a launch, an API call and a blit
-// kernel, some 8 us in all; up to kSmallCopy words one block reads them over the
-// host link in 3 to 4 us.
+// kernel, some 8 us in all; one block reads a few hundred words over the host link in
+// 3 us and 3,000 in 10 (a call with either takes as long with the line at 1,024).
 constexpr uint32_t kSmallCopy = 4096;
 struct SmallCopy {
   const uint32_t *from;
