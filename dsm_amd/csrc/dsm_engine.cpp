@@ -250,6 +250,8 @@ struct dsm_engine {
   DevBuf<unsigned long long> query_busy;  // per query: DFS task ticks since the last read
   uint32_t wave_slots = 0;       // waves of the largest grid
   uint32_t last_blocks = 0, last_wpb = 0;  // grid of the last DFS launch
+  uint32_t last_nrec = 0;                  // its records
+  double busy_per_record = -1;             // ms of its waves' task time a record, averaged (-1: no round yet)
   bool results_here = false;  // h_results holds the counts of the batch applied last
   uint32_t watchdog_ms = 60000;
   int wall_khz = 100000;
@@ -865,6 +867,18 @@ DfsArgs dfs_args(dsm_engine *e) {
   return da;
 }
 
+// The most blocks for a round with so much task time (ms, as the engine's last rounds
+// took it a record). Waves share a CU's issue slots and L1: at 12 a CU they take twice
+// as long for a task as at 4, and a round that ends with a few long tasks ends sooner
+// with 4. Measured at 4, 8 and 12 waves a CU: 20 ms of tasks (22 seeds, 100,000
+// vertices) 87, 100 and 106 us; 170 ms 186, 185 and 205; 270 ms 223, 221 and 220;
+// 880 ms (1,000,000 vertices) 541, 499 and 513; 2,600 ms 1,320, 932 and 948; 9,900 ms
+// 6.8, 4.3 and 3.7 ms.
+uint32_t blocks_for_work(const dsm_engine *e, double ms) {
+  const uint32_t waves_per_cu = ms <= 250 ? 4 : ms <= 2500 ? 8 : 0xFFFF;
+  return std::max(1u, waves_per_cu / e->dfs_wpb) * (uint32_t)e->num_cu;
+}
+
 // The grid: a round over a handful of records gets one block per CU, so that few
 // waves pay the start-up and termination atomics, and fewer where no list is long
 // enough to give a CU's waves anything to share (a record of a graph whose lists have
@@ -874,6 +888,8 @@ uint32_t dfs_grid(dsm_engine *e, uint32_t nrec) {
       ((uint64_t)nrec * std::max<uint32_t>(e->max_plans_per_key, 1) * 8 + e->dfs_wpb - 1) / e->dfs_wpb;
   const uint64_t least = std::min<uint64_t>((uint64_t)e->num_cu, want * std::max(1u, e->h_actl.p->max_deg / 16));
   uint32_t b = (uint32_t)std::min<uint64_t>(e->dfs_blocks, std::max<uint64_t>(want, least));
+  if (e->busy_per_record >= 0) b = std::min(b, blocks_for_work(e, e->busy_per_record * nrec));
+  e->last_nrec = nrec;
   e->last_wpb = e->tuples ? 4u : e->dfs_wpb;
   b = std::min(b, e->wave_slots / e->last_wpb);  // a mailbox for every wave
   e->last_blocks = b;
@@ -945,14 +961,21 @@ int run_round(dsm_engine *e, const uint32_t *rs, const uint32_t *rd, uint32_t nr
   return DSM_OK;
 }
 
-// The last round's errors: the records of its blocks, which have ended.
+// The last round's errors: the records of its blocks, which have ended; and its work
+// for the grids of later rounds.
 int round_error(dsm_engine *e) {
+  unsigned long long busy = 0;
   for (uint32_t b = 0; b < e->last_blocks; b++) {
     const BlockRec &r = e->h_rec.p[b];
     if (r.epoch != e->epoch) return e->fail_msg(DSM_EDEVICE, "DFS: block %u of %u left no record", b, e->last_blocks);
     if (r.seed_overflow)
       return e->fail_msg(DSM_ELIMIT, "seed table overflow (%llu seeds dropped)", r.seed_overflow);
     if (r.abort) return e->fail_msg(DSM_EDEVICE, "DFS watchdog: a wave waited more than %u ms for work", e->watchdog_ms);
+    busy += r.busy;
+  }
+  if (e->last_nrec) {
+    const double x = (double)busy / (double)e->wall_khz / e->last_nrec;
+    e->busy_per_record = e->busy_per_record < 0 ? x : (e->busy_per_record + x) / 2;
   }
   return DSM_OK;
 }

@@ -173,3 +173,32 @@ def test_update_rule_on_conflicting_batches(n, records):
             assert np.array_equal(np.where(dl > 2, 255, dl), l2)
     finally:
         eng.close()
+
+
+def test_grids_follow_the_work_of_earlier_rounds():
+    """Rounds of little work after a first one of unknown work start fewer blocks, and
+    batches of other sizes in between change the grid again: counts against the oracle."""
+    rng = np.random.default_rng(11)
+    n, m = 4000, 60000
+    u, v = rng.integers(0, n, m).astype(np.uint32), rng.integers(0, n, m).astype(np.uint32)
+    keep = u != v
+    u, v = u[keep], v[keep]
+    lab = rng.integers(0, 2, n).astype(np.uint32)
+    queries = [one_label("tri_pendant"), (3, np.array([0, 1, 0], np.uint32), np.array([0, 1], np.uint32),
+                                          np.array([1, 2], np.uint32))]
+    batches = []
+    for k in (400, 1, 400, 400, 3000, 2, 50, 6000, 400):
+        src, dst = rng.integers(0, n, k).astype(np.uint32), rng.integers(0, n, k).astype(np.uint32)
+        batches.append((rng.integers(0, 2, k).astype(np.uint8), src, dst, lab[dst]))
+    want = O.run_stream(O.Graph(n, lab, u, v), [O.Query(*q) for q in queries], batches)
+    eng = E.Engine((n, lab, u, v), queries)
+    try:
+        waves = []
+        for i, b in enumerate(batches):
+            pos, neg = eng.process_batch(*b)
+            assert pos.tolist() == want[i]["pos"] and neg.tolist() == want[i]["neg"], i
+            s = eng.stats()
+            waves.append(s["dfs_waves"] // s["dfs_launches"])
+        assert waves[3] < waves[0]
+    finally:
+        eng.close()
