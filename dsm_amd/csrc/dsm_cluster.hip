@@ -39,6 +39,11 @@ namespace {
 
 constexpr int kClusterWaves = 4;
 
+// A commit or merge of the update that the refinement follows found no room: some
+// lists have moved while their label-sorted copies wait to be built, so none is
+// walked. The refinement is launched again once there is room.
+__device__ __forceinline__ bool held_up(const ApplyCtl *actl) { return actl->overflow | actl->merge_overflow; }
+
 // The pass's targets at neighbours w[u] of candidates (lane-parallel: every lane its
 // own, those with `in`): the targets of the neighbour's label (every condition row
 // implies the target's label, and a combine into an existing cluster holds no bit of
@@ -169,7 +174,9 @@ __device__ __forceinline__ uint32_t nth_bit(uint64_t x, uint32_t n) {
 
 __global__ __launch_bounds__(256) void k_cluster_init(uint64_t *bm, uint32_t words, uint32_t first_row,
                                                       uint32_t nrows, uint64_t *alive, const uint32_t *alive_src,
-                                                      uint32_t nalive_src, uint32_t *ctl, uint32_t nctl) {
+                                                      uint32_t nalive_src, uint32_t *ctl, uint32_t nctl,
+                                                      const ApplyCtl *actl) {
+  if (held_up(actl)) return;
   const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
   const size_t zero = (size_t)nrows * words, copy = (size_t)nalive_src * words;
   uint64_t *z = bm + (size_t)first_row * words;
@@ -191,6 +198,7 @@ __global__ __launch_bounds__(kClusterWaves * 64) void k_cluster_pass(ClusterArgs
   const uint32_t lane = lane_id(), wv = bcast(threadIdx.x >> 6);
   const uint32_t wave = bcast((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
+  if (held_up(a.actl)) return;
   const uint32_t groups = (a.words + 63) >> 6;
   const uint64_t units = (uint64_t)a.nops * groups;
   for (uint64_t u = wave; u < units; u += nwaves) {
@@ -236,6 +244,7 @@ __global__ __launch_bounds__(kClusterWaves * 64) void k_cluster_pass(ClusterArgs
 // now.)
 __global__ __launch_bounds__(kClusterWaves * 64) void k_cluster_heavy(ClusterArgs a) {
   const uint32_t lane = lane_id();
+  if (held_up(a.actl)) return;
   const uint32_t total = min(bcast(a.ctl[0]), a.heavy_cap);
   for (uint32_t e = bcast((blockIdx.x * blockDim.x + threadIdx.x) >> 6); e < total; e += (gridDim.x * blockDim.x) >> 6) {
     const ClusterHeavy h = a.heavy[e];
@@ -264,11 +273,11 @@ __global__ __launch_bounds__(kClusterWaves * 64) void k_cluster_heavy(ClusterArg
 
 hipError_t launch_cluster_init(uint64_t *bm, uint32_t words, uint32_t first_row, uint32_t nrows, uint64_t *alive,
                                const uint32_t *alive_src, uint32_t nalive_src, uint32_t *ctl, uint32_t nctl,
-                               hipStream_t s) {
+                               const ApplyCtl *actl, hipStream_t s) {
   const size_t work = std::max<size_t>((size_t)nrows * words, (size_t)nalive_src * words);
   const uint32_t blocks = (uint32_t)std::min<size_t>(std::max<size_t>((work + 255) / 256, 1), 4096);
   hipLaunchKernelGGL(k_cluster_init, dim3(blocks), dim3(256), 0, s, bm, words, first_row, nrows, alive, alive_src,
-                     nalive_src, ctl, nctl);
+                     nalive_src, ctl, nctl, actl);
   return hipGetLastError();
 }
 

@@ -1322,13 +1322,14 @@ int cluster_refine(dsm_engine *e, uint32_t longest) {
   if (need > e->cheavy.n) HIPCHK(e->cheavy.alloc(need));
   HIPCHK(hipEventRecord(e->ev_ref[0], e->stream));
   HIPCHK(launch_cluster_init(e->bm.p, e->words, e->nsig_rows, e->npos_rows, e->calive.p, e->d_alive_src.p,
-                             e->nalive_src, e->cctl.p, nsteps, e->stream));
+                             e->nalive_src, e->cctl.p, nsteps, e->actl.p, e->stream));
   ClusterArgs a{};
   a.g = e->dev_graph();
   a.bm = e->bm.p;
   a.words = e->words;
   a.alive = e->calive.p;
   a.crow = e->d_crow.p;
+  a.actl = e->actl.p;
   a.heavy = e->cheavy.p;
   a.heavy_cap = (uint32_t)std::min<size_t>(e->cheavy.n, 0xFFFFFFF0u);
   for (uint32_t st = 0; st < nsteps; st++) {

@@ -370,13 +370,15 @@ struct ClusterArgs {
   ClusterHeavy *heavy;
   uint32_t heavy_cap;
   uint32_t *ctl;        // [1]: heavy entries queued
+  const ApplyCtl *actl; // status of the update before it
 };
 
 // Zeroes bm rows [first_row, first_row + nrows), copies the listed (alive row,
-// bm row) pairs into the alive rows and zeroes nctl counters.
+// bm row) pairs into the alive rows and zeroes nctl counters. Like the kernels of the
+// passes it does nothing while the update of actl is held up.
 hipError_t launch_cluster_init(uint64_t *bm, uint32_t words, uint32_t first_row, uint32_t nrows, uint64_t *alive,
                                const uint32_t *alive_src, uint32_t nalive_src, uint32_t *ctl, uint32_t nctl,
-                               hipStream_t s);
+                               const ApplyCtl *actl, hipStream_t s);
 hipError_t launch_cluster_pass(const ClusterArgs &a, uint32_t max_blocks, hipStream_t s);
 hipError_t launch_cluster_heavy(const ClusterArgs &a, uint32_t blocks, hipStream_t s);
 
