@@ -149,6 +149,8 @@ __device__ __forceinline__ void walk_candidates(const ClusterArgs &a, const Clus
       first = bcast(first) + before;
       for (uint32_t c = 0; c < nch; c++)
         if (first + c < a.heavy_cap) a.heavy[first + c] = ClusterHeavy{j, v, b0 + c * kClusterChunk, li};
+      // sized by the host so that this cannot happen
+      if (heavy && first + nch > a.heavy_cap) atomicAdd(&a.actl->chunks_dropped, 1u);
     }
     each_entry(wl, a.g.lpool, st + b0, heavy ? 0u : b1 - b0, [&](const uint32_t(&w)[4], const bool(&in)[4]) {
       const uint32_t lab[4] = {li, li, li, li};

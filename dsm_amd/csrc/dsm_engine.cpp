@@ -1207,6 +1207,9 @@ int status_error(dsm_engine *e) {
   if (e->h_actl.p->merge_overflow)
     return e->fail_msg(DSM_ELIMIT, "update: %u merged lists found no room in the merge scratch",
                        e->h_actl.p->merge_overflow);
+  if (e->h_actl.p->chunks_dropped)
+    return e->fail_msg(DSM_ELIMIT, "refinement: %u chunks of long lists found no room in their queue",
+                       e->h_actl.p->chunks_dropped);
   return DSM_OK;
 }
 
@@ -1312,12 +1315,12 @@ int upload_records(dsm_engine *e, const std::vector<uint32_t> &s, const std::vec
 // position rows are cleared, each core's alive row loaded, then pass step s of
 // every query runs as one k_cluster_pass launch plus one k_cluster_heavy
 // launch for the chunks of candidates with long lists (filter.cu:936-1177 runs
-// one kernel and one device synchronisation per cluster of one query).
-int cluster_refine(dsm_engine *e, uint32_t longest) {
+// one kernel and one device synchronisation per cluster of one query). No list is
+// longer than `longest`, and all together hold at most `entries`.
+int cluster_refine(dsm_engine *e, uint32_t longest, unsigned long long entries) {
   if (!e->cluster) return DSM_OK;
   const uint32_t nsteps = (uint32_t)e->cstep_off.size() - 1;
   // heavy chunks of one pass: at most 2 x (list entries) / kClusterChunk
-  const unsigned long long entries = std::max<unsigned long long>(e->h_actl.p->pool_used, 1);
   const size_t need = (size_t)e->cmax_step_ops * (2 * entries / kClusterChunk + 64);
   if (need > e->cheavy.n) HIPCHK(e->cheavy.alloc(need));
   HIPCHK(hipEventRecord(e->ev_ref[0], e->stream));
@@ -1408,6 +1411,8 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine:
   // no list is longer before the update, or after it
   const uint32_t before = e->h_actl.p->max_deg;
   const uint32_t longest = (uint32_t)std::min<uint64_t>((uint64_t)before + most_ins, 0xFFFFFFFFull);
+  // nor do the lists hold more than the pool's used part before, and the inserts
+  const unsigned long long entries = e->h_actl.p->pool_used + d.ins.size();
   Slice part;
   RoundArrays ra{};
   for (uint32_t rd = 0; rd < rounds; rd++) {
@@ -1471,7 +1476,7 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine:
   e->stats.touched_vertices = T;
   for (bool done_small = small;; done_small = false) {
     if (done_small) {
-      if (int rc = cluster_refine(e, longest)) return rc;
+      if (int rc = cluster_refine(e, longest, entries)) return rc;
       if (done) HIPCHK(hipEventRecord(done, e->stream));
       HIPCHK(hipStreamSynchronize(e->stream));
       if (int rc = status_error(e)) return rc;
@@ -1493,7 +1498,7 @@ int apply_delta_and_refresh(dsm_engine *e, const HostDelta &d, const dsm_engine:
     HIPCHK(launch_lbuild(e->dev_graph(), e->tables(), list, list ? &e->actl.p->ndirty : nullptr, e->sorted_build(),
                          longest, true, e->stream));
     HIPCHK(launch_filter_dirty(e->dev_graph(), e->tables(), e->dirty(), e->stream));
-    if (int rc = cluster_refine(e, longest)) return rc;
+    if (int rc = cluster_refine(e, longest, entries)) return rc;
     if (done) HIPCHK(hipEventRecord(done, e->stream));
     if (int rc = take_status(e)) return rc;
     if (!e->h_actl.p->overflow) break;
@@ -1584,8 +1589,8 @@ int create_impl(dsm_engine *e, const dsm_graph_desc *graph, const dsm_query_desc
   HIPCHK(launch_build_reset(e->sorted_build(), e->stream));
   HIPCHK(launch_lbuild(e->dev_graph(), e->tables(), nullptr, nullptr, e->sorted_build(), e->h_actl.p->max_deg, false,
                        e->stream));
-  if ((rc = cluster_refine(e, e->h_actl.p->max_deg))) return rc;
-  HIPCHK(hipStreamSynchronize(e->stream));
+  if ((rc = cluster_refine(e, e->h_actl.p->max_deg, e->h_actl.p->pool_used))) return rc;
+  if ((rc = take_status(e))) return rc;
   e->refine_timed = false;
   return DSM_OK;
 }

@@ -120,7 +120,8 @@ struct alignas(64) ApplyCtl {
   unsigned long long filter_entries;  // list entries of the vertices re-filtered (work measure)
   uint32_t max_deg;                 // no list has been longer (never lowered): kernels of longer lists are skipped
   uint32_t sync_queued[4];          // long lists queued by the catch-up (block, grid) and the sorted catch-up
-  uint32_t pad[12];
+  uint32_t chunks_dropped;          // refinement: chunks of long lists past the queue's end (must stay 0)
+  uint32_t pad[11];
 };
 static_assert(sizeof(ApplyCtl) == 128, "apply status layout");
 
@@ -370,7 +371,7 @@ struct ClusterArgs {
   ClusterHeavy *heavy;
   uint32_t heavy_cap;
   uint32_t *ctl;        // [1]: heavy entries queued
-  const ApplyCtl *actl; // status of the update before it
+  ApplyCtl *actl;       // status of the update before it
 };
 
 // Zeroes bm rows [first_row, first_row + nrows), copies the listed (alive row,

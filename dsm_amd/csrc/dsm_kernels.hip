@@ -478,6 +478,7 @@ __device__ __forceinline__ void begin_update(ApplyCtl *actl, const ApplyCtl *fro
   put(actl->filter_bits, 0);
   put(actl->nsegs, 0);
   put(actl->nrelabel_segs, 0);
+  put(actl->chunks_dropped, 0);
   for (int i = 0; i < 4; i++) {
     put(actl->sync_queued[i], 0);
     put(bctl[i], 0);
