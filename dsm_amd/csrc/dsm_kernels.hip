@@ -688,17 +688,18 @@ __device__ __forceinline__ void filter_light(DevGraph g, FilterTables ft, DirtyA
     for (int k = 0; k < kMaxRel / 8; k++) s_cnt[wv][lane][k] = 0;
     wave_sync();
     const uint32_t total = pre[64];
-    for (uint32_t e = 0; e < total; e += 256) {
-      uint32_t k[WAVES], o[WAVES], w[WAVES];
+    constexpr int kU = 4;  // entries a lane in flight
+    for (uint32_t e = 0; e < total; e += 64 * kU) {
+      uint32_t k[kU], o[kU], w[kU];
 #pragma unroll
-      for (int u = 0; u < 4; u++) k[u] = min(e + u * 64 + lane, total - 1);
+      for (int u = 0; u < kU; u++) k[u] = min(e + u * 64 + lane, total - 1);
       ranges_of(pre, k, o);
 #pragma unroll
-      for (int u = 0; u < 4; u++) w[u] = g.pool[from[o[u]] + (k[u] - pre[o[u]])];
+      for (int u = 0; u < kU; u++) w[u] = g.pool[from[o[u]] + (k[u] - pre[o[u]])];
 #pragma unroll
-      for (int u = 0; u < 4; u++) w[u] = s_lmap[g.lab[w[u]]];
+      for (int u = 0; u < kU; u++) w[u] = s_lmap[g.lab[w[u]]];
 #pragma unroll
-      for (int u = 0; u < 4; u++)
+      for (int u = 0; u < kU; u++)
         if (e + u * 64 + lane < total && w[u] != 0xFF)
           atomicAdd(reinterpret_cast<uint32_t *>(s_cnt[wv][o[u]]) + (w[u] >> 2), 1u << (w[u] & 3) * 8);
     }
