@@ -251,7 +251,8 @@ struct dsm_engine {
   uint32_t wave_slots = 0;       // waves of the largest grid
   uint32_t last_blocks = 0, last_wpb = 0;  // grid of the last DFS launch
   uint32_t last_nrec = 0;                  // its records
-  double busy_per_record = -1;             // ms of its waves' task time a record, averaged (-1: no round yet)
+  double busy_per_record = -1;             // most ms of task time a record in recent rounds (-1: no round yet)
+  bool grid_given = false;                 // blocks_per_cu set by the caller or by dsm_autotune
   bool results_here = false;  // h_results holds the counts of the batch applied last
   uint32_t watchdog_ms = 60000;
   int wall_khz = 100000;
@@ -867,15 +868,16 @@ DfsArgs dfs_args(dsm_engine *e) {
   return da;
 }
 
-// The most blocks for a round with so much task time (ms, as the engine's last rounds
-// took it a record). Waves share a CU's issue slots and L1: at 12 a CU they take twice
-// as long for a task as at 4, and a round that ends with a few long tasks ends sooner
-// with 4. Measured at 4, 8 and 12 waves a CU: 20 ms of tasks (22 seeds, 100,000
-// vertices) 87, 100 and 106 us; 170 ms 186, 185 and 205; 270 ms 223, 221 and 220;
-// 880 ms (1,000,000 vertices) 541, 499 and 513; 2,600 ms 1,320, 932 and 948; 9,900 ms
-// 6.8, 4.3 and 3.7 ms.
+// The most blocks for a round with so much task time (ms, as the engine's recent rounds
+// took it a record). Waves share a CU's issue slots and L1: at 12 a CU a task takes
+// longer than at 8, and a round that ends with a few long tasks ends sooner with 8.
+// Measured at 4, 8 and 12 waves a CU: 20 ms of tasks (22 seeds, 100,000 vertices) 87,
+// 100 and 106 us; 170 ms 186, 185 and 205; 270 ms 223, 221 and 220; 880 ms (1,000,000
+// vertices) 541, 499 and 513; 2,600 ms 1,320, 932 and 948; 9,900 ms 6.8, 4.3 and 3.7 ms.
+// No fewer than 8: a first round of heavy records after light ones has this grid too,
+// and takes a sixth longer with 8, but nearly twice as long with 4.
 uint32_t blocks_for_work(const dsm_engine *e, double ms) {
-  const uint32_t waves_per_cu = ms <= 250 ? 4 : ms <= 2500 ? 8 : 0xFFFF;
+  const uint32_t waves_per_cu = ms <= 2500 ? 8 : 0xFFFF;
   return std::max(1u, waves_per_cu / e->dfs_wpb) * (uint32_t)e->num_cu;
 }
 
@@ -888,7 +890,7 @@ uint32_t dfs_grid(dsm_engine *e, uint32_t nrec) {
       ((uint64_t)nrec * std::max<uint32_t>(e->max_plans_per_key, 1) * 8 + e->dfs_wpb - 1) / e->dfs_wpb;
   const uint64_t least = std::min<uint64_t>((uint64_t)e->num_cu, want * std::max(1u, e->h_actl.p->max_deg / 16));
   uint32_t b = (uint32_t)std::min<uint64_t>(e->dfs_blocks, std::max<uint64_t>(want, least));
-  if (e->busy_per_record >= 0) b = std::min(b, blocks_for_work(e, e->busy_per_record * nrec));
+  if (!e->grid_given && e->busy_per_record >= 0) b = std::min(b, blocks_for_work(e, e->busy_per_record * nrec));
   e->last_nrec = nrec;
   e->last_wpb = e->tuples ? 4u : e->dfs_wpb;
   b = std::min(b, e->wave_slots / e->last_wpb);  // a mailbox for every wave
@@ -975,7 +977,8 @@ int round_error(dsm_engine *e) {
   }
   if (e->last_nrec) {
     const double x = (double)busy / (double)e->wall_khz / e->last_nrec;
-    e->busy_per_record = e->busy_per_record < 0 ? x : (e->busy_per_record + x) / 2;
+    // the most, fading: light rounds in between leave the heavy ones their grid
+    e->busy_per_record = std::max(x, 0.97 * e->busy_per_record);
   }
   return DSM_OK;
 }
@@ -1564,6 +1567,7 @@ int create_impl(dsm_engine *e, const dsm_graph_desc *graph, const dsm_query_desc
   int per_cu = (int)dfs_bpc(e, wpb);
   if (e->opt.blocks_per_cu && (int)e->opt.blocks_per_cu < per_cu) per_cu = (int)e->opt.blocks_per_cu;
   e->dfs_blocks = (uint32_t)(per_cu * e->num_cu);
+  e->grid_given = e->opt.blocks_per_cu != 0;
   // room for the largest grid any launch shape can have (the autotuner may
   // pick another shape later)
   {
@@ -2023,6 +2027,7 @@ int dsm_autotune(dsm_engine *e, const dsm_change *sample, uint32_t k, dsm_tune_r
   HIPCHK(hipSetDevice(e->opt.device));
   int rc;
   const uint32_t nq = (uint32_t)e->queries.size();
+  e->grid_given = true;  // a trial runs on the grid it stands for, and the one found is kept
   std::vector<uint32_t> s(k), d(k);
   for (uint32_t i = 0; i < k; i++) {
     s[i] = sample[i].src;

@@ -1,0 +1,63 @@
+"""The grid of a DFS round: what the caller or the autotuner set, and what earlier rounds
+of little work leave to heavy ones."""
+import numpy as np
+import pytest
+
+from dsm_amd import engine as E
+
+pytestmark = pytest.mark.gpu
+
+
+def _mixed_graph():
+    """6,000 vertices of 1,000 neighbours each beside 6,000 of two: (graph, queries,
+    heavy batch, light batch), 400 inserts of edges that are there each."""
+    n, rng = 6000, np.random.default_rng(4)
+    i = np.arange(n)
+    u = np.concatenate([np.repeat(i, 500), n + i])
+    v = np.concatenate([(np.repeat(i, 500) + np.tile(rng.choice(np.arange(1, n // 2), 500, replace=False), n)) % n,
+                        n + (i + 1) % n])
+    graph = (2 * n, np.zeros(2 * n, np.uint32), u.astype(np.uint32), v.astype(np.uint32))
+    sq = np.array([(0, 1), (1, 2), (2, 3), (3, 0)], np.uint32)
+    pick = rng.choice(500 * n, 400, replace=False)
+    heavy, light = ((np.ones(400, np.uint8), graph[2][p], graph[3][p], np.zeros(400, np.uint32))
+                    for p in (pick, 500 * n + rng.choice(n, 400, replace=False)))
+    return graph, [(4, np.zeros(4, np.uint32), sq[:, 0].copy(), sq[:, 1].copy())], heavy, light
+
+
+def _waves(eng, batch):
+    eng.process_batch(*batch)
+    s = eng.stats()
+    return s["dfs_waves"] // s["dfs_launches"]
+
+
+def test_a_given_or_tuned_grid_is_kept():
+    """Rounds of little work start as many blocks as the caller set, or dsm_autotune found."""
+    graph, queries, _, light = _mixed_graph()
+    eng = E.Engine(graph, queries, relabel=False, blocks_per_cu=3)
+    try:
+        waves = [_waves(eng, light) for _ in range(4)]
+        assert len(set(waves)) == 1 and waves[0] % 12 == 0
+        cus = waves[0] // 12
+    finally:
+        eng.close()
+    eng = E.Engine(graph, queries, relabel=False)
+    try:
+        rep = eng.autotune(*light)
+        want = rep["blocks_per_cu"] * rep["waves_per_block"] * cus
+        assert [_waves(eng, light) for _ in range(4)] == [want] * 4
+    finally:
+        eng.close()
+
+
+def test_light_rounds_leave_heavy_ones_their_grid():
+    """Rounds of heavy records among light ones start all blocks each time."""
+    graph, queries, heavy, light = _mixed_graph()
+    eng = E.Engine(graph, queries, relabel=False)
+    try:
+        first = _waves(eng, heavy)
+        for _ in range(3):
+            for _ in range(8):
+                eng.process_batch(*light)
+            assert _waves(eng, heavy) == first
+    finally:
+        eng.close()
