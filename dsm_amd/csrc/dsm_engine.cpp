@@ -843,7 +843,7 @@ DfsArgs dfs_args(dsm_engine *e) {
   da.seed_tag = e->seed_tag.p;
   da.mail = e->mail.p;
   da.idle = e->idle.p;
-  da.donate_cap = 0xFFFFFFFFu;
+  da.donate_cap = e->opt.queue_capacity ? e->opt.queue_capacity - 1 : kNoDonateCap;
   da.epoch = ++e->epoch;
   da.donate_min = e->donate_min;
   da.lane_work = e->lane_work;
@@ -901,12 +901,6 @@ uint32_t dfs_grid(dsm_engine *e, uint32_t nrec) {
 // The waiting words of a grid.
 uint32_t idle_words(uint32_t waves) { return (waves + kIdleGroup - 1) / kIdleGroup; }
 
-// queue_capacity bounds the tasks a round hands to waiting waves: an equal share
-// for every wave of the grid.
-void cap_donations(dsm_engine *e, DfsArgs &da) {
-  if (e->opt.queue_capacity) da.donate_cap = e->opt.queue_capacity / (e->last_blocks * e->last_wpb);
-}
-
 // One round. ev0 / ev1 / ev2 (may be null) mark its start, the end of seeding (its
 // start, unless seeding is timed on its own) and its end; `up` brings the records,
 // where they have not been sent. Three launches: as one HIP graph with its nodes
@@ -925,7 +919,6 @@ int dfs_round(dsm_engine *e, const RoundPart *parts, int nparts, hipEvent_t ev0,
   if (ev1 && !e->seeding_timed) HIPCHK(hipEventRecord(ev1, e->stream));
   DfsArgs da = dfs_args(e);
   const uint32_t blocks = dfs_grid(e, nrec);
-  cap_donations(e, da);
   HIPCHK(launch_ctl_reset(e->ctl.p, clear.tuple_count, clear.counts, clear.ncounts, e->idle.p,
                           idle_words(e->last_blocks * e->last_wpb), up, e->stream));
   HIPCHK(launch_seed(seed_args(e, parts, nparts), e->stream));

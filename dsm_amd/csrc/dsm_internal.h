@@ -79,6 +79,7 @@ struct DfsCtl {
   CtlLine<uint32_t> nseeds;        // seeds written by the seed kernel
   CtlLine<uint32_t> seed_head[kSeedHeads];  // seed shares claimed: head h counts shares h, h + kSeedHeads, ...
   CtlLine<uint32_t> seed_overflow; // seeds dropped for lack of capacity (must stay 0)
+  CtlLine<uint32_t> donated;       // tasks handed to waiting waves, counted where they have a limit
   CtlLine<uint32_t> abort;         // set when an idle wave outlived the watchdog
 };
 // The waiting state of 16 waves of the grid (wave w is in word w mod ngroups),
@@ -173,6 +174,7 @@ struct BatchDev {
   const uint32_t *rl_l;     // device label (already clamped)
 };
 
+constexpr uint32_t kNoDonateCap = 0xFFFFFFFFu;
 struct DfsArgs {
   DevGraph g;
   const uint64_t *bm;
@@ -183,7 +185,7 @@ struct DfsArgs {
   const uint32_t *seed_d;
   Mailbox *mail;                 // [waves of the grid]
   IdleWord *idle;                // [ceil(waves / kIdleGroup)]
-  uint32_t donate_cap;           // most tasks a wave may hand out
+  uint32_t donate_cap;           // most tasks the round may hand to waiting waves
   uint32_t epoch;
   uint32_t donate_min;
   uint32_t lane_work;            // longest leaf list one lane scans alone

@@ -1244,6 +1244,7 @@ __global__ __launch_bounds__(256) void k_ctl_reset(DfsCtl *ctl, unsigned long lo
     if (ctl) {
       ctl->nseeds.v = 0;
       ctl->seed_overflow.v = 0;
+      ctl->donated.v = 0;
       ctl->abort.v = 0;
     }
   }
@@ -1273,6 +1274,7 @@ struct WaveHdr {
   uint8_t qv[kMaxQ];
   uint8_t lix[kMaxQ];
   uint32_t n, query, plan, tag;
+  uint32_t donated;          // tasks the wave has handed out
   uint32_t fstate, fn;       // leaf set F of the current positions 0..n-3 (see leaf_count)
 };
 constexpr uint32_t kFCap = 1024;   // largest leaf set F kept in LDS
@@ -1801,12 +1803,14 @@ struct Crew {
   uint32_t nwaves, ngroups;
   uint32_t me;       // this wave
   uint32_t look;     // the waiting word it looks at next
-  uint32_t donated;  // tasks it has handed out
 };
 
 // One range to a wave that waits in word g; `word` (lane 0) is what lane 0 last
 // saw of it. The claim is a compare-and-swap of the word: its owner is no longer
-// waiting from then on, and finds the task in its mailbox.
+// waiting from then on, and finds the task in its mailbox. CAP: the round has a limit
+// of tasks handed out (a kernel of its own: the look at it in the others, never taken,
+// cost the 64-query search 0.8%).
+template <bool CAP>
 __device__ __forceinline__ bool donate_one(WaveHdr &S, const DfsArgs &a, uint32_t L0, uint32_t l, uint32_t n,
                                            Crew &cr, uint32_t g, unsigned long long &word) {
   uint32_t lv = 0xFFFFFFFFu, mid = 0, keep_cn = 0;
@@ -1849,6 +1853,13 @@ __device__ __forceinline__ bool donate_one(WaveHdr &S, const DfsArgs &a, uint32_
     }
   }
   if (lv == 0xFFFFFFFFu) return false;
+  // a place under the limit first, which goes back if no wave is waiting
+  if constexpr (CAP) {
+    uint32_t room = 0;
+    if (lane_id() == 0)
+      room = ld_relaxed(&a.ctl->donated.v) < a.donate_cap && atomicAdd(&a.ctl->donated.v, 1u) < a.donate_cap;
+    if (!bcast(room)) return false;
+  }
   const uint32_t e = S.end[lv];
   uint32_t who = 0xFFFFFFFFu;
   if (lane_id() == 0) {
@@ -1865,8 +1876,10 @@ __device__ __forceinline__ bool donate_one(WaveHdr &S, const DfsArgs &a, uint32_
     }
   }
   who = bcast(who);
-  if (who == 0xFFFFFFFFu) return false;
-  cr.donated++;
+  if (who == 0xFFFFFFFFu) {
+    if (CAP && lane_id() == 0) atomicSub(&a.ctl->donated.v, 1u);
+    return false;
+  }
   const uint32_t lane = lane_id();
   uint32_t pay = 0;
   if (lane == 0) pay = S.plan;
@@ -1884,19 +1897,21 @@ __device__ __forceinline__ bool donate_one(WaveHdr &S, const DfsArgs &a, uint32_
     // split there donates [mid', mid) only
     if (lv != l && keep_cn != S.cn[lv]) S.cn[lv] = keep_cn;
     S.end[lv] = mid;
+    S.donated++;
   }
   wave_sync();
   return true;
 }
 
+template <bool CAP>
 __device__ __forceinline__ void try_donate(WaveHdr &S, const DfsArgs &a, uint32_t L0, uint32_t l, uint32_t n, Crew &cr) {
   const uint32_t g = cr.look;
   cr.look = g + 1 < cr.ngroups ? g + 1 : 0u;
   unsigned long long word = 0;
   if (lane_id() == 0) word = ld_relaxed(&a.idle[g].v);
   const uint32_t waiting = bcast((uint32_t)__popcll(word & kIdleBits));
-  for (uint32_t k = 0; k < waiting && k < kDonateBurst && cr.donated < a.donate_cap; k++)
-    if (!donate_one(S, a, L0, l, n, cr, g, word)) break;
+  for (uint32_t k = 0; k < waiting && k < kDonateBurst; k++)
+    if (!donate_one<CAP>(S, a, L0, l, n, cr, g, word)) break;
 }
 
 // No started wave has work: every waiting word has all its started waves
@@ -1988,7 +2003,7 @@ __device__ __forceinline__ bool wait_for_task(const DfsArgs &a, const Crew &cr, 
 // of 4,096, beside the update): 8.1 ms at two blocks, 6.1 at three, 5.9 at four
 // (a 512-entry leaf set), where the update falls behind; 5.6 at three with hash
 // sets for the short leaf sets.
-template <int WPB, bool TUP>
+template <int WPB, bool TUP, bool CAP>
 __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_levels) {
   extern __shared__ __align__(16) uint8_t s_dyn[];
   const uint32_t lane = lane_id();
@@ -2005,7 +2020,10 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
     M.ftab = M.fbuf + kFCap;
   }
   WaveHdr &S = *M.h;
-  if (lane == 0) S.plan = 0xFFFFFFFFu;
+  if (lane == 0) {
+    S.plan = 0xFFFFFFFFu;
+    S.donated = 0;
+  }
   wave_sync();
   // what the block's waves did, for its record
   __shared__ unsigned long long s_rec[WPB][7];
@@ -2014,7 +2032,6 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
   cr.ngroups = (cr.nwaves + kIdleGroup - 1) / kIdleGroup;
   cr.me = blockIdx.x * WPB + wv;
   cr.look = (cr.me + 1) % cr.ngroups;
-  cr.donated = 0;
   // a seed table overflow leaves unwritten slots: match nothing, the host
   // reports the error (the table is sized so that it cannot happen)
   const uint32_t nseeds = a.ctl->seed_overflow.v ? 0u : a.ctl->nseeds.v;
@@ -2150,7 +2167,7 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
           for (;;) {
             if (++tick >= a.donate_every) {
               tick = 0;
-              try_donate(S, a, L0, l, n, cr);
+              try_donate<CAP>(S, a, L0, l, n, cr);
             }
             const uint32_t p = bcast(S.pos[l]), e = bcast(S.end[l]);
             if (p >= e) break;
@@ -2198,7 +2215,7 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
           for (;;) {
             if (++tick >= a.donate_every) {
               tick = 0;
-              try_donate(S, a, L0, l, n, cr);
+              try_donate<CAP>(S, a, L0, l, n, cr);
             }
             const uint32_t p = bcast(S.pos[l]), e = bcast(S.end[l]);
             if (p >= e) break;
@@ -2273,7 +2290,7 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
         }
         if (++tick >= a.donate_every) {
           tick = 0;
-          try_donate(S, a, L0, l, n, cr);
+          try_donate<CAP>(S, a, L0, l, n, cr);
         }
         const uint32_t p = bcast(S.pos[l]), e = bcast(S.end[l]);
         if (p < e) {
@@ -2330,7 +2347,7 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
     s_rec[wv][0] = busy;
     s_rec[wv][1] = first_t;
     s_rec[wv][2] = last_t;
-    s_rec[wv][3] = cr.donated;
+    s_rec[wv][3] = S.donated;
   }
   __syncthreads();
   if (wv == 0) {
@@ -2379,7 +2396,7 @@ template <int WPB>
 int max_blocks(uint32_t chunk_levels) {
   int nb = 0;
   const size_t lds = (size_t)WPB * wave_lds_bytes(chunk_levels);
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_dfs<WPB, false>, WPB * 64, lds) != hipSuccess) return 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_dfs<WPB, false, false>, WPB * 64, lds) != hipSuccess) return 1;
   return nb > 0 ? nb : 1;
 }
 
@@ -2596,21 +2613,29 @@ hipError_t launch_seed(const SeedArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_dfs(const DfsArgs &a, uint32_t blocks, uint32_t waves_per_block, uint32_t max_query_vertices,
-                      hipStream_t s) {
-  const uint32_t cl = max_query_vertices > 3 ? max_query_vertices - 3 : 1;
+namespace {
+template <bool CAP>
+hipError_t launch_dfs_shape(const DfsArgs &a, uint32_t blocks, uint32_t waves_per_block, uint32_t cl, hipStream_t s) {
   const size_t per = wave_lds_bytes(cl);
   if (a.tuples) {
-    hipLaunchKernelGGL((k_dfs<4, true>), dim3(blocks), dim3(256), 4 * per, s, a, cl);
+    hipLaunchKernelGGL((k_dfs<4, true, CAP>), dim3(blocks), dim3(256), 4 * per, s, a, cl);
     return hipGetLastError();
   }
   switch (waves_per_block) {
-    case 1: hipLaunchKernelGGL((k_dfs<1, false>), dim3(blocks), dim3(64), per, s, a, cl); break;
-    case 2: hipLaunchKernelGGL((k_dfs<2, false>), dim3(blocks), dim3(128), 2 * per, s, a, cl); break;
-    case 8: hipLaunchKernelGGL((k_dfs<8, false>), dim3(blocks), dim3(512), 8 * per, s, a, cl); break;
-    default: hipLaunchKernelGGL((k_dfs<4, false>), dim3(blocks), dim3(256), 4 * per, s, a, cl); break;
+    case 1: hipLaunchKernelGGL((k_dfs<1, false, CAP>), dim3(blocks), dim3(64), per, s, a, cl); break;
+    case 2: hipLaunchKernelGGL((k_dfs<2, false, CAP>), dim3(blocks), dim3(128), 2 * per, s, a, cl); break;
+    case 8: hipLaunchKernelGGL((k_dfs<8, false, CAP>), dim3(blocks), dim3(512), 8 * per, s, a, cl); break;
+    default: hipLaunchKernelGGL((k_dfs<4, false, CAP>), dim3(blocks), dim3(256), 4 * per, s, a, cl); break;
   }
   return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_dfs(const DfsArgs &a, uint32_t blocks, uint32_t waves_per_block, uint32_t max_query_vertices,
+                      hipStream_t s) {
+  const uint32_t cl = max_query_vertices > 3 ? max_query_vertices - 3 : 1;
+  if (a.donate_cap != kNoDonateCap) return launch_dfs_shape<true>(a, blocks, waves_per_block, cl, s);
+  return launch_dfs_shape<false>(a, blocks, waves_per_block, cl, s);
 }
 
 uint32_t dfs_lds_bytes_per_wave(uint32_t max_query_vertices) {

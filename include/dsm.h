@@ -76,8 +76,8 @@ typedef struct {
   uint32_t waves_per_block;  /* DFS launch shape; 0 = default */
   uint32_t blocks_per_cu;    /* 0 = as many as occupancy allows */
   uint32_t donate_min;       /* smallest source range split off to an idle wave (0 = default) */
-  uint32_t queue_capacity;   /* most tasks a round hands to idle waves, shared evenly by
-                                its waves (0 = no limit) */
+  uint32_t queue_capacity;   /* a round hands fewer tasks than this to idle waves (0 = no
+                                limit, 1 = none) */
   uint32_t watchdog_ms;      /* an idle DFS wave that waits longer than this for
                                 work aborts the round with DSM_EDEVICE (0 = 60 s) */
   uint32_t lane_work;        /* one level above the leaf: longest list a lane scans

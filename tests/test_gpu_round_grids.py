@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from dsm_amd import engine as E
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -59,5 +60,30 @@ def test_light_rounds_leave_heavy_ones_their_grid():
             for _ in range(8):
                 eng.process_batch(*light)
             assert _waves(eng, heavy) == first
+    finally:
+        eng.close()
+
+
+@pytest.mark.parametrize("queue_capacity", [0, 1, 2, 50, 100000])
+def test_few_hand_offs_are_allowed(queue_capacity):
+    """A limit on a round's hand-offs below the number of its waves allows some: 400
+    records of 200-entry lists, eight seeds each, more than the grid has waves."""
+    n, rng = 2000, np.random.default_rng(9)
+    i = np.arange(n)
+    u = np.repeat(i, 100)
+    v = (u + np.tile(rng.choice(np.arange(1, n // 2), 100, replace=False), n)) % n
+    u, v, lab = u.astype(np.uint32), v.astype(np.uint32), np.zeros(n, np.uint32)
+    sq = np.array([(0, 1), (1, 2), (2, 3), (3, 0)], np.uint32)
+    queries = [(4, np.zeros(4, np.uint32), sq[:, 0].copy(), sq[:, 1].copy())]
+    pick = rng.choice(len(u), 400, replace=False)
+    batch = (np.ones(400, np.uint8), u[pick], v[pick], np.zeros(400, np.uint32))
+    want = O.run_stream(O.Graph(n, lab, u, v), [O.Query(*queries[0])], [batch], relabel=False)[0]["pos"]
+    eng = E.Engine((n, lab, u, v), queries, relabel=False, queue_capacity=queue_capacity)
+    try:
+        for _ in range(3):
+            assert eng.process_batch(*batch)[0].tolist() == want
+            donated = eng.stats()["tasks_donated"]
+            assert (donated > 0) == (queue_capacity != 1)
+            assert queue_capacity == 0 or donated < queue_capacity
     finally:
         eng.close()
