@@ -6,7 +6,9 @@
 // entry point; it lets the primitive be checked against a set intersection on
 // its own, outside the DFS.
 #include <algorithm>
+#include <memory>
 #include <mutex>
+#include <new>
 
 #include "../../include/dsm.h"
 #include "dsm_device.h"
@@ -139,39 +141,55 @@ bool sorted_set(const uint32_t *a, uint32_t n) {
 
 namespace {
 
-// Short calls. At most kShortA entries of A go to k_intersect_short (two rounds of
-// its block); inputs of at most kShortCopy entries together are uploaded in one
-// copy, and results of at most as many come back in one with their number: a copy
-// costs some 8 us, however small. 1,000 x 3,000 entries: 67 us with a copy per array
-// and three launches, 36 with one of each.
-constexpr uint32_t kShortA = 2048, kShortCopy = 8192;
+// Calls that are not long. At most kShortA entries of A go to k_intersect_short (two
+// rounds of its block); inputs of at most kShortCheck entries together are checked on
+// the host. Inputs of at most `staged` entries together go up in one copy, the word that
+// says whether they are in order with them, and results of at most half as many come
+// back in one copy with their number: a copy costs some 8 us, however small, and the
+// release of device memory 25 more once a call has sent eight copies and launches. Of
+// more entries, the copy into the staging buffer costs more than that.
+// 1,000 x 3,000 entries: 67 us with a copy per array and three launches, 36 with one of
+// each. With the device memory allocated, 5,000 x 5,000: 113 us with a copy per array
+// and five launches, 68 in six steps; 40,000 x 40,000 116 and 69, 130,000 x 130,000 211
+// and 154, 132,000 x 132,000 (unstaged) 187. In the fixed array, without that release:
+// 65,000 x 65,000 89 and 82 us, 80,000 x 80,000 96 and 92, 130,000 x 130,000 112 and 123.
+constexpr uint32_t kShortA = 2048, kShortCheck = 8192, kStaged = 262144, kStagedFixed = 131072;
+
+// kStaged + 1 words of the calling thread, or null. Kept until it ends: fresh pages
+// would cost each call more than the copies it saves.
+uint32_t *staging() {
+  static thread_local std::unique_ptr<uint32_t[]> words;
+  if (!words) words.reset(new (std::nothrow) uint32_t[kStaged + 1]);
+  return words.get();
+}
 
 uint32_t chunks_of(uint32_t na) { return (na + 63) / 64; }
 
-// Words of device memory: a | b | hits (64 per chunk) | cnt | off | total | result
+// Words of device memory: a | b | total | result | hits (64 per chunk) | cnt | off
 size_t words_of(uint32_t na, uint32_t nb) {
   const size_t nch = chunks_of(na);
   return (size_t)na + nb + nch * 64 + 2 * nch + 1 + std::min(na, nb);
 }
 
 // a and b, not empty, intersected in the words_of(na, nb) words at base; kBadInput
-// as the size if they are not in order, which the device checks with `check`.
-hipError_t intersect_in(uint32_t *base, const uint32_t *a, uint32_t na, const uint32_t *b, uint32_t nb, bool check,
-                        uint32_t *out, uint32_t *num_out) {
+// as the size if they are not in order, which the device checks past kShortCheck entries.
+hipError_t intersect_in(uint32_t *base, const uint32_t *a, uint32_t na, const uint32_t *b, uint32_t nb,
+                        uint32_t staged, uint32_t *out, uint32_t *num_out) {
   const uint32_t nch = chunks_of(na), most = std::min(na, nb);
-  uint32_t *dA = base, *dB = dA + na, *dH = dB + nb, *dC = dH + (size_t)nch * 64, *dO = dC + nch, *dT = dO + nch,
-           *dR = dT + 1;
-  uint32_t buf[kShortCopy + 1];
+  uint32_t *dA = base, *dB = dA + na, *dT = dB + nb, *dR = dT + 1, *dH = dR + most, *dC = dH + (size_t)nch * 64,
+           *dO = dC + nch;
+  const size_t both = (size_t)na + nb;
+  const bool check = both > kShortCheck;
+  uint32_t *buf = most <= staged / 2 ? staging() : nullptr;
   hipError_t e;
-  if ((size_t)na + nb <= kShortCopy) {
+  if (buf && both <= staged) {
     std::copy(a, a + na, buf);
     std::copy(b, b + nb, buf + na);
-    if ((e = hipMemcpy(dA, buf, ((size_t)na + nb) * 4, hipMemcpyHostToDevice)) != hipSuccess) return e;
+    buf[both] = 0;
+    if ((e = hipMemcpy(dA, buf, (both + 1) * 4, hipMemcpyHostToDevice)) != hipSuccess) return e;
   } else {
     if ((e = hipMemcpy(dA, a, (size_t)na * 4, hipMemcpyHostToDevice)) != hipSuccess) return e;
     if ((e = hipMemcpy(dB, b, (size_t)nb * 4, hipMemcpyHostToDevice)) != hipSuccess) return e;
-  }
-  if (check || na > kShortA) {
     hipLaunchKernelGGL(k_check_clear, dim3(1), dim3(1), 0, nullptr, dT);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
@@ -193,7 +211,7 @@ hipError_t intersect_in(uint32_t *base, const uint32_t *a, uint32_t na, const ui
                        dT, dR);
   }
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if (most <= kShortCopy) {
+  if (buf) {
     if ((e = hipMemcpy(buf, dT, ((size_t)most + 1) * 4, hipMemcpyDeviceToHost)) != hipSuccess) return e;
     *num_out = buf[0];
     if (buf[0] != kBadInput) std::copy(buf + 1, buf + 1 + buf[0], out);
@@ -229,7 +247,7 @@ int settled(const char *who, const uint32_t *a, uint32_t na, const uint32_t *b, 
     return DSM_EINVAL;
   }
   const bool none = na == 0 || nb == 0;
-  if ((none || all || (size_t)na + nb <= kShortCopy) && (!sorted_set(a, na) || !sorted_set(b, nb)))
+  if ((none || all || (size_t)na + nb <= kShortCheck) && (!sorted_set(a, na) || !sorted_set(b, nb)))
     return not_sorted(who);
   if (!none) return 1;
   *num_out = 0;
@@ -257,7 +275,7 @@ extern "C" int dsm_intersect_sorted(int device, const uint32_t *a, uint32_t na, 
   uint32_t *base = nullptr, size = 0;
   hipError_t e = hipSetDevice(device);
   if (e == hipSuccess) e = hipMalloc(&base, words_of(na, nb) * 4);
-  if (e == hipSuccess) e = intersect_in(base, a, na, b, nb, (size_t)na + nb > kShortCopy, out, &size);
+  if (e == hipSuccess) e = intersect_in(base, a, na, b, nb, kStaged, out, &size);
   if (base) (void)hipFree(base);
   return finished(who, e, a, na, b, nb, size, num_out);
 }
@@ -313,6 +331,6 @@ extern "C" int dsm_intersect_sorted_noalloc(int device, const uint32_t *a, uint3
   uint32_t *base = nullptr, size = 0;
   hipError_t e = hipSetDevice(device);
   if (e == hipSuccess) e = scratch_of(device, &base);
-  if (e == hipSuccess) e = intersect_in(base, a, na, b, nb, (size_t)na + nb > kShortCopy, out, &size);
+  if (e == hipSuccess) e = intersect_in(base, a, na, b, nb, kStagedFixed, out, &size);
   return finished(who, e, a, na, b, nb, size, num_out);
 }
