@@ -190,7 +190,8 @@ __device__ __forceinline__ void bounds2(const uint32_t *L, uint32_t d, uint32_t 
   r1 = __builtin_amdgcn_readlane(a, 32);
 }
 
-__device__ __forceinline__ bool lds_contains(const uint32_t *a, uint32_t n, uint32_t x) {
+template <typename T>
+__device__ __forceinline__ bool lds_contains(const T *a, uint32_t n, uint32_t x) {
   if (n == 0) return false;
   uint32_t lo = 0;
   while (n > 1) {

@@ -1277,7 +1277,7 @@ struct WaveHdr {
   uint32_t donated;          // tasks the wave has handed out
   uint32_t fstate, fn;       // leaf set F of the current positions 0..n-3 (see leaf_count)
 };
-constexpr uint32_t kFCap = 1024;   // largest leaf set F kept in LDS
+constexpr uint32_t kFCap = 1024;   // largest leaf set F kept in LDS as whole ids
 constexpr uint32_t kFScan = 2048;  // longest list it is computed from
 // Membership in F goes through a table beside it, of one of two kinds.
 // - Up to kFHash entries: a hash set of the ids, kFBuckets buckets of four, a full
@@ -1288,6 +1288,9 @@ constexpr uint32_t kFScan = 2048;  // longest list it is computed from
 //   bucket. A test reads two offsets and searches the bucket's few entries.
 //   Filling the buckets between two entries is a loop per entry, as long as F is
 //   short, which is why the short sets, nearly all of them, take the hash set.
+// A set of more than kFCap entries lies in the same words as the low halves of its
+// ids, two a word: the bucket gives the rest, where an id has at most 16 bits below its
+// bucket's (up to 2^25 vertices; in larger graphs such a set is not kept).
 constexpr uint32_t kFIdx = 512;
 constexpr uint32_t kFHash = 128;
 constexpr uint32_t kFBuckets = 64;
@@ -1300,7 +1303,7 @@ constexpr uint32_t kFEmpty = 0xFFFFFFFFu;
 // states of the leaf set F
 constexpr uint32_t kFStale = 0;  // not computed for the current positions
 constexpr uint32_t kFReady = 1;  // fbuf[0, fn) holds F, ftab its table
-constexpr uint32_t kFLarge = 2;  // the shortest fixed list exceeds kFScan, or F kFCap: per-candidate descent
+constexpr uint32_t kFLarge = 2;  // the shortest fixed list exceeds kFScan, or F kFCap unhalved: per-candidate descent
 constexpr uint32_t kFNone = 3;   // the leaf's only backward neighbour is position n-2
 
 struct WaveMem {
@@ -1309,10 +1312,11 @@ struct WaveMem {
   uint32_t *cand;   // [levels][64]
   uint32_t *cst;    // [levels][64] list start of each candidate
   uint32_t *cdg;    // [levels][64] degree of each candidate
-  uint32_t *fbuf;   // [kFCap] leaf set F, ascending
+  uint32_t *fbuf;   // [kFCap] leaf set F, ascending (past kFCap entries, halves: [2 kFCap])
   uint32_t *ftab;   // F's table: kFBuckets x 4 ids, or kFIdx + 1 16-bit bucket offsets into fbuf
 };
 constexpr uint32_t kFTabBytes = ((kFIdx + 1) * 2 + 15) / 16 * 16;
+static_assert(kFScan <= 2 * kFCap, "every set in halves fits");
 static_assert(kFBuckets * 16 <= kFTabBytes && kFBuckets == 64, "the hash set fits the table, a bucket per lane");
 
 __host__ __device__ constexpr uint32_t wave_lds_bytes(uint32_t chunk_levels) {
@@ -1423,7 +1427,10 @@ __device__ __forceinline__ uint32_t f_hash(uint32_t y) { return (y * 0x9E3779B1u
 // entries of the intersection of their lists (label bucket of the shortest)
 // that carry the leaf's signature bit and differ from the earlier images of
 // its label. F is sorted. Sets fstate: kFReady (F in fbuf), kFLarge (shortest
-// such list longer than kFScan, or F than kFCap) or kFNone (no such neighbour).
+// such list longer than kFScan, or F than kFCap with ids too long for halves) or kFNone
+// (no such neighbour). A set found to pass kFCap is computed anew, in halves, with its
+// bucket offsets: squares over lists of 1,900 entries (12,000 vertices) take 8.4 ms for 8
+// records and 79 for 256 with a descent per candidate instead, 3.4 and 29 in halves.
 __device__ __forceinline__ void compute_leaf_set(const WaveMem &M, const DfsArgs &a, uint32_t leaf, uint32_t &scanned,
                                  uint32_t &loads) {
   WaveHdr &S = *M.h;
@@ -1431,6 +1438,10 @@ __device__ __forceinline__ void compute_leaf_set(const WaveMem &M, const DfsArgs
   const uint32_t pv = leaf - 1;
   const uint32_t bp = S.back[leaf] & ~(1u << pv);
   uint32_t state = kFReady, cnt = 0;
+  uint16_t *fidx = reinterpret_cast<uint16_t *>(M.ftab);
+  const uint32_t sh = a.fshift;
+  bool halves = false;
+  uint32_t open = 0;  // of halves: the first bucket without an offset
   if (bp == 0) {
     state = kFNone;
   } else {
@@ -1448,17 +1459,38 @@ __device__ __forceinline__ void compute_leaf_set(const WaveMem &M, const DfsArgs
         const bool ok = test_entries(M, a, src, oth, inj, sig, p, len, w, loads);
         scanned += p + lane < len ? 1u : 0u;
         const uint64_t m = ballot(ok);
-        if (cnt + (uint32_t)__popcll(m) > kFCap) {
-          state = kFLarge;
-          break;
+        if (!halves && cnt + (uint32_t)__popcll(m) > kFCap) {
+          if (sh > 16) {
+            state = kFLarge;
+            break;
+          }
+          halves = true;
+          cnt = 0;
+          p = 0u - 64;
+          continue;
         }
-        if (ok) M.fbuf[cnt + mbcnt(m)] = w;
+        const uint32_t at = cnt + mbcnt(m);
+        if (!halves) {
+          if (ok) M.fbuf[at] = w;
+        } else if (m) {
+          // entry `at` opens every bucket after its predecessor's up to its own
+          const uint32_t b = w >> sh;
+          const uint64_t below = m & ((1ull << lane) - 1);
+          const uint32_t before = __shfl(b, below ? 63 - __builtin_clzll(below) : 0) + 1;
+          if (ok) {
+            for (uint32_t k = below ? before : open; k <= b; k++) fidx[k] = (uint16_t)at;
+            reinterpret_cast<uint16_t *>(M.fbuf)[at] = (uint16_t)w;
+          }
+          open = __builtin_amdgcn_readlane(b, 63 - __builtin_clzll(m)) + 1;
+        }
         cnt += (uint32_t)__popcll(m);
       }
     }
   }
   wave_sync();
-  if (state == kFReady && cnt <= kFHash) {
+  if (halves) {
+    for (uint32_t k = open + lane; k <= kFIdx; k += 64) fidx[k] = (uint16_t)cnt;
+  } else if (state == kFReady && cnt <= kFHash) {
     reinterpret_cast<uint4 *>(M.ftab)[lane] = uint4{kFEmpty, kFEmpty, kFEmpty, kFEmpty};
     wave_sync();
     for (uint32_t i = lane; i < cnt; i += 64) {
@@ -1469,8 +1501,6 @@ __device__ __forceinline__ void compute_leaf_set(const WaveMem &M, const DfsArgs
   } else if (state == kFReady) {
     // bucket offsets: entry i opens every bucket after its predecessor's up
     // to its own; buckets past the last entry start at cnt
-    uint16_t *fidx = reinterpret_cast<uint16_t *>(M.ftab);
-    const uint32_t sh = a.fshift;
     for (uint32_t i = lane; i < cnt; i += 64) {
       const uint32_t b = M.fbuf[i] >> sh;
       const uint32_t pb = i ? (M.fbuf[i - 1] >> sh) + 1 : 0u;
@@ -1494,6 +1524,15 @@ __device__ __forceinline__ bool f_look(const uint4 &t, uint32_t y, bool &found) 
   return found || t.w == kFEmpty;
 }
 
+// y in F of more than kFHash entries, which are whole ids or, past kFCap, halves.
+template <typename T>
+__device__ __forceinline__ bool in_leaf_range(const WaveMem &M, const DfsArgs &a, uint32_t y) {
+  const uint16_t *fidx = reinterpret_cast<const uint16_t *>(M.ftab);
+  const uint32_t b = y >> a.fshift;
+  const uint32_t lo = fidx[b], hi = fidx[b + 1];
+  return lds_contains(reinterpret_cast<const T *>(M.fbuf) + lo, hi - lo, (T)y);
+}
+
 // y in F (state kFReady, fn entries), through F's table.
 __device__ __forceinline__ bool in_leaf_set(const WaveMem &M, const DfsArgs &a, uint32_t fn, uint32_t y) {
   if (fn <= kFHash) {
@@ -1501,10 +1540,16 @@ __device__ __forceinline__ bool in_leaf_set(const WaveMem &M, const DfsArgs &a, 
     for (uint32_t h = f_hash(y); !f_look(reinterpret_cast<const uint4 *>(M.ftab)[h], y, found);) h = (h + 1) % kFBuckets;
     return found;
   }
+  return fn <= kFCap ? in_leaf_range<uint32_t>(M, a, y) : in_leaf_range<uint16_t>(M, a, y);
+}
+
+// Entry k of F.
+__device__ __forceinline__ uint32_t f_entry(const WaveMem &M, const DfsArgs &a, uint32_t fn, uint32_t k) {
+  if (fn <= kFCap) return M.fbuf[k];
   const uint16_t *fidx = reinterpret_cast<const uint16_t *>(M.ftab);
-  const uint32_t b = y >> a.fshift;
-  const uint32_t lo = fidx[b], hi = fidx[b + 1];
-  return lds_contains(M.fbuf + lo, hi - lo, y);
+  uint32_t b = 0;  // the last bucket that starts at or before k, and so holds it
+  for (uint32_t half = kFIdx / 2; half; half >>= 1) b = fidx[b + half] <= k ? b + half : b;
+  return b << a.fshift | (reinterpret_cast<const uint16_t *>(M.fbuf)[k] & ((1u << a.fshift) - 1));
 }
 
 // Leaf images of the partial match whose position n-2 holds w (this lane's
@@ -1579,10 +1624,14 @@ __device__ __forceinline__ uint32_t leaf_accept(const WaveMem &M, const DfsArgs 
         if (!f_look(t[u], y[u], found)) found = in_leaf_set(M, a, r.fn, y[u]);
         c += ok[u] && found && !(r.injw && y[u] == w[u]) ? 1u : 0u;
       }
+    } else if (r.fn <= kFCap) {
+#pragma unroll
+      for (int u = 0; u < K; u++)
+        c += ok[u] && !(r.injw && y[u] == w[u]) && in_leaf_range<uint32_t>(M, a, y[u]) ? 1u : 0u;
     } else {
 #pragma unroll
       for (int u = 0; u < K; u++)
-        c += ok[u] && !(r.injw && y[u] == w[u]) && in_leaf_set(M, a, r.fn, y[u]) ? 1u : 0u;
+        c += ok[u] && !(r.injw && y[u] == w[u]) && in_leaf_range<uint16_t>(M, a, y[u]) ? 1u : 0u;
     }
     return c;
   }
@@ -1740,7 +1789,7 @@ __device__ __forceinline__ uint32_t leaf_count_wave(const WaveMem &M, const DfsA
         uint32_t x[K];
         bool in[K];
 #pragma unroll
-        for (int u = 0; u < K; u++) x[u] = k0 + 64 * u + lane < r.fn ? M.fbuf[k0 + 64 * u + lane] : 0xFFFFFFFFu;
+        for (int u = 0; u < K; u++) x[u] = k0 + 64 * u + lane < r.fn ? f_entry(M, a, r.fn, k0 + 64 * u + lane) : 0xFFFFFFFFu;
         contains_each(L, len, x, in);
 #pragma unroll
         for (int u = 0; u < K; u++) c += in[u] && !(r.injw && x[u] == ww) ? 1u : 0u;
