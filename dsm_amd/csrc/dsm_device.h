@@ -95,10 +95,6 @@ template <typename T>
 __device__ __forceinline__ void st_release(T *p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ bool cas_u32(uint32_t *p, uint32_t expect, uint32_t desire) {
-  return __hip_atomic_compare_exchange_strong(p, &expect, desire, __ATOMIC_ACQ_REL, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // # elements < x in sorted a[0, n)
 __device__ __forceinline__ uint32_t lower_bound(const uint32_t *a, uint32_t n, uint32_t x) {
