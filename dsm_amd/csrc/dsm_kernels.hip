@@ -1902,11 +1902,13 @@ __device__ __forceinline__ bool donate_one(WaveHdr &S, const DfsArgs &a, uint32_
     }
   }
   if (lv == 0xFFFFFFFFu) return false;
-  // a place under the limit first, which goes back if no wave is waiting
+  // a place under the limit first, which goes back if no wave is waiting, as does one past it
   if constexpr (CAP) {
     uint32_t room = 0;
-    if (lane_id() == 0)
-      room = ld_relaxed(&a.ctl->donated.v) < a.donate_cap && atomicAdd(&a.ctl->donated.v, 1u) < a.donate_cap;
+    if (lane_id() == 0 && ld_relaxed(&a.ctl->donated.v) < a.donate_cap) {
+      room = atomicAdd(&a.ctl->donated.v, 1u) < a.donate_cap;
+      if (!room) atomicSub(&a.ctl->donated.v, 1u);
+    }
     if (!bcast(room)) return false;
   }
   const uint32_t e = S.end[lv];
