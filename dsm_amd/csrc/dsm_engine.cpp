@@ -882,13 +882,23 @@ uint32_t blocks_for_work(const dsm_engine *e, double ms) {
 }
 
 // The grid: a round over a handful of records gets one block per CU, so that few
-// waves pay the start-up and termination atomics, and fewer where no list is long
-// enough to give a CU's waves anything to share (a record of a graph whose lists have
-// 30 entries is matched by a few waves; 256 blocks' records cost more than that).
+// waves pay the start-up and termination atomics, and fewer where neither a list is long
+// enough to give a CU's waves anything to share nor a query deep enough: a 4-vertex query
+// on lists of 30 entries is matched by a few waves, and 256 blocks' records cost more than
+// that. What a seed can expand is at most the longest list's length to the power of the
+// positions after it. One record, lists of 16 entries, paths of 6, 7 and 8 vertices, in
+// two calls: 317, 992 and 7,061 us with a block per 4,096 entries of that, 334, 997 and
+// 7,109 per 16,384, 476, 4,109 and 58,452 by the lists' length alone; of 5 vertices 202
+// with either.
 uint32_t dfs_grid(dsm_engine *e, uint32_t nrec) {
   const uint64_t want =
       ((uint64_t)nrec * std::max<uint32_t>(e->max_plans_per_key, 1) * 8 + e->dfs_wpb - 1) / e->dfs_wpb;
-  const uint64_t least = std::min<uint64_t>((uint64_t)e->num_cu, want * std::max(1u, e->h_actl.p->max_deg / 16));
+  const uint32_t longest = e->h_actl.p->max_deg;
+  uint64_t tree = 1;
+  for (uint32_t l = 2; l < e->max_qn && tree < (1ull << 32); l++) tree *= longest;
+  const uint64_t share = std::max<uint64_t>({1, longest / 16, tree / 4096});
+  const uint64_t least = share >= (uint64_t)e->num_cu ? (uint64_t)e->num_cu
+                                                      : std::min<uint64_t>((uint64_t)e->num_cu, want * share);
   uint32_t b = (uint32_t)std::min<uint64_t>(e->dfs_blocks, std::max<uint64_t>(want, least));
   if (!e->grid_given && e->busy_per_record >= 0) b = std::min(b, blocks_for_work(e, e->busy_per_record * nrec));
   e->last_nrec = nrec;

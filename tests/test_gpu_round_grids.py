@@ -87,3 +87,31 @@ def test_few_hand_offs_are_allowed(queue_capacity):
             assert queue_capacity == 0 or donated < queue_capacity
     finally:
         eng.close()
+
+
+@pytest.mark.parametrize("k,whole", [(4, False), (6, True), (9, True)])
+def test_deep_queries_over_short_lists_get_a_block_per_cu(k, whole):
+    """One record of a graph whose lists have 8 or 16 entries: a path of many vertices gives
+    a whole grid work, one of four does not."""
+    n, half, rng = 3000, 8 if k < 9 else 4, np.random.default_rng(k)
+    i = np.arange(n)
+    u = np.repeat(i, half).astype(np.uint32)
+    v = ((u + np.tile(rng.choice(np.arange(1, n // 2), half, replace=False), n)) % n).astype(np.uint32)
+    graph = (n, np.zeros(n, np.uint32), u, v)
+    queries = [(k, np.zeros(k, np.uint32), np.arange(k - 1, dtype=np.uint32), np.arange(1, k, dtype=np.uint32))]
+    one = (np.ones(1, np.uint8), u[:1], v[:1], np.zeros(1, np.uint32))
+    full = (np.ones(2000, np.uint8), u[:2000], v[:2000], np.zeros(2000, np.uint32))
+    eng = E.Engine(graph, [(2, np.zeros(2, np.uint32), np.zeros(1, np.uint32), np.ones(1, np.uint32))], relabel=False,
+                   blocks_per_cu=1)
+    try:
+        grid = _waves(eng, full)  # a block per CU
+    finally:
+        eng.close()
+    want = O.run_stream(O.Graph(*graph), [O.Query(*queries[0])], [one], relabel=False)[0]["pos"]
+    eng = E.Engine(graph, queries, relabel=False)
+    try:
+        assert eng.process_batch(*one)[0].tolist() == want and want[0] > 0
+        waves = _waves(eng, one)
+        assert waves >= grid if whole else waves < grid
+    finally:
+        eng.close()
