@@ -250,6 +250,7 @@ struct dsm_engine {
   DevBuf<unsigned long long> query_busy;  // per query: DFS task ticks since the last read
   uint32_t wave_slots = 0;       // waves of the largest grid
   uint32_t last_blocks = 0, last_wpb = 0;  // grid of the last DFS launch
+  uint32_t last_crew = 0;                  // its blocks that began at once
   uint32_t last_nrec = 0;                  // its records
   double busy_per_record = -1;             // most ms of task time a record in recent rounds (-1: no round yet)
   bool grid_given = false;                 // blocks_per_cu set by the caller or by dsm_autotune
@@ -868,17 +869,24 @@ DfsArgs dfs_args(dsm_engine *e) {
   return da;
 }
 
-// The most blocks for a round with so much task time (ms, as the engine's recent rounds
-// took it a record). Waves share a CU's issue slots and L1: at 12 a CU a task takes
-// longer than at 8, and a round that ends with a few long tasks ends sooner with 8.
-// Measured at 4, 8 and 12 waves a CU: 20 ms of tasks (22 seeds, 100,000 vertices) 87,
-// 100 and 106 us; 170 ms 186, 185 and 205; 270 ms 223, 221 and 220; 880 ms (1,000,000
-// vertices) 541, 499 and 513; 2,600 ms 1,320, 932 and 948; 9,900 ms 6.8, 4.3 and 3.7 ms.
-// No fewer than 8: a first round of heavy records after light ones has this grid too,
-// and takes a sixth longer with 8, but nearly twice as long with 4.
+// The blocks that begin a round with so much task time (ms, as the engine's recent
+// rounds took it a record). Waves share a CU's issue slots and L1: at 12 a CU they take
+// twice as long for a task as at 4, and a round that ends with a few long tasks ends
+// sooner with 4. Measured at 4, 8 and 12 waves a CU: 20 ms of tasks (22 seeds, 100,000
+// vertices) 87, 100 and 106 us; 170 ms 186, 185 and 205; 270 ms 223, 221 and 220;
+// 880 ms (1,000,000 vertices) 541, 499 and 513; 2,600 ms 1,320, 932 and 948; 9,900 ms
+// 6.8, 4.3 and 3.7 ms.
+//
+// As many more as give every CU four waves are a reserve that joins the round when it has
+// lasted kJoinUs, so that heavy records after light ones do not stay with the few waves
+// that those need: 400 records of squares over lists of 1,000 entries after 300 rounds of
+// lists of two take 17.7 ms, without the reserve 32.1, and 9.9 with all blocks from the
+// start. (All other blocks as a reserve: 12.8 ms, but the light rounds take 91 us, not 87
+// or, without a reserve, 83. Joining after 100 or 400 us makes no difference.)
+constexpr uint32_t kJoinUs = 200;
+uint32_t dfs_layer(const dsm_engine *e) { return std::max(1u, 4 / e->dfs_wpb) * (uint32_t)e->num_cu; }
 uint32_t blocks_for_work(const dsm_engine *e, double ms) {
-  const uint32_t waves_per_cu = ms <= 2500 ? 8 : 0xFFFF;
-  return std::max(1u, waves_per_cu / e->dfs_wpb) * (uint32_t)e->num_cu;
+  return ms <= 250 ? dfs_layer(e) : ms <= 2500 ? 2 * dfs_layer(e) : 0xFFFF0000u;
 }
 
 // The grid: a round over a handful of records gets one block per CU, so that few
@@ -900,12 +908,14 @@ uint32_t dfs_grid(dsm_engine *e, uint32_t nrec) {
   const uint64_t least = share >= (uint64_t)e->num_cu ? (uint64_t)e->num_cu
                                                       : std::min<uint64_t>((uint64_t)e->num_cu, want * share);
   uint32_t b = (uint32_t)std::min<uint64_t>(e->dfs_blocks, std::max<uint64_t>(want, least));
-  if (!e->grid_given && e->busy_per_record >= 0) b = std::min(b, blocks_for_work(e, e->busy_per_record * nrec));
   e->last_nrec = nrec;
   e->last_wpb = e->tuples ? 4u : e->dfs_wpb;
   b = std::min(b, e->wave_slots / e->last_wpb);  // a mailbox for every wave
-  e->last_blocks = b;
-  return b;
+  uint32_t crew = b;
+  if (!e->grid_given && e->busy_per_record >= 0) crew = std::min(b, blocks_for_work(e, e->busy_per_record * nrec));
+  e->last_crew = crew;
+  e->last_blocks = std::min(b, crew + dfs_layer(e));
+  return e->last_blocks;
 }
 
 // The waiting words of a grid.
@@ -929,8 +939,12 @@ int dfs_round(dsm_engine *e, const RoundPart *parts, int nparts, hipEvent_t ev0,
   if (ev1 && !e->seeding_timed) HIPCHK(hipEventRecord(ev1, e->stream));
   DfsArgs da = dfs_args(e);
   const uint32_t blocks = dfs_grid(e, nrec);
+  da.crew = e->last_crew * e->last_wpb;
+  da.cgroups = idle_words(da.crew);
+  da.ngroups = da.cgroups + idle_words((blocks - e->last_crew) * e->last_wpb);
+  da.join_after = (unsigned long long)e->wall_khz * kJoinUs / 1000;
   HIPCHK(launch_ctl_reset(e->ctl.p, clear.tuple_count, clear.counts, clear.ncounts, e->idle.p,
-                          idle_words(e->last_blocks * e->last_wpb), up, e->stream));
+                          da.ngroups, up, e->stream));
   HIPCHK(launch_seed(seed_args(e, parts, nparts), e->stream));
   if (ev1 && e->seeding_timed) HIPCHK(hipEventRecord(ev1, e->stream));
   HIPCHK(launch_dfs(da, blocks, e->dfs_wpb, e->max_qn, e->stream));
@@ -972,7 +986,10 @@ int round_error(dsm_engine *e) {
   unsigned long long busy = 0;
   for (uint32_t b = 0; b < e->last_blocks; b++) {
     const BlockRec &r = e->h_rec.p[b];
-    if (r.epoch != e->epoch) return e->fail_msg(DSM_EDEVICE, "DFS: block %u of %u left no record", b, e->last_blocks);
+    if (r.epoch != e->epoch) {
+      if (b >= e->last_crew) continue;  // the round did without it
+      return e->fail_msg(DSM_EDEVICE, "DFS: block %u of %u left no record", b, e->last_blocks);
+    }
     if (r.seed_overflow)
       return e->fail_msg(DSM_ELIMIT, "seed table overflow (%llu seeds dropped)", r.seed_overflow);
     if (r.abort) return e->fail_msg(DSM_EDEVICE, "DFS watchdog: a wave waited more than %u ms for work", e->watchdog_ms);
@@ -989,12 +1006,14 @@ int round_error(dsm_engine *e) {
 // The last round's errors, and its work and balance into the statistics.
 int check_round(dsm_engine *e, uint64_t *seeds) {
   if (int rc = round_error(e)) return rc;
-  const uint32_t nb = e->last_blocks, nw = nb * e->last_wpb;
-  *seeds = nb ? e->h_rec.p[0].nseeds : 0;
+  uint32_t nb = 0;  // blocks that took part
+  *seeds = e->last_blocks ? e->h_rec.p[0].nseeds : 0;
   unsigned long long busy = 0, busiest = 0, active = 0, t0 = ~0ull, t1 = 0;
   double first = 0, last = 0;  // summed over the active waves
-  for (uint32_t b = 0; b < nb; b++) {
+  for (uint32_t b = 0; b < e->last_blocks; b++) {
     const BlockRec &r = e->h_rec.p[b];
+    if (r.epoch != e->epoch) continue;
+    nb++;
     e->stats.tasks_donated += r.donated;
     e->stats.dfs_entries += r.scanned;
     e->stats.dfs_search_loads += r.loads;
@@ -1008,6 +1027,7 @@ int check_round(dsm_engine *e, uint64_t *seeds) {
     first += (double)r.first_sum;
     last += (double)r.last_sum;
   }
+  const uint32_t nw = nb * e->last_wpb;
   e->stats.dfs_busy_ms += (double)busy / (double)e->wall_khz;
   e->stats.dfs_waves += nw;
   if (busy) e->stats.dfs_block_imbalance += (double)busiest / ((double)busy / nb);
@@ -1579,7 +1599,7 @@ int create_impl(dsm_engine *e, const dsm_graph_desc *graph, const dsm_query_desc
     e->wave_slots = most * (uint32_t)e->num_cu;
     HIPCHK(e->mail.alloc(e->wave_slots));
     HIPCHK(hipMemset(e->mail.p, 0, (size_t)e->wave_slots * sizeof(Mailbox)));  // stop = 0: no epoch
-    HIPCHK(e->idle.alloc(idle_words(e->wave_slots)));
+    HIPCHK(e->idle.alloc(idle_words(e->wave_slots) + 1));  // the reserve's begin with a word of their own
     HIPCHK(e->h_rec.ensure(e->wave_slots));
   }
   e->donate_min = e->opt.donate_min ? e->opt.donate_min : 256;

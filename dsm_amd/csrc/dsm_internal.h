@@ -82,7 +82,8 @@ struct DfsCtl {
   CtlLine<uint32_t> donated;       // tasks handed to waiting waves, counted where they have a limit
   CtlLine<uint32_t> abort;         // set when an idle wave outlived the watchdog
 };
-// The waiting state of 16 waves of the grid (wave w is in word w mod ngroups),
+// The waiting state of 16 waves of the grid (wave w of those that begin at once, or of the
+// reserve, is in word w mod the words of its kind),
 // a line each: bits 0..15 waiting for work, bits 16..31 started, bits 32..63 the
 // number of claims so far. Busy waves look at one word after another for a
 // waiting wave, so that no line is polled by the whole grid.
@@ -90,7 +91,8 @@ using IdleWord = CtlLine<unsigned long long>;
 constexpr uint32_t kIdleGroup = 16;
 
 // What a block of a DFS launch did, written to pinned host memory by the block
-// when it ends; valid when epoch is the launch's. Times are wall-clock ticks.
+// when it ends; valid when epoch is the launch's (a block of the reserve that the round
+// did without leaves it as it was). Times are wall-clock ticks.
 struct alignas(128) BlockRec {
   unsigned long long epoch;
   unsigned long long active;       // waves that had a task
@@ -184,8 +186,11 @@ struct DfsArgs {
   const uint32_t *seed_s;
   const uint32_t *seed_d;
   Mailbox *mail;                 // [waves of the grid]
-  IdleWord *idle;                // [ceil(waves / kIdleGroup)]
+  IdleWord *idle;                // [ceil(waves / kIdleGroup)] of those that begin at once, then of the reserve
   uint32_t donate_cap;           // most tasks the round may hand to waiting waves
+  uint32_t crew;                 // waves of the blocks that begin at once; the others are a reserve
+  uint32_t cgroups, ngroups;     // their waiting words, and all
+  unsigned long long join_after; // wall-clock ticks after which the reserve joins
   uint32_t epoch;
   uint32_t donate_min;
   uint32_t lane_work;            // longest leaf list one lane scans alone

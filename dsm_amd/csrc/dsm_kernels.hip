@@ -1275,6 +1275,7 @@ struct WaveHdr {
   uint8_t lix[kMaxQ];
   uint32_t n, query, plan, tag;
   uint32_t donated;          // tasks the wave has handed out
+  uint64_t since;            // when it began
   uint32_t fstate, fn;       // leaf set F of the current positions 0..n-3 (see leaf_count)
 };
 constexpr uint32_t kFCap = 1024;   // largest leaf set F kept in LDS as whole ids
@@ -1847,9 +1848,10 @@ constexpr uint32_t kDonateBurst = DSM_DONATE_BURST;
 constexpr uint32_t kMaxParts = 64;  // shares a seed is cut into at most
 constexpr unsigned long long kIdleBits = (1ull << kIdleGroup) - 1;
 
-// The waves of the grid as try_donate and the waiting waves see them.
+// A wave among the grid's. Those of the blocks that begin at once (a.crew waves) have the
+// first a.cgroups waiting words, the reserve's the rest.
 struct Crew {
-  uint32_t nwaves, ngroups;
+  uint32_t nwaves;
   uint32_t me;       // this wave
   uint32_t look;     // the waiting word it looks at next
 };
@@ -1919,7 +1921,7 @@ __device__ __forceinline__ bool donate_one(WaveHdr &S, const DfsArgs &a, uint32_
       const unsigned long long next = (word & ~(1ull << b)) + (1ull << 32);
       const unsigned long long was = atomicCAS(&a.idle[g].v, word, next);
       if (was == word) {
-        who = b * cr.ngroups + g;
+        who = g < a.cgroups ? b * a.cgroups + g : a.crew + b * (a.ngroups - a.cgroups) + g - a.cgroups;
         word = next;
         break;
       }
@@ -1957,7 +1959,10 @@ __device__ __forceinline__ bool donate_one(WaveHdr &S, const DfsArgs &a, uint32_
 template <bool CAP>
 __device__ __forceinline__ void try_donate(WaveHdr &S, const DfsArgs &a, uint32_t L0, uint32_t l, uint32_t n, Crew &cr) {
   const uint32_t g = cr.look;
-  cr.look = g + 1 < cr.ngroups ? g + 1 : 0u;
+  // the reserve's words too once it has joined
+  const bool last = g + 1 == a.cgroups ? a.cgroups == a.ngroups || wall_clock64() - bcast64(S.since) < a.join_after
+                                       : g + 1 == a.ngroups;
+  cr.look = last ? 0u : g + 1;
   unsigned long long word = 0;
   if (lane_id() == 0) word = ld_relaxed(&a.idle[g].v);
   const uint32_t waiting = bcast((uint32_t)__popcll(word & kIdleBits));
@@ -1965,17 +1970,27 @@ __device__ __forceinline__ void try_donate(WaveHdr &S, const DfsArgs &a, uint32_
     if (!donate_one<CAP>(S, a, L0, l, n, cr, g, word)) break;
 }
 
+// Where wave `me` marks that it has started and that it waits.
+struct IdlePlace {
+  uint32_t word, bit;
+};
+__device__ __forceinline__ IdlePlace idle_place(const DfsArgs &a, uint32_t me) {
+  const bool crew = me < a.crew;
+  const uint32_t w = crew ? me : me - a.crew, words = crew ? a.cgroups : a.ngroups - a.cgroups;
+  return IdlePlace{(crew ? 0u : a.cgroups) + w % words, w / words};
+}
+
 // No started wave has work: every waiting word has all its started waves
 // waiting, twice in a row with no claim between. Work can only come from a
 // busy wave, so nothing is left then, apart from waves that start later, which
 // bring a seed of their own and finish it alone.
-__device__ __forceinline__ bool all_waiting(const DfsArgs &a, const Crew &cr) {
+__device__ __forceinline__ bool all_waiting(const DfsArgs &a) {
   uint32_t claims = 0;
   for (int pass = 0; pass < 2; pass++) {
     wave_sync();  // keeps the passes apart; the words are read past the caches
     uint32_t c = 0;
     bool all = true;
-    for (uint32_t g = lane_id(); g < cr.ngroups; g += 64) {
+    for (uint32_t g = lane_id(); g < a.ngroups; g += 64) {
       const unsigned long long v = ld_relaxed(&a.idle[g].v);
       all = all && (v & kIdleBits) == (v >> kIdleGroup & kIdleBits);
       c += (uint32_t)(v >> 32);
@@ -1995,8 +2010,9 @@ __device__ __forceinline__ bool all_waiting(const DfsArgs &a, const Crew &cr) {
 // after the others had been told to stop), it takes that task instead.
 __device__ __forceinline__ bool wait_for_task(const DfsArgs &a, const Crew &cr, uint32_t &seen) {
   const uint32_t lane = lane_id();
-  unsigned long long *word = &a.idle[cr.me % cr.ngroups].v;
-  const uint32_t b = cr.me / cr.ngroups;
+  const IdlePlace at = idle_place(a, cr.me);
+  unsigned long long *word = &a.idle[at.word].v;
+  const uint32_t b = at.bit;
   const unsigned long long bits = 1ull << b | 1ull << (b + kIdleGroup);
   uint32_t full = 0;
   if (lane == 0) {
@@ -2007,7 +2023,7 @@ __device__ __forceinline__ bool wait_for_task(const DfsArgs &a, const Crew &cr, 
   Mailbox *mb = &a.mail[cr.me];
   const uint64_t since = wall_clock64();
   for (uint32_t naps = 0;; naps++) {
-    if (look && all_waiting(a, cr))
+    if (look && all_waiting(a))
       for (uint32_t w = lane; w < cr.nwaves; w += 64)
         __hip_atomic_store(&a.mail[w].stop, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     look = false;
@@ -2044,6 +2060,30 @@ __device__ __forceinline__ bool wait_for_task(const DfsArgs &a, const Crew &cr, 
   }
 }
 
+// A block of the reserve (whose waves come after the first a.crew): waits until the round is over
+// (false) or has lasted long enough to be worth its waves (true). It joins as a block does
+// that starts late, which the words above allow for: it takes what seeds are left and then
+// waits for tasks. Its first wave watches its mailbox for the round's end, the others wait
+// at the barrier.
+__device__ __forceinline__ bool reserve_joins(const DfsArgs &a, uint32_t total, uint32_t me, uint64_t since) {
+  __shared__ uint32_t s_joins;
+  if (total == 0) return false;  // nobody will say that the round is over
+  if (threadIdx.x < 64) {
+    uint32_t joins = 0;
+    for (;;) {
+      uint32_t stop = 0;
+      if (lane_id() == 0) stop = ld_relaxed(&a.mail[me].stop);
+      if (bcast(stop) == a.epoch) break;
+      joins = wall_clock64() - since >= a.join_after;
+      if (joins) break;
+      for (uint32_t r = 0; r < 4; r++) __builtin_amdgcn_s_sleep(8);
+    }
+    if (lane_id() == 0) s_joins = joins;
+  }
+  __syncthreads();
+  return s_joins != 0;
+}
+
 // Bound by latency: dependent scattered reads and LDS steps, on few waves. What
 // counts is how many waves fit. Registers: the wave's index is made uniform, so
 // that its LDS addresses live in scalar registers (135 -> 96 vector registers; at
@@ -2074,15 +2114,15 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
   if (lane == 0) {
     S.plan = 0xFFFFFFFFu;
     S.donated = 0;
+    S.since = wall_clock64();
   }
   wave_sync();
   // what the block's waves did, for its record
   __shared__ unsigned long long s_rec[WPB][7];
   Crew cr;
   cr.nwaves = gridDim.x * WPB;
-  cr.ngroups = (cr.nwaves + kIdleGroup - 1) / kIdleGroup;
   cr.me = blockIdx.x * WPB + wv;
-  cr.look = (cr.me + 1) % cr.ngroups;
+  cr.look = (cr.me + 1) % a.cgroups;
   // a seed table overflow leaves unwritten slots: match nothing, the host
   // reports the error (the table is sized so that it cannot happen)
   const uint32_t nseeds = a.ctl->seed_overflow.v ? 0u : a.ctl->nseeds.v;
@@ -2096,14 +2136,18 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
   // kSeedHeads counters, a wave starting at one of its own, so that the grid's
   // first claims do not queue up on one line. With more shares than waves a wave
   // whose counter has run out moves on to one that has not.
-  const uint32_t parts = nseeds && nseeds < cr.nwaves ? min(cr.nwaves / nseeds, kMaxParts) : 1u;
+  const uint32_t parts = nseeds && nseeds < a.crew ? min(a.crew / nseeds, kMaxParts) : 1u;
   const uint32_t total = nseeds * parts;
+  if (cr.me >= a.crew && !reserve_joins(a, total, cr.me, bcast64(S.since))) return;
   uint32_t head = cr.me % kSeedHeads;
   bool seeds_left = total > 0;
   uint32_t seen = 0;  // mail taken so far
   if (lane == 0) {
     seen = ld_relaxed(&a.mail[cr.me].mail);
-    if (seeds_left) atomicOr(&a.idle[cr.me % cr.ngroups].v, 1ull << (cr.me / cr.ngroups + kIdleGroup));
+    if (seeds_left) {
+      const IdlePlace at = idle_place(a, cr.me);
+      atomicOr(&a.idle[at.word].v, 1ull << (at.bit + kIdleGroup));
+    }
   }
   seen = bcast(seen);
   uint64_t busy = 0;            // wall-clock ticks spent on tasks
@@ -2120,7 +2164,7 @@ __global__ __launch_bounds__(WPB * 64, 4) void k_dfs(DfsArgs a, uint32_t chunk_l
         break;
       }
       uint64_t open = 0;
-      if (total > cr.nwaves) {
+      if (total > a.crew) {
         const uint32_t h = lane % kSeedHeads;
         open = ballot(lane < kSeedHeads && h + kSeedHeads * ld_relaxed(&a.ctl->seed_head[h].v) < total);
       }

@@ -64,6 +64,25 @@ def test_light_rounds_leave_heavy_ones_their_grid():
         eng.close()
 
 
+def test_a_heavy_round_after_many_light_ones_is_joined_by_the_reserve():
+    """Once light rounds have settled on few blocks, a heavy one gets as many again while it
+    runs, and counts what it did; the light ones do without them."""
+    graph, queries, heavy, light = _mixed_graph()
+    eng = E.Engine(graph, queries, relabel=False)
+    try:
+        want = eng.process_batch(*heavy)[0].tolist()
+        most = _waves(eng, heavy)
+        for _ in range(400):
+            eng.process_batch(*light)
+        few = _waves(eng, light)
+        assert 2 * few <= most
+        assert eng.process_batch(*heavy)[0].tolist() == want and want[0] > 0
+        s = eng.stats()
+        assert s["dfs_waves"] // s["dfs_launches"] == 2 * few
+    finally:
+        eng.close()
+
+
 @pytest.mark.parametrize("queue_capacity", [0, 1, 2, 50, 100000])
 def test_few_hand_offs_are_allowed(queue_capacity):
     """A limit on a round's hand-offs below the number of its waves allows some: 400
