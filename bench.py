@@ -22,8 +22,10 @@ Legs (one JSON line on stdout, details on stderr):
   cpu      the CPU oracle (single core) on one batch of the same stream
 """
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -41,6 +43,15 @@ def log(*a):
 
 def pct(xs, p):
     return float(np.percentile(np.asarray(xs, dtype=np.float64), p)) if len(xs) else None
+
+
+def kernel_code():
+    """SHA-256 of the sources of k_dfs without comments and white space."""
+    h = hashlib.sha256()
+    for f in ("dsm_kernels.hip", "dsm_device.h", "dsm_internal.h"):
+        with open(os.path.join(ROOT, "dsm_amd", "csrc", f)) as src:
+            h.update(re.sub(r"//[^\n]*|\s+", "", src.read()).encode())
+    return h.hexdigest()
 
 
 def make_workload(name):
@@ -440,7 +451,7 @@ def main():
     ap.add_argument("--donate-min-n2", type=int, default=0)
     ap.add_argument("--leaf-segments", type=int, default=1)
     ap.add_argument("--poll-max", type=int, default=0)
-    ap.add_argument("--leaf-budget", type=int, default=0, help="0: the engine's default (2048)")
+    ap.add_argument("--leaf-budget", type=int, default=0, help="0: the engine's default (8192)")
     ap.add_argument("--overlap-apply", type=int, default=1,
                     help="1: pipelined batches update a second copy of the graph during the round")
     ap.add_argument("--cluster-filter", type=int, default=0,
@@ -503,16 +514,18 @@ def main():
     merge_rate = merge_per_launch / (dfs_ms_avg * 1e-3) / 1e9 if dfs_ms_avg > 0 else 0.0
     # HBM bytes per launch measured by rocprofv3 (FETCH_SIZE / WRITE_SIZE runs
     # scaled by a copy of known size), kept in profiles/
-    # The profile was taken on this workload's default run (the same command
-    # under rocprofv3, tuned shape passed explicitly); it carries the
-    # algorithmic bytes of its own launches, so traffic / algorithmic bytes is
-    # a ratio of one run, not of two.
+    # A profile was taken with the command it names, under rocprofv3; it carries the
+    # algorithmic bytes of its own launches, so traffic / algorithmic bytes is a ratio
+    # of one run, not of two. The traffic is given as this kernel's only if the profile
+    # is of these sources.
     traffic = prof = None
+    prof_is_ours = False
     tpath = os.path.join(ROOT, "profiles", "k_dfs_%s_traffic.json" % w.name)
     if os.path.exists(tpath):
         with open(tpath) as f:
             prof = json.load(f)
-        traffic = prof.get("traffic_bytes_per_launch")
+        prof_is_ours = prof.get("kernel_code") == kernel_code()
+        traffic = prof["traffic_bytes_per_launch"] if prof_is_ours else None
     roofline = {"bound": "hbm", "kernel": "k_dfs", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
                 "bytes_per_launch": int(bytes_per_launch), "avg_launch_ms": round(dfs_ms_avg, 4),
@@ -541,8 +554,8 @@ def main():
     if prof and prof.get("algorithmic_bytes_per_launch"):
         roofline["traffic_run"] = {"algorithmic_bytes_per_launch": prof["algorithmic_bytes_per_launch"],
                                    "avg_launch_ms": prof.get("avg_launch_ms"),
-                                   "traffic_over_algorithmic": round(traffic / prof["algorithmic_bytes_per_launch"],
-                                                                     3),
+                                   "same_kernel": prof_is_ours,
+                                   "traffic_over_algorithmic": prof.get("traffic_over_algorithmic"),
                                    "dram_GB_per_s": prof.get("dram_GB_per_s"),
                                    "profile": os.path.relpath(tpath, ROOT)}
 
