@@ -2,7 +2,7 @@
 // two 64-bit keys (source, target), a radix sort puts them in order, equal
 // neighbours are dropped, and the lists go to their slots in the pool. With the
 // lists counted, scattered and sorted by one host core, an engine for 2,000,003
-// edges on 200,003 vertices took 82.8 ms to make; it takes 4.2 ms this way, most
+// edges on 200,003 vertices took 82.8 ms to make; it takes 4.4 ms this way, most
 // of it allocations and the upload of the edges.
 //
 //   k_csr_keys                          the keys; the first edge out of range

@@ -1399,9 +1399,9 @@ DevGraph graph_of(const dsm_engine *e, const dsm_engine::GraphCopy &c) {
 // An update that one block does in less time than the launches of many take
 // (k_update_small): few lists, none with pieces, and few vertices that can become dirty
 // (the relabelled ones' neighbours), in a graph whose marks one block looks through
-// in a few steps. One record on lists of 30: 25 to 28 us instead of 37. With 560
-// vertices that may be dirty it takes 38 instead of 49, but behind the negatives'
-// round instead of beside it: 880 us for four such calls instead of 830.
+// in a few steps. One record on lists of 30: 81 us a call instead of 105. With 500
+// vertices that may be dirty (8 records, 400 vertices) it takes 30 us, but behind the
+// negatives' round instead of beside it: 1,180 us for four such calls instead of 1,120.
 bool small_update(const dsm_engine *e, const HostDelta &d) {
   const size_t T = d.tv.size(), R = d.rl_v.size(), changes = d.ins.size() + d.del.size();
   const size_t longest = (size_t)e->h_actl.p->max_deg + d.ins.size();

@@ -1046,10 +1046,11 @@ __global__ __launch_bounds__(256) void k_lbuild_place(DevGraph g, const uint8_t 
   }
 }
 
-// A whole update by one block, its phases a block barrier apart instead of a launch:
-// for one record on lists of 30 entries the ten kernels took 37 us, most of it between
-// them, and this takes 25 to 28 in one launch. Lists of at most kBuildSeg entries (no pieces), at most kSmallChanges changes.
-// It ends with the update's status in pinned host memory.
+// A whole update by one block, its phases a block barrier apart instead of a launch: one
+// record on lists of 30 entries takes it 18.5 us, and the call 81 where the ten kernels,
+// most of whose time lies between them, made it 105. Lists of at most kBuildSeg entries
+// (no pieces), at most kSmallChanges changes. It ends with the update's status in pinned
+// host memory.
 constexpr uint32_t kOneWaves = 8;
 static_assert(kOneWaves * 64 == kPlanBlock && kOneWaves * 64 == kCompactBlock, "the phases' strides");
 __global__ __launch_bounds__(kOneWaves * 64) void k_update_small(DevGraph g, BatchDev b, FilterTables ft, DirtyArgs d,
