@@ -74,7 +74,8 @@ typedef struct {
   uint64_t tuple_capacity; /* tuples kept per batch (0: counts only) */
   int tuples_in_host_memory; /* 1: tuple buffer in pinned host memory (spill) */
   uint32_t waves_per_block;  /* DFS launch shape; 0 = default */
-  uint32_t blocks_per_cu;    /* 0 = as many as occupancy allows */
+  uint32_t blocks_per_cu;    /* 0 = as many as occupancy allows, fewer where the recent
+                                rounds had little work; else so many in every round */
   uint32_t donate_min;       /* smallest source range split off to an idle wave (0 = default) */
   uint32_t queue_capacity;   /* a round hands fewer tasks than this to idle waves (0 = no
                                 limit, 1 = none) */
@@ -138,7 +139,7 @@ typedef struct {
    * expanded: the bytes merge intersections over whole lists would read */
   uint64_t dfs_merge_bytes;
   /* balance of the persistent DFS grid, summed over the launches: time the
-   * waves spent on tasks (ms, all waves), waves launched, and per launch the
+   * waves spent on tasks (ms, all waves), waves that took part, and per launch the
    * busiest block's task time over the mean block's */
   double dfs_busy_ms;
   uint64_t dfs_waves;
